@@ -49,7 +49,7 @@ struct DevBuf
 // Every device buffer a context keeps between calls.
 struct Buffers
 {
-    DevBuf hRes, vRes, hOff, vOff, order, items, queue, rowbuf, scores, tTable, dnaProf, ids32, scratchOff32,
+    DevBuf hRes, vRes, hOff, vOff, order, items, queue, rowbuf, strips, scores, tTable, dnaProf, ids32, scratchOff32,
         scratch32, table32, emptyIds;
     // Traceback (sqmi_align_counts).
     DevBuf trace, traceOff, locs, endEF, endIJ, counts;
@@ -63,7 +63,7 @@ struct Buffers
     template <class F>
     void forEach(F f)
     {
-        for (DevBuf *b : {&hRes, &vRes, &hOff, &vOff, &order, &items, &queue, &rowbuf, &scores, &tTable, &dnaProf,
+        for (DevBuf *b : {&hRes, &vRes, &hOff, &vOff, &order, &items, &queue, &rowbuf, &strips, &scores, &tTable, &dnaProf,
                           &ids32, &scratchOff32, &scratch32, &table32, &emptyIds, &trace, &traceOff, &locs, &endEF,
                           &endIJ, &counts, &longCk, &longPairs, &longWalk, &longTrace, &longBest, &longSched, &ops, &opOff, &opLen,
                           &begins, &opsPacked, &opStart, &bandIds, &bandScratch})
@@ -72,6 +72,10 @@ struct Buffers
 };
 
 }  // namespace
+
+namespace {
+struct Planned;
+}
 
 struct sqmi_context
 {
@@ -95,10 +99,14 @@ struct sqmi_context
     std::vector<int4> longRanges;
     bool longStreamed = false;
     Buffers b;
+    Planned *planned = nullptr;   // the calls' plans, one after the other (owned)
     // The no-allocation entry point: this device's scratch array (its device
     // address, from hipGetSymbolAddress at creation) and, during such a
     // call, the arena carved from it.
     void *scratchPtr = nullptr;
+    // Host memory the packed score kernel raises when a strip's wait runs
+    // past its bound (never expected).
+    uint32_t *waitFlag = nullptr;
     Arena arena;
     bool noAlloc = false;   // inside sqmi_align_score_noalloc
     // The last sqmi_align_score call, kept for an identical next call: the
@@ -211,13 +219,39 @@ struct ScoringInfo
     int o = 0, e = 0;
     int sMax = 0, sMin = 0;
     bool dna = false;   // v_perm profile path possible
+    bool dnaDrift = false;   // and for the drifted scores t + drift (global score kernels)
 };
 
-// Local table kernels fuse the two lookups and the diagonal add into one
-// 32-bit add when every table value s - gapOpen is >= 0.
-int32_t tNonNeg(const ScoringInfo &si, uint32_t mode)
+// The score kernels' drifted representation (kernels.hpp, Drift; local:
+// score16.hpp).  Scores t below 0 raise the bias, so that a diagonal step
+// never leaves the value range.
+Drift driftOf(const ScoringInfo &si, bool local)
 {
-    return (mode & SQMI_LOCAL) != 0 && !si.dna && si.sMin >= si.o ? 1 : 0;
+    Drift r;
+    const int ext = std::max(si.o, si.e);
+    r.d = -ext;
+    r.cost = ext - si.o;
+    const int tMin = std::min(0, si.sMin - si.o - (local ? 0 : ext));
+    if (local) {
+        r.bias = r.cost + 2 * r.d + 2 - tMin;
+        r.neg = r.bias - r.cost;
+    } else {
+        r.neg = r.cost - tMin + 1;
+        r.bias = r.neg + 3 * r.cost + 1;
+    }
+    return r;
+}
+
+// Whether a pair's stored values stay within kDriftNarrowMax (and no t is
+// below 0): at most bias + sMax * min(n, m) + drift * (n + m), local + drift
+// * 17 instead.  Pairs inside the int16 window (fitsInt16) always stay within
+// 65535: there sMax * min(n, m) is at most 30719 and drift * (n + m) at most
+// 26624, the bias of costs up to 1024 at most 6146 (local: 17 * 1024 and 4098).
+bool driftNarrow(const ScoringInfo &si, const Drift &dr, bool local, int64_t n, int64_t m)
+{
+    const int64_t span = local ? 17 : n + m + 2 * kDriftSlack;
+    return dr.neg == (local ? 2 * dr.d + 2 : dr.cost + 1) &&
+           dr.bias + (int64_t)std::max(0, si.sMax) * (std::min(n, m) + kDriftSlack) + dr.d * span <= kDriftNarrowMax;
 }
 
 // Conservative range of every value a pair can produce inside the DP (H, E, F
@@ -244,6 +278,9 @@ bool fitsLong32(const ScoringInfo &si, int64_t n, int64_t m)
     return up < (1LL << 28) && low > -(1LL << 28) && n < (1LL << 30) && m < (1LL << 30);
 }
 
+// The pairs of one shape: for groups of 16 or 64 lanes the items become units
+// of the packed score kernel (Planned::units), for the one-pair-per-lane and
+// trace kernels they are launched as they are.
 struct Plan16
 {
     Variant16 var;
@@ -254,9 +291,14 @@ struct Plan16
 
 int pairsPerWave(const Variant16 &v) { return 2 * (64 / v.G); }
 
-// Shapes compiled for the packed forward: groups of 16 lanes (kFwd16) or one
-// pair couple per lane (kLane16).
-bool shapeSupported(const Variant16 &v) { return v.G == 1 ? laneSupported(v) : variantSupported(v); }
+// Shapes of the score calls: a pair couple per 16 or 64 lanes (kScore16) or
+// per lane (kLane16).
+bool shapeSupported(const Variant16 &v)
+{
+    if (v.G == 1)
+        return laneSupported(v);
+    return (v.G == 16 && (v.R == 8 || v.R == 16)) || (v.G == 64 && (v.R == 4 || v.R == 8 || v.R == 16));
+}
 
 // The planner's shape table (seqan_amd/tuning/shapes.json, turned into C++
 // by the build): per category (DNA byte profile or substitution table,
@@ -276,27 +318,44 @@ int lengthBin(int64_t m)
 
 int shapeCategory(bool dna, bool local) { return (dna ? 0 : 2) + (local ? 1 : 0); }
 
-// SQMI_SHAPE_RULE=fixed: the rule the table replaced (G = 16; R = 8 when
-// |V| + 1 <= 128, else 16), for comparing tuned and untuned plans.
+// SQMI_SHAPE_RULE=fixed: groups of 16 lanes and whole items for every pair,
+// for comparing the shape rules with one shape.
 bool fixedShapeRule()
 {
     const char *env = std::getenv("SQMI_SHAPE_RULE");
     return env && std::strcmp(env, "fixed") == 0;
 }
 
-// The shape of length bin `bin` for a call holding pairs16 pairs on the
-// packed route (all bins: the shapes' launches run side by side, so the
-// whole call is what fills the GPU).
-Variant16 tableShape(int category, int bin, int64_t pairs16, bool dna, uint32_t track)
+// Whether the shape table gives length bin `bin` the one-pair-per-lane
+// kernel, for a call holding pairs16 pairs on the packed route (all bins: the
+// launches run side by side, so the whole call is what fills the GPU), and
+// its rows per lane.
+int laneRows(int category, int bin, int64_t pairs16)
 {
-    if (fixedShapeRule())
-        return Variant16{16, bin <= 7 ? 8 : 16, dna, track};
     int cls = 0;
     while (cls + 1 < kTabNClasses && pairs16 >= kTabCountClasses[cls + 1])
         ++cls;
     const int idx = kTabChoice[category][bin][cls];
-    return Variant16{kTabShapes[idx][0], kTabShapes[idx][1], dna, track};
+    return kTabShapes[idx][0] == 1 ? kTabShapes[idx][1] : 0;
 }
+
+// Lanes per pair couple and whole items or strips, by the time a pair takes
+// against the whole call's.  A wave of 16-lane groups sweeps n x m cells (of
+// eight pairs at once) in about 5.7 n m cycles at three waves per SIMD, a wave
+// of one 64-lane group (one couple) in a quarter of that; the call's cells
+// take about 2.3e-4 cycles each on the whole chip.  An item may take a
+// quarter of the call's time: longer ones end after the others have left the
+// chip.  So couples go to 64 lanes from 1.0e-5 of the call's cells on, and
+// their row blocks to different waves (strips) from 4e-5 on.  Measured (MI355X):
+// 3,001 uneven pairs (100 bp - 10 kbp, semi-global) 14.2 -> 1.8 ms, where four
+// waves of one workgroup used to share an item's blocks; 1,048,576 of them
+// 99 -> 69 ms, of which the shorter recurrence gives most.
+constexpr double kCouple64Share = 1.0e-5, kStripShare = 4.0e-5;
+// Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
+constexpr int64_t kResidentWaves = 3072;
+// Rows per unit of the group shapes' row counts.
+constexpr int kUnitRows = 64;
+inline int64_t unitsOfRows(int64_t m) { return (m + kUnitRows) / kUnitRows; }   // m + 1 rows
 
 // Row blocks of a pair with m rows under shape v (at most 255 fit the keys).
 // Row blocks of G * R rows (a power of two for every compiled shape).
@@ -304,16 +363,6 @@ int64_t blocksFor(const Variant16 &v, int64_t m)
 {
     const int64_t br = (int64_t)v.G * v.R;
     return (br & (br - 1)) == 0 ? (m + br) >> __builtin_ctzll((unsigned long long)br) : (m + br) / br;
-}
-
-// One pair per launch: one wavefront, whose first 16-lane group sweeps the
-// pair (the other pair slots of the wavefront stay empty).
-Variant16 plainVariant(bool dna, uint32_t track, int64_t m)
-{
-    Variant16 v{16, 16, dna, track};
-    if (m + 1 <= 128)
-        v.R = 8;
-    return v;
 }
 
 sqmi_status checkSet(sqmi_context *ctx, const sqmi_sequences *s, const char *name)
@@ -343,11 +392,22 @@ struct Key
 {
     uint32_t key;
     int32_t id;
-    // Left uninitialised: the planner's key arrays (8 MB for a million
-    // pairs) are written in full, in parallel, right after allocation.
-    Key() {}
-    Key(uint32_t k, int32_t i) : key(k), id(i) {}
 };
+
+// A vector whose new elements are left uninitialised: the planner's large
+// arrays are written in full, in parallel, right after they are sized.
+template <class T>
+struct RawAlloc : std::allocator<T>
+{
+    template <class U>
+    struct rebind { using other = RawAlloc<U>; };
+    template <class U>
+    void construct(U *p) noexcept { ::new (static_cast<void *>(p)) U; }
+    template <class U, class... A>
+    void construct(U *p, A &&...a) { ::new (static_cast<void *>(p)) U(std::forward<A>(a)...); }
+};
+template <class T>
+using RawVec = std::vector<T, RawAlloc<T>>;
 
 struct Planned
 {
@@ -360,10 +420,31 @@ struct Planned
     std::vector<int32_t> idsLong;   // int32 pairs for the tiled long-pair kernels
     std::vector<int64_t> scratchOff32;
     int64_t scratch32 = 0;
-    std::vector<Key> keys16;        // int16 pairs, sorted by bucket key
+    RawVec<Key> keys16, keysTmp;    // int16 pairs, sorted by bucket key; the sort's other half
+    std::vector<uint32_t> sortHist;
     std::vector<Variant16> shapes;  // int16 shape slots (key classes 0..)
-    std::vector<Plan16> plans;      // one per kernel variant in use
+    std::vector<Plan16> plans;      // one per one-pair-per-lane or trace shape in use
+    // Packed score kernel: pair ids grouped by item, units, buffers.
+    RawVec<int32_t> order16;
+    RawVec<ScoreUnit> units;
+    int64_t slotWords = 0, stripWords = 0;
+    int64_t items16 = 0, padded16 = 0;
+    bool dna16 = false;             // profile path of the packed kernels
+    Drift drift{};
     int64_t cells = 0;
+
+    // Back to an empty plan that keeps its arrays (a context's calls share
+    // one, so that large calls don't fault their pages in every time).
+    void reset()
+    {
+        emptyIds.clear();
+        ids32.clear();
+        idsLong.clear();
+        scratchOff32.clear();
+        shapes.clear();
+        plans.clear();
+        scratch32 = slotWords = stripWords = items16 = padded16 = cells = 0;
+    }
 };
 
 // int32 pairs whose sides are both at least this long (and that are DNA,
@@ -427,6 +508,16 @@ sqmi_status longStreamCheck(sqmi_context *ctx)
     return SQMI_OK;
 }
 
+// After a call's final synchronisation: whether a strip's wait ran past its
+// bound (the flag is raised by the kernel, in host memory).
+sqmi_status stripCheck(sqmi_context *ctx)
+{
+    if (*static_cast<volatile uint32_t *>(ctx->waitFlag) == 0)
+        return SQMI_OK;
+    *ctx->waitFlag = 0;
+    return fail(ctx, SQMI_ERR_DEVICE, "a row block's wait for the one above it ran past its bound; results are not valid");
+}
+
 // Streams the long-pair forward spreads its pair couples over (1..4).  On
 // 64 pairs of 100 kbp with 128-column tiles: 1 stream 263 ms, 2 streams
 // 164 ms, 3 streams 157 ms (with 256-column tiles: 220, 170, 170 ms; 4
@@ -447,21 +538,20 @@ constexpr int64_t kParallelMin = 32768;
 // Stable LSD radix sort of 28-bit keys in two passes of 14 bits, each pass
 // split into contiguous per-thread ranges so that equal digits keep their
 // input order.
-void radixSort(std::vector<Key> &keys)
+void radixSort(RawVec<Key> &keys, RawVec<Key> &tmp, std::vector<uint32_t> &hist)
 {
     const size_t n = keys.size();
     if (n < 2)
         return;
-    std::vector<Key> tmp(n);
+    tmp.resize(n);
     int T = 1;
 #ifdef _OPENMP
     T = std::max(1, std::min(omp_get_max_threads(), (int)(n / 16384) + 1));
 #endif
     constexpr int B = 14, NB = 1 << B;
-    std::vector<uint32_t> hist((size_t)T * NB);
+    hist.resize((size_t)T * NB);
     for (int shift = 0; shift < 2 * B; shift += B) {
         const uint32_t mask = (uint32_t)NB - 1;
-        std::fill(hist.begin(), hist.end(), 0u);
 #pragma omp parallel num_threads(T)
         {
             int t = 0;
@@ -470,6 +560,7 @@ void radixSort(std::vector<Key> &keys)
 #endif
             const size_t lo = n * t / T, hi = n * (t + 1) / T;
             uint32_t *h = hist.data() + (size_t)t * NB;
+            std::fill(h, h + NB, 0u);
             for (size_t k = lo; k < hi; ++k)
                 ++h[(keys[k].key >> shift) & mask];
 #pragma omp barrier
@@ -491,27 +582,27 @@ void radixSort(std::vector<Key> &keys)
     }
 }
 
-// Bucket keys (28 bits): class (3 bits: 0..5 int16 shape slot, 6 int32,
-// 7 empty) | 1023 - row units (10 bits) | 32767 - |H| (15 bits).  Ascending
+// Bucket keys (28 bits): class (3 bits: 0..6 int16 shape slot, 7 int32 or
+// empty) | 1023 - row units (10 bits) | 32767 - |H| (15 bits).  Ascending
 // order puts int16 pairs first, grouped by shape and row units (most first),
-// widest first, then the int32 and the empty pairs in input order.  A row
-// unit is a quarter of a G*R-row block for the packed kernels with groups
-// of 16 or 64 lanes (their block 0 may be 1..4 quarters tall), a whole
-// block for the one-pair-per-lane kernel and the trace kernel.
+// widest first, then the int32 and empty pairs in input order.  A row
+// unit is 64 rows for the group shapes (their block 0 is as tall as the item
+// needs), a whole block for the one-pair-per-lane and the trace kernels.
 constexpr int kKeyNBits = 15, kKeyUnitBits = 10, kKeyClassShift = kKeyNBits + kKeyUnitBits;
-constexpr uint32_t kClassInt32 = 6, kClassEmpty = 7, kMaxShapeSlots = 6;
+constexpr uint32_t kClassRest = 7;
+// Shape slots of the score calls: group shapes (the longest pairs first; + 0
+// wide values, + 1 narrow), then lanes.
+constexpr uint32_t kSlot64 = 0, kSlot16 = 2, kSlotLane16 = 4, kSlotLane32 = 5, kSlotLaneWide = 6;
 constexpr int64_t kMaxBlocks16 = 255;   // row blocks per pair of a packed work item
 inline uint32_t bucketOf(uint32_t key) { return key >> kKeyNBits; }
 inline int32_t widthOf(uint32_t key) { return (int32_t)((1u << kKeyNBits) - 1 - (key & ((1u << kKeyNBits) - 1))); }
 inline int32_t unitsOf(uint32_t key) { return (int32_t)(1023u - ((key >> kKeyNBits) & 1023u)); }
-// Row units of a shape: quarter blocks where block 0 may be shortened.
-inline bool quarterUnits(const Variant16 &v, bool traceShape) { return v.G >= 16 && v.R % 4 == 0 && !traceShape; }
-// Quarter-block shapes: a pair takes just enough quarters (fine), or whole
-// blocks counted as 4 quarters each (coarse).  Fine units cut the rows of
-// block 0 but split the pairs of a length bin over 4 times as many buckets,
-// which widens the spread of |H| inside a work item when the bin holds few
-// pairs; so a bin takes fine units from kFineUnitPairs pairs on
-// (SQMI_ROW_UNITS=block / quarter: always coarse / fine).
+// Row units of the group shapes: 64 rows (fine), or 256 (coarse: units rounded
+// up to 4).  Fine units cut the rows of block 0 but split the pairs of a
+// length bin over 4 times as many buckets, which widens the spread of |H|
+// inside an item when the bin holds few pairs; so a bin takes fine units from
+// kFineUnitPairs pairs on (SQMI_ROW_UNITS=block / quarter: always coarse /
+// fine).
 constexpr int64_t kFineUnitPairs = 8192;
 int rowUnitsMode()   // 0 by bin size, 1 coarse, 2 fine
 {
@@ -522,20 +613,142 @@ int rowUnitsMode()   // 0 by bin size, 1 coarse, 2 fine
         return 2;
     return 0;
 }
-inline int64_t unitsFor(const Variant16 &v, int64_t m, bool quarter, bool fine)
+// Work items with at least this many row blocks become strips
+// (SQMI_COOP_MIN_BLOCKS; 0: none, unset: the rule of kStripShare).
+int stripMinBlocks()
 {
-    if (!quarter)
-        return blocksFor(v, m);
-    if (!fine)
-        return 4 * blocksFor(v, m);
-    const int64_t rows = (int64_t)v.G * v.R / 4;
-    return (rows & (rows - 1)) == 0 ? (m + rows) >> __builtin_ctzll((unsigned long long)rows) : (m + rows) / rows;
+    const char *env = std::getenv("SQMI_COOP_MIN_BLOCKS");
+    return env && *env ? std::max(0, std::atoi(env)) : -1;
+}
+
+// Units of the packed score kernel from the sorted keys of the group shapes,
+// which come first, in slot order (the longest items first).  starts /
+// itemOff: the buckets' first keys and items.
+void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &starts,
+               const std::vector<size_t> &itemOff, int R16, int R64, double cellsStrip, bool noStrips)
+{
+    const RawVec<Key> &keys = P.keys16;
+    const size_t nb = starts.size() - 1;
+    size_t bG = 0, b64 = 0;   // buckets of the group shapes, and of 64 lanes
+    while (bG < nb && (keys[starts[bG]].key >> kKeyClassShift) < kSlotLane16) {
+        if ((keys[starts[bG]].key >> kKeyClassShift) < kSlot16)
+            b64 = bG + 1;
+        ++bG;
+    }
+    const size_t nPairs = starts[bG], nItems = itemOff[bG], n64 = itemOff[b64];
+    const bool par = (int64_t)nPairs > kParallelMin;
+    P.order16.resize(nPairs);
+#pragma omp parallel for schedule(static) if (par)
+    for (int64_t k = 0; k < (int64_t)nPairs; ++k)
+        P.order16[k] = keys[k].id;
+    const int minBlocks = noStrips ? 0 : fixedShapeRule() && stripMinBlocks() < 0 ? 0 : stripMinBlocks();
+    // An item as one unit, with its row units in `pad`.  Few pairs: the
+    // units of its tallest pair (buckets may be coarse).
+    auto item = [&](size_t b, size_t k, size_t e) {
+        const uint32_t key = keys[starts[b]].key, slot = key >> kKeyClassShift;
+        int64_t units = unitsOf(key);
+        if (!par || slot < kSlot16) {
+            int64_t maxM = 0;
+            for (size_t x = k; x < e; ++x)
+                maxM = std::max(maxM, V.offsets[keys[x].id + 1] - V.offsets[keys[x].id]);
+            units = unitsOfRows(maxM);
+        }
+        return ScoreUnit{(int32_t)k, (int32_t)(e - k), widthOf(keys[k].key), 0, 0,
+                         (slot < kSlot16 ? kUnit64 : 0) | (slot % 2 == 0 ? kUnitWide : 0), -1, (int32_t)units, 0};
+    };
+    // Rows: blocks of R rows per lane, block 0 as tall as needed.
+    auto split = [](ScoreUnit &u, int R) {
+        const int G = (u.shape & kUnit64) ? 64 : 16, rowsPerUnit = kUnitRows / G, per = R / rowsPerUnit;
+        u.nblocks = (u.pad + per - 1) / per;
+        int RH = (u.pad - per * (u.nblocks - 1)) * rowsPerUnit;
+        if (G == 64 && RH > 4)   // compiled heights 1, 2, 3, 4, 6, 8, 12, 16
+            RH = RH <= 6 ? 6 : RH <= 8 ? 8 : RH <= 12 ? 12 : 16;
+        u.rows = R | std::min(RH, R) << 8;
+    };
+    auto padded = [](const ScoreUnit &u) -> int64_t {
+        return (int64_t)2 * 64 * u.maxN * ((u.rows >> 8) + (int64_t)(u.nblocks - 1) * (u.rows & 0xff));
+    };
+    auto words = [](const ScoreUnit &u) -> int64_t { return ((u.shape & kUnit64) ? 1 : 4) * (int64_t)(u.maxN + 1); };
+    auto strips = [&](const ScoreUnit &u) {
+        if (u.nblocks < 2 || minBlocks == 0)
+            return false;
+        return minBlocks > 0 ? u.nblocks >= minBlocks
+                             : (u.shape & kUnit64) && (double)u.maxN * u.pad * kUnitRows > cellsStrip;
+    };
+    auto addStrips = [&](ScoreUnit u) {
+        u.rowOff = P.stripWords;
+        P.stripWords += words(u) * u.nblocks;
+        for (int b = 0; b < u.nblocks; ++b) {
+            u.block = b;
+            P.units.push_back(u);
+        }
+    };
+    P.units.clear();
+    P.items16 = (int64_t)nItems;
+
+    // 64 lanes.  Strips of as few rows as give every resident wave about two.
+    int stripR = R64 ? R64 : 4;
+    if (!R64 && minBlocks < 0) {
+        int64_t strips4 = 0;
+        for (size_t b = 0; b < b64; ++b)
+            strips4 += (int64_t)((starts[b + 1] - starts[b] + 1) / 2) * ((unitsOf(keys[starts[b]].key) + 3) / 4);
+        while (stripR < 16 && strips4 * 4 / stripR > 2 * kResidentWaves)
+            stripR *= 2;
+    }
+    P.units.reserve(nItems);
+    for (size_t b = 0; b < b64; ++b)
+        for (size_t k = starts[b]; k < starts[b + 1]; k += 2) {
+            ScoreUnit u = item(b, k, std::min(starts[b + 1], k + 2));
+            split(u, R64 ? R64 : stripR);
+            const bool s = strips(u);
+            if (!s && !R64)
+                split(u, 16);
+            P.padded16 += padded(u);
+            if (s) {
+                addStrips(u);
+            } else {
+                P.slotWords = std::max(P.slotWords, words(u));
+                P.units.push_back(u);
+            }
+        }
+    // 16 lanes: whole items (strips on request only).
+    if (minBlocks > 0) {
+        for (size_t b = b64; b < bG; ++b)
+            for (size_t k = starts[b]; k < starts[b + 1]; k += 8) {
+                ScoreUnit u = item(b, k, std::min(starts[b + 1], k + 8));
+                split(u, R16);
+                P.padded16 += padded(u);
+                if (strips(u)) {
+                    addStrips(u);
+                } else {
+                    P.slotWords = std::max(P.slotWords, words(u));
+                    P.units.push_back(u);
+                }
+            }
+        return;
+    }
+    const size_t at = P.units.size();
+    P.units.resize(at + nItems - n64);
+    int64_t slotWords = P.slotWords, pad = 0;
+#pragma omp parallel for schedule(dynamic, 8) reduction(max : slotWords) reduction(+ : pad) if (par)
+    for (int64_t b = (int64_t)b64; b < (int64_t)bG; ++b) {
+        size_t it = at + itemOff[b] - n64;
+        for (size_t k = starts[b]; k < starts[b + 1]; k += 8, ++it) {
+            ScoreUnit u = item(b, k, std::min(starts[b + 1], k + 8));
+            split(u, R16);
+            slotWords = std::max(slotWords, words(u));
+            pad += padded(u);
+            P.units[it] = u;
+        }
+    }
+    P.slotWords = slotWords;
+    P.padded16 += pad;
 }
 
 // Routing (empty / int16 / int32) and length bucketing into work items.
 // Pure host code: needs no device.
 void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &scoring, uint32_t mode,
-          uint32_t flags, Planned &P, bool traceShape = false, bool noLong = false)
+          uint32_t flags, Planned &P, bool traceShape = false, bool noLong = false, bool noStrips = false)
 {
     P.flags = flags;
     const int64_t N = H.count;
@@ -559,6 +772,11 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
     // cells past n stay at or below the maximum over columns 1..n, and an
     // equal one follows its source in column order.
     si.dna = si.alpha <= 4 && si.sMin - si.o >= 0 && si.sMax - si.o <= 255;
+    si.dnaDrift = si.dna && si.sMax - si.o - std::max(si.o, si.e) <= 255;
+    P.drift = driftOf(si, local);
+    P.dna16 = local || traceShape ? si.dna : si.dnaDrift;
+    const Drift dr = P.drift;
+    const bool dna16 = P.dna16;
     uint32_t track;
     if (local)
         track = kTrackLocal;
@@ -578,7 +796,8 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
     // the shape table's choice for the number of the call's pairs in that
     // bin (a pair that needs more than 255 row blocks of its bin's shape
     // takes G = 16, R = 16).
-    std::vector<Key> keys((size_t)N);
+    RawVec<Key> &keys = P.keys16;
+    keys.resize((size_t)N);
     int64_t cells = 0;
     // The long route: every AlignConfig and local for scores, global only
     // for the traceback.
@@ -590,122 +809,147 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
     };
     std::vector<Variant16> &shapes = P.shapes;
     shapes.clear();
-    uint8_t binSlot[16];
     bool fineBin[16] = {};
-    int fallbackSlot = -1;
     const int forcedG = (int)((flags >> 8) & 0xFF), forcedR = (int)((flags >> 16) & 0xFF);
-    if (traceShape || (forcedG && forcedR)) {
-        shapes.push_back(traceShape ? Variant16{kTraceLanes, kTraceRows / kTraceLanes, si.dna, track}
-                                    : Variant16{forcedG, forcedR, si.dna, track});
-        std::fill(binSlot, binSlot + 16, (uint8_t)0);
-        std::fill(fineBin, fineBin + 16, rowUnitsMode() == 2);
-        if (shapes[0].G == 1) {
-            // Pairs taller than 255 blocks of the forced lane shape.
-            shapes.push_back(Variant16{16, 16, si.dna, track});
-            fallbackSlot = 1;
-        }
+    int R16 = 16, R64 = 0;          // rows per lane of the group shapes (R64 = 0: by the rule)
+    int binLane[16] = {};           // one-pair-per-lane rows of a length bin, or 0
+    int binG[16] = {};              // forced group size of a bin, or 0 (the rule)
+    double cells64 = 0, cellsStrip = 0;
+    if (traceShape) {
+        shapes.push_back(Variant16{kTraceLanes, kTraceRows / kTraceLanes, si.dna, track});
     } else {
-        // Pairs per length bin (int16 route only), then one slot per shape.
-        int64_t binCount[16] = {};
+        for (int w = 1; w >= 0; --w)
+            shapes.push_back(Variant16{64, 16, dna16, track, w != 0});
+        for (int w = 1; w >= 0; --w)
+            shapes.push_back(Variant16{16, 16, dna16, track, w != 0});
+        shapes.push_back(Variant16{1, 16, dna16, track});
+        shapes.push_back(Variant16{1, 32, dna16, track});
+        shapes.push_back(Variant16{1, forcedG == 1 ? forcedR : 16, dna16, track, true});
+        // Pairs per length bin and cells of the int16 route.
+        int64_t binCount[16] = {}, cells16 = 0;
 #pragma omp parallel if (N > kParallelMin)
         {
-            int64_t local16[16] = {};
+            int64_t local16[16] = {}, localCells = 0;
 #pragma omp for schedule(static) nowait
             for (int64_t i = 0; i < N; ++i) {
                 const int64_t n = H.offsets[i + 1] - H.offsets[i];
                 const int64_t m = V.offsets[i + 1] - V.offsets[i];
-                if (n != 0 && m != 0 && route16(n, m))
+                if (n != 0 && m != 0 && route16(n, m)) {
                     ++local16[lengthBin(m)];
+                    localCells += n * m;
+                }
             }
 #pragma omp critical
-            for (int b = 0; b < 16; ++b)
-                binCount[b] += local16[b];
+            {
+                for (int b = 0; b < 16; ++b)
+                    binCount[b] += local16[b];
+                cells16 += localCells;
+            }
         }
-        const int cat = shapeCategory(si.dna, local);
-        auto slotOf = [&](const Variant16 &v) {
-            for (size_t k = 0; k < shapes.size(); ++k)
-                if (shapes[k].G == v.G && shapes[k].R == v.R)
-                    return (int)k;
-            shapes.push_back(v);
-            return (int)shapes.size() - 1;
-        };
         int64_t pairs16 = 0;
         for (int b = 0; b < 16; ++b)
             pairs16 += binCount[b];
-        // SQMI_BIN_SHAPES="b:G:R,...": the shape of bin b, in place of the
-        // table's (the shape tuner times whole calls with it).
-        int overG[16] = {}, overR[16] = {};
+        cells64 = kCouple64Share * (double)cells16;
+        cellsStrip = kStripShare * (double)cells16;
+        if (fixedShapeRule()) {
+            std::fill(binG, binG + 16, 16);
+        } else {
+            for (int b = 0; b < 16; ++b)
+                binLane[b] = laneRows(shapeCategory(dna16, local), b, pairs16);
+        }
+        // SQMI_BIN_SHAPES="b:G:R,...": the shape of bin b (the shape tuner
+        // times whole calls with it); forced shapes: every bin's.
+        auto force = [&](int b, int g, int r) {
+            if (!shapeSupported(Variant16{g, r, dna16, track}))
+                return;
+            binG[b] = g == 1 ? 0 : g;
+            binLane[b] = g == 1 ? r : 0;
+            if (g == 16)
+                R16 = r;
+            if (g == 64)
+                R64 = r;
+        };
         if (const char *env = std::getenv("SQMI_BIN_SHAPES")) {
             for (const char *c = env; *c;) {
                 int b = -1, g = 0, r = 0, used = 0;
                 if (std::sscanf(c, "%d:%d:%d%n", &b, &g, &r, &used) != 3)
                     break;
-                if (b >= 0 && b < 16) {
-                    overG[b] = g;
-                    overR[b] = r;
-                }
+                if (b >= 0 && b < 16)
+                    force(b, g, r);
                 c += used;
                 if (*c == ',')
                     ++c;
             }
         }
-        for (int b = 0; b < 16; ++b) {
-            Variant16 v = overG[b] ? Variant16{overG[b], overR[b], si.dna, track}
-                                   : tableShape(cat, b, pairs16, si.dna, track);
-            if (!shapeSupported(v))
-                v = Variant16{16, 16, si.dna, track};
-            binSlot[b] = (uint8_t)(binCount[b] ? slotOf(v) : 0);
-        }
-        fallbackSlot = slotOf(Variant16{16, 16, si.dna, track});
+        if (forcedG && forcedR)
+            for (int b = 0; b < 16; ++b)
+                force(b, forcedG, forcedR);
         const int unitsMode = rowUnitsMode();
         for (int b = 0; b < 16; ++b)
             fineBin[b] = unitsMode == 2 || (unitsMode == 0 && binCount[b] >= kFineUnitPairs);
     }
+    // Shape slot and row units of an int16 pair.
+    auto slotOf = [&](int64_t n, int64_t m, int64_t &units) -> uint32_t {
+        if (traceShape) {
+            units = blocksFor(shapes[0], m);
+            return 0;
+        }
+        const int b = lengthBin(m);
+        const bool wide = !driftNarrow(si, dr, local, n, m);
+        if (binLane[b] && (local || !wide || forcedG == 1)) {
+            const uint32_t slot = !local && wide ? kSlotLaneWide : binLane[b] == 32 ? kSlotLane32 : kSlotLane16;
+            units = blocksFor(shapes[slot], m);
+            if (units <= kMaxBlocks16)
+                return slot;
+        }
+        const bool g64 = binG[b] ? binG[b] == 64 : (double)n * (double)m > cells64;
+        units = unitsOfRows(m);
+        if (!fineBin[b]) {
+            // Pairs of an item have their row 0 in block 0: coarse units span
+            // no more than a block (R = 8 on 16 lanes: 128 rows).
+            const int64_t per = !g64 && R16 == 8 ? 2 : 4;
+            units = (units + per - 1) / per * per;
+        }
+        return (g64 ? kSlot64 : kSlot16) + (wide ? 0u : 1u);
+    };
 #pragma omp parallel for schedule(static) reduction(+ : cells) if (N > kParallelMin)
     for (int64_t i = 0; i < N; ++i) {
         const int64_t n = H.offsets[i + 1] - H.offsets[i];
         const int64_t m = V.offsets[i + 1] - V.offsets[i];
-        uint32_t key = kClassEmpty << kKeyClassShift;
+        uint32_t key = kClassRest << kKeyClassShift;
         if (n != 0 && m != 0) {
             cells += n * m;
-            key = kClassInt32 << kKeyClassShift;
             if (route16(n, m)) {
-                uint32_t slot = binSlot[lengthBin(m)];
-                int64_t nblocks = blocksFor(shapes[slot], m);
-                if (nblocks > kMaxBlocks16 && fallbackSlot >= 0) {
-                    slot = (uint32_t)fallbackSlot;
-                    nblocks = blocksFor(shapes[slot], m);
-                }
-                if (nblocks <= kMaxBlocks16) {
-                    const int64_t units =
-                        unitsFor(shapes[slot], m, quarterUnits(shapes[slot], traceShape), fineBin[lengthBin(m)]);
+                int64_t units = 0;
+                const uint32_t slot = slotOf(n, m, units);
+                if (units <= 1023 && !(traceShape && units > kMaxBlocks16))
                     key = (slot << kKeyClassShift) | ((1023u - (uint32_t)units) << kKeyNBits) |
                           ((1u << kKeyNBits) - 1 - (uint32_t)n);
-                }
             }
         }
         keys[i] = Key{key, (int32_t)i};
     }
     P.cells = cells;
-    radixSort(keys);
-    // Segments of the sorted order: int16 (by shape), int32, empty.
+    radixSort(keys, P.keysTmp, P.sortHist);
+    // Segments of the sorted order: int16 (by shape), then int32 and empty.
     size_t n16 = 0;
-    while (n16 < keys.size() && (keys[n16].key >> kKeyClassShift) < kClassInt32) {
+    while (n16 < keys.size() && (keys[n16].key >> kKeyClassShift) < kClassRest) {
         // Jump by bucket boundaries found with a binary search.
         const uint32_t cls = keys[n16].key >> kKeyClassShift;
         n16 = (size_t)(std::upper_bound(keys.begin() + n16, keys.end(), ((cls + 1) << kKeyClassShift) - 1,
                                         [](uint32_t v, const Key &k) { return v < k.key; }) -
                        keys.begin());
     }
-    size_t e32 = n16;
-    while (e32 < keys.size() && (keys[e32].key >> kKeyClassShift) == kClassInt32)
-        ++e32;
     const int64_t longMin = longMinSide();
     const bool longOk = si.dna && (mode == 0 || !traceShape) && !noLong;
-    for (size_t k = n16; k < e32; ++k) {
+    for (size_t k = n16; k < keys.size(); ++k) {
         const int32_t i = keys[k].id;
         const int64_t n = H.offsets[i + 1] - H.offsets[i];
         const int64_t m = V.offsets[i + 1] - V.offsets[i];
+        if (n == 0 || m == 0) {
+            P.emptyIds.push_back(i);
+            continue;
+        }
         if (longOk && n >= longMin && m >= longMin && fitsLong32(si, n, m)) {
             P.idsLong.push_back(i);
             continue;
@@ -716,11 +960,8 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
         // one trace byte per cell, 16-byte aligned.
         P.scratch32 += traceShape ? ((8 * (m + 1) + (n + 1) * (m + 1) + 15) & ~(int64_t)15) : m + 1;
     }
-    for (size_t k = e32; k < keys.size(); ++k)
-        P.emptyIds.push_back(keys[k].id);
     keys.resize(n16);
-    std::vector<Key> &keys16 = P.keys16;
-    keys16.swap(keys);
+    RawVec<Key> &keys16 = P.keys16;
 
     // Work items: each bucket (shape, row blocks) is cut into runs of up to
     // pairs-per-wave pairs, in sorted order.  Bucket starts are found in
@@ -754,7 +995,9 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
         itemOff[b + 1] = itemOff[b] + (starts[b + 1] - starts[b] + PP - 1) / PP;
     }
     std::vector<Plan16> &plans = P.plans;
-    for (uint32_t v = 0; v < (uint32_t)shapes.size(); ++v) {
+    if (!traceShape)
+        makeUnits(V, P, starts, itemOff, R16, R64, cellsStrip, noStrips);
+    for (uint32_t v = traceShape ? 0 : kSlotLane16; v < (uint32_t)shapes.size(); ++v) {
         // The shape's contiguous range of buckets and of sorted pairs.
         size_t b0 = 0;
         while (b0 < nb && (keys16[starts[b0]].key >> kKeyClassShift) < v)
@@ -770,7 +1013,6 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
         const size_t p0 = starts[b0], p1 = starts[b1];
         const size_t i0 = itemOff[b0];
         const int PP = pairsPerWave(pl.var);
-        const bool quarter = quarterUnits(pl.var, traceShape);
         pl.order.resize(p1 - p0);
         pl.items.resize(itemOff[b1] - i0);
         int32_t maxN = 0;
@@ -783,14 +1025,11 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
 #pragma omp parallel for schedule(dynamic, 8) if (p1 - p0 > (size_t)kParallelMin)
         for (int64_t b = (int64_t)b0; b < (int64_t)b1; ++b) {
             size_t it = itemOff[b] - i0;
-            const int32_t units = unitsOf(keys16[starts[b]].key);
-            const int32_t nblocks = quarter ? (units + 3) / 4 : units;
-            const int32_t headQ = quarter ? units - 4 * (nblocks - 1) : 4;   // quarters in block 0
+            const int32_t nblocks = unitsOf(keys16[starts[b]].key);
             for (size_t k = starts[b]; k < starts[b + 1]; k += PP, ++it) {
                 const size_t e = std::min(starts[b + 1], k + PP);
                 // Widest first inside a bucket: the first pair has the item's width.
-                pl.items[it] = WorkItem{(int32_t)(k - p0), (int32_t)(e - k) | ((headQ & 3) << 16),
-                                        widthOf(keys16[k].key), nblocks};
+                pl.items[it] = WorkItem{(int32_t)(k - p0), (int32_t)(e - k), widthOf(keys16[k].key), nblocks};
             }
         }
     }
@@ -804,16 +1043,14 @@ void fillStats(const Planned &P, sqmi_stats &st)
     st.pairs_long = (int64_t)P.idsLong.size();
     st.pairs_long_packed = (longPacked(P.si, P.flags) && P.mode == 0) ? st.pairs_long : 0;
     st.pairs_int16 = (int64_t)P.keys16.size();
-    int64_t items = 0, padded = 0;
+    int64_t items = P.items16, padded = P.padded16;
     st.pairs_lane = 0;
     for (const Plan16 &pl : P.plans) {
         items += (int64_t)pl.items.size();
         if (pl.var.G == 1)
             st.pairs_lane += (int64_t)pl.order.size();
-        for (const WorkItem &w : pl.items) {
-            const int64_t BR = (int64_t)pl.var.G * pl.var.R, headQ = ((w.count >> 16) & 3) ? ((w.count >> 16) & 3) : 4;
-            padded += 2LL * (64 / pl.var.G) * (int64_t)w.maxN * ((w.nblocks - 1) * BR + headQ * BR / 4);
-        }
+        for (const WorkItem &w : pl.items)
+            padded += 2LL * (64 / pl.var.G) * (int64_t)w.maxN * w.nblocks * pl.var.G * pl.var.R;
     }
     st.work_items = items;
     st.padded_cells = padded;
@@ -862,17 +1099,6 @@ int64_t traceBudget(const sqmi_context *ctx)
     }
     const int64_t quarter = ctx ? ctx->totalMem / 4 : 0;
     return std::min<int64_t>(std::max<int64_t>(quarter, (int64_t)8 << 30), (int64_t)64 << 30);
-}
-
-// Work items with at least this many row blocks are swept by the four waves
-// of a workgroup together (10, i.e. more than 2304 rows, or
-// SQMI_COOP_MIN_BLOCKS; 0 disables).  Shorter items gain nothing from it.
-int coopMinBlocks()
-{
-    const char *env = std::getenv("SQMI_COOP_MIN_BLOCKS");
-    if (env && *env)
-        return std::max(0, std::atoi(env));
-    return kTabCoopMinBlocks;
 }
 
 // Device copies of what every entry point needs: residues (unless already on
@@ -1267,12 +1493,18 @@ sqmi_status sqmi_create(int device, sqmi_context **out)
     sqmi_context *ctx = new (std::nothrow) sqmi_context();
     if (!ctx)
         return SQMI_ERR_OUT_OF_MEMORY;
+    ctx->planned = new (std::nothrow) Planned();
+    if (!ctx->planned) {
+        delete ctx;
+        return SQMI_ERR_OUT_OF_MEMORY;
+    }
     ctx->device = device;
     ctx->numCUs = prop.multiProcessorCount;
     ctx->l2PerCU = (int64_t)prop.l2CacheSize / 32;
     ctx->totalMem = (int64_t)prop.totalGlobalMem;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&ctx->ownStream) != hipSuccess ||
         hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&ctx->waitFlag), 64, hipHostMallocDefault) != hipSuccess ||
         scratchAddress(device, &ctx->scratchPtr) != hipSuccess) {
         if (ctx->ev0)
             (void)hipEventDestroy(ctx->ev0);
@@ -1280,9 +1512,13 @@ sqmi_status sqmi_create(int device, sqmi_context **out)
             (void)hipEventDestroy(ctx->ev1);
         if (ctx->ownStream)
             (void)hipStreamDestroy(ctx->ownStream);
+        if (ctx->waitFlag)
+            (void)hipHostFree(ctx->waitFlag);
+        delete ctx->planned;
         delete ctx;
         return SQMI_ERR_DEVICE;
     }
+    *ctx->waitFlag = 0;
     ctx->stream = ctx->ownStream;
     *out = ctx;
     return SQMI_OK;
@@ -1312,6 +1548,9 @@ sqmi_status sqmi_destroy(sqmi_context *ctx)
         (void)hipEventDestroy(ctx->longFork);
     if (ctx->ownStream)
         (void)hipStreamDestroy(ctx->ownStream);
+    if (ctx->waitFlag)
+        (void)hipHostFree(ctx->waitFlag);
+    delete ctx->planned;
     delete ctx;
     return SQMI_OK;
 }
@@ -1405,7 +1644,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             if ((err = hipStreamSynchronize(stream)) != hipSuccess)
                 return hipFail(ctx, err, "alignment kernels");
             ctx->longStreamed = ctx->replay.longStreamed;
-            if ((st = longStreamCheck(ctx)) != SQMI_OK)
+            if ((st = longStreamCheck(ctx)) != SQMI_OK || (st = stripCheck(ctx)) != SQMI_OK)
                 return st;
             ctx->stats = ctx->replay.stats;
             ctx->stats.host_plan_ms = keyMs;
@@ -1418,9 +1657,10 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
     }
     dropReplay(ctx);
 
-    Planned P;
+    Planned &P = *ctx->planned;
+    P.reset();
     const auto tPlan = std::chrono::steady_clock::now();
-    plan(*setH, *setV, *scoring, mode, flags, P);
+    plan(*setH, *setV, *scoring, mode, flags, P, false, false, ctx->noAlloc);
     ctx->stats.host_plan_ms = msSince(tPlan);
     fillStats(P, ctx->stats);
     const ScoringInfo &si = P.si;
@@ -1430,6 +1670,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
     const int64_t scratch32 = P.scratch32;
     const auto &keys16 = P.keys16;
     const uint32_t track = P.track;
+    const int kind = P.local ? kScoreLocal : (track & kTrackRight) ? kScoreRight : kScoreGlobal;
 
     // The no-allocation call: everything but the row buffers has a fixed
     // size; the row buffers need at least one workgroup's worth per shape.
@@ -1450,12 +1691,16 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         for (const Plan16 &pl : plans) {
             nOrder += pl.order.size();
             nItems += pl.items.size();
-            const Variant16 &v = pl.var;
-            const int rc = v.G == 1 ? laneRowCols(pl.maxN, v.R) : pl.maxN + v.G + 2;
-            minRb = std::max(minRb, (size_t)wavesPerBlock16() * 64 / (v.G == 1 ? 1 : v.G) * rc * 8);
+            minRb = std::max(minRb, (size_t)wavesPerBlock16() * 64 * laneRowCols(pl.maxN, pl.var.R) * 8);
         }
         if (!plans.empty())
-            need += arenaBytes(4 * nOrder) + arenaBytes(sizeof(WorkItem) * nItems) + arenaBytes(64 * plans.size());
+            need += arenaBytes(4 * nOrder) + arenaBytes(sizeof(WorkItem) * nItems);
+        if (!P.units.empty()) {
+            need += arenaBytes(4 * P.order16.size()) + arenaBytes(sizeof(ScoreUnit) * P.units.size());
+            minRb = std::max(minRb, (size_t)wavesPerBlock16() * P.slotWords * 8);
+        }
+        if (!plans.empty() || !P.units.empty())
+            need += arenaBytes(64 * (plans.size() + 1));
         if (!ids32.empty())
             need += arenaBytes(4 * ids32.size()) + arenaBytes(8 * ids32.size()) + arenaBytes((size_t)8 * scratch32);
         if (!emptyIds.empty())
@@ -1479,115 +1724,154 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
     // Kernel launches wait in `launches` until every upload is enqueued.
     Deferred launches;
 
+    // ---- packed score kernel: its arguments but for the units ----------
+    ScoreArgs sa{};
+    sa.hRes = dH;
+    sa.vRes = dV;
+    sa.hOff = static_cast<const int64_t *>(ctx->b.hOff.p);
+    sa.vOff = static_cast<const int64_t *>(ctx->b.vOff.p);
+    sa.error = ctx->waitFlag;
+    sa.scores = dScores;
+    sa.mode = mode;
+    sa.alpha = A;
+    sa.tTable = static_cast<const int16_t *>(ctx->b.tTable.p);
+    sa.dnaProfile = static_cast<const uint32_t *>(ctx->b.dnaProf.p);
+    sa.drift = P.drift;
+
     // ---- plain form: one launch per pair (baseline for the batched form) --
     // Host data staged by hipMemcpyAsync must outlive the copies: the plain
     // form's lists live at function scope, like the planner's.
     std::vector<int32_t> plainIds;
-    std::vector<WorkItem> plainItems;
+    std::vector<ScoreUnit> plainUnits;
     if ((flags & SQMI_PLAIN_PER_PAIR) && (err = hipEventRecord(ctx->ev0, stream)) != hipSuccess)
         return hipFail(ctx, err, "event");
     if (flags & SQMI_PLAIN_PER_PAIR) {
-        std::vector<int32_t> &ids16 = plainIds;
-        std::vector<WorkItem> &items = plainItems;
-        int maxN = 0;
+        // One wavefront, whose first 16-lane group sweeps the pair (the other
+        // pair slots of the wavefront stay empty).
+        int64_t slotWords = 1;
         for (const Key &k : keys16) {
             const int32_t id = k.id;
             const int64_t n = setH->offsets[id + 1] - setH->offsets[id];
             const int64_t m = setV->offsets[id + 1] - setV->offsets[id];
-            const Variant16 v = plainVariant(si.dna, track, m);
-            const int64_t BR = (int64_t)v.G * v.R;
-            items.push_back(WorkItem{(int32_t)ids16.size(), 1, (int32_t)n, (int32_t)((m + 1 + BR - 1) / BR)});
-            ids16.push_back(id);
-            maxN = std::max<int>(maxN, (int)n);
+            const int units = (int)unitsOfRows(m), nb = (units + 3) / 4;
+            plainUnits.push_back(ScoreUnit{(int32_t)plainIds.size(), 1, (int32_t)n, nb,
+                                           16 | (4 * (units - 4 * (nb - 1))) << 8,
+                                           driftNarrow(si, P.drift, P.local, n, m) ? 0 : kUnitWide, -1, 0, 0});
+            plainIds.push_back(id);
+            slotWords = std::max<int64_t>(slotWords, 4 * (n + 1));
         }
-        const size_t np = ids16.size();
+        const size_t np = plainIds.size();
         if ((err = ensure(ctx->b.order, 4 * np)) != hipSuccess ||
-            (err = ensure(ctx->b.items, sizeof(WorkItem) * np)) != hipSuccess ||
+            (err = ensure(ctx->b.items, sizeof(ScoreUnit) * np)) != hipSuccess ||
             (err = ensure(ctx->b.queue, 4 * np + 64)) != hipSuccess ||
-            (err = ensure(ctx->b.rowbuf, (size_t)4 * (maxN + 18) * 2 * sizeof(uint32_t))) != hipSuccess)
+            (err = ensure(ctx->b.rowbuf, (size_t)slotWords * 8)) != hipSuccess)
             return hipFail(ctx, err, "allocating plain work lists");
-        if (np && ((err = hipMemcpyAsync(ctx->b.order.p, ids16.data(), 4 * np, hipMemcpyHostToDevice, stream)) !=
+        if (np && ((err = hipMemcpyAsync(ctx->b.order.p, plainIds.data(), 4 * np, hipMemcpyHostToDevice, stream)) !=
                        hipSuccess ||
-                   (err = hipMemcpyAsync(ctx->b.items.p, items.data(), sizeof(WorkItem) * np, hipMemcpyHostToDevice,
-                                         stream)) != hipSuccess ||
+                   (err = hipMemcpyAsync(ctx->b.items.p, plainUnits.data(), sizeof(ScoreUnit) * np,
+                                         hipMemcpyHostToDevice, stream)) != hipSuccess ||
                    (err = hipMemsetAsync(ctx->b.queue.p, 0, 4 * np, stream)) != hipSuccess))
             return hipFail(ctx, err, "uploading plain work lists");
         for (size_t k = 0; k < np; ++k) {
-            const int32_t id = ids16[k];
-            const Variant16 v = plainVariant(si.dna, track, setV->offsets[id + 1] - setV->offsets[id]);
-            FwdArgs a{};
-            a.hRes = dH;
-            a.vRes = dV;
-            a.hOff = static_cast<const int64_t *>(ctx->b.hOff.p);
-            a.vOff = static_cast<const int64_t *>(ctx->b.vOff.p);
+            ScoreArgs a = sa;
             a.order = static_cast<const int32_t *>(ctx->b.order.p);
-            a.items = static_cast<const WorkItem *>(ctx->b.items.p) + k;
-            a.nItems = 1;
+            a.units = static_cast<const ScoreUnit *>(ctx->b.items.p) + k;
+            a.nUnits = 1;
             a.queue = static_cast<uint32_t *>(ctx->b.queue.p) + k;
-            a.rowbuf = static_cast<uint32_t *>(ctx->b.rowbuf.p);
-            a.rowCols = maxN + 18;
-            a.scores = dScores;
-            a.gapOpen = si.o;
-            a.gapExtend = si.e;
-            a.mode = mode;
-            a.alpha = A;
-            a.tTable = static_cast<const int16_t *>(ctx->b.tTable.p);
-            a.dnaProfile = static_cast<const uint32_t *>(ctx->b.dnaProf.p);
-            a.tNonNeg = tNonNeg(si, mode);
-            if ((err = launchFwd16(v, a, 1, stream, 64)) != hipSuccess)
+            a.rowbuf = static_cast<uint64_t *>(ctx->b.rowbuf.p);
+            a.slotWords = slotWords;
+            if ((err = launchScore16(P.dna16, kind, a, 1, stream, 64)) != hipSuccess)
                 return hipFail(ctx, err, "launching plain kernel");
         }
         plans.clear();
+        P.units.clear();
     }
 
     // ---- packed int16 kernels -------------------------------------------
-    // One launch per shape in use, in order on the stream.  Each plan has its
-    // own slices of the work lists and its own queue counters (cleared by one
-    // fill kernel), so the uploads of a later plan never touch what an
-    // earlier launch still reads; the launches share the row buffers, which a
-    // launch only uses while it runs.
-    if (!plans.empty()) {
+    // The packed score kernel takes every group unit in one launch; the
+    // one-pair-per-lane shapes in use one launch each, in order on the
+    // stream.  Each has its own slices of the work lists and its own queue
+    // counter (cleared by one fill kernel), so the uploads of a later launch
+    // never touch what an earlier one still reads; the launches share the row
+    // buffers, which a launch only uses while it runs.
+    if (!plans.empty() || !P.units.empty()) {
         const int wpb = wavesPerBlock16();
-        std::vector<size_t> orderOff(plans.size() + 1, 0), itemOff(plans.size() + 1, 0);
+        const size_t unitBytes = sizeof(ScoreUnit) * P.units.size(), unitOrder = P.order16.size();
+        std::vector<size_t> orderOff(plans.size() + 1, unitOrder), itemOff(plans.size() + 1, 0);
         std::vector<int> grids(plans.size()), rowColsOf(plans.size());
         size_t rbMax = 0;
+        int unitGrid = 0;
+        if (!P.units.empty()) {
+            unitGrid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occupancyScore16(P.dna16, kind),
+                                                          ((int64_t)P.units.size() + wpb - 1) / wpb));
+            const size_t perBlock = std::max<size_t>((size_t)wpb * P.slotWords * 8, 8);
+            if (ctx->noAlloc)   // the persistent grid shrinks to the scratch that is left
+                unitGrid = (int)std::max<size_t>(1, std::min<size_t>((size_t)unitGrid, rowbufBudget / perBlock));
+            rbMax = (size_t)unitGrid * perBlock;
+        }
         for (size_t k = 0; k < plans.size(); ++k) {
             const Plan16 &pl = plans[k];
             const Variant16 &v = pl.var;
-            if (!shapeSupported(v))
+            if (!laneSupported(v))
                 return fail(ctx, SQMI_ERR_UNSUPPORTED, "kernel variant not compiled");
-            const int occ = v.G == 1 ? occupancyLane16(v) : occupancy16(v);
             const int64_t nIt = (int64_t)pl.items.size();
-            grids[k] = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occ, (nIt + wpb - 1) / wpb));
-            // Row buffers per wave slot: G = 16, one row of (G, F) per group;
-            // G = 1, one per lane, column-major across the 64 lanes.
-            rowColsOf[k] = v.G == 1 ? laneRowCols(pl.maxN, v.R) : pl.maxN + v.G + 2;
-            const size_t perBlock = (size_t)wpb * 64 / (v.G == 1 ? 1 : v.G) * rowColsOf[k] * 8;
-            if (ctx->noAlloc)   // the persistent grid shrinks to the scratch that is left
+            grids[k] = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occupancyLane16(v), (nIt + wpb - 1) / wpb));
+            // Row buffers per wave slot: one per lane, column-major across the 64 lanes.
+            rowColsOf[k] = laneRowCols(pl.maxN, v.R);
+            const size_t perBlock = (size_t)wpb * 64 * rowColsOf[k] * 8;
+            if (ctx->noAlloc)
                 grids[k] = (int)std::max<size_t>(1, std::min<size_t>((size_t)grids[k], rowbufBudget / perBlock));
             rbMax = std::max(rbMax, (size_t)grids[k] * perBlock);
             orderOff[k + 1] = orderOff[k] + pl.order.size();
             itemOff[k + 1] = itemOff[k] + pl.items.size();
         }
-        const size_t nq = 16 * plans.size();   // queue counters: 16 dwords per plan
+        const size_t nq = 16 * (plans.size() + 1);   // queue counters: 16 dwords per launch
         if ((err = ensure(ctx->b.order, 4 * orderOff.back())) != hipSuccess ||
-            (err = ensure(ctx->b.items, sizeof(WorkItem) * itemOff.back())) != hipSuccess ||
-            (err = ensure(ctx->b.queue, 4 * nq)) != hipSuccess || (err = ensure(ctx->b.rowbuf, rbMax)) != hipSuccess)
+            (err = ensure(ctx->b.items, unitBytes + sizeof(WorkItem) * itemOff.back())) != hipSuccess ||
+            (err = ensure(ctx->b.queue, 4 * nq)) != hipSuccess || (err = ensure(ctx->b.rowbuf, rbMax)) != hipSuccess ||
+            (P.stripWords && (err = ensure(ctx->b.strips, (size_t)P.stripWords * 8)) != hipSuccess))
             return hipFail(ctx, err, "allocating work lists");
         uint32_t *dQueues = static_cast<uint32_t *>(ctx->b.queue.p);
         launches.push_back([=] { return launchZero32(dQueues, nq, stream); });
+        if (!P.units.empty()) {
+            if ((err = hipMemcpyAsync(ctx->b.order.p, P.order16.data(), 4 * unitOrder, hipMemcpyHostToDevice, stream)) !=
+                    hipSuccess ||
+                (err = hipMemcpyAsync(ctx->b.items.p, P.units.data(), unitBytes, hipMemcpyHostToDevice, stream)) !=
+                    hipSuccess)
+                return hipFail(ctx, err, "uploading work lists");
+            ScoreArgs a = sa;
+            a.order = static_cast<const int32_t *>(ctx->b.order.p);
+            a.units = static_cast<const ScoreUnit *>(ctx->b.items.p);
+            a.nUnits = (int32_t)P.units.size();
+            a.queue = dQueues;
+            a.rowbuf = static_cast<uint64_t *>(ctx->b.rowbuf.p);
+            a.slotWords = P.slotWords;
+            a.strips = static_cast<uint64_t *>(ctx->b.strips.p);
+            a.stripWords = P.stripWords;
+            if (P.stripWords > 0) {
+                // Strips find their input words by their not being 0, and
+                // merge the results of modes that track every block's cells.
+                const size_t words = 2 * (size_t)P.stripWords;
+                uint32_t *dStrips = static_cast<uint32_t *>(ctx->b.strips.p);
+                launches.push_back([=] { return launchZero32(dStrips, words, stream); });
+                if (kind != kScoreGlobal)
+                    launches.push_back([=] {
+                        return launchFill32(reinterpret_cast<uint32_t *>(dScores), (size_t)N, (uint32_t)INT32_MIN, stream);
+                    });
+            }
+            const bool dna = P.dna16;
+            launches.push_back([=] { return launchScore16(dna, kind, a, unitGrid, stream); });
+        }
         for (size_t k = 0; k < plans.size(); ++k) {
             const Plan16 &pl = plans[k];
             const Variant16 &v = pl.var;
             int32_t *dOrder = static_cast<int32_t *>(ctx->b.order.p) + orderOff[k];
-            WorkItem *dItems = static_cast<WorkItem *>(ctx->b.items.p) + itemOff[k];
-            uint32_t *dQueue = static_cast<uint32_t *>(ctx->b.queue.p) + 16 * k;
+            WorkItem *dItems = reinterpret_cast<WorkItem *>(static_cast<char *>(ctx->b.items.p) + unitBytes) + itemOff[k];
             if ((err = hipMemcpyAsync(dOrder, pl.order.data(), 4 * pl.order.size(), hipMemcpyHostToDevice,
                                       stream)) != hipSuccess ||
                 (err = hipMemcpyAsync(dItems, pl.items.data(), sizeof(WorkItem) * pl.items.size(),
                                       hipMemcpyHostToDevice, stream)) != hipSuccess)
                 return hipFail(ctx, err, "uploading work lists");
-            const int64_t nIt = (int64_t)pl.items.size();
             FwdArgs a{};
             a.hRes = dH;
             a.vRes = dV;
@@ -1595,19 +1879,8 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             a.vOff = static_cast<const int64_t *>(ctx->b.vOff.p);
             a.order = dOrder;
             a.items = dItems;
-            a.nItems = (int32_t)nIt;
-            a.queue = dQueue;
-            // Items are ordered by row blocks, most first: the leading ones with
-            // at least coopMinBlocks() blocks are shared by a workgroup's waves
-            // (groups of 16 lanes only).
-            {
-                const int minBlocks = v.G == 1 ? 0 : coopMinBlocks();
-                int32_t nLong = 0;
-                while (minBlocks > 0 && nLong < (int32_t)nIt && pl.items[nLong].nblocks >= minBlocks)
-                    ++nLong;
-                a.nLong = nLong;
-                a.queueLong = dQueue + 1;
-            }
+            a.nItems = (int32_t)pl.items.size();
+            a.queue = dQueues + 16 * (k + 1);
             a.rowbuf = static_cast<uint32_t *>(ctx->b.rowbuf.p);
             a.rowCols = rowColsOf[k];
             a.scores = dScores;
@@ -1617,10 +1890,9 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             a.alpha = A;
             a.tTable = static_cast<const int16_t *>(ctx->b.tTable.p);
             a.dnaProfile = static_cast<const uint32_t *>(ctx->b.dnaProf.p);
-            a.tNonNeg = tNonNeg(si, mode);
+            a.drift = P.drift;
             const int grid = grids[k];
-            launches.push_back(
-                [=] { return v.G == 1 ? launchLane16(v, a, grid, stream) : launchFwd16(v, a, grid, stream); });
+            launches.push_back([=] { return launchLane16(v, a, grid, stream); });
         }
     }
 
@@ -1712,8 +1984,10 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         return hipFail(ctx, err, "alignment kernels");
     if (ctx->replay.valid)
         ctx->replay.longStreamed = ctx->longStreamed;
-    if ((st = longStreamCheck(ctx)) != SQMI_OK)
+    if ((st = longStreamCheck(ctx)) != SQMI_OK || (st = stripCheck(ctx)) != SQMI_OK) {
+        dropReplay(ctx);
         return st;
+    }
     float ms = 0;
     if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess)
         ctx->stats.device_ms = ms;
@@ -1817,7 +2091,8 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         return fail(ctx, SQMI_ERR_DEVICE, "hipSetDevice failed");
     hipStream_t stream = ctx->stream;
 
-    Planned P;
+    Planned &P = *ctx->planned;
+    P.reset();
     Inputs in;
     // Host residue sets of 4 MB and more are copied in on a second host
     // thread while this one plans (the planner reads only the offsets; a

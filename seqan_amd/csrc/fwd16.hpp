@@ -1018,19 +1018,6 @@ struct Fwd16 {
     }
 };
 
-// Waves per SIMD the register budget is set for: three (168 VGPRs) for the
-// DNA kernels and the R = 8 table kernels; two (256 VGPRs) for the R = 16
-// table kernels, whose table-row offsets and scores read one column ahead
-// would spill at three.
-template <int R, bool DNA>
-constexpr int kFwdWaves = (!DNA && R >= 16) ? 2 : 3;
-
-template <int G, int R, bool DNA, uint32_t TRK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFwdWaves<R, DNA>))) void kFwd16(FwdArgs a)
-{
-    Fwd16<G, R, DNA, TRK>::run(a);
-}
-
 // Forward pass with trace records (global alignment under any AlignConfig,
 // G = 16, R = 16).
 template <bool DNA, uint32_t TRK>
@@ -1038,58 +1025,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 {
     Fwd16<16, 16, DNA, TRK, true>::run(a);
 }
-
-template <int G, int R, bool DNA>
-hipError_t launchTrk(const Variant16 &v, const FwdArgs &args, int gridBlocks, hipStream_t stream,
-                     int threadsPerBlock)
-{
-    dim3 grid(gridBlocks), block(threadsPerBlock);
-    switch (v.track) {
-        case kTrackEnd:
-            hipLaunchKernelGGL((kFwd16<G, R, DNA, kTrackEnd>), grid, block, 0, stream, args);
-            break;
-        case kTrackBottom:
-            hipLaunchKernelGGL((kFwd16<G, R, DNA, kTrackBottom>), grid, block, 0, stream, args);
-            break;
-        case kTrackRight:
-            hipLaunchKernelGGL((kFwd16<G, R, DNA, kTrackRight>), grid, block, 0, stream, args);
-            break;
-        case kTrackBottom | kTrackRight:
-            hipLaunchKernelGGL((kFwd16<G, R, DNA, kTrackBottom | kTrackRight>), grid, block, 0, stream, args);
-            break;
-        case kTrackLocal:
-            if constexpr (!DNA) {
-                if (args.tNonNeg) {
-                    hipLaunchKernelGGL((kFwd16<G, R, DNA, kTrackLocal | kLocalAdd3>), grid, block, 0, stream, args);
-                    break;
-                }
-            }
-            hipLaunchKernelGGL((kFwd16<G, R, DNA, kTrackLocal>), grid, block, 0, stream, args);
-            break;
-        default:
-            return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-template <int G, int R, bool DNA>
-const void *kernelTrk(uint32_t track)
-{
-    switch (track) {
-        case kTrackEnd: return (const void *)&kFwd16<G, R, DNA, kTrackEnd>;
-        case kTrackBottom: return (const void *)&kFwd16<G, R, DNA, kTrackBottom>;
-        case kTrackRight: return (const void *)&kFwd16<G, R, DNA, kTrackRight>;
-        case kTrackBottom | kTrackRight: return (const void *)&kFwd16<G, R, DNA, kTrackBottom | kTrackRight>;
-        case kTrackLocal: return (const void *)&kFwd16<G, R, DNA, kTrackLocal>;
-        default: return nullptr;
-    }
-}
-
-// The compiled (G, R) family of this template: a pair couple per group of
-// 16 lanes, or per wavefront (G = 64: the short-batch shapes, four times the
-// lanes per pair for the same rows).  The one-pair-per-lane form is a
-// separate kernel (lane.hip).
-#define SQMI_FOR_EACH_GR(X) X(16, 16) X(16, 8) X(64, 4) X(64, 8) X(64, 16)
 
 }  // namespace
 }  // namespace sqmi

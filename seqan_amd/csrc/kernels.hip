@@ -1,13 +1,14 @@
 // kernels.hip -- gfx950 kernels of the batched affine-gap alignment engine
 // other than the packed forward (fwd16.hpp): the int32 per-pair sweep, the
 // traceback walks and count kernels, the fills; and the dispatch to the
-// packed forward's instantiation units (fwd16.hip).
+// packed kernels' instantiation units (score16.hip, fwd16.hip).
 #include <algorithm>
 #include <type_traits>
 
 #include "fwd16_parts.hpp"
 #include "kernels.hpp"
 #include "packed16.hpp"
+#include "score16_parts.hpp"
 #include "seqan_amd.h"
 
 namespace sqmi {
@@ -103,10 +104,18 @@ __global__ void kFillScores(int32_t *scores, const int32_t *ids, int n, int32_t 
         scores[ids[t]] = value;
 }
 
-__global__ void kZero32(uint32_t *p, size_t n)
+__global__ void kFill32(uint32_t *p, size_t n, uint32_t value)
 {
-    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x)
-        p[t] = 0;
+    // 16 bytes a thread from the first 16-byte boundary on.
+    const size_t head = min(n, (size_t)((16 - (reinterpret_cast<uintptr_t>(p) & 15)) & 15) / 4);
+    const size_t quads = (n - head) / 4, t0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    uint4 *q = reinterpret_cast<uint4 *>(p + head);
+    for (size_t t = t0; t < quads; t += (size_t)gridDim.x * blockDim.x)
+        q[t] = make_uint4(value, value, value, value);
+    if (t0 < head)
+        p[t0] = value;
+    if (t0 < n - head - 4 * quads)
+        p[head + 4 * quads + t0] = value;
 }
 
 // Exclusive prefix sums of the row lengths (one workgroup of 1024 threads:
@@ -552,55 +561,48 @@ int wavesPerBlock16() { return 4; }
 
 namespace {
 
-// The instantiation unit of a shape: DNA profile or table, 16 or 64 lanes.
-const Fwd16Part *partOf(bool dna, int G)
+const void *scoreKernel(bool dna, int kind)
 {
-    if (G == 16)
-        return dna ? &kFwdPartDna16 : &kFwdPartTab16;
-    if (G == 64)
-        return dna ? &kFwdPartDna64 : &kFwdPartTab64;
-    return nullptr;
-}
-
-const void *kernelFor(const Variant16 &v)
-{
-    const Fwd16Part *p = partOf(v.dna, v.G);
-    return p ? p->kernel(v) : nullptr;
+    switch (kind) {
+        case kScoreGlobal: return dna ? scoreDnaGlobal() : scoreTabGlobal();
+        case kScoreRight: return dna ? scoreDnaRight() : scoreTabRight();
+        case kScoreLocal: return dna ? scoreDnaLocal() : scoreTabLocal();
+        default: return nullptr;
+    }
 }
 
 }  // namespace
 
-bool variantSupported(const Variant16 &v) { return kernelFor(v) != nullptr; }
-
-int occupancy16(const Variant16 &v)
+int occupancyScore16(bool dna, int kind)
 {
-    const void *k = kernelFor(v);
-    if (!k)
-        return 0;
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, scoreKernel(dna, kind), 256, 0) != hipSuccess)
         return 1;
     return blocks > 0 ? blocks : 1;
 }
 
-hipError_t launchFwd16(const Variant16 &v, const FwdArgs &args, int gridBlocks, hipStream_t stream,
-                       int threadsPerBlock)
+hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBlocks, hipStream_t stream,
+                         int threadsPerBlock)
 {
-    const Fwd16Part *p = partOf(v.dna, v.G);
-    return p ? p->launch(v, args, gridBlocks, stream, threadsPerBlock) : hipErrorInvalidValue;
+    const void *k = scoreKernel(dna, kind);
+    if (!k)
+        return hipErrorInvalidValue;
+    ScoreArgs copy = args;
+    void *params[] = {&copy};
+    return hipLaunchKernel(k, dim3(gridBlocks), dim3(threadsPerBlock), params, 0, stream);
 }
 
-int traceSteps(int maxN) { return kFwdPartDna16.traceSteps(maxN); }
+int traceSteps(int maxN) { return kFwdPartDna.traceSteps(maxN); }
 
 hipError_t launchFwdTrace16(bool dna, uint32_t track, const FwdArgs &args, int gridBlocks, hipStream_t stream)
 {
-    return (dna ? kFwdPartDna16 : kFwdPartTab16).launchTrace(track, args, gridBlocks, stream);
+    return (dna ? kFwdPartDna : kFwdPartTab).launchTrace(track, args, gridBlocks, stream);
 }
 
 int occupancyTrace16(bool dna)
 {
     int blocks = 0;
-    const void *k = (dna ? kFwdPartDna16 : kFwdPartTab16).traceKernel();
+    const void *k = (dna ? kFwdPartDna : kFwdPartTab).traceKernel();
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, 0) != hipSuccess)
         return 1;
     return blocks > 0 ? blocks : 1;
@@ -644,12 +646,12 @@ hipError_t launchSimple32(const Simple32Args &args, hipStream_t stream)
     return hipGetLastError();
 }
 
-hipError_t launchZero32(uint32_t *p, size_t n, hipStream_t stream)
+hipError_t launchFill32(uint32_t *p, size_t n, uint32_t value, hipStream_t stream)
 {
     if (n == 0)
         return hipSuccess;
-    const size_t blocks = std::min<size_t>((n + 255) / 256, 1024);
-    hipLaunchKernelGGL(kZero32, dim3((unsigned)blocks), dim3(256), 0, stream, p, n);
+    const size_t blocks = std::min<size_t>((n + 1023) / 1024, 2048);
+    hipLaunchKernelGGL(kFill32, dim3((unsigned)blocks), dim3(256), 0, stream, p, n, value);
     return hipGetLastError();
 }
 

@@ -25,8 +25,36 @@ enum Track : uint32_t {
     // Kernel variant flag beside kTrackLocal (table kernels): every table
     // value t = s - gapOpen is >= 0, so the two lookups and the diagonal
     // add fuse into one 32-bit add (FwdArgs::tNonNeg).
-    kLocalAdd3 = 16
+    kLocalAdd3 = 16,
+    // Kernel variant flag of the global score kernels (drifted values): the
+    // values need all 16 bits (Variant16::wide).
+    kWideVals = 32
 };
+
+// The global score kernels (packed, every AlignConfig) hold drifted values
+// (the local ones drift along the sweep only, score16.hpp):
+//   stored(i, j) = value(i, j) + drift * (i + j) + bias,   drift = -max(e, o)
+// (extending past max(e, o) is never better than reopening, so max(e, o)
+// stands for e).  A gap extension is then a step without cost, so
+//   E = max(E, G), F = max(F, G), H = max(G(i-1,j-1) + t, E, F), G = H - cost
+// with cost = max(e, o) - o and t = s + cost + 2 drift: five operations and
+// the score lookup per cell instead of eight.  Every stored value is >= 0:
+// `neg` stands for minus infinity, and no operation on a value >= neg gives a
+// value below 1 (E never falls below neg, G not below neg - cost, a
+// diagonal not below neg - cost + min t).  True values are at least bias -
+// 3 cost (the all-gap path) and above neg.
+struct Drift {
+    int32_t d, cost, neg, bias;
+};
+// Stored values of at most this take the three-operand packed maximum
+// (v_pk_maximum3_f16: as bit patterns, non-negative finite halves order like
+// integers) and 32-bit sums and differences of both halves at once; above,
+// up to 65535, unsigned packed maxima, sums and differences (kWideVals).
+constexpr int kDriftNarrowMax = 0x7bff;
+// Rows and columns past a pair's own that its item may sweep with real
+// residues (one-pair-per-lane kernels): pairs of an item differ by less than
+// a row block in |V|, and columns are swept in groups of 4.
+constexpr int kDriftSlack = 64;
 
 // A work item: up to `pairs per wave` pairs that share the same number of
 // row blocks; processed together by one wavefront.
@@ -61,6 +89,7 @@ struct FwdArgs {
     const int16_t *tTable;      // (alpha+1)^2 entries: s(h,v) - gapOpen, pad row/col
     const uint32_t *dnaProfile; // dwords 0..4: bytes v=0..3 of s(h,v)-gapOpen, h=0..3, pad;
                                 // dwords 8..12: bytes h=0..3 of s(h,v)-gapOpen, v=0..3, pad
+    Drift drift;                // global score kernels
     int32_t tNonNeg;            // local table kernels: every s(h,v) - gapOpen >= 0
     int32_t bandLo, bandUp;     // banded kernels: cells with bandLo <= j - i <= bandUp
     int32_t bandCols;           // banded kernels: row-buffer ring columns (a power of two <= rowCols)
@@ -154,22 +183,58 @@ struct Simple32Args {
     const int32_t *table;       // alpha^2 substitution scores
 };
 
+// The packed score kernels (score16.hpp).  Kinds: global modes without a free
+// last column, with one, local.
+enum ScoreKind : int { kScoreGlobal = 0, kScoreRight = 1, kScoreLocal = 2 };
+// A unit of work: all row blocks of an item (block < 0), or one of them (a
+// strip).  Up to 2 * 64 / G pairs whose row 0 lies in block 0.
+constexpr int32_t kUnit64 = 1, kUnitWide = 2;   // ScoreUnit::shape: G = 64 (else 16), wide values
+struct ScoreUnit {
+    int32_t first;      // index of the first pair in `order`
+    int32_t count;      // pairs
+    int32_t maxN;       // max |H|
+    int32_t nblocks;    // block 0 of G * RH rows, the others of G * R
+    int32_t rows;       // R | RH << 8 (R: 8 or 16, and 4 for G = 64; RH: 4, 8, 12 or 16, and 1, 2, 3, 6 for G = 64)
+    int32_t shape;
+    int32_t block;      // strip: its block, else -1
+    int32_t pad;
+    int64_t rowOff;     // strips: the item's words in ScoreArgs::strips (nblocks x 64 / G x (maxN + 1))
+};
+struct ScoreArgs {
+    const uint8_t *hRes;
+    const uint8_t *vRes;
+    const int64_t *hOff;
+    const int64_t *vOff;
+    const int32_t *order;
+    const ScoreUnit *units;
+    int32_t nUnits;
+    uint32_t *queue;            // unit counter (zeroed before the launch)
+    uint64_t *rowbuf;           // slotWords (G, F) words per wave of the grid
+    int64_t slotWords;
+    uint64_t *strips;           // strips' bottom rows (zeroed before the launch)
+    int64_t stripWords;
+    uint32_t *error;            // host memory: set when a strip's wait runs past its bound
+    int32_t *scores;            // indexed by pair id
+    uint32_t mode;
+    int32_t alpha;
+    const int16_t *tTable;
+    const uint32_t *dnaProfile;
+    Drift drift;
+};
+hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBlocks, hipStream_t stream,
+                         int threadsPerBlock = 256);
+int occupancyScore16(bool dna, int kind);
+
 // Kernel variant of the packed int16 family.
 struct Variant16 {
     int G;      // lanes per pair group
     int R;      // rows per lane
-    bool dna;   // v_perm profile path (alphabet <= 4, not local)
+    bool dna;   // v_perm profile path (alphabet <= 4)
     uint32_t track;
+    bool wide = false;  // global scores: drifted values above kDriftNarrowMax
 };
 
-// Returns the number of work-item slots (waves) the launch should use and the
-// device function; launches onto `stream`.
-hipError_t launchFwd16(const Variant16 &v, const FwdArgs &args, int gridBlocks, hipStream_t stream,
-                       int threadsPerBlock = 256);
 int wavesPerBlock16();
-// Maximum resident blocks per CU for the variant (occupancy query).
-int occupancy16(const Variant16 &v);
-bool variantSupported(const Variant16 &v);
 hipError_t launchSimple32(const Simple32Args &args, hipStream_t stream);
 
 // One pair couple per lane (lane.hip): Variant16 with G = 1 and R in {16,
@@ -256,9 +321,10 @@ hipError_t launchFillScores(int32_t *scores, const int32_t *ids, int n, int32_t 
 // n + 1 exclusive prefix sums of len (device memory throughout).
 hipError_t launchPackRows(const uint8_t *src, const int64_t *off, const int64_t *len, int64_t *start, uint8_t *dst,
                           int64_t n, hipStream_t stream);
-// p[0 .. n) = 0 by a kernel (no memset node, so the call can be captured in a
+// p[0 .. n) = value by a kernel (no memset node, so the call can be captured in a
 // HIP graph).
-hipError_t launchZero32(uint32_t *p, size_t n, hipStream_t stream);
+hipError_t launchFill32(uint32_t *p, size_t n, uint32_t value, hipStream_t stream);
+inline hipError_t launchZero32(uint32_t *p, size_t n, hipStream_t stream) { return launchFill32(p, n, 0, stream); }
 
 // The no-allocation entry point's device array (scratch.hip): its size and
 // its device address on `device`, which must be the current device; the

@@ -18,12 +18,16 @@
 //   H(i,j) = max(G(i-1,j-1) + t(h,v), E(i,j), F(i,j))   [local: max(., 0)]
 //   G(i,j) = H(i,j) + o,   t = s - o
 //
+// Global scores hold drifted values (kernels.hpp, Drift), which make a gap
+// step free of additions and keep every value >= 0; local scores hold the
+// values themselves and saturate.
+//
 // A lane sweeps its couple in blocks of R rows (rows bottom-aligned: row m
 // is the last row of the last block, the rows above row 0 are virtual), all
-// columns of one block before the next.  Adds saturate (v_pk_add_i16 with
-// clamp), so the virtual rows sink towards -32768 and stay below every real
-// value without a floor; only a free first row needs one (rows up to row 0
-// floored at 0, in the first block).  No value crosses lanes, so there is no
+// columns of one block before the next.  The virtual rows need no floor:
+// under drift they stay at or below minus infinity's stand-in, in the local
+// kernels the saturating adds let them sink.  Under a free first row, row 0
+// of the first block gains drift per column (H(0, j) = 0).  No value crosses lanes, so there is no
 // skew and no lane shift; the bottom row of a block (G, F per column) goes
 // to a per-wave row buffer laid out column-major across the 64 lanes (one
 // coalesced 512-byte load and store per column), read back by the next
@@ -45,6 +49,8 @@ namespace {
 
 template <int R, bool DNA, uint32_t TRK>
 struct Lane16 {
+    static constexpr bool LOC = (TRK & kTrackLocal) != 0;
+    static constexpr bool WIDE = (TRK & kWideVals) != 0;
     static constexpr int QD = 4;   // columns per group: one dword of residues per pair
 
     struct Couple {
@@ -80,15 +86,20 @@ struct Lane16 {
 
     // One block of R rows: column 0, then columns 1 .. Nw (rounded up to QD;
     // the extra columns cannot change a result).  FIRST: block 0, with no
-    // row above it (-inf).  TOPFLOOR: block 0 under a free first row, whose
-    // rows up to row 0 are floored at 0 (H(0, j) = 0; the virtual rows above
-    // it then hold 0 too, which leaves row 1 exactly as the border would).
-    template <bool FIRST, bool TOPFLOOR>
+    // row above it (-inf).  TOPFREE: block 0 under a free first row: row 0
+    // takes E(0, j) = H(0, j) = E(0, j - 1) + drift.
+    template <bool FIRST, bool TOPFREE>
     __device__ __forceinline__ static void block(const FwdArgs &a, const Couple &c, int b, int Nw, bool last,
-                                                 uint2 *rb, const uint32_t *sProf, const int16_t *sT, s16x2 &best)
+                                                 uint2 *rb, const uint32_t *sProf, const int16_t *sT, s16x2 &best,
+                                                 int2 &bestH)
     {
         const int o = a.gapOpen, e = a.gapExtend;
-        const s16x2 o2 = splat(o), e2 = splat(e), neg2 = splat(kNeg16);
+        const Drift dr = a.drift;
+        const s16x2 o2 = splat(o), e2 = splat(e), neg2 = splat(LOC ? kNeg16 : dr.neg);
+        // In vector registers: 32-bit adds with scalar operands issue slower.
+        uint32_t cost2 = (uint32_t)dr.cost * 0x10001u, d2 = (uint32_t)dr.d * 0x10001u;
+        if constexpr (!LOC)
+            asm volatile("" : "+v"(cost2), "+v"(d2));
         const bool leftFree = (a.mode & (SQMI_FREE_LEFT | SQMI_LOCAL)) != 0;
         const int eo = max(e, o);   // the first column's gap chain grows by max(e, o) per row
         const int PAD = a.alpha;
@@ -98,6 +109,7 @@ struct Lane16 {
         // Per row: DNA the row words of both pairs, else the two row codes.
         uint32_t rowA[R], rowB[DNA ? R : 1];
         s16x2 Gk[R], Ek[R];
+        uint32_t rowD[TOPFREE ? R : 1];
 #pragma unroll
         for (int k = 0; k < R; ++k) {
             int code[2], g0[2];
@@ -112,6 +124,9 @@ struct Lane16 {
                 code[x] = cc;
                 // G at column 0: virtual rows -inf, H(0,0) = 0, the first column.
                 g0[x] = (i < 0) ? kNeg16 : (i == 0) ? o : ((leftFree ? 0 : o + (i - 1) * eo) + o);
+                if constexpr (!LOC)
+                    g0[x] = (i < 0) ? dr.neg : (i == 0) ? dr.bias - dr.cost
+                            : leftFree ? dr.bias + dr.d * i - dr.cost : dr.bias - 2 * dr.cost;
             }
             if constexpr (DNA) {
                 rowA[k] = sProf[8 + code[0]];
@@ -121,11 +136,17 @@ struct Lane16 {
             }
             Gk[k] = pack(g0[0], g0[1]);
             Ek[k] = neg2;
+            if constexpr (TOPFREE) {
+                const uint32_t top = (rowbase + k == c.p[0] ? 0xffffu : 0u) | (rowbase + k == c.p[1] ? 0xffff0000u : 0u);
+                rowD[k] = d2 & top;
+                Ek[k] = as16(bfi(top, asu(splat(dr.bias)), asu(neg2)));
+            }
         }
-        // TOPFLOOR: row k is floored at 0 in the halves whose row 0 lies at or
-        // below it.  The threshold is made opaque in every step, so that the
-        // compiler recomputes the R masks instead of keeping them live.
-        s16x2 top1 = pack(c.p[0] + 1, c.p[1] + 1);
+        // Free last row: the running maximum of the bottom row's stored G,
+        // gaining drift per column so that it stays comparable; its true
+        // value is taken at column n.
+        uint32_t botM = asu(Gk[R - 1]);
+        const int base[2] = {dr.cost - dr.bias - dr.d * c.m[0], dr.cost - dr.bias - dr.d * c.m[1]};
 
         // Column 0 of the previous block's bottom row (the diagonal input of
         // column 1), then this block's own column-0 entry.
@@ -134,10 +155,6 @@ struct Lane16 {
             upGprev = as16(rb[0].x);
         if (!last)
             rb[0] = make_uint2(asu(Gk[R - 1]), asu(neg2));
-        if constexpr (TRK & kTrackBottom) {
-            if (last)
-                best = vmax(best, Gk[R - 1]);   // H(m, 0) is a tracked cell
-        }
 
         const int NwP = padded(Nw);
         const s16x2 nHalf = pack(c.n[0], c.n[1]);
@@ -195,57 +212,79 @@ struct Lane16 {
                 };
                 s16x2 uG = as16(up.x), uF = as16(up.y);
                 const s16x2 upG = uG;
-                if constexpr (TOPFLOOR)
-                    asm volatile("" : "+v"(top1));
                 // The diagonal term of row k comes from the old G of row k - 1
                 // before it is overwritten.
-                s16x2 D = addSat(upGprev, as16(tOf(0)));
+                auto dOf = [&](s16x2 g, int k) -> s16x2 {
+                    if constexpr (LOC)
+                        return addSat(g, as16(tOf(k)));
+                    else if constexpr (DNA && !WIDE)
+                        return as16(asu(g) + tOf(k));   // t >= 0 and halves below 0x8000: no carry
+                    else
+                        return as16(uadd2(asu(g), tOf(k)));
+                };
+                s16x2 D = dOf(upGprev, 0);
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
-                    Ek[k] = vmax(addSat(Ek[k], e2), Gk[k]);
-                    const s16x2 F = vmax(addSat(uF, e2), uG);
-                    s16x2 H = vmax(vmax(D, Ek[k]), F);
-                    if constexpr (TRK & kTrackLocal) {
-                        H = vmax(H, splat(0));
-                    } else if constexpr (TOPFLOOR) {
-                        // 0 in the halves with k <= p (row k is row 0 or above it).
-                        const uint32_t atOrAbove = asu(subSat(splat(k), top1) >> splat(15));
-                        H = vmax(H, as16(~atOrAbove & 0x80008000u));
-                    }
-                    if (k + 1 < R)
-                        D = addSat(Gk[k], as16(tOf(k + 1)));
-                    const s16x2 Gn = addSat(H, o2);
-                    Gk[k] = Gn;
-                    if constexpr (TRK & kTrackLocal)
+                    s16x2 F, Gn;
+                    if constexpr (LOC) {
+                        Ek[k] = vmax(addSat(Ek[k], e2), Gk[k]);
+                        F = vmax(addSat(uF, e2), uG);
+                        const s16x2 H = vmax(vmax(vmax(D, Ek[k]), F), splat(0));
+                        if (k + 1 < R)
+                            D = dOf(Gk[k], k + 1);
+                        Gn = addSat(H, o2);
                         best = vmax(best, Gn);
+                    } else {
+                        uint32_t Ev = asu(Ek[k]);
+                        if constexpr (TOPFREE)
+                            Ev = uadd2(Ev, rowD[k]);
+                        Ev = umax2(Ev, asu(Gk[k]));
+                        const uint32_t Fv = umax2(asu(uF), asu(uG));
+                        const uint32_t H = WIDE ? umax2(umax2(asu(D), Ev), Fv) : max3Pos(asu(D), Ev, Fv);
+                        if (k + 1 < R)
+                            D = dOf(Gk[k], k + 1);
+                        Ek[k] = as16(Ev);
+                        F = as16(Fv);
+                        Gn = as16(WIDE ? usub2(H, cost2) : H - cost2);
+                    }
+                    Gk[k] = Gn;
                     uG = Gn;
                     uF = F;
                 }
                 upGprev = upG;
                 if (!last)
                     rb[j * 64] = make_uint2(asu(uG), asu(uF));
-                if constexpr (TRK & (kTrackEnd | kTrackBottom | kTrackRight)) {
-                    // 0xffff in the halves where j == n.
-                    auto eqMaskN = [&]() -> uint32_t {
-                        const s16x2 rem = nHalf - splat(j);
-                        return ((uint16_t)rem.x == 0 ? 0xffffu : 0u) | ((uint16_t)rem.y == 0 ? 0xffff0000u : 0u);
-                    };
-                    if constexpr (TRK & kTrackBottom) {
-                        if (last)
-                            best = vmax(best, as16(bfi(afterMask(), asu(neg2), asu(uG))));
-                    }
-                    if constexpr (TRK & kTrackEnd) {
-                        if (last)
-                            best = as16(bfi(eqMaskN(), asu(uG), asu(best)));
+                if constexpr (!LOC) {
+                    const s16x2 rem = nHalf - splat(j);   // n - j per half
+                    if constexpr (TRK & (kTrackEnd | kTrackBottom)) {
+                        if (last) {
+                            botM = (TRK & kTrackBottom) ? umax2(uadd2(botM, d2), asu(uG)) : asu(uG);
+                            if ((uint16_t)rem.x == 0)
+                                bestH.x = max(bestH.x, (int)(botM & 0xffffu) + base[0] - dr.d * j);
+                            if ((uint16_t)rem.y == 0)
+                                bestH.y = max(bestH.y, (int)(botM >> 16) + base[1] - dr.d * j);
+                        }
                     }
                     if constexpr (TRK & kTrackRight) {
-                        const uint32_t eq = eqMaskN();
-                        if (eq != 0) {
-                            s16x2 cm = Gk[0];
+                        // The maximum of the block's rows in column n, per
+                        // half: down the rows the running maximum gains drift
+                        // per row; rows above row 0 are left out.
+                        if ((uint16_t)rem.x == 0 || (uint16_t)rem.y == 0) {
+                            const int iTop[2] = {rowbase - c.p[0], rowbase - c.p[1]};
+                            uint32_t mx = asu(Gk[0]);
 #pragma unroll
-                            for (int k = 1; k < R; ++k)
-                                cm = vmax(cm, Gk[k]);
-                            best = vmax(best, as16(bfi(eq, asu(cm), asu(neg2))));
+                            for (int k = 1; k < R; ++k) {
+                                mx = uadd2(mx, d2);
+                                if constexpr (FIRST)
+                                    mx &= ~((iTop[0] + k - 1 < 0 ? 0xffffu : 0u) | (iTop[1] + k - 1 < 0 ? 0xffff0000u : 0u));
+                                mx = umax2(mx, asu(Gk[k]));
+                            }
+                            if ((uint16_t)rem.x == 0 && iTop[0] + R > 0)
+                                bestH.x = max(bestH.x, (int)(mx & 0xffffu) + dr.cost - dr.bias -
+                                                           dr.d * (iTop[0] + R - 1 + j));
+                            if ((uint16_t)rem.y == 0 && iTop[1] + R > 0)
+                                bestH.y = max(bestH.y, (int)(mx >> 16) + dr.cost - dr.bias -
+                                                           dr.d * (iTop[1] + R - 1 + j));
                         }
                     }
                 }
@@ -269,13 +308,20 @@ struct Lane16 {
     {
         __shared__ uint32_t sProf[16];
         __shared__ int16_t sT[33 * 33];
+        // Under drift t = s - o + drift for real codes, 0 for the padding code.
         if constexpr (DNA) {
-            if (threadIdx.x < 16)
-                sProf[threadIdx.x] = a.dnaProfile[threadIdx.x];
+            if (threadIdx.x < 16) {
+                uint32_t w = a.dnaProfile[threadIdx.x];
+                if (!LOC && (int)(threadIdx.x & 7) < a.alpha)
+                    w += (uint32_t)a.drift.d * (0x01010101u >> (32 - 8 * min(a.alpha, 4)));
+                sProf[threadIdx.x] = w;
+            }
         } else {
-            const int nT = (a.alpha + 1) * (a.alpha + 1);
-            for (int i = threadIdx.x; i < nT; i += blockDim.x)
-                sT[i] = a.tTable[i];
+            const int TW = a.alpha + 1;
+            for (int i = threadIdx.x; i < TW * TW; i += blockDim.x) {
+                const bool pad = i / TW == a.alpha || i % TW == a.alpha;
+                sT[i] = LOC ? a.tTable[i] : pad ? (int16_t)0 : (int16_t)(a.tTable[i] + a.drift.d);
+            }
         }
         __syncthreads();
 
@@ -313,21 +359,24 @@ struct Lane16 {
                 c.pid[x] = pid;
                 c.p[x] = w.nblocks * R - 1 - m;
             }
-            s16x2 best = (TRK & kTrackLocal) ? splat(a.gapOpen) : splat(kNeg16);
+            s16x2 best = splat(a.gapOpen);                  // local: G of the best cell
+            int2 bestH = make_int2(INT32_MIN, INT32_MIN);   // global modes: H
             const int nb = ok ? w.nblocks : 0;
             const bool topFree = !(TRK & kTrackLocal) && (a.mode & SQMI_FREE_TOP) != 0;
             if (nb > 0) {
                 if (topFree)
-                    block<true, true>(a, c, 0, w.maxN, nb == 1, rb, sProf, sT, best);
+                    block<true, true>(a, c, 0, w.maxN, nb == 1, rb, sProf, sT, best, bestH);
                 else
-                    block<true, false>(a, c, 0, w.maxN, nb == 1, rb, sProf, sT, best);
+                    block<true, false>(a, c, 0, w.maxN, nb == 1, rb, sProf, sT, best, bestH);
             }
             for (int b = 1; b < nb; ++b)
-                block<false, false>(a, c, b, w.maxN, b == nb - 1, rb, sProf, sT, best);
+                block<false, false>(a, c, b, w.maxN, b == nb - 1, rb, sProf, sT, best, bestH);
+            if constexpr (LOC)
+                bestH = make_int2((int)best.x - a.gapOpen, (int)best.y - a.gapOpen);
             if (c.pid[0] >= 0)
-                a.scores[c.pid[0]] = (int)best.x - a.gapOpen;
+                a.scores[c.pid[0]] = bestH.x;
             if (c.pid[1] >= 0)
-                a.scores[c.pid[1]] = (int)best.y - a.gapOpen;
+                a.scores[c.pid[1]] = bestH.y;
         }
     }
 };
@@ -345,16 +394,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(laneWaves<R
 }
 
 template <int R, bool DNA>
-const void *laneKernel(uint32_t track)
+const void *laneKernel(const Variant16 &v)
 {
-    switch (track) {
-        case kTrackEnd: return (const void *)&kLane16<R, DNA, kTrackEnd>;
-        case kTrackBottom: return (const void *)&kLane16<R, DNA, kTrackBottom>;
-        case kTrackRight: return (const void *)&kLane16<R, DNA, kTrackRight>;
-        case kTrackBottom | kTrackRight: return (const void *)&kLane16<R, DNA, kTrackBottom | kTrackRight>;
+#define SQMI_TRK(t)                                                                                        \
+    case t:                                                                                                \
+        return v.wide ? (const void *)&kLane16<R, DNA, (t) | kWideVals> : (const void *)&kLane16<R, DNA, (t)>;
+    switch (v.track) {
+        SQMI_TRK(kTrackEnd)
+        SQMI_TRK(kTrackBottom)
+        SQMI_TRK(kTrackRight)
+        SQMI_TRK(kTrackBottom | kTrackRight)
         case kTrackLocal: return (const void *)&kLane16<R, DNA, kTrackLocal>;
         default: return nullptr;
     }
+#undef SQMI_TRK
 }
 
 const void *laneKernelFor(const Variant16 &v)
@@ -362,9 +415,9 @@ const void *laneKernelFor(const Variant16 &v)
     if (v.G != 1)
         return nullptr;
     if (v.R == 16)
-        return v.dna ? laneKernel<16, true>(v.track) : laneKernel<16, false>(v.track);
+        return v.dna ? laneKernel<16, true>(v) : laneKernel<16, false>(v);
     if (v.R == 32)
-        return v.dna ? laneKernel<32, true>(v.track) : laneKernel<32, false>(v.track);
+        return v.dna ? laneKernel<32, true>(v) : laneKernel<32, false>(v);
     return nullptr;
 }
 

@@ -31,6 +31,28 @@ __device__ __forceinline__ s16x2 addSat(s16x2 a, s16x2 b) { return __builtin_ele
 // Saturating a - b per half: its sign bit is exactly (a < b), whatever the
 // magnitudes (v_pk_sub_i16 with clamp).
 __device__ __forceinline__ s16x2 subSat(s16x2 a, s16x2 b) { return __builtin_elementwise_sub_sat(a, b); }
+__device__ __forceinline__ uint32_t umax2(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t uadd2(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, a) + __builtin_bit_cast(u16x2, b));
+}
+__device__ __forceinline__ uint32_t usub2(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, a) - __builtin_bit_cast(u16x2, b));
+}
+// max(a, b, c) per half, for halves of at most 0x7bff: read as half floats
+// those are non-negative and finite (subnormals included, which the
+// instruction does not flush), and their order is the integers'.
+__device__ __forceinline__ uint32_t max3Pos(uint32_t a, uint32_t b, uint32_t c)
+{
+    uint32_t r;
+    asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 // 0xffff in the halves where a > b.
 __device__ __forceinline__ uint32_t gtMask(s16x2 a, s16x2 b) { return asu(subSat(b, a) >> splat(15)); }
 
