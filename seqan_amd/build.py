@@ -22,13 +22,13 @@ LIB = os.path.join(PKG, "libseqan_amd.so")
 ARCH = os.environ.get("SQMI_OFFLOAD_ARCH", "gfx950")
 
 # (source, object name, defines).  score16.hip is built once per DNA profile /
-# substitution table and kind, fwd16.hip per profile / table; the sources
+# substitution table and kind, trace16.hip per profile / table; the sources
 # compile in parallel, the longest first.
 SOURCES = [("score16.hip", f"score16_{t}_{k}", {"SQMI_SCORE_DNA": d, "SQMI_SCORE_KIND": f"kScore{k}",
                                                 "SQMI_SCORE_PART": f"score{t}{k}"})
            for d, t in ((0, "Tab"), (1, "Dna")) for k in ("Local", "Right", "Global")]
-SOURCES += [("fwd16.hip", "fwd16_dna", {"SQMI_FWD_DNA": 1, "SQMI_FWD_PART": "kFwdPartDna"}),
-            ("fwd16.hip", "fwd16_tab", {"SQMI_FWD_DNA": 0, "SQMI_FWD_PART": "kFwdPartTab"}),
+SOURCES += [("trace16.hip", "trace16_tab", {"SQMI_TRACE_DNA": 0, "SQMI_TRACE_PART": "traceTab"}),
+            ("trace16.hip", "trace16_dna", {"SQMI_TRACE_DNA": 1, "SQMI_TRACE_PART": "traceDna"}),
             ("kernels.hip", "kernels", {}), ("lane.hip", "lane", {}), ("band16.hip", "band16", {}),
             ("long.hip", "long", {}), ("banded.hip", "banded", {}), ("scratch.hip", "scratch", {}),
             ("engine.cpp", "engine", {}), ("scoring.cpp", "scoring", {}), ("workload.cpp", "workload", {})]

@@ -52,7 +52,7 @@ struct Buffers
     DevBuf hRes, vRes, hOff, vOff, order, items, queue, rowbuf, strips, scores, tTable, dnaProf, ids32, scratchOff32,
         scratch32, table32, emptyIds;
     // Traceback (sqmi_align_counts).
-    DevBuf trace, traceOff, locs, endEF, endIJ, counts;
+    DevBuf trace, traceOff, locs, ends, endOff, endEF, endIJ, counts;
     // Long pairs (tiled int32 kernels).
     DevBuf longCk, longPairs, longWalk, longTrace, longBest, longSched;
     // Alignment rows (sqmi_align_rows, sqmi_align_local_rows).
@@ -64,7 +64,7 @@ struct Buffers
     void forEach(F f)
     {
         for (DevBuf *b : {&hRes, &vRes, &hOff, &vOff, &order, &items, &queue, &rowbuf, &strips, &scores, &tTable, &dnaProf,
-                          &ids32, &scratchOff32, &scratch32, &table32, &emptyIds, &trace, &traceOff, &locs, &endEF,
+                          &ids32, &scratchOff32, &scratch32, &table32, &emptyIds, &trace, &traceOff, &locs, &ends, &endOff, &endEF,
                           &endIJ, &counts, &longCk, &longPairs, &longWalk, &longTrace, &longBest, &longSched, &ops, &opOff, &opLen,
                           &begins, &opsPacked, &opStart, &bandIds, &bandScratch})
             f(*b);
@@ -774,7 +774,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
     si.dna = si.alpha <= 4 && si.sMin - si.o >= 0 && si.sMax - si.o <= 255;
     si.dnaDrift = si.dna && si.sMax - si.o - std::max(si.o, si.e) <= 255;
     P.drift = driftOf(si, local);
-    P.dna16 = local || traceShape ? si.dna : si.dnaDrift;
+    P.dna16 = local ? si.dna : si.dnaDrift;
     const Drift dr = P.drift;
     const bool dna16 = P.dna16;
     uint32_t track;
@@ -816,7 +816,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
     int binG[16] = {};              // forced group size of a bin, or 0 (the rule)
     double cells64 = 0, cellsStrip = 0;
     if (traceShape) {
-        shapes.push_back(Variant16{kTraceLanes, kTraceRows / kTraceLanes, si.dna, track});
+        shapes.push_back(Variant16{kTraceLanes, kTraceRows / kTraceLanes, dna16, track});
     } else {
         for (int w = 1; w >= 0; --w)
             shapes.push_back(Variant16{64, 16, dna16, track, w != 0});
@@ -2118,36 +2118,89 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
     const int A = si.alpha, S = A * A + 2;
     const int64_t budget = traceBudget(ctx);
 
-    // Host-side chunking of the int16 items and of the int32 pairs.
+    // Host-side chunking of the int16 items and of the int32 pairs.  An
+    // item's blocks become strips when a wave would take more than a quarter
+    // of the chunk's time for it (3,072 resident waves), as in the score
+    // calls; SQMI_COOP_MIN_BLOCKS as there.
     const Plan16 *pl = P.plans.empty() ? nullptr : &P.plans[0];
-    std::vector<int64_t> itemOff;           // per item: first record within its chunk (units of 64 records)
-    std::vector<size_t> chunkEnd;           // item index after each chunk
-    std::vector<TraceLoc> locs;             // per pair in plan order
-    int64_t traceRecs = 0;                  // largest chunk, in units of 64 records
+    std::vector<int64_t> itemOff, endOff;   // per item: first record within its chunk (steps), first end candidate
+    std::vector<size_t> chunkEnd, chunkUnits;   // item and unit index after each chunk
+    RawVec<TraceLoc> locs;                  // per pair in plan order
+    int64_t traceRecs = 0;                  // largest chunk, in steps
+    int64_t slotWords = 1, stripWords = 0, nEnds = 0;
+    std::vector<int64_t> chunkStrips;       // strip words of each chunk
     if (pl) {
+        const size_t nIt = pl->items.size();
         const int64_t recBytes = 64 * 16;
-        itemOff.resize(pl->items.size());
+        itemOff.resize(nIt);
+        endOff.resize(nIt);
         locs.resize(pl->order.size());
+        std::vector<uint8_t> wide(nIt);
         int64_t run = 0;
-        for (size_t k = 0; k < pl->items.size(); ++k) {
+        for (size_t k = 0; k < nIt; ++k) {
             const WorkItem &w = pl->items[k];
-            const int steps = traceSteps(w.maxN);
-            const int64_t recs = (int64_t)w.nblocks * steps;
+            const int64_t recs = (int64_t)w.nblocks * traceSteps(w.maxN);
             if (run > 0 && (run + recs) * recBytes > budget) {
                 chunkEnd.push_back(k);
                 run = 0;
             }
             itemOff[k] = run;
-            for (int x = 0; x < w.count; ++x) {
-                const int32_t pid = pl->order[w.first + x];
-                const int64_t m = setV->offsets[pid + 1] - setV->offsets[pid];
-                locs[w.first + x] = TraceLoc{run, steps, (int32_t)((int64_t)w.nblocks * kTraceRows - 1 - m),
-                                             (x / 2) * kTraceLanes, x % 2};
-            }
             run += recs;
             traceRecs = std::max(traceRecs, run);
         }
-        chunkEnd.push_back(pl->items.size());
+        chunkEnd.push_back(nIt);
+#pragma omp parallel for schedule(static) if (N > kParallelMin)
+        for (int64_t k = 0; k < (int64_t)nIt; ++k) {
+            const WorkItem &w = pl->items[k];
+            bool any = false;
+            for (int x = 0; x < w.count; ++x) {
+                const int32_t pid = pl->order[w.first + x];
+                any |= !driftNarrow(si, P.drift, P.local, setH->offsets[pid + 1] - setH->offsets[pid],
+                                    setV->offsets[pid + 1] - setV->offsets[pid]);
+            }
+            wide[k] = any;
+        }
+        const int minBlocks = stripMinBlocks();
+        P.units.clear();
+        for (size_t c = 0, b = 0; c < chunkEnd.size(); b = chunkEnd[c], ++c) {
+            int64_t total = 0, off = 0;
+            for (size_t k = b; k < chunkEnd[c]; ++k)
+                total += (int64_t)pl->items[k].nblocks * traceSteps(pl->items[k].maxN);
+            for (size_t k = b; k < chunkEnd[c]; ++k) {
+                const WorkItem &w = pl->items[k];
+                const bool strips = w.nblocks > 1 &&
+                                    (minBlocks < 0 ? (int64_t)w.nblocks * traceSteps(w.maxN) * 4 * kResidentWaves > total
+                                                   : minBlocks > 0 && w.nblocks >= minBlocks);
+                ScoreUnit u{w.first, w.count, w.maxN, w.nblocks, 16 | 16 << 8, wide[k] ? kUnitWide : 0, -1,
+                            (int32_t)(k - b), 0};
+                endOff[k] = nEnds;
+                nEnds += (int64_t)w.count * (strips ? w.nblocks : 1);
+                if (strips) {
+                    u.rowOff = off;
+                    off += (int64_t)4 * (w.maxN + 1) * w.nblocks;
+                    for (u.block = 0; u.block < w.nblocks; ++u.block)
+                        P.units.push_back(u);
+                } else {
+                    slotWords = std::max<int64_t>(slotWords, (int64_t)4 * (w.maxN + 1));
+                    P.units.push_back(u);
+                }
+                wide[k] = strips;   // from here on: whether the item has strips
+            }
+            chunkUnits.push_back(P.units.size());
+            chunkStrips.push_back(off);
+            stripWords = std::max(stripWords, off);
+        }
+#pragma omp parallel for schedule(static) if (N > kParallelMin)
+        for (int64_t k = 0; k < (int64_t)nIt; ++k) {
+            const WorkItem &w = pl->items[k];
+            for (int x = 0; x < w.count; ++x) {
+                const int32_t pid = pl->order[w.first + x];
+                const int64_t m = setV->offsets[pid + 1] - setV->offsets[pid];
+                locs[w.first + x] = TraceLoc{itemOff[k], traceSteps(w.maxN),
+                                             (int32_t)((int64_t)w.nblocks * kTraceRows - 1 - m),
+                                             (x / 2) * kTraceLanes, x % 2, endOff[k] + x, w.count, wide[k] ? w.nblocks : 1};
+            }
+        }
     }
     std::vector<size_t> chunk32End;         // int32 pairs per chunk
     std::vector<int64_t> off32(P.ids32.size());
@@ -2222,63 +2275,66 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
     if (pl) {
         const size_t nIt = pl->items.size(), np = pl->order.size();
         const int wpb = wavesPerBlock16();
-        const int occ = occupancyTrace16(si.dna);
-        const int rowCols = pl->maxN + kTraceLanes + 2;
-        int64_t maxChunkItems = 0;
-        for (size_t c = 0, b = 0; c < chunkEnd.size(); b = chunkEnd[c], ++c)
-            maxChunkItems = std::max<int64_t>(maxChunkItems, (int64_t)(chunkEnd[c] - b));
-        const int grid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occ, (maxChunkItems + wpb - 1) / wpb));
-        const size_t rbBytes = (size_t)grid * wpb * (64 / kTraceLanes) * rowCols * 2 * sizeof(uint32_t);
+        size_t maxUnits = 0;
+        for (size_t c = 0, b = 0; c < chunkUnits.size(); b = chunkUnits[c], ++c)
+            maxUnits = std::max(maxUnits, chunkUnits[c] - b);
+        const int grid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occupancyTrace16(P.dna16, P.track),
+                                                            ((int64_t)maxUnits + wpb - 1) / wpb));
         if ((err = ensure(ctx->b.order, 4 * np)) != hipSuccess ||
-            (err = ensure(ctx->b.items, sizeof(WorkItem) * nIt)) != hipSuccess ||
-            (err = ensure(ctx->b.traceOff, 8 * nIt)) != hipSuccess ||
+            (err = ensure(ctx->b.items, sizeof(ScoreUnit) * P.units.size())) != hipSuccess ||
+            (err = ensure(ctx->b.traceOff, 8 * nIt)) != hipSuccess || (err = ensure(ctx->b.endOff, 8 * nIt)) != hipSuccess ||
             (err = ensure(ctx->b.locs, sizeof(TraceLoc) * np)) != hipSuccess ||
             (err = ensure(ctx->b.queue, 4 * chunkEnd.size() + 64)) != hipSuccess ||
-            (err = ensure(ctx->b.rowbuf, rbBytes)) != hipSuccess ||
-            (err = ensure(ctx->b.endEF, (size_t)8 * N)) != hipSuccess ||
-            (P.track != kTrackEnd && (err = ensure(ctx->b.endIJ, (size_t)8 * N)) != hipSuccess) ||
+            (err = ensure(ctx->b.rowbuf, (size_t)grid * wpb * slotWords * 8)) != hipSuccess ||
+            (err = ensure(ctx->b.strips, (size_t)stripWords * 8)) != hipSuccess ||
+            (err = ensure(ctx->b.ends, sizeof(TraceEnd) * (size_t)nEnds)) != hipSuccess ||
             (err = ensure(ctx->b.trace, (size_t)traceRecs * 64 * 16)) != hipSuccess)
             return hipFail(ctx, err, "allocating traceback buffers");
-        int32_t *dEndIJ = P.track != kTrackEnd ? static_cast<int32_t *>(ctx->b.endIJ.p) : nullptr;
         if ((err = hipMemcpyAsync(ctx->b.order.p, pl->order.data(), 4 * np, hipMemcpyHostToDevice, stream)) !=
                 hipSuccess ||
-            (err = hipMemcpyAsync(ctx->b.items.p, pl->items.data(), sizeof(WorkItem) * nIt, hipMemcpyHostToDevice,
-                                  stream)) != hipSuccess ||
+            (err = hipMemcpyAsync(ctx->b.items.p, P.units.data(), sizeof(ScoreUnit) * P.units.size(),
+                                  hipMemcpyHostToDevice, stream)) != hipSuccess ||
             (err = hipMemcpyAsync(ctx->b.traceOff.p, itemOff.data(), 8 * nIt, hipMemcpyHostToDevice, stream)) !=
+                hipSuccess ||
+            (err = hipMemcpyAsync(ctx->b.endOff.p, endOff.data(), 8 * nIt, hipMemcpyHostToDevice, stream)) !=
                 hipSuccess ||
             (err = hipMemcpyAsync(ctx->b.locs.p, locs.data(), sizeof(TraceLoc) * np, hipMemcpyHostToDevice, stream)) !=
                 hipSuccess ||
             (err = hipMemsetAsync(ctx->b.queue.p, 0, 4 * chunkEnd.size() + 64, stream)) != hipSuccess)
             return hipFail(ctx, err, "uploading traceback work lists");
-        const WorkItem *dItems = static_cast<const WorkItem *>(ctx->b.items.p);
         const int32_t *dOrder = static_cast<const int32_t *>(ctx->b.order.p);
-        size_t b = 0;
+        size_t b = 0, ub = 0;
         for (size_t c = 0; c < chunkEnd.size(); ++c) {
-            const size_t e = chunkEnd[c];
-            FwdArgs a{};
+            const size_t e = chunkEnd[c], ue = chunkUnits[c];
+            TraceArgs a{};
             a.hRes = in.dH;
             a.vRes = in.dV;
             a.hOff = static_cast<const int64_t *>(ctx->b.hOff.p);
             a.vOff = static_cast<const int64_t *>(ctx->b.vOff.p);
             a.order = dOrder;
-            a.items = dItems + b;
-            a.nItems = (int32_t)(e - b);
+            a.units = static_cast<const ScoreUnit *>(ctx->b.items.p) + ub;
+            a.nUnits = (int32_t)(ue - ub);
             a.queue = static_cast<uint32_t *>(ctx->b.queue.p) + c;
-            a.rowbuf = static_cast<uint32_t *>(ctx->b.rowbuf.p);
-            a.rowCols = rowCols;
-            a.scores = in.dScores;
-            a.gapOpen = si.o;
-            a.gapExtend = si.e;
+            a.rowbuf = static_cast<uint64_t *>(ctx->b.rowbuf.p);
+            a.slotWords = slotWords;
+            a.strips = static_cast<uint64_t *>(ctx->b.strips.p);
+            a.stripWords = chunkStrips[c];
+            a.error = ctx->waitFlag;
             a.mode = mode;
             a.alpha = A;
             a.tTable = static_cast<const int16_t *>(ctx->b.tTable.p);
             a.dnaProfile = static_cast<const uint32_t *>(ctx->b.dnaProf.p);
+            a.drift = P.drift;
             a.trace = static_cast<uint4 *>(ctx->b.trace.p);
+            a.traceRecs = traceRecs;
             a.traceOff = static_cast<const int64_t *>(ctx->b.traceOff.p) + b;
-            a.endEF = static_cast<int32_t *>(ctx->b.endEF.p);
-            a.endIJ = dEndIJ;
-            const int cg = std::max(1, std::min(grid, (int)((e - b + wpb - 1) / wpb)));
-            if ((err = launchFwdTrace16(si.dna, P.track, a, cg, stream)) != hipSuccess)
+            a.ends = static_cast<TraceEnd *>(ctx->b.ends.p);
+            a.endOff = static_cast<const int64_t *>(ctx->b.endOff.p) + b;
+            if (chunkStrips[c] > 0 && (err = launchZero32(static_cast<uint32_t *>(ctx->b.strips.p),
+                                                          2 * (size_t)chunkStrips[c], stream)) != hipSuccess)
+                return hipFail(ctx, err, "launching fill kernel");
+            const int cg = std::max(1, std::min(grid, (int)((ue - ub + wpb - 1) / wpb)));
+            if ((err = launchTrace16(P.dna16, P.track, a, cg, stream)) != hipSuccess)
                 return hipFail(ctx, err, "launching trace kernel");
             const int32_t p0 = pl->items[b].first;
             const int32_t p1 = pl->items[e - 1].first + pl->items[e - 1].count;
@@ -2291,12 +2347,11 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
             wa.locs = static_cast<const TraceLoc *>(ctx->b.locs.p) + p0;
             wa.nPairs = p1 - p0;
             wa.trace = a.trace;
+            wa.ends = a.ends;
             wa.scores = in.dScores;
-            wa.endEF = a.endEF;
             wa.counts = dCounts;
             wa.alpha = A;
             wa.linear = si.o == si.e;
-            wa.endIJ = dEndIJ;
             wa.local = P.local ? 1 : 0;
             wa.table = static_cast<const int32_t *>(ctx->b.table32.p);
             wa.gapOpen = si.o;
@@ -2308,6 +2363,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
             if ((err = launchWalk16(wa, stream)) != hipSuccess)
                 return hipFail(ctx, err, "launching walk kernel");
             b = e;
+            ub = ue;
         }
     }
     // Banded pairs whose band, clipped to the matrix, has at most 64
@@ -2508,7 +2564,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
     }
     if ((err = hipStreamSynchronize(stream)) != hipSuccess)
         return hipFail(ctx, err, "traceback kernels");
-    if ((st = longStreamCheck(ctx)) != SQMI_OK)
+    if ((st = longStreamCheck(ctx)) != SQMI_OK || (st = stripCheck(ctx)) != SQMI_OK)
         return st;
     float ms = 0;
     if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess)

@@ -1,11 +1,10 @@
 // kernels.hip -- gfx950 kernels of the batched affine-gap alignment engine
-// other than the packed forward (fwd16.hpp): the int32 per-pair sweep, the
+// other than the packed kernels (score16.hpp, trace16.hpp): the int32 per-pair sweep, the
 // traceback walks and count kernels, the fills; and the dispatch to the
-// packed kernels' instantiation units (score16.hip, fwd16.hip).
+// packed kernels' instantiation units (score16.hip, trace16.hip).
 #include <algorithm>
 #include <type_traits>
 
-#include "fwd16_parts.hpp"
 #include "kernels.hpp"
 #include "packed16.hpp"
 #include "score16_parts.hpp"
@@ -317,25 +316,160 @@ __device__ __forceinline__ void walkCounts(int n, int m, const uint8_t *h, const
         *opLen = nOps;
 }
 
-// Trace bits of cell (i, j) of one pair from the packed records of
-// kFwdTrace16, with the last record read kept (moves up inside a lane reuse
-// it).  The walk is latency-bound (each move depends on the last record
-// read); plain per-move reads measured faster than prefetching a lane's next
-// records, batching the residue loads or a branch-free move loop.
+// The same walk by a group of 16 lanes per pair: the lanes read the bits of
+// the next 16 cells of the diagonal (or of the gap) at once, so a walk waits
+// for memory once per run of equal moves (or per 16 of them) instead of once
+// per move.  What bounds it then is the records' traffic: each cell's record
+// sits in a line of its own (65,536 pairs of 1 kbp 1.85 -> 1.47 ms; 8,191
+// uneven pairs of up to 10 kbp, where the longest walk counts, 13.8 -> 1.2 ms;
+// 8,192 protein pairs local 1.24 -> 0.12 ms; 65,536 banded pairs of 150 bp
+// 0.67 -> 0.17 ms).  The state is kept alike in all lanes of the group;
+// groups of a wave diverge as they like (a group's lanes never do, outside
+// predicated statements).
+constexpr int kWalkLanes = 16;
+
+__device__ __forceinline__ uint32_t groupBallot(bool p)
+{
+    return (uint32_t)(__ballot(p) >> (threadIdx.x & 48)) & 0xffffu;
+}
+
+struct WalkEnd {
+    int score, i, j, e, f;   // the end cell
+};
+
+template <class Bits>
+__device__ __forceinline__ void walkGroup(int n, int m, const uint8_t *h, const uint8_t *v, int A, const WalkEnd &end,
+                                          const Bits &bits, int32_t *cnt, uint8_t *opEnd, int64_t *opLen, bool local,
+                                          int64_t *begins, bool linear, bool alwaysOpen, const int32_t *lTab, int go,
+                                          int ge)
+{
+    const int t = threadIdx.x & (kWalkLanes - 1);
+    int cur = end.score, i = end.i, j = end.j;
+    if (local) {
+        m = i;
+        n = j;
+    }
+    int prev = 0, opens = 0, exts = 0;
+    int64_t nOps = 0;
+    // A run of k equal moves: 0 aligned pairs, 1 gap in H ('V'), 2 gap in V.
+    auto emit = [&](int kind, int k) {
+        if (kind > 0 && k > 0) {
+            opens += prev == kind ? 0 : 1;
+            exts += prev == kind ? k : k - 1;
+        }
+        if (k > 0)
+            prev = kind;
+        if (opEnd)
+            for (int q = t; q < k; q += kWalkLanes)
+                opEnd[-1 - nOps - q] = kind == 0 ? 'M' : kind == 1 ? 'V' : 'H';
+        nOps += k;
+    };
+    emit(1, m - i);   // trailing gaps after the end cell
+    emit(2, n - j);
+    bool walk = i > 0 && j > 0, first = true;
+    int known = -1;   // direction of (i, j) by the end-cell rule
+    if (walk) {
+        const uint32_t b0 = bits(i, j);
+        known = linear ? dirOf(b0) : end.f == end.score ? 1 : end.e == end.score ? 2 : dirOf(b0);
+        if (local && (lTab ? cur <= 0 : (b0 & kBitStop) != 0))
+            walk = false;
+    }
+    while (walk) {
+        // Aligned pairs from (i, j) up the diagonal.
+        const int ii = i - t, jj = j - t;
+        const bool valid = ii > 0 && jj > 0;
+        const uint32_t b = valid ? bits(ii, jj) : 0;
+        int d = valid ? dirOf(b) : 3;
+        if (t == 0 && first)
+            d = known;
+        const bool none = local && !lTab && (b & kBitStop) != 0 && !(first && t == 0);
+        const uint32_t end16 = groupBallot(d != 0 || none);
+        int r = end16 ? __builtin_ctz(end16) : kWalkLanes;
+        bool stopped = false;
+        int hv = 0;
+        if (t < r)
+            hv = min((int)h[jj - 1], A - 1) * A + min((int)v[ii - 1], A - 1);
+        if (lTab) {
+            // H along the run; the walk stops on the first cell where it is 0.
+            int sum = t < r ? lTab[hv] : 0;
+#pragma unroll
+            for (int q = 1; q < kWalkLanes; q <<= 1) {
+                const int o = __shfl_up(sum, q, kWalkLanes);
+                sum += t >= q ? o : 0;
+            }
+            const uint32_t zero = groupBallot(t < r && cur == sum && ii > 1 && jj > 1);
+            if (zero) {
+                r = __builtin_ctz(zero) + 1;
+                stopped = true;
+            }
+            if (r > 0)
+                cur -= __shfl(sum, r - 1, kWalkLanes);
+        }
+        if (t < r)
+            atomicAdd(cnt + hv, 1);
+        emit(0, r);
+        i -= r;
+        j -= r;
+        if (stopped || i <= 0 || j <= 0)
+            break;
+        if (r == kWalkLanes) {
+            first = false;
+            continue;
+        }
+        if (__shfl((int)none, r, kWalkLanes))
+            break;
+        const bool vert = __shfl(d, r, kWalkLanes) == 1;
+        first = false;
+        // A gap: up to the cell that opened it, or row / column 1.
+        for (;;) {
+            const int gi = vert ? i - t : i, gj = vert ? j : j - t, at = vert ? gi : gj;
+            const uint32_t gb = at > 0 ? bits(gi, gj) : 0;
+            const bool open = alwaysOpen || (gb & (vert ? kBitFOpen : kBitEOpen)) != 0;
+            const uint32_t gEnd = groupBallot(at > 0 && (linear || open || at == 1));
+            const int g = gEnd ? __builtin_ctz(gEnd) + 1 : kWalkLanes;
+            const bool opened = linear || __shfl((int)open, g - 1, kWalkLanes) != 0;
+            emit(vert ? 1 : 2, g);
+            cur -= ge * (g - 1) + (gEnd && opened ? go : ge);
+            if (vert)
+                i -= g;
+            else
+                j -= g;
+            if (gEnd)
+                break;
+        }
+        if (i <= 0 || j <= 0 || (lTab && cur == 0))
+            break;
+    }
+    if (local) {
+        // The window starts where the walk stopped (dp_traceback_adaptor.h:
+        // 87-93); an empty window keeps both begins at 0.
+        if (begins && nOps > 0 && t == 0) {
+            begins[0] = j;
+            begins[1] = i;
+        }
+        i = j = 0;
+    }
+    // Leading gaps down to the origin: first the column, then the row
+    // (dp_traceback_impl.h:522-545).
+    emit(1, i);
+    emit(2, j);
+    if (t == 0) {
+        atomicAdd(cnt + A * A, opens);
+        atomicAdd(cnt + A * A + 1, exts);
+        if (opLen)
+            *opLen = nOps;
+    }
+}
+
+// Trace bits of cell (i, j) of one pair from the packed records of kTrace16.
 struct Bits16 {
     const uint4 *trace;
     TraceLoc loc;
-    int64_t key = -1;
-    uint4 w = make_uint4(0, 0, 0, 0);
-    __device__ __forceinline__ uint32_t operator()(int i, int j)
+    __device__ __forceinline__ uint32_t operator()(int i, int j) const
     {
         const int r = loc.p + i;
         const int b = r / kTraceRows, rr = r % kTraceRows, l = rr / 16, k = rr % 16;
-        const int64_t idx = (loc.rec0 + (int64_t)b * loc.steps + (j + l)) * 64 + loc.lane0 + l;
-        if (idx != key) {
-            w = trace[idx];
-            key = idx;
-        }
+        const uint4 w = trace[(loc.rec0 + (int64_t)b * loc.steps + (j + l)) * 64 + loc.lane0 + l];
         const uint32_t ef = k < 8 ? w.x : w.y, dx = k < 8 ? w.z : w.w;
         const int sh = (k & 7) + 8 * loc.half;
         return ((ef >> sh) & 1u) | (((ef >> (sh + 16)) & 1u) << 1) | (((dx >> sh) & 1u) << 2) |
@@ -363,58 +497,95 @@ struct BandBits {
     }
 };
 
-__global__ __launch_bounds__(64) void kBandedWalk(BandedWalkArgs a)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.nIds)
-        return;
-    const int pid = a.ids[t];
-    const int A = a.alpha, S = A * A + 2;
-    const int64_t ho = a.hOff[pid], vo = a.vOff[pid];
-    const int n = (int)(a.hOff[pid + 1] - ho), m = (int)(a.vOff[pid + 1] - vo);
-    int32_t *cnt = a.counts + (int64_t)pid * S;
-    const int lo = (int)(a.lower > -(int64_t)m ? a.lower : -(int64_t)m);   // the band clipped to the matrix
-    const int up = (int)(a.upper < (int64_t)n ? a.upper : (int64_t)n);
-    BandBits bits{a.trace + a.traceOff[t], a.segLanes, lo, min(up - lo + 1, a.segLanes), n};
-    walkCounts(n, m, a.hRes + ho, a.vRes + vo, A, a.scores[pid], a.endEF[2 * pid], a.endEF[2 * pid + 1], bits, cnt,
-               a.ops ? a.ops + a.opOff[pid + 1] : nullptr, a.ops ? a.opLen + pid : nullptr, a.endIJ[2 * pid],
-               a.endIJ[2 * pid + 1], a.local != 0, a.begins ? a.begins + 2 * pid : nullptr, a.linear != 0);
-}
+// Threads of a walk workgroup: counts accumulate in LDS (alpha^2 + 2 words per
+// pair, at most 1,026), so large alphabets take fewer pairs per workgroup.
+int walkThreads(int alpha) { return alpha <= 7 ? 256 : 64; }
 
-constexpr int kWalkThreads = 64;
-// Counts live in LDS while walking when alpha^2 + 2 <= kWalkLdsStride.
-constexpr int kWalkLdsStride = 51;
-
-// One thread per pair.  LDS: counts accumulate in LDS, else in the output
-// row itself (two kernels rather than one pointer of unknown address space).
-template <bool LDS>
-__global__ __launch_bounds__(kWalkThreads) void kWalk16(WalkArgs a)
+__global__ __launch_bounds__(256) void kBandedWalk(BandedWalkArgs a)
 {
     extern __shared__ int32_t sCnt[];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.nPairs)
-        return;
-    const int pid = a.ids[t];
     const int A = a.alpha, S = A * A + 2;
-    const int64_t ho = a.hOff[pid], vo = a.vOff[pid];
-    const int n = (int)(a.hOff[pid + 1] - ho), m = (int)(a.vOff[pid + 1] - vo);
-    int32_t *out = a.counts + (int64_t)pid * S;
-    int32_t *cnt;
-    if constexpr (LDS)
-        cnt = sCnt + threadIdx.x * S;
-    else
-        cnt = out;
-    for (int q = 0; q < S; ++q)
-        cnt[q] = 0;
-    Bits16 bits{a.trace, a.locs[t]};
-    walkCounts(n, m, a.hRes + ho, a.vRes + vo, A, a.scores[pid], a.endEF[2 * pid], a.endEF[2 * pid + 1], bits, cnt,
-               a.ops ? a.ops + a.opOff[pid + 1] : nullptr, a.ops ? a.opLen + pid : nullptr,
-               a.endIJ ? a.endIJ[2 * pid] : -1, a.endIJ ? a.endIJ[2 * pid + 1] : -1, a.local != 0,
-               a.begins ? a.begins + 2 * pid : nullptr, a.linear != 0, a.local ? a.table : nullptr, a.gapOpen,
-               a.gapExtend);
-    if constexpr (LDS)
-        for (int q = 0; q < S; ++q)
-            out[q] = cnt[q];
+    const int t = threadIdx.x & (kWalkLanes - 1), q = threadIdx.x / kWalkLanes;
+    const int id = blockIdx.x * (blockDim.x / kWalkLanes) + q;
+    int32_t *cnt = sCnt + q * S;
+    for (int k = t; k < S; k += kWalkLanes)
+        cnt[k] = 0;
+    __syncthreads();
+    if (id < a.nIds) {
+        const int pid = a.ids[id];
+        const int64_t ho = a.hOff[pid], vo = a.vOff[pid];
+        const int n = (int)(a.hOff[pid + 1] - ho), m = (int)(a.vOff[pid + 1] - vo);
+        const int lo = (int)(a.lower > -(int64_t)m ? a.lower : -(int64_t)m);   // the band clipped to the matrix
+        const int up = (int)(a.upper < (int64_t)n ? a.upper : (int64_t)n);
+        const BandBits bits{a.trace + a.traceOff[id], a.segLanes, lo, min(up - lo + 1, a.segLanes), n};
+        const WalkEnd end{a.scores[pid], a.endIJ[2 * pid], a.endIJ[2 * pid + 1], a.endEF[2 * pid], a.endEF[2 * pid + 1]};
+        walkGroup(n, m, a.hRes + ho, a.vRes + vo, A, end, bits, cnt, a.ops ? a.ops + a.opOff[pid + 1] : nullptr,
+                  a.ops ? a.opLen + pid : nullptr, a.local != 0, a.begins ? a.begins + 2 * pid : nullptr,
+                  a.linear != 0, false, nullptr, 0, 0);
+    }
+    __syncthreads();
+    if (id < a.nIds) {
+        int32_t *out = a.counts + (int64_t)a.ids[id] * S;
+        for (int k = t; k < S; k += kWalkLanes)
+            out[k] = cnt[k];
+    }
+}
+
+__global__ __launch_bounds__(256) void kWalk16(WalkArgs a)
+{
+    extern __shared__ int32_t sCnt[];
+    const int A = a.alpha, S = A * A + 2;
+    const int t = threadIdx.x & (kWalkLanes - 1), q = threadIdx.x / kWalkLanes;
+    const int id = blockIdx.x * (blockDim.x / kWalkLanes) + q;
+    int32_t *cnt = sCnt + q * S;
+    for (int k = t; k < S; k += kWalkLanes)
+        cnt[k] = 0;
+    __syncthreads();
+    if (id < a.nPairs) {
+        const int pid = a.ids[id];
+        const TraceLoc loc = a.locs[id];
+        const int64_t ho = a.hOff[pid], vo = a.vOff[pid];
+        const int n = (int)(a.hOff[pid + 1] - ho), m = (int)(a.vOff[pid + 1] - vo);
+        // The end cell.  Local: the candidates' first strict maximum in
+        // column order.  Global: the last unit's bottom-row candidate, unless
+        // a cell of column n beats it (rows ascend with the units).
+        WalkEnd end{INT32_MIN, 0x7fffffff, 0x7fffffff, INT32_MIN, INT32_MIN};
+        for (int k = t; k < loc.nEnds; k += kWalkLanes) {
+            const TraceEnd c = a.ends[loc.end0 + (int64_t)k * loc.endStride];
+            const bool take = a.local ? c.v > end.score || (c.v == end.score && (c.j < end.j || (c.j == end.j && c.i < end.i)))
+                                      : c.rv > end.score || (c.rv == end.score && c.ri < end.i);
+            if (take)
+                end = a.local ? WalkEnd{c.v, c.i, c.j, c.e, c.f} : WalkEnd{c.rv, c.ri, c.rj, c.re, c.rf};
+        }
+#pragma unroll
+        for (int d = 1; d < kWalkLanes; d <<= 1) {
+            const WalkEnd o{__shfl_xor(end.score, d, kWalkLanes), __shfl_xor(end.i, d, kWalkLanes),
+                            __shfl_xor(end.j, d, kWalkLanes), __shfl_xor(end.e, d, kWalkLanes),
+                            __shfl_xor(end.f, d, kWalkLanes)};
+            if (o.score > end.score || (o.score == end.score && (o.j < end.j || (o.j == end.j && o.i < end.i))))
+                end = o;
+        }
+        if (a.local) {
+            if (end.j == 0x7fffffff)   // no cell above 0: an empty window
+                end = WalkEnd{0, 0, 0, INT32_MIN, INT32_MIN};
+        } else {
+            const TraceEnd c = a.ends[loc.end0 + (int64_t)(loc.nEnds - 1) * loc.endStride];
+            if (c.v != INT32_MIN && c.v >= end.score)
+                end = WalkEnd{c.v, c.i, c.j, c.e, c.f};
+        }
+        if (t == 0)
+            a.scores[pid] = end.score;
+        const Bits16 bits{a.trace, loc};
+        walkGroup(n, m, a.hRes + ho, a.vRes + vo, A, end, bits, cnt, a.ops ? a.ops + a.opOff[pid + 1] : nullptr,
+                  a.ops ? a.opLen + pid : nullptr, a.local != 0, a.begins ? a.begins + 2 * pid : nullptr,
+                  a.linear != 0, a.gapExtend < a.gapOpen, a.local ? a.table : nullptr, a.gapOpen, a.gapExtend);
+    }
+    __syncthreads();
+    if (id < a.nPairs) {
+        int32_t *out = a.counts + (int64_t)a.ids[id] * S;
+        for (int k = t; k < S; k += kWalkLanes)
+            out[k] = cnt[k];
+    }
 }
 
 // int32 forward with trace bytes (same encoding), column-major with column
@@ -592,18 +763,21 @@ hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBloc
     return hipLaunchKernel(k, dim3(gridBlocks), dim3(threadsPerBlock), params, 0, stream);
 }
 
-int traceSteps(int maxN) { return kFwdPartDna.traceSteps(maxN); }
-
-hipError_t launchFwdTrace16(bool dna, uint32_t track, const FwdArgs &args, int gridBlocks, hipStream_t stream)
+hipError_t launchTrace16(bool dna, uint32_t track, const TraceArgs &args, int gridBlocks, hipStream_t stream)
 {
-    return (dna ? kFwdPartDna : kFwdPartTab).launchTrace(track, args, gridBlocks, stream);
+    const void *k = dna ? traceDna(track) : traceTab(track);
+    if (!k)
+        return hipErrorInvalidValue;
+    TraceArgs copy = args;
+    void *params[] = {&copy};
+    return hipLaunchKernel(k, dim3(gridBlocks), dim3(256), params, 0, stream);
 }
 
-int occupancyTrace16(bool dna)
+int occupancyTrace16(bool dna, uint32_t track)
 {
     int blocks = 0;
-    const void *k = (dna ? kFwdPartDna : kFwdPartTab).traceKernel();
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, dna ? traceDna(track) : traceTab(track), 256, 0) !=
+        hipSuccess)
         return 1;
     return blocks > 0 ? blocks : 1;
 }
@@ -612,12 +786,9 @@ hipError_t launchWalk16(const WalkArgs &args, hipStream_t stream)
 {
     if (args.nPairs <= 0)
         return hipSuccess;
-    const int S = args.alpha * args.alpha + 2;
-    const dim3 grid((args.nPairs + kWalkThreads - 1) / kWalkThreads), block(kWalkThreads);
-    if (S <= kWalkLdsStride)
-        hipLaunchKernelGGL(kWalk16<true>, grid, block, (size_t)kWalkThreads * S * sizeof(int32_t), stream, args);
-    else
-        hipLaunchKernelGGL(kWalk16<false>, grid, block, 0, stream, args);
+    const int threads = walkThreads(args.alpha), pairs = threads / kWalkLanes;
+    hipLaunchKernelGGL(kWalk16, dim3((args.nPairs + pairs - 1) / pairs), dim3(threads),
+                       (size_t)pairs * (args.alpha * args.alpha + 2) * sizeof(int32_t), stream, args);
     return hipGetLastError();
 }
 
@@ -625,7 +796,9 @@ hipError_t launchBandedWalk(const BandedWalkArgs &args, hipStream_t stream)
 {
     if (args.nIds <= 0)
         return hipSuccess;
-    hipLaunchKernelGGL(kBandedWalk, dim3((args.nIds + 63) / 64), dim3(64), 0, stream, args);
+    const int threads = walkThreads(args.alpha), pairs = threads / kWalkLanes;
+    hipLaunchKernelGGL(kBandedWalk, dim3((args.nIds + pairs - 1) / pairs), dim3(threads),
+                       (size_t)pairs * (args.alpha * args.alpha + 2) * sizeof(int32_t), stream, args);
     return hipGetLastError();
 }
 

@@ -22,12 +22,8 @@ enum Track : uint32_t {
     kTrackBottom = 2,   // last row free: max over row m, j <= n
     kTrackRight = 4,    // last column free: max over column n, i <= m
     kTrackLocal = 8,    // local: max over all cells
-    // Kernel variant flag beside kTrackLocal (table kernels): every table
-    // value t = s - gapOpen is >= 0, so the two lookups and the diagonal
-    // add fuse into one 32-bit add (FwdArgs::tNonNeg).
-    kLocalAdd3 = 16,
-    // Kernel variant flag of the global score kernels (drifted values): the
-    // values need all 16 bits (Variant16::wide).
+    // Kernel variant flag of the one-pair-per-lane kernels (drifted values):
+    // the values need all 16 bits (Variant16::wide).
     kWideVals = 32
 };
 
@@ -77,8 +73,6 @@ struct FwdArgs {
     const WorkItem *items;
     int32_t nItems;
     uint32_t *queue;            // work-queue counter of the per-wave items (zeroed before launch)
-    int32_t nLong;              // items [0, nLong) are shared by the 4 waves of a workgroup
-    uint32_t *queueLong;        // work-queue counter of those (zeroed before launch)
     uint32_t *rowbuf;           // per wave slot: GROUPS * rowCols * 2 dwords
     int32_t rowCols;            // columns per group row buffer
     int32_t *scores;            // indexed by pair id
@@ -90,14 +84,8 @@ struct FwdArgs {
     const uint32_t *dnaProfile; // dwords 0..4: bytes v=0..3 of s(h,v)-gapOpen, h=0..3, pad;
                                 // dwords 8..12: bytes h=0..3 of s(h,v)-gapOpen, v=0..3, pad
     Drift drift;                // global score kernels
-    int32_t tNonNeg;            // local table kernels: every s(h,v) - gapOpen >= 0
     int32_t bandLo, bandUp;     // banded kernels: cells with bandLo <= j - i <= bandUp
     int32_t bandCols;           // banded kernels: row-buffer ring columns (a power of two <= rowCols)
-    // Trace variant only:
-    uint4 *trace;               // 16-byte trace records (64 per step)
-    const int64_t *traceOff;    // per item: first record (units of 64 records)
-    int32_t *endEF;             // per pair id: E and F of the end cell
-    int32_t *endIJ;             // free ends: per pair id, the end cell (i, j)
 };
 
 // Where the trace records of one pair live: rows are bottom-aligned in the
@@ -109,24 +97,37 @@ struct TraceLoc {
     int32_t p;                  // item row of the pair's row 0
     int32_t lane0;              // first lane of the pair's group
     int32_t half;               // 0: low int16 half, 1: high
+    // The end-cell candidates of the pair's units (strips of the item, or the
+    // whole item): ends[end0 + q * endStride], q < nEnds.
+    int64_t end0;
+    int32_t endStride;
+    int32_t nEnds;
 };
 
-// Traceback walk: one thread per pair.
+// End-cell candidates a trace unit leaves per pair, values in H: b, the best
+// cell of the bottom row (global; only the last unit's counts) or of all its
+// cells (local, none: j = INT32_MAX); r, the best cell of column n (free last
+// column).
+struct TraceEnd {
+    int32_t v, i, j, e, f;
+    int32_t rv, ri, rj, re, rf;
+};
+
+// Traceback walk: 16 lanes per pair.
 struct WalkArgs {
     const uint8_t *hRes;
     const uint8_t *vRes;
     const int64_t *hOff;
     const int64_t *vOff;
-    const int32_t *ids;         // pair ids, one per thread
-    const TraceLoc *locs;       // per thread
+    const int32_t *ids;         // pair ids
+    const TraceLoc *locs;       // per id
     int32_t nPairs;
     const uint4 *trace;
-    const int32_t *scores;      // per pair id: H(m, n)
-    const int32_t *endEF;       // per pair id: E(m, n), F(m, n)
+    const TraceEnd *ends;       // end-cell candidates (TraceLoc::end0)
+    int32_t *scores;            // per pair id (output)
     int32_t *counts;            // per pair id: alpha^2 + 2 counts
     int32_t alpha;
     int32_t linear;             // gap open == gap extend: the linear-gap walk
-    const int32_t *endIJ;       // free ends, local: per pair id, the end cell (i, j); null: (m, n)
     int32_t local;              // local walk: stops where H falls to 0, no leading / trailing gaps
     const int32_t *table;       // local: alpha^2 substitution scores (H along the path)
     int32_t gapOpen;
@@ -413,13 +414,39 @@ hipError_t launchLongResult(const TileArgs &args, hipStream_t stream);
 hipError_t launchTileWalkInit(const TileArgs &args, hipStream_t stream);
 hipError_t launchTileWalk32(const TileArgs &args, hipStream_t stream);
 
-// Trace family.
+// Trace family (trace16.hpp).
 constexpr int kTraceRows = 256;       // rows per block of the trace kernel (G = 16, R = 16)
 constexpr int kTraceLanes = 16;
-int traceSteps(int maxN);             // column steps per block for an item of width maxN
-// track: kTrackEnd (global) or the bottom / right bits of free end gaps.
-hipError_t launchFwdTrace16(bool dna, uint32_t track, const FwdArgs &args, int gridBlocks, hipStream_t stream);
-int occupancyTrace16(bool dna);
+inline int traceSteps(int maxN) { return (maxN + kTraceLanes + 3) / 4 * 4; }   // column steps per block
+// Units as ScoreArgs', 256-row blocks throughout, `pad` the item's index.
+struct TraceArgs {
+    const uint8_t *hRes;
+    const uint8_t *vRes;
+    const int64_t *hOff;
+    const int64_t *vOff;
+    const int32_t *order;
+    const ScoreUnit *units;
+    int32_t nUnits;
+    uint32_t *queue;
+    uint64_t *rowbuf;
+    int64_t slotWords;
+    uint64_t *strips;
+    int64_t stripWords;
+    uint32_t *error;
+    uint32_t mode;
+    int32_t alpha;
+    const int16_t *tTable;
+    const uint32_t *dnaProfile;
+    Drift drift;
+    uint4 *trace;               // 16-byte trace records (64 per step)
+    int64_t traceRecs;          // steps the buffer holds
+    const int64_t *traceOff;    // per item: its first step
+    TraceEnd *ends;
+    const int64_t *endOff;      // per item: its first candidate
+};
+// track: kTrackEnd (global), the bottom / right bits of free end gaps, or kTrackLocal.
+hipError_t launchTrace16(bool dna, uint32_t track, const TraceArgs &args, int gridBlocks, hipStream_t stream);
+int occupancyTrace16(bool dna, uint32_t track);
 hipError_t launchWalk16(const WalkArgs &args, hipStream_t stream);
 hipError_t launchCounts32(const Counts32Args &args, hipStream_t stream);
 

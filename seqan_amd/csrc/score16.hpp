@@ -116,6 +116,73 @@ __device__ __forceinline__ void rowStore(uint64_t *p, uint64_t v, bool strip)
         __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
+// A refill's words of the strip above (columns j0, j0 + 1, ... of the lane):
+// waits until they are there.  Ends: see the file's head; `stop` once a wait
+// has run past its bound.
+template <int C>
+__device__ __forceinline__ void waitWords(uint64_t (&rv)[C], const uint64_t *rowIn, int Nw, int j0, uint32_t *error,
+                                          bool &stop)
+{
+    int spins = 0;
+    for (;;) {
+        bool missing = false;
+#pragma unroll
+        for (int q = 0; q < C; ++q)
+            missing |= (uint32_t)rv[q] == 0;
+        if (stop || __ballot(missing) == 0)
+            break;
+        __builtin_amdgcn_s_sleep(8);
+        if (++spins > (1 << 21)) {
+            __hip_atomic_store(error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            stop = true;
+        } else if ((spins & 1023) == 0) {
+            stop = __hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0;
+        }
+#pragma unroll
+        for (int q = 0; q < C; ++q)
+            if ((uint32_t)rv[q] == 0)
+                rv[q] = rowLoad(rowIn + min(max(j0 + q, 0), Nw), true);
+    }
+}
+
+// The unit's fields as wave-uniform values.
+__device__ __forceinline__ ScoreUnit uniformUnit(ScoreUnit w)
+{
+    w.first = __builtin_amdgcn_readfirstlane(w.first);
+    w.count = __builtin_amdgcn_readfirstlane(w.count);
+    w.maxN = __builtin_amdgcn_readfirstlane(w.maxN);
+    w.nblocks = __builtin_amdgcn_readfirstlane(w.nblocks);
+    w.rows = __builtin_amdgcn_readfirstlane(w.rows);
+    w.shape = __builtin_amdgcn_readfirstlane(w.shape);
+    w.block = __builtin_amdgcn_readfirstlane(w.block);
+    w.pad = __builtin_amdgcn_readfirstlane(w.pad);
+    return w;
+}
+
+// The score tables in LDS: t = s - o + tAdd for real codes, 0 for the padding
+// code (tAdd: the drift under drift in both directions, the diagonal step's
+// second half; 0 local).
+template <bool DNA, class Args>
+__device__ __forceinline__ void loadScores(const Args &a, int tAdd, uint32_t *sProf, char *sT)
+{
+    if constexpr (DNA) {
+        if (threadIdx.x < 5) {
+            uint32_t w = a.dnaProfile[threadIdx.x];
+            if ((int)threadIdx.x < a.alpha)
+                w += (uint32_t)tAdd * (0x01010101u >> (32 - 8 * min(a.alpha, 4)));
+            sProf[threadIdx.x] = w;
+        }
+    } else {
+        const int TW = a.alpha + 1;
+        for (int i = threadIdx.x; i < TW * TW * kTabCopies; i += blockDim.x) {
+            const int w = i / kTabCopies, h = w / TW, v = w % TW;
+            const uint32_t t = (h == a.alpha || v == a.alpha) ? 0u : (uint32_t)(uint16_t)(a.tTable[w] + tAdd);
+            *reinterpret_cast<uint32_t *>(sT + 4 * i) = t << 16;
+        }
+    }
+    __syncthreads();
+}
+
 // Per-lane state of one pair couple (lo = pair A, hi = pair B).
 struct Couple {
     const uint8_t *h[2];
@@ -249,29 +316,8 @@ struct Score16 {
         };
         auto refillStore = [&](int s) {
             if constexpr (!HEAD) {
-                if (strip) {
-                    // The words of the strip above: wait until they are there.
-                    int spins = 0;
-                    for (;;) {
-                        bool missing = false;
-#pragma unroll
-                        for (int q = 0; q < CPL; ++q)
-                            missing |= (uint32_t)rv[q] == 0;
-                        if (stop || __ballot(missing) == 0)
-                            break;
-                        __builtin_amdgcn_s_sleep(8);
-                        if (++spins > (1 << 21)) {
-                            __hip_atomic_store(a.error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                            stop = true;
-                        } else if ((spins & 1023) == 0) {
-                            stop = __hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0;
-                        }
-#pragma unroll
-                        for (int q = 0; q < CPL; ++q)
-                            if ((uint32_t)rv[q] == 0)
-                                rv[q] = rowLoad(rowIn + min(max(colOf(s, q), 0), Nw), true);
-                    }
-                }
+                if (strip)
+                    waitWords(rv, rowIn, Nw, colOf(s, 0), a.error, stop);
             }
 #pragma unroll
             for (int q = 0; q < CPL; ++q) {
@@ -649,25 +695,7 @@ __device__ __forceinline__ void scoreRun(const ScoreArgs &a)
 {
     __shared__ uint32_t sProf[8];
     __shared__ __align__(16) char sT[DNA ? 16 : kTabLdsBytes];
-    // t for real codes, 0 for the padding code: s - o, plus the drift of the
-    // diagonal step's second half under drift in both directions (global).
-    const int tAdd = KIND == kScoreLocal ? 0 : a.drift.d;
-    if constexpr (DNA) {
-        if (threadIdx.x < 5) {
-            uint32_t w = a.dnaProfile[threadIdx.x];
-            if ((int)threadIdx.x < a.alpha)
-                w += (uint32_t)tAdd * (0x01010101u >> (32 - 8 * min(a.alpha, 4)));
-            sProf[threadIdx.x] = w;
-        }
-    } else {
-        const int TW = a.alpha + 1;
-        for (int i = threadIdx.x; i < TW * TW * kTabCopies; i += blockDim.x) {
-            const int w = i / kTabCopies, h = w / TW, v = w % TW;
-            const uint32_t t = (h == a.alpha || v == a.alpha) ? 0u : (uint32_t)(uint16_t)(a.tTable[w] + tAdd);
-            *reinterpret_cast<uint32_t *>(sT + 4 * i) = t << 16;
-        }
-    }
-    __syncthreads();
+    loadScores<DNA>(a, KIND == kScoreLocal ? 0 : a.drift.d, sProf, sT);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     uint64_t *slotRow = a.rowbuf + (size_t)(blockIdx.x * (blockDim.x >> 6) + wave) * a.slotWords;
@@ -681,14 +709,7 @@ __device__ __forceinline__ void scoreRun(const ScoreArgs &a)
         it = __builtin_amdgcn_readfirstlane(it);
         if (it >= a.nUnits)
             break;
-        ScoreUnit w = a.units[it];
-        w.first = __builtin_amdgcn_readfirstlane(w.first);
-        w.count = __builtin_amdgcn_readfirstlane(w.count);
-        w.maxN = __builtin_amdgcn_readfirstlane(w.maxN);
-        w.nblocks = __builtin_amdgcn_readfirstlane(w.nblocks);
-        w.rows = __builtin_amdgcn_readfirstlane(w.rows);
-        w.shape = __builtin_amdgcn_readfirstlane(w.shape);
-        w.block = __builtin_amdgcn_readfirstlane(w.block);
+        const ScoreUnit w = uniformUnit(a.units[it]);
         if (w.shape & kUnit64) {
             if (w.shape & kUnitWide)
                 Score16<64, DNA, KIND, true>::unit(a, w, slotRow, sProf, sT, stop);
