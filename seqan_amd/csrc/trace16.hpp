@@ -255,7 +255,10 @@ struct Trace16 {
 
         uint32_t botG = Gk[RB - 1], botF = neg2, upGprev = neg2;
         uint32_t z2 = asu(splat(dr.bias));                              // local: the stored 0
-        uint32_t best2 = asu(splat(dr.bias - dr.cost + 1));             // local: G of the best cell, H >= 1
+        // Local: G of the lane's best cell so far (a whole item's earlier
+        // blocks included), H >= 1.
+        uint32_t best2 = asu(pack(dr.bias - dr.cost + max(LOC ? cb.v[0] : 0, 1),
+                                  dr.bias - dr.cost + max(LOC ? cb.v[1] : 0, 1)));
         constexpr int DL = 4;
         uint32_t qa[DNA ? 1 : DL], qb[DNA ? 1 : DL];
         auto ldA = [&](uint32_t col, int k) -> uint32_t { return *reinterpret_cast<const uint16_t *>(sT + (col + selA[k])); };

@@ -74,3 +74,19 @@ def test_counts_in_chunks_with_strips(ctx, monkeypatch):
     score = sa.simple_score(2, -3, -1, -5)
     for mode in (0, 9, 15, sa.LOCAL):
         _check_rows(ctx, H, V, score, mode)
+
+
+def test_local_best_in_an_early_block(ctx, monkeypatch):
+    # Whole items of several row blocks whose best cell lies in the first
+    # ones: a later block's lower cells must not replace it.
+    monkeypatch.setenv("SQMI_COOP_MIN_BLOCKS", "0")
+    rng = np.random.default_rng(14)
+    for alpha, score in ((4, sa.simple_score(2, -3, -1, -5)), (24, sa.blosum62(-1, -11))):
+        hs, vs = [], []
+        for n in (300, 600, 900, 1200):
+            for at in (0, n // 3, n - 120):
+                h, v = (rng.integers(0, alpha, n).astype(np.uint8) for _ in range(2))
+                v[at:at + 60] = h[n // 2:n // 2 + 60]
+                hs.append(h)
+                vs.append(v)
+        _check_rows(ctx, sa.SeqSet.from_list(hs), sa.SeqSet.from_list(vs), score, sa.LOCAL)
