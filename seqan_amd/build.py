@@ -30,7 +30,7 @@ SOURCES = [("score16.hip", f"score16_{t}_{k}", {"SQMI_SCORE_DNA": d, "SQMI_SCORE
 SOURCES += [("trace16.hip", "trace16_tab", {"SQMI_TRACE_DNA": 0, "SQMI_TRACE_PART": "traceTab"}),
             ("trace16.hip", "trace16_dna", {"SQMI_TRACE_DNA": 1, "SQMI_TRACE_PART": "traceDna"}),
             ("kernels.hip", "kernels", {}), ("lane.hip", "lane", {}), ("band16.hip", "band16", {}),
-            ("long.hip", "long", {}), ("banded.hip", "banded", {}), ("scratch.hip", "scratch", {}),
+            ("long16.hip", "long16", {}), ("long.hip", "long", {}), ("banded.hip", "banded", {}), ("scratch.hip", "scratch", {}),
             ("engine.cpp", "engine", {}), ("scoring.cpp", "scoring", {}), ("workload.cpp", "workload", {})]
 JOBS = max(1, min(8, os.cpu_count() or 1))
 

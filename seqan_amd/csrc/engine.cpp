@@ -18,6 +18,7 @@
 #endif
 #include <chrono>
 #include <climits>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -93,11 +94,6 @@ struct sqmi_context
     static constexpr int kMaxLongStreams = 4;
     hipStream_t longStreams[kMaxLongStreams] = {};
     hipEvent_t longFork = nullptr, longJoin[kMaxLongStreams] = {};
-    // Streaming long-pair forward: its item ranges (kept until the next
-    // call, as a pending upload may read them) and whether the call used it
-    // (then the call checks the kernel's wait-bound flag after its sync).
-    std::vector<int4> longRanges;
-    bool longStreamed = false;
     Buffers b;
     Planned *planned = nullptr;   // the calls' plans, one after the other (owned)
     // The no-allocation entry point: this device's scratch array (its device
@@ -118,7 +114,6 @@ struct sqmi_context
         uint64_t key = 0;
         hipGraphExec_t exec = nullptr;
         sqmi_stats stats{};
-        bool longStreamed = false;   // the graph holds the streaming long-pair forward
     } replay;
 };
 
@@ -351,6 +346,12 @@ int laneRows(int category, int bin, int64_t pairs16)
 // waves of one workgroup used to share an item's blocks; 1,048,576 of them
 // 99 -> 69 ms, of which the shorter recurrence gives most.
 constexpr double kCouple64Share = 1.0e-5, kStripShare = 4.0e-5;
+// Time of a strip's step (ns), by its rows per lane: alone on a SIMD, and of a full one.
+struct LongCost {
+    int rows;
+    double alone, full;
+};
+constexpr LongCost kLongCosts[] = {{4, 115, 63}, {8, 153, 111}, {16, 230, 203}};
 // Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
 constexpr int64_t kResidentWaves = 3072;
 // Rows per unit of the group shapes' row counts.
@@ -450,14 +451,22 @@ struct Planned
 // int32 pairs whose sides are both at least this long (and that are DNA,
 // global) run the tiled long-pair kernels instead of one thread per pair
 // (2048, or SQMI_LONG_MIN_SIDE).
-// The packed long-pair forward keeps tile values relative to a base: it
-// needs kLong16Span steps of at most D = max|s| + |o| + |e| inside the int16
-// window.
-bool longPacked(const ScoringInfo &si, uint32_t flags)
+// The packed long-pair kernels (long16.hip) hold values relative to a base;
+// target: where a strip's top row is kept; a strip of 64 R rows needs every
+// value below kDriftNarrowMax, the cells of a wave growing by at most sMax + 2
+// drift per row and column.
+int longTarget(const ScoringInfo &si, const Drift &dr)
 {
-    const int64_t D = std::max(std::abs(si.sMax), std::abs(si.sMin)) + std::abs(si.o) + std::abs(si.e);
-    return !(flags & SQMI_FORCE_INT32) && (int64_t)kLong16Span * D <= std::min(-kNeg16 - kGuard16, 32767 - kGuard16);
+    return dr.neg + 8 * dr.cost + 64 * (std::max(si.sMax, 0) + 2 * dr.d) + 16;
 }
+bool longRowsFit(const ScoringInfo &si, int R)
+{
+    const Drift dr = driftOf(si, false);
+    const int64_t grow = std::max(si.sMax, 0) + 2 * (int64_t)dr.d;
+    return si.dnaDrift && si.o <= 0 && si.e <= 0 && dr.neg == dr.cost + 1 &&
+           longTarget(si, dr) + kLongSlackV + (64 * R + 256 + kLongT) * grow + 8 * dr.cost <= kDriftNarrowMax;
+}
+bool longPacked(const ScoringInfo &si, uint32_t flags) { return !(flags & SQMI_FORCE_INT32) && longRowsFit(si, 4); }
 
 // Test and tuning switch: SQMI_LONG_ALL=1 sends every pair the long route
 // can take there, also those the packed kernels could score.
@@ -479,33 +488,6 @@ int64_t longMinSide()
     if (env && *env && std::atoll(env) > 0)
         return std::atoll(env);
     return 2048;
-}
-
-// The packed long-pair forward as one persistent launch over every tile
-// (SQMI_LONG_STREAM=1), or one launch per tile anti-diagonal (default).  On
-// 64 pairs of 100 kbp the persistent form measured 382 ms against 161 ms:
-// 323 ms even without its agent-scope fences, so the dataflow schedule
-// itself, not only the cross-XCD coherence, costs more than the launches.
-bool longStreaming()
-{
-    const char *env = std::getenv("SQMI_LONG_STREAM");
-    return env && *env == '1';
-}
-
-// After a call's final synchronisation: the streaming forward's waits are
-// bounded, and one that ran past its bound leaves a flag (never expected:
-// every wait is for tiles that running waves hold).
-sqmi_status longStreamCheck(sqmi_context *ctx)
-{
-    if (!ctx->longStreamed)
-        return SQMI_OK;
-    ctx->longStreamed = false;
-    uint32_t flag = 0;
-    if (hipMemcpy(&flag, static_cast<const uint32_t *>(ctx->b.longSched.p) + 1, 4, hipMemcpyDeviceToHost) != hipSuccess)
-        return fail(ctx, SQMI_ERR_DEVICE, "reading the long-pair forward's wait flag");
-    if (flag)
-        return fail(ctx, SQMI_ERR_DEVICE, "long-pair forward: a tile wait ran past its bound; scores are not valid");
-    return SQMI_OK;
 }
 
 // After a call's final synchronisation: whether a strip's wait ran past its
@@ -1217,10 +1199,210 @@ struct RowsDev {
     int64_t *begins = nullptr;   // local windows only
 };
 
+// Host copies of the long pairs' descriptors (kept until the caller has
+// synchronised).
+struct LongStage {
+    std::vector<LongPair> pairs;
+    std::vector<LongCouple> couples;
+    std::vector<int2> units;
+};
+
+// The packed kernels' long pairs (`ids`, longest first, so that couples hold
+// similar shapes), in chunks of couples whose buffers fit traceBudget().
+sqmi_status runLong16(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_sequences *setV, const Planned &P,
+                      const Inputs &in, int32_t *dCounts, const RowsDev &rows, const std::vector<int32_t> &ids,
+                      LongStage &stage, Deferred *deferred)
+{
+    hipStream_t stream = ctx->stream;
+    const int64_t budget = traceBudget(ctx), N = setH->count;
+    const size_t nc = (ids.size() + 1) / 2;
+    auto sides = [&](size_t k, int32_t &n, int32_t &m) {
+        n = (int32_t)(setH->offsets[ids[k] + 1] - setH->offsets[ids[k]]);
+        m = (int32_t)(setV->offsets[ids[k] + 1] - setV->offsets[ids[k]]);
+    };
+    // Rows per lane by the time the call should take.  A step of a strip of 4,
+    // 8 or 16 rows per lane takes a wave alone on its SIMD 115, 153 or 230
+    // ns, and 63, 111 or 203 ns of a full one's; a strip starts about 160
+    // steps behind the one above.  Either the chain of one couple's strips
+    // bounds the call or the rounds of strips on the chip's SIMDs do, plus
+    // their start.  Forward of 100 kbp pairs, R = 8 / 16: 10 pairs 20.1 / 27
+    // ms, 20: 28.3 / 27.2, 40: 45.5 / 43.6, 64: 68 / 77 (a fourth round
+    // for 64 strips).  SQMI_LONG_ROWS sets R for tests.
+    int R = 4;
+    double best = 0;
+    for (const LongCost &q : kLongCosts) {
+        double strips = 0, chain = 0, lead = 0, steps = 0;
+        for (size_t k = 0; k < ids.size(); k += 2) {
+            int32_t n, m, n1 = 0, m1 = 0;
+            sides(k, n, m);
+            if (k + 1 < ids.size())
+                sides(k + 1, n1, m1);
+            const double nb = std::max(m, m1) / (64 * q.rows) + 1, len = std::max(n, n1);
+            strips += nb;
+            steps += nb * len;
+            lead = std::max(lead, 160 * nb * q.alone);
+            chain = std::max(chain, (len + 160 * nb) * q.alone);
+        }
+        const double rounds = strips / (4 * std::max(1, ctx->numCUs));
+        const double t = std::max(chain, std::ceil(rounds) * (steps / strips) * q.full + lead);
+        if (longRowsFit(P.si, q.rows) && (best == 0 || t < best)) {
+            best = t;
+            R = q.rows;
+        }
+    }
+    if (const char *env = std::getenv("SQMI_LONG_ROWS")) {
+        const int r = std::atoi(env);
+        if ((r == 4 || r == 8 || r == 16) && longRowsFit(P.si, r))
+            R = r;
+    }
+    std::vector<LongCouple> &couples = stage.couples;
+    couples.assign(nc, LongCouple{});
+    std::vector<size_t> chunkEnd, unitEnd;
+    int64_t rowWords = 0, stateWords = 0, bytes = 0, maxRows = 1, maxState = 0;
+    const int64_t traceBytes = dCounts ? (int64_t)2 * longWinStrips(R) * kWinCouples * kLongT * 64 * longRecBytes(R) : 0;
+    size_t maxCouples = 1, first = 0;
+    for (size_t c = 0; c < nc; ++c) {
+        LongCouple &q = couples[c];
+        for (int x = 0; x < 2; ++x) {
+            const size_t k = 2 * c + x;
+            q.pid[x] = -1;
+            if (k < ids.size()) {
+                q.pid[x] = ids[k];
+                sides(k, q.n[x], q.m[x]);
+            }
+        }
+        q.maxN = std::max(q.n[0], q.n[1]);
+        q.nb = std::max(q.m[0], q.m[1]) / (64 * R) + 1;
+        for (int x = 0; x < 2; ++x)
+            q.p[x] = q.nb * 64 * R - 1 - q.m[x];
+        q.chunks = (longSteps(q.maxN) + kLongT - 1) / kLongT;
+        const int64_t rw = (int64_t)(q.nb - 1) * (q.maxN + 1);
+        const int64_t sw = dCounts ? (int64_t)q.nb * q.chunks * longStateWords(R) * 64 : 0;
+        const int64_t need = 8 * rw + 4 * sw + traceBytes;
+        if (bytes > 0 && bytes + need > budget) {
+            chunkEnd.push_back(c);
+            first = c;
+            rowWords = stateWords = bytes = 0;
+        }
+        q.rows = rowWords;
+        q.state = stateWords;
+        rowWords += rw;
+        stateWords += sw;
+        bytes += need;
+        maxRows = std::max(maxRows, rowWords);
+        maxState = std::max(maxState, stateWords);
+        maxCouples = std::max(maxCouples, c + 1 - first);
+    }
+    chunkEnd.push_back(nc);
+    std::vector<int2> &units = stage.units;
+    units.clear();
+    size_t b = 0;
+    for (size_t e : chunkEnd) {
+        int nb = 0;
+        for (size_t c = b; c < e; ++c)
+            nb = std::max(nb, couples[c].nb);
+        for (int s = 0; s < nb; ++s)
+            for (size_t c = b; c < e; ++c)
+                if (s < couples[c].nb)
+                    units.push_back(make_int2((int)(c - b), s));
+        unitEnd.push_back(units.size());
+        b = e;
+    }
+    if (units.size() >= (size_t)INT32_MAX)
+        return fail(ctx, SQMI_ERR_UNSUPPORTED, "long pairs: too many strips for one launch");
+    hipError_t err;
+    const size_t qWords = 16 * chunkEnd.size();
+    if ((err = ensure(ctx->b.strips, (size_t)maxRows * 8)) != hipSuccess ||
+        (err = ensure(ctx->b.longPairs, sizeof(LongCouple) * nc)) != hipSuccess ||
+        (err = ensure(ctx->b.longSched, 4 * qWords + sizeof(int2) * units.size())) != hipSuccess ||
+        (err = ensure(ctx->b.endEF, (size_t)8 * N)) != hipSuccess)
+        return hipFail(ctx, err, "allocating long-pair buffers");
+    if (dCounts && ((err = ensure(ctx->b.longCk, (size_t)maxState * 4)) != hipSuccess ||
+                    (err = ensure(ctx->b.longWalk, (size_t)8 * kLongWalkInts * maxCouples)) != hipSuccess ||
+                    (err = ensure(ctx->b.longTrace, (size_t)traceBytes * maxCouples)) != hipSuccess))
+        return hipFail(ctx, err, "allocating long-pair traceback buffers");
+    uint32_t *queues = static_cast<uint32_t *>(ctx->b.longSched.p);
+    int2 *dUnits = reinterpret_cast<int2 *>(queues + qWords);
+    if ((err = hipMemcpyAsync(ctx->b.longPairs.p, couples.data(), sizeof(LongCouple) * nc, hipMemcpyHostToDevice, stream)) !=
+            hipSuccess ||
+        (err = hipMemcpyAsync(dUnits, units.data(), sizeof(int2) * units.size(), hipMemcpyHostToDevice, stream)) != hipSuccess)
+        return hipFail(ctx, err, "uploading long pairs");
+    hipError_t opErr = hipSuccess;
+    auto op = [&](std::function<hipError_t()> f) {
+        if (deferred)
+            deferred->push_back(std::move(f));
+        else if (opErr == hipSuccess)
+            opErr = f();
+        return opErr;
+    };
+    if ((err = op([=] { return launchZero32(queues, qWords, stream); })) != hipSuccess)
+        return hipFail(ctx, err, "launching queue reset");
+    b = 0;
+    size_t ub = 0;
+    for (size_t k = 0; k < chunkEnd.size(); ++k) {
+        const size_t e = chunkEnd[k], ue = unitEnd[k];
+        LongArgs a{};
+        a.hRes = in.dH;
+        a.vRes = in.dV;
+        a.hOff = static_cast<const int64_t *>(ctx->b.hOff.p);
+        a.vOff = static_cast<const int64_t *>(ctx->b.vOff.p);
+        a.couples = static_cast<const LongCouple *>(ctx->b.longPairs.p) + b;
+        a.nCouples = (int32_t)(e - b);
+        a.units = dUnits + ub;
+        a.nUnits = (int32_t)(ue - ub);
+        a.queue = queues + 16 * k;
+        a.rows = static_cast<uint64_t *>(ctx->b.strips.p);
+        a.state = dCounts ? static_cast<uint32_t *>(ctx->b.longCk.p) : nullptr;
+        a.error = ctx->waitFlag;
+        a.target = longTarget(P.si, P.drift);
+        a.alpha = P.si.alpha;
+        a.dnaProfile = static_cast<const uint32_t *>(ctx->b.dnaProf.p);
+        a.drift = P.drift;
+        a.scores = in.dScores;
+        a.endEF = static_cast<int32_t *>(ctx->b.endEF.p);
+        int64_t words = 0, maxM = 0, maxN = 0;
+        for (size_t c = b; c < e; ++c) {
+            words = std::max(words, couples[c].rows + (int64_t)(couples[c].nb - 1) * (couples[c].maxN + 1));
+            maxM = std::max<int64_t>(maxM, std::max(couples[c].m[0], couples[c].m[1]));
+            maxN = std::max<int64_t>(maxN, couples[c].maxN);
+        }
+        const int numCUs = std::max(1, ctx->numCUs);
+        if ((err = op([=] {
+                 const hipError_t z = launchZero32(reinterpret_cast<uint32_t *>(a.rows), 2 * (size_t)words, stream);
+                 return z != hipSuccess ? z : launchLong16(R, a, numCUs, stream);
+             })) != hipSuccess)
+            return hipFail(ctx, err, "launching long-pair forward");
+        if (dCounts) {
+            a.trace = ctx->b.longTrace.p;
+            a.walk = static_cast<int32_t *>(ctx->b.longWalk.p);
+            a.counts = dCounts;
+            a.linear = P.si.o == P.si.e;
+            a.alwaysOpen = P.si.e < P.si.o;
+            a.ops = rows.ops;
+            a.opOff = rows.opOff;
+            a.opLen = rows.opLen;
+            if ((err = op([=] { return launchLong16WalkInit(a, stream); })) != hipSuccess)
+                return hipFail(ctx, err, "launching long-pair walk init");
+            // A round leaves its window through the top (at least winStrips
+            // - 1 strips up) or the left side (all its chunks but one, less
+            // the 63 columns between a strip's first and last lane).
+            const int64_t up = (int64_t)(longWinStrips(R) - 1) * 64 * R, left = (kWinChunks - 1) * kLongT - 63;
+            const int64_t rounds = (maxM + up - 1) / up + (maxN + left - 1) / left + 2;
+            for (int64_t r = 0; r < rounds; ++r)
+                if ((err = op([=] { return launchLong16Round(R, a, stream); })) != hipSuccess)
+                    return hipFail(ctx, err, "launching long-pair traceback");
+        }
+        b = e;
+        ub = ue;
+    }
+    return SQMI_OK;
+}
+
 sqmi_status runLong(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_sequences *setV, const Planned &P,
                     const Inputs &in, uint32_t flags, int32_t *dCounts, const RowsDev &rows,
-                    std::vector<LongPair> &pairs, Deferred *deferred = nullptr)
+                    LongStage &stage, Deferred *deferred = nullptr)
 {
+    std::vector<LongPair> &pairs = stage.pairs;
     // Stream operations run at once, or are appended to `deferred` (all
     // uploads and allocations still happen here).
     hipError_t opErr = hipSuccess;
@@ -1237,16 +1419,17 @@ sqmi_status runLong(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_se
     const int C = kLongTileC;
     const int64_t budget = traceBudget(ctx);
     const int64_t N = setH->count;
-    // The packed forward is global only; free end gaps and local take the
+    // The packed kernels are global only; free end gaps and local take the
     // int32 forward and a result pass over its checkpoints.
-    const bool packed = longPacked(P.si, flags) && P.mode == 0;
-    // Longest first, so that the couples of the packed forward pair similar shapes.
+    // Longest first, so that the couples of the packed kernels pair similar shapes.
     std::vector<int32_t> ids(P.idsLong);
     std::stable_sort(ids.begin(), ids.end(), [&](int32_t x, int32_t y) {
         const int64_t mx = setV->offsets[x + 1] - setV->offsets[x], my = setV->offsets[y + 1] - setV->offsets[y];
         const int64_t nx = setH->offsets[x + 1] - setH->offsets[x], ny = setH->offsets[y + 1] - setH->offsets[y];
         return mx != my ? mx > my : nx > ny;
     });
+    if (longPacked(P.si, flags) && P.mode == 0)
+        return runLong16(ctx, setH, setV, P, in, dCounts, rows, ids, stage, deferred);
     // Descriptors with checkpoint offsets relative to the pair's chunk.
     std::vector<size_t> chunkEnd;
     int64_t run = 0, maxRun = 0, bestRun = 0;
@@ -1312,63 +1495,6 @@ sqmi_status runLong(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_se
             maxT = std::max(maxT, pairs[k].ntiles);
         }
         a.wavesPerPair = (maxB + 3) / 4;
-        // (One chunk only: the schedule's upload happens now, and with
-        // deferred launches a second chunk's would overwrite the first's.)
-        if (packed && longStreaming() && chunkEnd.size() == 1 && maxB + maxT < 32768) {
-            // One persistent launch: items = groups of four row blocks of a
-            // couple on one anti-diagonal, in anti-diagonal order (ranges of
-            // consecutive groups of a couple).
-            const int couples = (int)((e - b + 1) / 2);
-            std::vector<int> nbC(couples), ntC(couples);
-            int stride = 1, maxD = 0;
-            for (int c = 0; c < couples; ++c) {
-                const LongPair &p0 = pairs[b + 2 * c];
-                const LongPair &p1 = b + 2 * c + 1 < e ? pairs[b + 2 * c + 1] : p0;
-                nbC[c] = std::max(p0.nblocks, p1.nblocks);
-                ntC[c] = std::max(p0.ntiles, p1.ntiles);
-                stride = std::max(stride, nbC[c]);
-                maxD = std::max(maxD, nbC[c] + ntC[c] - 1);
-            }
-            std::vector<int4> &ranges = ctx->longRanges;
-            ranges.clear();
-            int64_t items = 0;
-            for (int d = 0; d < maxD; ++d)
-                for (int c = 0; c < couples; ++c) {
-                    const int blo = std::max(0, d - ntC[c] + 1), bhi = std::min(d, nbC[c] - 1);
-                    if (blo > bhi)
-                        continue;
-                    ranges.push_back(make_int4((int)items, c, d, blo / 4));
-                    items += bhi / 4 - blo / 4 + 1;
-                }
-            if (items >= INT32_MAX)
-                return fail(ctx, SQMI_ERR_UNSUPPORTED, "long pairs: too many tiles for one launch");
-            // longSched: [0] item counter, [1] wait flag, [16 ..) progress, then the ranges.
-            const size_t progWords = (size_t)couples * stride;
-            const size_t rangeOff = ((16 + progWords) * 4 + 15) / 16 * 16;
-            if ((err = ensure(ctx->b.longSched, rangeOff + sizeof(int4) * ranges.size())) != hipSuccess)
-                return hipFail(ctx, err, "allocating the long-pair schedule");
-            char *sched = static_cast<char *>(ctx->b.longSched.p);
-            if ((err = hipMemcpyAsync(sched + rangeOff, ranges.data(), sizeof(int4) * ranges.size(),
-                                      hipMemcpyHostToDevice, stream)) != hipSuccess)
-                return hipFail(ctx, err, "uploading the long-pair schedule");
-            TileArgs t = a;
-            t.ranges = reinterpret_cast<const int4 *>(sched + rangeOff);
-            t.nRanges = (int32_t)ranges.size();
-            t.nItems = (int32_t)items;
-            t.queue = reinterpret_cast<uint32_t *>(sched);
-            t.error = reinterpret_cast<uint32_t *>(sched) + 1;
-            t.progress = reinterpret_cast<uint32_t *>(sched) + 16;
-            t.progStride = stride;
-            const int grid = std::max(1, ctx->numCUs * occupancyTileFwd16Stream());
-            uint32_t *words = reinterpret_cast<uint32_t *>(sched);
-            const size_t nWords = 16 + progWords;
-            if ((err = op([=] {
-                     hipError_t e2 = launchZero32(words, nWords, stream);
-                     return e2 != hipSuccess ? e2 : launchTileFwd16Stream(t, grid, stream);
-                 })) != hipSuccess)
-                return hipFail(ctx, err, "launching long-pair forward");
-            ctx->longStreamed = true;
-        } else {
         // Every launch sweeps one tile anti-diagonal and ends with a barrier
         // for its whole grid.  Groups of pair couples on separate streams do
         // not wait for each other's slowest tiles, so their launches fill
@@ -1407,7 +1533,7 @@ sqmi_status runLong(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_se
                 TileArgs t = sub[s];
                 t.diag = d;
                 hipStream_t st = s > 0 ? ctx->longStreams[s] : stream;
-                if ((err = op([=] { return packed ? launchTileFwd16(t, st) : launchTileFwd32(t, st); })) !=
+                if ((err = op([=] { return launchTileFwd32(t, st); })) !=
                     hipSuccess)
                     return hipFail(ctx, err, "launching long-pair forward");
             }
@@ -1422,7 +1548,6 @@ sqmi_status runLong(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_se
                      })) != hipSuccess)
                     return hipFail(ctx, err, "long-pair join");
             }
-        }
         }
         if (P.mode != 0) {
             const TileArgs ta = a;
@@ -1618,7 +1743,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         }
         if (flags & SQMI_SCORES_ON_DEVICE)
             scal.push_back((int64_t)(uintptr_t)scores);
-        for (const char *name : {"SQMI_COOP_MIN_BLOCKS", "SQMI_LONG_ALL", "SQMI_LONG_MIN_SIDE", "SQMI_LONG_STREAMS",
+        for (const char *name : {"SQMI_COOP_MIN_BLOCKS", "SQMI_LONG_ALL", "SQMI_LONG_MIN_SIDE", "SQMI_LONG_STREAMS", "SQMI_LONG_ROWS",
                                  "SQMI_SHAPE_RULE", "SQMI_TRACE_BUDGET_MB", "SQMI_ROW_UNITS", "SQMI_BIN_SHAPES"}) {
             const char *v = std::getenv(name);
             for (const char *c = v ? v : ""; *c; ++c)
@@ -1643,8 +1768,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
                 return hipFail(ctx, err, "copying scores");
             if ((err = hipStreamSynchronize(stream)) != hipSuccess)
                 return hipFail(ctx, err, "alignment kernels");
-            ctx->longStreamed = ctx->replay.longStreamed;
-            if ((st = longStreamCheck(ctx)) != SQMI_OK || (st = stripCheck(ctx)) != SQMI_OK)
+            if ((st = stripCheck(ctx)) != SQMI_OK)
                 return st;
             ctx->stats = ctx->replay.stats;
             ctx->stats.host_plan_ms = keyMs;
@@ -1924,8 +2048,8 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         a.table = static_cast<const int32_t *>(ctx->b.table32.p);
         launches.push_back([=] { return launchSimple32(a, stream); });
     }
-    std::vector<LongPair> longPairs;
-    if ((st = runLong(ctx, setH, setV, P, in, flags, nullptr, RowsDev{}, longPairs, &launches)) != SQMI_OK)
+    LongStage longStage;
+    if ((st = runLong(ctx, setH, setV, P, in, flags, nullptr, RowsDev{}, longStage, &launches)) != SQMI_OK)
         return st;
     if (!emptyIds.empty()) {
         if ((err = ensure(ctx->b.emptyIds, 4 * emptyIds.size())) != hipSuccess)
@@ -1982,9 +2106,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
     }
     if ((err = hipStreamSynchronize(stream)) != hipSuccess)
         return hipFail(ctx, err, "alignment kernels");
-    if (ctx->replay.valid)
-        ctx->replay.longStreamed = ctx->longStreamed;
-    if ((st = longStreamCheck(ctx)) != SQMI_OK || (st = stripCheck(ctx)) != SQMI_OK) {
+    if ((st = stripCheck(ctx)) != SQMI_OK) {
         dropReplay(ctx);
         return st;
     }
@@ -2503,8 +2625,8 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
             b = e;
         }
     }
-    std::vector<LongPair> longPairs;
-    if ((st = runLong(ctx, setH, setV, P, in, flags, dCounts, rows, longPairs)) != SQMI_OK)
+    LongStage longStage;
+    if ((st = runLong(ctx, setH, setV, P, in, flags, dCounts, rows, longStage)) != SQMI_OK)
         return st;
     if (!P.emptyIds.empty()) {
         if ((err = ensure(ctx->b.emptyIds, 4 * P.emptyIds.size())) != hipSuccess)
@@ -2564,7 +2686,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
     }
     if ((err = hipStreamSynchronize(stream)) != hipSuccess)
         return hipFail(ctx, err, "traceback kernels");
-    if ((st = longStreamCheck(ctx)) != SQMI_OK || (st = stripCheck(ctx)) != SQMI_OK)
+    if ((st = stripCheck(ctx)) != SQMI_OK)
         return st;
     float ms = 0;
     if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess)

@@ -366,7 +366,7 @@ struct TileArgs {
     const uint32_t *dnaProfile;
     int32_t *scores;            // per pair id
     int32_t *endEF;             // per pair id: E, F of cell (m, n)
-    uint32_t mode;              // SQMI_FREE_* / SQMI_LOCAL (int32 forward; the packed one is global only)
+    uint32_t mode;              // SQMI_FREE_* / SQMI_LOCAL
     int32_t *best;              // local: per row block of each pair (LongPair::bestck), the maximum G so far
     // traceback
     uint2 *trace;               // per long pair: kRoundSlots tiles x kTileRecSteps steps x 16 lanes records
@@ -376,43 +376,75 @@ struct TileArgs {
     uint8_t *ops;               // rows, as in WalkArgs (optional)
     const int64_t *opOff;
     int64_t *opLen;
-    // Streaming packed forward (kTileFwd16S): items = row-block groups of a
-    // couple on an anti-diagonal, claimed in anti-diagonal order.  ranges[r]
-    // = (first item, couple, diagonal, first group) of the consecutive
-    // groups of one couple on one diagonal.
-    const int4 *ranges;
-    int32_t nRanges;
-    int32_t nItems;
-    uint32_t *queue;            // item counter (zeroed before the launch)
-    uint32_t *progress;         // per couple x row block: tiles done (zeroed)
-    int32_t progStride;         // row blocks per couple in `progress`
-    uint32_t *error;            // set when a wait runs past its bound
 };
 constexpr int kTileSlack = 24;        // steps per tile beyond its width (skew + prefetch)
 constexpr int kWalkStateInts = 8;
 // Traceback window of one round: kRoundBlocks row blocks x kRoundTiles column
-// tiles recomputed with trace records (tileC = kLongTileC).  Tiles of 128
-// columns: the forward of 64 pairs of 100 kbp takes 157 ms against 171 ms
-// with 256 columns (a lone tile's sweep, the per-anti-diagonal latency, is
-// halved) and 291 ms with 64 (per-tile overheads take over).
+// tiles recomputed with trace records (tileC = kLongTileC).
 constexpr int kLongTileC = 128;
 constexpr int kTileRecSteps = kLongTileC + kTileSlack;
 constexpr int kRoundBlocks = 8, kRoundTiles = 16, kRoundSlots = kRoundBlocks * kRoundTiles;
 hipError_t launchTileFwd32(const TileArgs &args, hipStream_t stream);
-// One persistent launch of the packed forward over every tile of the
-// chunk's pairs (kTileFwd16S); gridBlocks of 256 threads.
-hipError_t launchTileFwd16Stream(const TileArgs &args, int gridBlocks, hipStream_t stream);
-int occupancyTileFwd16Stream();
-// Packed variant: pair couples (2 c, 2 c + 1), values relative to a per-tile
-// base; valid when kLong16Span x (max|s| + |o| + |e|) fits the int16 window.
-constexpr int kLong16Span = 800;
-hipError_t launchTileFwd16(const TileArgs &args, hipStream_t stream);
 hipError_t launchTileTrace32(const TileArgs &args, hipStream_t stream);
 // Scores of long pairs under free end gaps or local alignment, from the
 // forward's checkpoints (free last row / column) or its running maximum.
 hipError_t launchLongResult(const TileArgs &args, hipStream_t stream);
 hipError_t launchTileWalkInit(const TileArgs &args, hipStream_t stream);
 hipError_t launchTileWalk32(const TileArgs &args, hipStream_t stream);
+
+// Packed long pairs, global (long16.hip): couples of pairs in strips of 64 R
+// rows, R = 4, 8 or 16 rows per lane, bottom-aligned (pair row i is strip row
+// p + i).  `state` and `rows` count words in LongArgs::state and ::rows.
+struct LongCouple {
+    int32_t pid[2];     // the second -1: none
+    int32_t n[2], m[2], p[2];
+    int32_t maxN;       // the larger |H|
+    int32_t nb;         // strips
+    int32_t chunks;     // checkpoints per strip
+    int32_t pad;
+    int64_t rows;       // (nb - 1) x (maxN + 1) words: bottom rows
+    int64_t state;      // nb x chunks x longStateWords(R) x 64 words
+};
+constexpr int kLongT = 128;             // steps between checkpoints
+constexpr int kLongSlackV = 512;        // growth of a strip's top row before its base is raised
+constexpr int kWinChunks = 14, kWinCouples = kWinChunks / 2;   // a traceback window's chunks, waves per strip of it
+constexpr int kLongWalkInts = 8;
+constexpr int longSteps(int maxN) { return (maxN + 64 + 3) / 4 * 4; }
+constexpr int longStateWords(int R) { return 2 * R + 4; }
+constexpr int longWinStrips(int R) { return 1024 / (64 * R) + 1; }
+constexpr int longRecBytes(int R) { return R == 16 ? 16 : 8; }
+struct LongArgs {
+    const uint8_t *hRes;
+    const uint8_t *vRes;
+    const int64_t *hOff;
+    const int64_t *vOff;
+    const LongCouple *couples;
+    int32_t nCouples;
+    const int2 *units;          // (couple, strip), strip by strip
+    int32_t nUnits;
+    uint32_t *queue;            // unit counter (zeroed before the launch)
+    uint64_t *rows;             // zeroed before the launch
+    uint32_t *state;            // null: no checkpoints
+    uint32_t *error;            // as in ScoreArgs
+    int32_t target;             // a strip's base is raised to keep its top row here
+    int32_t alpha;
+    const uint32_t *dnaProfile;
+    Drift drift;
+    int32_t *scores;            // per pair id
+    int32_t *endEF;             // per pair id: E, F of cell (m, n)
+    // Traceback.
+    void *trace;                // per pair: longWinStrips x kWinCouples x kLongT x 64 records
+    int32_t *walk;              // per pair: kLongWalkInts ints
+    int32_t *counts;            // per pair id: alpha^2 + 2 counts
+    int32_t linear, alwaysOpen; // gap open == / > gap extend
+    uint8_t *ops;               // rows, as in WalkArgs (optional)
+    const int64_t *opOff;
+    int64_t *opLen;
+};
+hipError_t launchLong16(int R, const LongArgs &args, int numCUs, hipStream_t stream);
+hipError_t launchLong16WalkInit(const LongArgs &args, hipStream_t stream);
+// One round: the windows' trace records, then the walks through them.
+hipError_t launchLong16Round(int R, const LongArgs &args, hipStream_t stream);
 
 // Trace family (trace16.hpp).
 constexpr int kTraceRows = 256;       // rows per block of the trace kernel (G = 16, R = 16)
