@@ -21,15 +21,18 @@ CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libseqan_amd.so")
 ARCH = os.environ.get("SQMI_OFFLOAD_ARCH", "gfx950")
 
-# (source, object name, defines).  score16.hip is built once per DNA profile /
-# substitution table and kind, trace16.hip per profile / table; the sources
+# (source, object name, defines).  score16.hip and band16.hip are built once per
+# DNA profile / substitution table and kind, trace16.hip per profile / table; the sources
 # compile in parallel, the longest first.
 SOURCES = [("score16.hip", f"score16_{t}_{k}", {"SQMI_SCORE_DNA": d, "SQMI_SCORE_KIND": f"kScore{k}",
                                                 "SQMI_SCORE_PART": f"score{t}{k}"})
            for d, t in ((0, "Tab"), (1, "Dna")) for k in ("Local", "Right", "Global")]
+SOURCES += [("band16.hip", f"band16_{t}_{k}", {"SQMI_BAND_DNA": d, "SQMI_BAND_KIND": f"kBand{k}",
+                                              "SQMI_BAND_PART": f"band{t}{k}"})
+            for d, t in ((0, "Tab"), (1, "Dna")) for k in ("Local", "Free", "End")]
 SOURCES += [("trace16.hip", "trace16_tab", {"SQMI_TRACE_DNA": 0, "SQMI_TRACE_PART": "traceTab"}),
             ("trace16.hip", "trace16_dna", {"SQMI_TRACE_DNA": 1, "SQMI_TRACE_PART": "traceDna"}),
-            ("kernels.hip", "kernels", {}), ("lane.hip", "lane", {}), ("band16.hip", "band16", {}),
+            ("kernels.hip", "kernels", {}), ("lane.hip", "lane", {}),
             ("long16.hip", "long16", {}), ("long.hip", "long", {}), ("banded.hip", "banded", {}), ("scratch.hip", "scratch", {}),
             ("engine.cpp", "engine", {}), ("scoring.cpp", "scoring", {}), ("workload.cpp", "workload", {})]
 JOBS = max(1, min(8, os.cpu_count() or 1))

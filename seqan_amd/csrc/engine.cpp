@@ -249,6 +249,17 @@ bool driftNarrow(const ScoringInfo &si, const Drift &dr, bool local, int64_t n, 
            dr.bias + (int64_t)std::max(0, si.sMax) * (std::min(n, m) + kDriftSlack) + dr.d * span <= kDriftNarrowMax;
 }
 
+// What a path inside a band of W1 + 1 diagonals can lose, in drifted values,
+// on the way to a cell up to maxM rows down: no more than by gaps of the
+// band's width right and down in turn, or by mismatches along a diagonal.
+// (The plain bias covers two gaps, which reach any cell of a whole matrix.)
+int64_t bandDrop(const ScoringInfo &si, const Drift &dr, int64_t W1, int64_t maxM)
+{
+    const int64_t zigzag = dr.cost * (2 * ((maxM + W1 - 1) / W1) + 6);
+    const int64_t diagonal = std::max<int64_t>(0, -((int64_t)si.sMin + 2 * dr.d)) * maxM + 3 * dr.cost;
+    return std::min(zigzag, diagonal);
+}
+
 // Conservative range of every value a pair can produce inside the DP (H, E, F
 // and H + gapOpen), from the sizes alone.  H <= max(0, sMax) * min(n, m) since
 // gap costs are <= 0.  H(i,j) >= the score of the all-gap path along row 0
@@ -352,6 +363,12 @@ struct LongCost {
     double alone, full;
 };
 constexpr LongCost kLongCosts[] = {{4, 115, 63}, {8, 153, 111}, {16, 230, 203}};
+// Banded scores, ns: a column of a packed item's block (one wave per SIMD);
+// a row of a pair on the int32 kernels, alone and per SIMD of a full chip
+// (wide: of 64 diagonals).  1,000 to 65,536 pairs: free ends, 1 kbp, 201
+// diagonals, packed 3.9-4.0 ms, int32 2.5, 3.3 (4,096), 12.9 (16,384) and
+// 51.8; local, 150 bp, 33 diagonals, 0.19-0.20 against 0.04, 0.06, 0.19, 0.67.
+constexpr double kBandColumn = 310, kBandNarrowLone = 270, kBandNarrowFull = 70, kBandWideLone = 615, kBandWideFull = 202;
 // Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
 constexpr int64_t kResidentWaves = 3072;
 // Rows per unit of the group shapes' row counts.
@@ -2777,9 +2794,9 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
                 upErr = uploadResidues(ctx, setH, setV, in);
         });
 
-    // Route: empty pairs (INT32_MIN), the packed int16 kernel (global
-    // alignment, values inside the int16 window, at least 8 diagonals past
-    // the first), narrow bands (<= 64 diagonals), wide bands.
+    // Route: empty pairs (INT32_MIN), the packed int16 kernel (values inside
+    // 16 bits, at least 8 diagonals past the first), narrow bands (<= 64
+    // diagonals), wide bands.
     const auto tPlan = std::chrono::steady_clock::now();
     ScoringInfo si{};
     si.alpha = scoring->alphabet_size;
@@ -2799,15 +2816,44 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     // bp: R = 12 1.64 ms, 16 1.74 ms; [-100, 100] on 65,536 pairs of 1 kbp:
     // R = 16 4.66 ms, 12 5.10 ms.
     int bandR = W1 >= 64 ? 16 : W1 >= 24 ? 12 : 8;
-    if (const char *env = std::getenv("SQMI_BAND_ROWS")) {   // tuning knob: 8, 12 or 16 rows per block
+    if (const char *env = std::getenv("SQMI_BAND_ROWS")) {   // tuning knob: 12 or 16 rows per block
         const int r = std::atoi(env);
-        bandR = r == 8 ? 8 : (r == 12 || r == 16) && W1 >= r ? r : bandR;
+        bandR = W1 >= 24 && (r == 12 || r == 16) ? r : bandR;
     }
-    const bool packedOk = mode == 0 && !(flags & SQMI_FORCE_INT32) && W1 >= bandR && si.o <= 0 && si.e <= 0 &&
-                          si.o >= -1024 && si.e >= -1024 && si.sMax <= 1024 && si.sMin >= -1024 && si.alpha + 1 <= 33 &&
-                          lower_diag > -30000 && upper_diag < 30000;
+    si.dnaDrift = si.dna && si.sMax - si.o - std::max(si.o, si.e) <= 255;
+    const bool bandCostsOk = !(flags & SQMI_FORCE_INT32) && W1 >= bandR && si.o <= 0 && si.e <= 0 && si.o >= -1024 &&
+                             si.e >= -1024 && si.sMax <= 1024 && si.sMin >= -1024 && si.alpha + 1 <= 33 &&
+                             lower_diag > -30000 && upper_diag < 30000;
+    // The packed kernel's values: the bias covers the longest pair of the
+    // call; columns run to the item's longest |H|, a group past the band.
+    Drift dr = driftOf(si, local);
+    int64_t maxN = 1, maxM = 1;
+#pragma omp parallel for schedule(static) reduction(max : maxN, maxM) if (N > kParallelMin)
+    for (int64_t i = 0; i < N; ++i) {
+        maxN = std::max(maxN, setH->offsets[i + 1] - setH->offsets[i]);
+        maxM = std::max(maxM, setV->offsets[i + 1] - setV->offsets[i]);
+    }
+    if (!local && bandCostsOk)
+        dr.bias += (int32_t)std::min<int64_t>(bandDrop(si, dr, W1, maxM), 1 << 20);
+    auto bandTop = [&](int64_t m) {   // the largest stored value of pairs with m rows
+        const int64_t cols = std::min(maxN, m + upper_diag) + 8;
+        return dr.bias + (int64_t)std::max(si.sMax, 0) * std::min(m, cols) + dr.d * (local ? 17 : m + cols);
+    };
+    const bool narrowT = dr.neg == (local ? 2 * dr.d + 2 : dr.cost + 1);   // no t below 0
+    bool bandWide = !narrowT;
+    const bool packedOk = bandCostsOk;
     std::vector<int32_t> narrow, wide, rejected, packed;
     int64_t wNarrow = 1, wWide = 0, cells = 0;
+    auto toInt32 = [&](int32_t id, int64_t n, int64_t m) {
+        const int64_t w = std::min<int64_t>(upper_diag, n) - std::max<int64_t>(lower_diag, -m) + 1;
+        if (w <= 64) {
+            narrow.push_back(id);
+            wNarrow = std::max(wNarrow, w);
+        } else {
+            wide.push_back(id);
+            wWide = std::max(wWide, w);
+        }
+    };
     for (int64_t i = 0; i < N; ++i) {
         const int64_t n = setH->offsets[i + 1] - setH->offsets[i], m = setV->offsets[i + 1] - setV->offsets[i];
         if (n == 0 || m == 0) {
@@ -2821,17 +2867,32 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
                                    : ": needs |H| >= 2 and lower_diag < min(0, |H| - |V|) < max(0, |H| - |V|) "
                                      "< upper_diag"));
         cells += n * m;
-        if (packedOk && fitsInt16(si, n, m, false)) {
+        if (packedOk && n <= 30000 && m <= 30000 && bandTop(m) <= 65535) {
             packed.push_back((int32_t)i);
+            bandWide |= bandTop(m) > kDriftNarrowMax;
             continue;
         }
-        const int64_t w = std::min<int64_t>(upper_diag, n) - std::max<int64_t>(lower_diag, -m) + 1;
-        if (w <= 64) {
-            narrow.push_back((int32_t)i);
-            wNarrow = std::max(wNarrow, w);
-        } else {
-            wide.push_back((int32_t)i);
-            wWide = std::max(wWide, w);
+        toInt32((int32_t)i, n, m);
+    }
+    // Free end gaps and local alignment, few pairs: a packed item takes its
+    // whole sweep, however few the items; the int32 kernels, which spread a
+    // pair's band over a wave, are done earlier.
+    if (mode != 0 && !packed.empty() && !envFlag("SQMI_BAND_PACKED")) {
+        double items = 0, blockCols = 0, lone = 0, full = 0;
+        std::vector<int32_t> perM((size_t)maxM + 1, 0);
+        for (int32_t id : packed) {
+            const int64_t n = setH->offsets[id + 1] - setH->offsets[id], m = setV->offsets[id + 1] - setV->offsets[id];
+            items += perM[(size_t)m]++ % 128 == 0;
+            const double w = (double)std::min<int64_t>(W1 + 1, n + m), chunks = std::ceil(w / 64);
+            blockCols = std::max(blockCols, (double)(m / bandR + 1) * std::min<double>(w + bandR, (double)n));
+            lone = std::max(lone, (double)m * (w <= 64 ? kBandNarrowLone : kBandWideLone * chunks));
+            full += (double)m * (w <= 64 ? kBandNarrowFull * w / 64 : kBandWideFull * chunks);
+        }
+        const double simds = 4.0 * std::max(1, ctx->numCUs);
+        if (std::max(lone, full / simds) < std::ceil(items / simds) * blockCols * kBandColumn) {
+            for (int32_t id : packed)
+                toInt32(id, setH->offsets[id + 1] - setH->offsets[id], setV->offsets[id + 1] - setV->offsets[id]);
+            packed.clear();
         }
     }
     int seg = 1;
@@ -2893,22 +2954,23 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
         (err = hipMemcpyAsync(dIds, all.data(), 4 * all.size(), hipMemcpyHostToDevice, stream)) != hipSuccess)
         return hipFail(ctx, err, "uploading banded pair lists");
     int bandGrid = 0, bandRowColsN = 0, bandLds = 0;
+    BandVariant bandVar{};
     if (!bandItems.empty()) {
         // Workgroups of 4 waves per CU: the occupancy limit, but no more than
         // keep the row-buffer rings of a CU's waves within its share of L2
         // (at least one).  On 1 M pairs of 150 bp, band [-16, 16] (rings of
         // 32 KB per wave), 1, 2 and 3 workgroups per CU ran 1.92, 2.09 and
         // 2.61 ms: the rings of more waves than L2 holds go to memory.
-        // Rings of up to 64 columns (128 KB per workgroup) live in LDS
-        // (SQMI_BAND_LDS=0 keeps them in global memory), which also limits
-        // the CU to the workgroups whose rings fit.
+        // Rings of up to 64 columns (128 KB per workgroup) live in LDS, which
+        // also limits the CU to the workgroups whose rings fit.
         bandRowColsN = bandRingCols(bandMaxN, lower_diag, upper_diag, bandR);
-        const char *ldsEnv = std::getenv("SQMI_BAND_LDS");
-        bandLds = (ldsEnv && ldsEnv[0] == '0') ? 0 : bandLdsRingBytes(bandR, si.dna, bandRowColsN);
+        bandLds = bandR == 16 ? 0 : bandLdsRingBytes(bandRowColsN);
+        bandVar = BandVariant{bandR, local ? si.dna : si.dnaDrift,
+                              local ? kBandLocal : (mode & (SQMI_FREE_BOTTOM | SQMI_FREE_RIGHT)) ? kBandFree : kBandEnd,
+                              bandWide, bandLds > 0};
         const int64_t ringBytes = (int64_t)64 * bandRowColsN * 8;   // per wave
-        const int occ = bandLds ? occupancyBand16(bandR, si.dna, bandLds)
-                                : (int)std::max<int64_t>(1, std::min<int64_t>(occupancyBand16(bandR, si.dna, 0),
-                                                                              ctx->l2PerCU / (4 * ringBytes)));
+        const int most = occupancyBand16(bandVar, bandLds);
+        const int occ = bandLds ? most : (int)std::max<int64_t>(1, std::min<int64_t>(most, ctx->l2PerCU / (4 * ringBytes)));
         const int64_t nIt = (int64_t)bandItems.size();
         bandGrid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occ, (nIt + 3) / 4));
         if ((err = ensure(ctx->b.order, 4 * bandOrder.size())) != hipSuccess ||
@@ -2946,9 +3008,10 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
         f.alpha = si.alpha;
         f.tTable = static_cast<const int16_t *>(ctx->b.tTable.p);
         f.dnaProfile = static_cast<const uint32_t *>(ctx->b.dnaProf.p);
+        f.drift = dr;
         f.bandLo = (int32_t)lower_diag;
         f.bandUp = (int32_t)upper_diag;
-        if ((err = launchBand16(bandR, si.dna, f, bandGrid, bandLds, stream)) != hipSuccess)
+        if ((err = launchBand16(bandVar, f, bandGrid, bandLds, stream)) != hipSuccess)
             return hipFail(ctx, err, "launching packed banded kernel");
     }
     BandedArgs a{};

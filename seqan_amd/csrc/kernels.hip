@@ -7,6 +7,7 @@
 
 #include "kernels.hpp"
 #include "packed16.hpp"
+#include "band16_parts.hpp"
 #include "score16_parts.hpp"
 #include "seqan_amd.h"
 
@@ -750,6 +751,54 @@ int occupancyScore16(bool dna, int kind)
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, scoreKernel(dna, kind), 256, 0) != hipSuccess)
         return 1;
     return blocks > 0 ? blocks : 1;
+}
+
+static const void *bandKernel(const BandVariant &v)
+{
+    using Part = const void *(*)(int, bool, bool);
+    static constexpr Part parts[2][3] = {{bandTabEnd, bandTabFree, bandTabLocal}, {bandDnaEnd, bandDnaFree, bandDnaLocal}};
+    return v.kind < 0 || v.kind > 2 ? nullptr : parts[v.dna][v.kind](v.R, v.wide, v.lds);
+}
+
+int bandRingCols(int maxN, int64_t lower, int64_t upper, int R)
+{
+    // The smallest power of two of at least W - 1 + R + 10 columns; when that
+    // reaches the pair's whole width the buffer is linear (a power of two
+    // no smaller than bandRowCols).
+    const int64_t need = std::min<int64_t>(upper - lower + R + 10, (int64_t)bandRowCols(maxN));
+    int c = 1;
+    while (c < need)
+        c <<= 1;
+    return c;
+}
+
+int bandLdsRingBytes(int bandCols)
+{
+    // Four waves' rings of bandCols columns x 64 lanes x 8 bytes, when they
+    // leave room for the static tables in the 160 KB of LDS per CU.
+    const int64_t bytes = (int64_t)4 * 64 * bandCols * 8;
+    return bytes > 128 * 1024 ? 0 : (int)bytes;
+}
+
+int occupancyBand16(const BandVariant &v, int ringLdsBytes)
+{
+    const void *k = bandKernel(v);
+    int blocks = 0;
+    if (!k || (v.lds && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, ringLdsBytes) != hipSuccess))
+        return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, (size_t)ringLdsBytes) != hipSuccess)
+        return 1;
+    return blocks > 0 ? blocks : 1;
+}
+
+hipError_t launchBand16(const BandVariant &v, const FwdArgs &args, int gridBlocks, int ringLdsBytes, hipStream_t stream)
+{
+    const void *k = bandKernel(v);
+    if (!k)
+        return hipErrorInvalidValue;
+    FwdArgs copy = args;
+    void *params[] = {&copy};
+    return hipLaunchKernel(k, dim3(gridBlocks), dim3(256), params, (size_t)ringLdsBytes, stream);
 }
 
 hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBlocks, hipStream_t stream,

@@ -244,17 +244,26 @@ hipError_t launchSimple32(const Simple32Args &args, hipStream_t stream);
 // x 64 lanes of (G, F) pairs (8 bytes each).
 bool laneSupported(const Variant16 &v);
 int laneRowCols(int maxN, int R);
-// Packed banded global alignment (band16.hip): one pair couple per lane, R in
-// {8, 12, 16} rows per block, bandUp - bandLo >= R; work items hold up to 128
-// pairs of one length m (WorkItem.count = pairs | m << 16, nblocks =
-// (m + R) / R).  Row buffer per wave slot: a ring of bandRingCols(...)
-// columns x 64 lanes x 8 bytes.
-int bandRowCols(int maxN);
+// Packed banded scores (band16.hpp): one pair couple per lane, R rows per
+// block, bandUp - bandLo >= R; work items hold up to 128 pairs of one length m
+// (WorkItem.count = pairs | m << 16, nblocks = (m + R) / R).  Row buffer per
+// wave slot: a ring of bandRingCols(...) columns x 64 lanes x 8 bytes, in LDS
+// where bandLdsRingBytes() > 0.  R: 8 with LDS rings, 12 with either, 16 with
+// rings in memory.
+enum BandKind : int { kBandEnd = 0, kBandFree = 1, kBandLocal = 2 };   // cell (m, n); free last row / column; local
+struct BandVariant {
+    int R;
+    bool dna;
+    int kind;
+    bool wide;      // values above kDriftNarrowMax
+    bool lds;
+};
+constexpr int bandRowCols(int maxN) { return (maxN + 3) / 4 * 4 + 5; }
 int bandRingCols(int maxN, int64_t lower, int64_t upper, int R);
-// LDS bytes of the rings when they fit in LDS (the kernel's LDS form), else 0.
-int bandLdsRingBytes(int R, bool dna, int bandCols);
-int occupancyBand16(int R, bool dna, int ringLdsBytes);
-hipError_t launchBand16(int R, bool dna, const FwdArgs &args, int gridBlocks, int ringLdsBytes, hipStream_t stream);
+// LDS bytes of a workgroup's rings, 0 where they do not fit.
+int bandLdsRingBytes(int bandCols);
+int occupancyBand16(const BandVariant &v, int ringLdsBytes);
+hipError_t launchBand16(const BandVariant &v, const FwdArgs &args, int gridBlocks, int ringLdsBytes, hipStream_t stream);
 int occupancyLane16(const Variant16 &v);
 hipError_t launchLane16(const Variant16 &v, const FwdArgs &args, int gridBlocks, hipStream_t stream);
 
