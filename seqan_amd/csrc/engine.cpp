@@ -45,6 +45,10 @@ struct DevBuf
     void *p = nullptr;
     size_t cap = 0;
     Arena *arena = nullptr;   // set: carve from this arena instead of hipMalloc
+    // p lies in the context's stage; the buffer's own memory waits here.
+    bool view = false;
+    void *own = nullptr;
+    size_t ownCap = 0;
 };
 
 // Every device buffer a context keeps between calls.
@@ -95,6 +99,20 @@ struct sqmi_context
     hipStream_t longStreams[kMaxLongStreams] = {};
     hipEvent_t longFork = nullptr, longJoin[kMaxLongStreams] = {};
     Buffers b;
+    // A call's offsets, tables and work lists go through pinned memory to
+    // one device buffer (stageBegin, put, stageFlush).
+    DevBuf stage;
+    char *pin = nullptr;
+    size_t pinCap = 0, pinUsed = 0, pinSent = 0;
+    bool pinOn = false;      // the running call stages its uploads
+    struct Down {
+        void *dst;
+        const void *src;
+        size_t bytes;
+    };
+    std::vector<Down> down;  // results on their way through `pin` (fetch, deliver)
+    size_t downUsed = 0, downCap = 0;
+    bool pinBusy = false;    // copies from `pin` may be in flight
     Planned *planned = nullptr;   // the calls' plans, one after the other (owned)
     // The no-allocation entry point: this device's scratch array (its device
     // address, from hipGetSymbolAddress at creation) and, during such a
@@ -106,12 +124,14 @@ struct sqmi_context
     Arena arena;
     bool noAlloc = false;   // inside sqmi_align_score_noalloc
     // The last sqmi_align_score call, kept for an identical next call: the
-    // key of its inputs, its statistics and its launches as an instantiated
-    // HIP graph.  Its plan lives on in the context's device buffers, so any
+    // key of its inputs, its statistics and its launches, from the second
+    // such call on as an instantiated HIP graph (to capture and instantiate one
+    // takes 60-80 us, which a call that comes once does not get back).  Its plan lives on in the context's device buffers, so any
     // other call on the context drops it.
     struct Replay {
         bool valid = false;
         uint64_t key = 0;
+        std::vector<std::function<hipError_t()>> launches;   // until the second such call captures them
         hipGraphExec_t exec = nullptr;
         sqmi_stats stats{};
     } replay;
@@ -132,10 +152,20 @@ sqmi_status hipFail(sqmi_context *ctx, hipError_t err, const char *what)
     return fail(ctx, err == hipErrorOutOfMemory ? SQMI_ERR_OUT_OF_MEMORY : SQMI_ERR_DEVICE, msg);
 }
 
+void endView(DevBuf &b)
+{
+    if (!b.view)
+        return;
+    b.p = b.own;
+    b.cap = b.ownCap;
+    b.view = false;
+}
+
 hipError_t ensure(DevBuf &b, size_t bytes)
 {
     if (bytes == 0)
         bytes = 16;
+    endView(b);
     if (b.cap >= bytes)
         return hipSuccess;
     if (b.arena) {
@@ -176,6 +206,26 @@ void dropReplay(sqmi_context *ctx)
     ctx->replay = sqmi_context::Replay{};
 }
 
+// The kept launches as an instantiated graph; a capture the runtime refuses
+// leaves them to be run one by one.
+void captureReplay(sqmi_context *ctx)
+{
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    if (hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal) == hipSuccess) {
+        hipError_t err = hipSuccess;
+        for (auto &f : ctx->replay.launches)
+            if (err == hipSuccess)
+                err = f();
+        const hipError_t end = hipStreamEndCapture(ctx->stream, &graph);
+        if (err == hipSuccess && end == hipSuccess && graph && hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess)
+            ctx->replay.exec = exec;
+        if (graph)
+            (void)hipGraphDestroy(graph);
+    }
+    (void)hipGetLastError();   // a refused capture leaves its error behind
+}
+
 uint64_t mix64(uint64_t x)
 {
     x ^= x >> 33;
@@ -202,10 +252,153 @@ size_t arenaBytes(size_t bytes) { return ((bytes ? bytes : 16) + 255) & ~(size_t
 
 void release(DevBuf &b)
 {
+    endView(b);
     if (b.p && !b.arena)
         (void)hipFree(b.p);
     b.p = nullptr;
     b.cap = 0;
+}
+
+// Staged uploads.  A call's small arrays (offsets, tables, work lists) are
+// gathered in pinned memory and sent together: a copy from pageable memory
+// takes 8-12 us each, whatever its size, and large ones run at one thread's
+// memcpy.  Results come back the same way (20 MB to pageable memory 1.13 ms,
+// to pinned memory 0.38 and 0.03 from there).  stageBegin: `bytes` bounds what the call will put (each array
+// rounded up to 256 bytes), `down` what it will fetch; more than kMaxDown goes
+// straight to the caller's memory.
+constexpr size_t kMaxDown = (size_t)256 << 20;
+hipError_t stageBegin(sqmi_context *ctx, size_t bytes, size_t down = 0)
+{
+    ctx->pinOn = false;
+    ctx->downUsed = ctx->downCap = 0;
+    ctx->down.clear();
+    if (ctx->pinBusy) {   // an earlier call failed between its uploads and its end
+        const hipError_t e = hipDeviceSynchronize();
+        if (e != hipSuccess)
+            return e;
+        ctx->pinBusy = false;
+    }
+    if (ctx->noAlloc)
+        return hipSuccess;
+    if (down > kMaxDown)
+        down = 0;
+    if (ctx->pinCap < std::max(bytes, down)) {
+        if (ctx->pin)
+            (void)hipHostFree(ctx->pin);
+        ctx->pin = nullptr;
+        ctx->pinCap = 0;
+        const size_t cap = std::max(bytes, down) + std::max(bytes, down) / 4;
+        void *p = nullptr;
+        const hipError_t e = hipHostMalloc(&p, cap, hipHostMallocDefault);
+        if (e != hipSuccess)
+            return e;
+        ctx->pin = static_cast<char *>(p);
+        ctx->pinCap = cap;
+    }
+    const hipError_t e = ensure(ctx->stage, bytes);
+    if (e != hipSuccess)
+        return e;
+    ctx->downCap = down;
+    ctx->pinUsed = ctx->pinSent = 0;
+    ctx->pinOn = true;
+    return hipSuccess;
+}
+
+// Sends what has been put since the last flush.
+hipError_t stageFlush(sqmi_context *ctx)
+{
+    if (!ctx->pinOn || ctx->pinSent == ctx->pinUsed)
+        return hipSuccess;
+    ctx->pinBusy = true;
+    const hipError_t e = hipMemcpyAsync(static_cast<char *>(ctx->stage.p) + ctx->pinSent, ctx->pin + ctx->pinSent,
+                                        ctx->pinUsed - ctx->pinSent, hipMemcpyHostToDevice, ctx->stream);
+    ctx->pinSent = ctx->pinUsed;
+    return e;
+}
+
+// The call's stream is synchronised.
+void stageEnd(sqmi_context *ctx) { ctx->pinOn = ctx->pinBusy = false; }
+
+size_t stageBytes(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+
+// A host copy, by all threads from 2 MB on.
+constexpr size_t kParallelCopy = (size_t)2 << 20;
+void copyBytes(void *dst, const void *src, size_t len)
+{
+    if (len < kParallelCopy) {
+        if (len)
+            std::memcpy(dst, src, len);
+        return;
+    }
+    constexpr size_t kPart = (size_t)512 << 10;
+    const int64_t parts = (int64_t)((len + kPart - 1) / kPart);
+#pragma omp parallel for schedule(static)
+    for (int64_t q = 0; q < parts; ++q)
+        std::memcpy(static_cast<char *>(dst) + q * kPart, static_cast<const char *>(src) + q * kPart,
+                    std::min(kPart, len - (size_t)q * kPart));
+}
+
+// dst receives src[0 .. bytes) of device memory by the next deliver() after a
+// synchronisation of the stream.  (The uploads from the same pinned memory
+// precede the results in the stream.)
+hipError_t fetch(sqmi_context *ctx, void *dst, const void *src, size_t bytes)
+{
+    if (ctx->downUsed + stageBytes(bytes) > ctx->downCap)
+        return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream);
+    ctx->down.push_back({dst, ctx->pin + ctx->downUsed, bytes});
+    ctx->pinBusy = true;
+    const hipError_t e = hipMemcpyAsync(ctx->pin + ctx->downUsed, src, bytes, hipMemcpyDeviceToHost, ctx->stream);
+    ctx->downUsed += stageBytes(bytes);
+    return e;
+}
+
+// The first n fetched arrays, to their places.
+void deliver(sqmi_context *ctx, size_t n)
+{
+    for (size_t k = 0; k < n; ++k)
+        copyBytes(ctx->down[k].dst, ctx->down[k].src, ctx->down[k].bytes);
+    ctx->down.erase(ctx->down.begin(), ctx->down.begin() + n);
+}
+void deliver(sqmi_context *ctx) { deliver(ctx, ctx->down.size()); }
+
+struct Piece {
+    const void *src;
+    size_t bytes;
+};
+
+// b holds the pieces, one after the other, in device memory once the stage is
+// flushed (or, where the call does not stage or they do not fit, once the
+// stream has run the copies).
+hipError_t put(sqmi_context *ctx, DevBuf &b, const Piece *pieces, size_t n)
+{
+    size_t bytes = 0, at = 0;
+    for (size_t k = 0; k < n; ++k)
+        bytes += pieces[k].bytes;
+    if (!ctx->pinOn || ctx->pinUsed + stageBytes(bytes) > std::min(ctx->pinCap, ctx->stage.cap)) {
+        hipError_t e = ensure(b, bytes);
+        for (size_t k = 0; k < n && e == hipSuccess; at += pieces[k++].bytes)
+            if (pieces[k].bytes)
+                e = hipMemcpyAsync(static_cast<char *>(b.p) + at, pieces[k].src, pieces[k].bytes, hipMemcpyHostToDevice,
+                                   ctx->stream);
+        return e;
+    }
+    endView(b);
+    b.own = b.p;
+    b.ownCap = b.cap;
+    b.view = true;
+    b.p = static_cast<char *>(ctx->stage.p) + ctx->pinUsed;
+    b.cap = bytes;
+    char *dst = ctx->pin + ctx->pinUsed;
+    ctx->pinUsed += stageBytes(bytes);
+    for (size_t k = 0; k < n; at += pieces[k++].bytes)
+        copyBytes(dst + at, pieces[k].src, pieces[k].bytes);
+    // Large arrays are on their way while the next one is gathered.
+    return bytes < kParallelCopy ? hipSuccess : stageFlush(ctx);
+}
+hipError_t put(sqmi_context *ctx, DevBuf &b, const void *src, size_t bytes)
+{
+    const Piece one{src, bytes};
+    return put(ctx, b, &one, 1);
 }
 
 struct ScoringInfo
@@ -383,6 +576,10 @@ int64_t blocksFor(const Variant16 &v, int64_t m)
     return (br & (br - 1)) == 0 ? (m + br) >> __builtin_ctzll((unsigned long long)br) : (m + br) / br;
 }
 
+// Calls with at most this many pairs plan on one thread: waking the thread
+// team costs more than it saves.
+constexpr int64_t kParallelMin = 32768;
+
 sqmi_status checkSet(sqmi_context *ctx, const sqmi_sequences *s, const char *name)
 {
     if (!s)
@@ -395,9 +592,14 @@ sqmi_status checkSet(sqmi_context *ctx, const sqmi_sequences *s, const char *nam
         return fail(ctx, SQMI_ERR_UNSUPPORTED, std::string(name) + ": more than 2^31-2 sequences");
     if (s->count > 0 && s->offsets[0] < 0)
         return fail(ctx, SQMI_ERR_INVALID_ARGUMENT, std::string(name) + ": negative offset");
-    for (int64_t i = 0; i < s->count; ++i)
-        if (s->offsets[i + 1] < s->offsets[i])
-            return fail(ctx, SQMI_ERR_INVALID_ARGUMENT, std::string(name) + ": offsets not monotone");
+    const int64_t n = s->count;
+    const int64_t *off = s->offsets;
+    bool bad = false;
+#pragma omp parallel for schedule(static) reduction(|| : bad) if (n > kParallelMin)
+    for (int64_t i = 0; i < n; ++i)
+        bad = bad || off[i + 1] < off[i];
+    if (bad)
+        return fail(ctx, SQMI_ERR_INVALID_ARGUMENT, std::string(name) + ": offsets not monotone");
     return SQMI_OK;
 }
 
@@ -530,10 +732,6 @@ int longStreams()
 }
 
 
-// Calls with at most this many pairs plan on one thread: waking the thread
-// team costs more than it saves.
-constexpr int64_t kParallelMin = 32768;
-
 // Stable LSD radix sort of 28-bit keys in two passes of 14 bits, each pass
 // split into contiguous per-thread ranges so that equal digits keep their
 // input order.
@@ -542,6 +740,10 @@ void radixSort(RawVec<Key> &keys, RawVec<Key> &tmp, std::vector<uint32_t> &hist)
     const size_t n = keys.size();
     if (n < 2)
         return;
+    if (n <= 1024) {   // clearing and summing the digit counts takes longer (30 us)
+        std::stable_sort(keys.begin(), keys.end(), [](const Key &a, const Key &b) { return a.key < b.key; });
+        return;
+    }
     tmp.resize(n);
     int T = 1;
 #ifdef _OPENMP
@@ -1117,6 +1319,21 @@ struct Inputs
     uint32_t prof[16] = {};
 };
 
+// Residue sets of up to this many bytes go through the stage.
+constexpr int64_t kStageResidues = (int64_t)1 << 20;
+
+// Bytes uploadInputs() puts into the stage, at most.
+size_t stageInputs(const sqmi_sequences *setH, const sqmi_sequences *setV, const sqmi_scoring *scoring, uint32_t flags)
+{
+    const int64_t N = setH->count, A = scoring->alphabet_size;
+    size_t bytes = 2 * stageBytes(8 * (N + 1)) + stageBytes(2 * (A + 1) * (A + 1)) + stageBytes(64) + stageBytes(4 * A * A);
+    if (!(flags & SQMI_RESIDUES_ON_DEVICE) && setH->offsets[N] + setV->offsets[N] <= kStageResidues)
+        bytes += stageBytes(setH->offsets[N]) + stageBytes(setV->offsets[N]) + 512;
+    return bytes;
+}
+
+size_t downScores(int64_t N, uint32_t flags) { return flags & SQMI_SCORES_ON_DEVICE ? 0 : stageBytes(4 * (size_t)N); }
+
 // A host thread that is joined when it goes out of scope (early returns
 // included).
 struct JoinedThread {
@@ -1139,7 +1356,15 @@ hipError_t uploadResidues(sqmi_context *ctx, const sqmi_sequences *setH, const s
     const int64_t N = setH->count;
     const int64_t hTot = setH->offsets[N], vTot = setV->offsets[N];
     hipError_t err;
-    if ((err = ensure(ctx->b.hRes, hTot + 64)) != hipSuccess || (err = ensure(ctx->b.vRes, vTot + 64)) != hipSuccess ||
+    if (ctx->pinOn && hTot + vTot <= kStageResidues) {
+        // (64 bytes of slack after the residues, as below.)
+        if ((err = put(ctx, ctx->b.hRes, setH->residues, hTot)) != hipSuccess)
+            return err;
+        ctx->pinUsed = std::min(std::min(ctx->pinCap, ctx->stage.cap), ctx->pinUsed + 256);
+        if ((err = put(ctx, ctx->b.vRes, setV->residues, vTot)) != hipSuccess)
+            return err;
+        ctx->pinUsed = std::min(std::min(ctx->pinCap, ctx->stage.cap), ctx->pinUsed + 256);
+    } else if ((err = ensure(ctx->b.hRes, hTot + 64)) != hipSuccess || (err = ensure(ctx->b.vRes, vTot + 64)) != hipSuccess ||
         (err = hipMemcpyAsync(ctx->b.hRes.p, setH->residues, hTot, hipMemcpyHostToDevice, ctx->stream)) !=
             hipSuccess ||
         (err = hipMemcpyAsync(ctx->b.vRes.p, setV->residues, vTot, hipMemcpyHostToDevice, ctx->stream)) != hipSuccess)
@@ -1154,7 +1379,6 @@ sqmi_status uploadInputs(sqmi_context *ctx, const sqmi_sequences *setH, const sq
                          const sqmi_scoring *scoring, const ScoringInfo &si, int32_t *scores, uint32_t flags,
                          Inputs &in)
 {
-    hipStream_t stream = ctx->stream;
     const int64_t N = setH->count;
     hipError_t err;
     const uint8_t *dH = setH->residues, *dV = setV->residues;
@@ -1164,10 +1388,8 @@ sqmi_status uploadInputs(sqmi_context *ctx, const sqmi_sequences *setH, const sq
         dH = in.dH;
         dV = in.dV;
     }
-    if ((err = ensure(ctx->b.hOff, 8 * (N + 1))) != hipSuccess || (err = ensure(ctx->b.vOff, 8 * (N + 1))) != hipSuccess)
-        return hipFail(ctx, err, "allocating offsets");
-    if ((err = hipMemcpyAsync(ctx->b.hOff.p, setH->offsets, 8 * (N + 1), hipMemcpyHostToDevice, stream)) != hipSuccess ||
-        (err = hipMemcpyAsync(ctx->b.vOff.p, setV->offsets, 8 * (N + 1), hipMemcpyHostToDevice, stream)) != hipSuccess)
+    if ((err = put(ctx, ctx->b.hOff, setH->offsets, 8 * (N + 1))) != hipSuccess ||
+        (err = put(ctx, ctx->b.vOff, setV->offsets, 8 * (N + 1))) != hipSuccess)
         return hipFail(ctx, err, "copying offsets");
     int32_t *dScores = scores;
     if (!(flags & SQMI_SCORES_ON_DEVICE)) {
@@ -1190,12 +1412,9 @@ sqmi_status uploadInputs(sqmi_context *ctx, const sqmi_sequences *setH, const sq
                 prof[h] |= (uint32_t)(scoring->table[h * A + v] - si.o) << (8 * v);
                 prof[8 + v] |= (uint32_t)(scoring->table[h * A + v] - si.o) << (8 * h);
             }
-    if ((err = ensure(ctx->b.tTable, tTab.size() * 2)) != hipSuccess || (err = ensure(ctx->b.dnaProf, 64)) != hipSuccess ||
-        (err = ensure(ctx->b.table32, 4 * A * A)) != hipSuccess)
-        return hipFail(ctx, err, "allocating tables");
-    if ((err = hipMemcpyAsync(ctx->b.tTable.p, tTab.data(), tTab.size() * 2, hipMemcpyHostToDevice, stream)) != hipSuccess ||
-        (err = hipMemcpyAsync(ctx->b.dnaProf.p, prof, 64, hipMemcpyHostToDevice, stream)) != hipSuccess ||
-        (err = hipMemcpyAsync(ctx->b.table32.p, scoring->table, 4 * A * A, hipMemcpyHostToDevice, stream)) != hipSuccess)
+    if ((err = put(ctx, ctx->b.tTable, tTab.data(), tTab.size() * 2)) != hipSuccess ||
+        (err = put(ctx, ctx->b.dnaProf, prof, 64)) != hipSuccess ||
+        (err = put(ctx, ctx->b.table32, scoring->table, 4 * A * A)) != hipSuccess)
         return hipFail(ctx, err, "copying tables");
     in.dH = dH;
     in.dV = dV;
@@ -1690,6 +1909,9 @@ sqmi_status sqmi_destroy(sqmi_context *ctx)
         (void)hipEventDestroy(ctx->longFork);
     if (ctx->ownStream)
         (void)hipStreamDestroy(ctx->ownStream);
+    release(ctx->stage);
+    if (ctx->pin)
+        (void)hipHostFree(ctx->pin);
     if (ctx->waitFlag)
         (void)hipHostFree(ctx->waitFlag);
     delete ctx->planned;
@@ -1760,6 +1982,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         }
         if (flags & SQMI_SCORES_ON_DEVICE)
             scal.push_back((int64_t)(uintptr_t)scores);
+        scal.push_back((int64_t)(uintptr_t)stream);   // the kept launches name it
         for (const char *name : {"SQMI_COOP_MIN_BLOCKS", "SQMI_LONG_ALL", "SQMI_LONG_MIN_SIDE", "SQMI_LONG_STREAMS", "SQMI_LONG_ROWS",
                                  "SQMI_SHAPE_RULE", "SQMI_TRACE_BUDGET_MB", "SQMI_ROW_UNITS", "SQMI_BIN_SHAPES"}) {
             const char *v = std::getenv(name);
@@ -1776,10 +1999,20 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
                 ((err = hipMemcpyAsync(ctx->b.hRes.p, rH, hTot, hipMemcpyHostToDevice, stream)) != hipSuccess ||
                  (err = hipMemcpyAsync(ctx->b.vRes.p, rV, vTot, hipMemcpyHostToDevice, stream)) != hipSuccess))
                 return hipFail(ctx, err, "copying residues");
-            if ((err = hipEventRecord(ctx->ev0, stream)) != hipSuccess ||
-                (err = hipGraphLaunch(ctx->replay.exec, stream)) != hipSuccess ||
-                (err = hipEventRecord(ctx->ev1, stream)) != hipSuccess)
-                return hipFail(ctx, err, "launching the call's graph");
+            if (!ctx->replay.exec)
+                captureReplay(ctx);
+            if ((err = hipEventRecord(ctx->ev0, stream)) != hipSuccess)
+                return hipFail(ctx, err, "event");
+            if (ctx->replay.exec) {
+                if ((err = hipGraphLaunch(ctx->replay.exec, stream)) != hipSuccess)
+                    return hipFail(ctx, err, "launching the call's graph");
+            } else {
+                for (auto &f : ctx->replay.launches)
+                    if ((err = f()) != hipSuccess)
+                        return hipFail(ctx, err, "launching alignment kernels");
+            }
+            if ((err = hipEventRecord(ctx->ev1, stream)) != hipSuccess)
+                return hipFail(ctx, err, "event");
             if (!(flags & SQMI_SCORES_ON_DEVICE) &&
                 (err = hipMemcpyAsync(scores, ctx->b.scores.p, 4 * N, hipMemcpyDeviceToHost, stream)) != hipSuccess)
                 return hipFail(ctx, err, "copying scores");
@@ -1857,6 +2090,16 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
 
     // ---- device buffers --------------------------------------------------
     Inputs in;
+    {
+        // Offsets, tables and the packed kernels' lists; the other routes'
+        // lists are copied by themselves.
+        size_t bytes = stageInputs(setH, setV, scoring, flags) + stageBytes(4 * (P.order16.size() + (size_t)N)) +
+                       stageBytes(sizeof(ScoreUnit) * P.units.size());
+        for (const Plan16 &pl : plans)
+            bytes += stageBytes(sizeof(WorkItem) * pl.items.size()) + 256;
+        if ((err = stageBegin(ctx, bytes + 1024, downScores(N, flags))) != hipSuccess)
+            return hipFail(ctx, err, "allocating upload staging");
+    }
     if ((st = uploadInputs(ctx, setH, setV, scoring, si, scores, flags, in)) != SQMI_OK)
         return st;
     const uint8_t *dH = in.dH, *dV = in.dV;
@@ -1884,9 +2127,12 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
     // form's lists live at function scope, like the planner's.
     std::vector<int32_t> plainIds;
     std::vector<ScoreUnit> plainUnits;
-    if ((flags & SQMI_PLAIN_PER_PAIR) && (err = hipEventRecord(ctx->ev0, stream)) != hipSuccess)
-        return hipFail(ctx, err, "event");
     if (flags & SQMI_PLAIN_PER_PAIR) {
+        // Its kernels are launched right here: they need the offsets and tables.
+        if ((err = stageFlush(ctx)) != hipSuccess)
+            return hipFail(ctx, err, "uploading");
+        if ((err = hipEventRecord(ctx->ev0, stream)) != hipSuccess)
+            return hipFail(ctx, err, "event");
         // One wavefront, whose first 16-lane group sweeps the pair (the other
         // pair slots of the wavefront stay empty).
         int64_t slotWords = 1;
@@ -1967,19 +2213,24 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             itemOff[k + 1] = itemOff[k] + pl.items.size();
         }
         const size_t nq = 16 * (plans.size() + 1);   // queue counters: 16 dwords per launch
-        if ((err = ensure(ctx->b.order, 4 * orderOff.back())) != hipSuccess ||
-            (err = ensure(ctx->b.items, unitBytes + sizeof(WorkItem) * itemOff.back())) != hipSuccess ||
-            (err = ensure(ctx->b.queue, 4 * nq)) != hipSuccess || (err = ensure(ctx->b.rowbuf, rbMax)) != hipSuccess ||
+        std::vector<Piece> orders, lists;
+        if (!P.units.empty()) {
+            orders.push_back({P.order16.data(), 4 * unitOrder});
+            lists.push_back({P.units.data(), unitBytes});
+        }
+        for (const Plan16 &pl : plans) {
+            orders.push_back({pl.order.data(), 4 * pl.order.size()});
+            lists.push_back({pl.items.data(), sizeof(WorkItem) * pl.items.size()});
+        }
+        if ((err = put(ctx, ctx->b.order, orders.data(), orders.size())) != hipSuccess ||
+            (err = put(ctx, ctx->b.items, lists.data(), lists.size())) != hipSuccess)
+            return hipFail(ctx, err, "uploading work lists");
+        if ((err = ensure(ctx->b.queue, 4 * nq)) != hipSuccess || (err = ensure(ctx->b.rowbuf, rbMax)) != hipSuccess ||
             (P.stripWords && (err = ensure(ctx->b.strips, (size_t)P.stripWords * 8)) != hipSuccess))
             return hipFail(ctx, err, "allocating work lists");
         uint32_t *dQueues = static_cast<uint32_t *>(ctx->b.queue.p);
         launches.push_back([=] { return launchZero32(dQueues, nq, stream); });
         if (!P.units.empty()) {
-            if ((err = hipMemcpyAsync(ctx->b.order.p, P.order16.data(), 4 * unitOrder, hipMemcpyHostToDevice, stream)) !=
-                    hipSuccess ||
-                (err = hipMemcpyAsync(ctx->b.items.p, P.units.data(), unitBytes, hipMemcpyHostToDevice, stream)) !=
-                    hipSuccess)
-                return hipFail(ctx, err, "uploading work lists");
             ScoreArgs a = sa;
             a.order = static_cast<const int32_t *>(ctx->b.order.p);
             a.units = static_cast<const ScoreUnit *>(ctx->b.items.p);
@@ -2008,11 +2259,6 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             const Variant16 &v = pl.var;
             int32_t *dOrder = static_cast<int32_t *>(ctx->b.order.p) + orderOff[k];
             WorkItem *dItems = reinterpret_cast<WorkItem *>(static_cast<char *>(ctx->b.items.p) + unitBytes) + itemOff[k];
-            if ((err = hipMemcpyAsync(dOrder, pl.order.data(), 4 * pl.order.size(), hipMemcpyHostToDevice,
-                                      stream)) != hipSuccess ||
-                (err = hipMemcpyAsync(dItems, pl.items.data(), sizeof(WorkItem) * pl.items.size(),
-                                      hipMemcpyHostToDevice, stream)) != hipSuccess)
-                return hipFail(ctx, err, "uploading work lists");
             FwdArgs a{};
             a.hRes = dH;
             a.vRes = dV;
@@ -2079,60 +2325,36 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         launches.push_back([=] { return launchFillScores(dScores, dEmpty, ne, INT32_MIN, stream); });
     }
 
-    // ---- the launches: captured into a graph that an identical next call
-    // relaunches, or run directly (plain form, no-allocation calls, or
-    // SQMI_GRAPH=0); a capture the runtime refuses falls back to running them.
+    // ---- the launches: run, and kept for an identical next call ----------
+    if ((err = stageFlush(ctx)) != hipSuccess)
+        return hipFail(ctx, err, "uploading");
     if (!(flags & SQMI_PLAIN_PER_PAIR) && (err = hipEventRecord(ctx->ev0, stream)) != hipSuccess)
         return hipFail(ctx, err, "event");
-    bool ran = false;
-    if (replayable && !launches.empty()) {
-        hipGraph_t graph = nullptr;
-        hipGraphExec_t exec = nullptr;
-        err = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
-        if (err == hipSuccess) {
-            hipError_t capErr = hipSuccess;
-            for (auto &f : launches)
-                if (capErr == hipSuccess)
-                    capErr = f();
-            err = hipStreamEndCapture(stream, &graph);
-            if (capErr == hipSuccess && err == hipSuccess && graph &&
-                hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess &&
-                (err = hipGraphLaunch(exec, stream)) == hipSuccess) {
-                ran = true;
-                ctx->replay.valid = true;
-                ctx->replay.key = key;
-                ctx->replay.exec = exec;
-                exec = nullptr;
-            }
-            if (graph)
-                (void)hipGraphDestroy(graph);
-            if (exec)
-                (void)hipGraphExecDestroy(exec);
-        }
-        (void)hipGetLastError();   // a refused capture leaves its error behind
-    }
-    if (!ran)
-        for (auto &f : launches)
-            if ((err = f()) != hipSuccess)
-                return hipFail(ctx, err, "launching alignment kernels");
+    for (auto &f : launches)
+        if ((err = f()) != hipSuccess)
+            return hipFail(ctx, err, "launching alignment kernels");
     if ((err = hipEventRecord(ctx->ev1, stream)) != hipSuccess)
         return hipFail(ctx, err, "event");
     if (!(flags & SQMI_SCORES_ON_DEVICE)) {
-        if ((err = hipMemcpyAsync(scores, dScores, 4 * N, hipMemcpyDeviceToHost, stream)) != hipSuccess)
+        if ((err = fetch(ctx, scores, dScores, 4 * N)) != hipSuccess)
             return hipFail(ctx, err, "copying scores");
     }
     if ((err = hipStreamSynchronize(stream)) != hipSuccess)
         return hipFail(ctx, err, "alignment kernels");
-    if ((st = stripCheck(ctx)) != SQMI_OK) {
-        dropReplay(ctx);
+    deliver(ctx);
+    stageEnd(ctx);
+    if ((st = stripCheck(ctx)) != SQMI_OK)
         return st;
-    }
     float ms = 0;
     if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess)
         ctx->stats.device_ms = ms;
     ctx->stats.total_ms = msSince(tStart);
-    if (ctx->replay.valid)
+    if (replayable && !launches.empty()) {
+        ctx->replay.valid = true;
+        ctx->replay.key = key;
+        ctx->replay.launches = std::move(launches);
         ctx->replay.stats = ctx->stats;
+    }
     return SQMI_OK;
 }
 
@@ -2364,6 +2586,20 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
 
     // ---- device buffers --------------------------------------------------
     hipError_t err;
+    {
+        size_t bytes = stageInputs(setH, setV, scoring, flags) + stageBytes(8 * (N + 1)) + stageBytes(4 * P.ids32.size()) + stageBytes(8 * P.ids32.size()) + 4096;
+        if (pl)
+            bytes += stageBytes(4 * pl->order.size()) + stageBytes(sizeof(ScoreUnit) * P.units.size()) +
+                     2 * stageBytes(8 * pl->items.size()) + stageBytes(sizeof(TraceLoc) * pl->order.size());
+        size_t down = downScores(N, flags);
+        if (down) {
+            down += stageBytes((size_t)4 * S * N) + 256;
+            if (wantRows)
+                down += stageBytes(8 * N) + stageBytes(16 * N) + stageBytes((size_t)(opOffsets[N] - opOffsets[0]));
+        }
+        if ((err = stageBegin(ctx, bytes, down)) != hipSuccess)
+            return hipFail(ctx, err, "allocating upload staging");
+    }
     if ((st = uploadInputs(ctx, setH, setV, scoring, si, scores, flags, in)) != SQMI_OK)
         return st;
     int32_t *dCounts = counts;
@@ -2379,9 +2615,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         // Offsets always come from the host; ops and lengths live where the
         // scores do.
         const int64_t opBytes = opOffsets[N];
-        if ((err = ensure(ctx->b.opOff, 8 * (N + 1))) != hipSuccess)
-            return hipFail(ctx, err, "allocating op offsets");
-        if ((err = hipMemcpyAsync(ctx->b.opOff.p, opOffsets, 8 * (N + 1), hipMemcpyHostToDevice, stream)) != hipSuccess)
+        if ((err = put(ctx, ctx->b.opOff, opOffsets, 8 * (N + 1))) != hipSuccess)
             return hipFail(ctx, err, "uploading op offsets");
         rows.opOff = static_cast<const int64_t *>(ctx->b.opOff.p);
         if (flags & SQMI_SCORES_ON_DEVICE) {
@@ -2419,26 +2653,18 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
             maxUnits = std::max(maxUnits, chunkUnits[c] - b);
         const int grid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occupancyTrace16(P.dna16, P.track),
                                                             ((int64_t)maxUnits + wpb - 1) / wpb));
-        if ((err = ensure(ctx->b.order, 4 * np)) != hipSuccess ||
-            (err = ensure(ctx->b.items, sizeof(ScoreUnit) * P.units.size())) != hipSuccess ||
-            (err = ensure(ctx->b.traceOff, 8 * nIt)) != hipSuccess || (err = ensure(ctx->b.endOff, 8 * nIt)) != hipSuccess ||
-            (err = ensure(ctx->b.locs, sizeof(TraceLoc) * np)) != hipSuccess ||
-            (err = ensure(ctx->b.queue, 4 * chunkEnd.size() + 64)) != hipSuccess ||
+        if ((err = ensure(ctx->b.queue, 4 * chunkEnd.size() + 64)) != hipSuccess ||
             (err = ensure(ctx->b.rowbuf, (size_t)grid * wpb * slotWords * 8)) != hipSuccess ||
             (err = ensure(ctx->b.strips, (size_t)stripWords * 8)) != hipSuccess ||
             (err = ensure(ctx->b.ends, sizeof(TraceEnd) * (size_t)nEnds)) != hipSuccess ||
             (err = ensure(ctx->b.trace, (size_t)traceRecs * 64 * 16)) != hipSuccess)
             return hipFail(ctx, err, "allocating traceback buffers");
-        if ((err = hipMemcpyAsync(ctx->b.order.p, pl->order.data(), 4 * np, hipMemcpyHostToDevice, stream)) !=
-                hipSuccess ||
-            (err = hipMemcpyAsync(ctx->b.items.p, P.units.data(), sizeof(ScoreUnit) * P.units.size(),
-                                  hipMemcpyHostToDevice, stream)) != hipSuccess ||
-            (err = hipMemcpyAsync(ctx->b.traceOff.p, itemOff.data(), 8 * nIt, hipMemcpyHostToDevice, stream)) !=
-                hipSuccess ||
-            (err = hipMemcpyAsync(ctx->b.endOff.p, endOff.data(), 8 * nIt, hipMemcpyHostToDevice, stream)) !=
-                hipSuccess ||
-            (err = hipMemcpyAsync(ctx->b.locs.p, locs.data(), sizeof(TraceLoc) * np, hipMemcpyHostToDevice, stream)) !=
-                hipSuccess ||
+        if ((err = put(ctx, ctx->b.order, pl->order.data(), 4 * np)) != hipSuccess ||
+            (err = put(ctx, ctx->b.items, P.units.data(), sizeof(ScoreUnit) * P.units.size())) != hipSuccess ||
+            (err = put(ctx, ctx->b.traceOff, itemOff.data(), 8 * nIt)) != hipSuccess ||
+            (err = put(ctx, ctx->b.endOff, endOff.data(), 8 * nIt)) != hipSuccess ||
+            (err = put(ctx, ctx->b.locs, locs.data(), sizeof(TraceLoc) * np)) != hipSuccess ||
+            (err = stageFlush(ctx)) != hipSuccess ||
             (err = hipMemsetAsync(ctx->b.queue.p, 0, 4 * chunkEnd.size() + 64, stream)) != hipSuccess)
             return hipFail(ctx, err, "uploading traceback work lists");
         const int32_t *dOrder = static_cast<const int32_t *>(ctx->b.order.p);
@@ -2543,13 +2769,11 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
     }
     if (bandLanes > 0) {
         const size_t n32 = P.ids32.size();
-        if ((err = ensure(ctx->b.ids32, 4 * n32)) != hipSuccess || (err = ensure(ctx->b.scratchOff32, 8 * n32)) != hipSuccess ||
-            (err = ensure(ctx->b.scratch32, (size_t)std::max<int64_t>(bandBytes, 1))) != hipSuccess ||
+        if ((err = ensure(ctx->b.scratch32, (size_t)std::max<int64_t>(bandBytes, 1))) != hipSuccess ||
             (err = ensure(ctx->b.endEF, (size_t)8 * N)) != hipSuccess || (err = ensure(ctx->b.endIJ, (size_t)8 * N)) != hipSuccess)
             return hipFail(ctx, err, "allocating banded traceback buffers");
-        if ((err = hipMemcpyAsync(ctx->b.ids32.p, P.ids32.data(), 4 * n32, hipMemcpyHostToDevice, stream)) != hipSuccess ||
-            (err = hipMemcpyAsync(ctx->b.scratchOff32.p, bandOff.data(), 8 * n32, hipMemcpyHostToDevice, stream)) !=
-                hipSuccess)
+        if ((err = put(ctx, ctx->b.ids32, P.ids32.data(), 4 * n32)) != hipSuccess ||
+            (err = put(ctx, ctx->b.scratchOff32, bandOff.data(), 8 * n32)) != hipSuccess || (err = stageFlush(ctx)) != hipSuccess)
             return hipFail(ctx, err, "uploading banded traceback lists");
         size_t cb = 0;
         for (size_t ce : bandChunkEnd) {
@@ -2603,12 +2827,10 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         }
     } else if (!P.ids32.empty()) {
         const size_t n32 = P.ids32.size();
-        if ((err = ensure(ctx->b.ids32, 4 * n32)) != hipSuccess || (err = ensure(ctx->b.scratchOff32, 8 * n32)) != hipSuccess ||
-            (err = ensure(ctx->b.scratch32, (size_t)scratch32)) != hipSuccess)
+        if ((err = ensure(ctx->b.scratch32, (size_t)scratch32)) != hipSuccess)
             return hipFail(ctx, err, "allocating int32 traceback buffers");
-        if ((err = hipMemcpyAsync(ctx->b.ids32.p, P.ids32.data(), 4 * n32, hipMemcpyHostToDevice, stream)) != hipSuccess ||
-            (err = hipMemcpyAsync(ctx->b.scratchOff32.p, off32.data(), 8 * n32, hipMemcpyHostToDevice, stream)) !=
-                hipSuccess)
+        if ((err = put(ctx, ctx->b.ids32, P.ids32.data(), 4 * n32)) != hipSuccess ||
+            (err = put(ctx, ctx->b.scratchOff32, off32.data(), 8 * n32)) != hipSuccess || (err = stageFlush(ctx)) != hipSuccess)
             return hipFail(ctx, err, "uploading int32 traceback lists");
         size_t b = 0;
         for (size_t e : chunk32End) {
@@ -2642,6 +2864,8 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
             b = e;
         }
     }
+    if ((err = stageFlush(ctx)) != hipSuccess)   // offsets and tables, where no list above sent them
+        return hipFail(ctx, err, "uploading");
     LongStage longStage;
     if ((st = runLong(ctx, setH, setV, P, in, flags, dCounts, rows, longStage)) != SQMI_OK)
         return st;
@@ -2675,34 +2899,38 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
     if ((err = hipEventRecord(ctx->ev1, stream)) != hipSuccess)
         return hipFail(ctx, err, "event");
     if (!(flags & SQMI_SCORES_ON_DEVICE)) {
-        if ((err = hipMemcpyAsync(scores, in.dScores, 4 * N, hipMemcpyDeviceToHost, stream)) != hipSuccess ||
-            (err = hipMemcpyAsync(counts, dCounts, (size_t)4 * S * N, hipMemcpyDeviceToHost, stream)) != hipSuccess)
+        if ((err = fetch(ctx, scores, in.dScores, 4 * N)) != hipSuccess ||
+            (err = fetch(ctx, counts, dCounts, (size_t)4 * S * N)) != hipSuccess)
             return hipFail(ctx, err, "copying results");
-        if (wantRows &&
-            ((err = hipMemcpyAsync(opLengths, rows.opLen, 8 * N, hipMemcpyDeviceToHost, stream)) != hipSuccess ||
-             (begins && (err = hipMemcpyAsync(begins, rows.begins, 16 * N, hipMemcpyDeviceToHost, stream)) !=
-                            hipSuccess)))
+        if (wantRows && ((err = fetch(ctx, opLengths, rows.opLen, 8 * N)) != hipSuccess ||
+                         (begins && (err = fetch(ctx, begins, rows.begins, 16 * N)) != hipSuccess)))
             return hipFail(ctx, err, "copying rows");
         if (wantRows) {
             // Packed rows fill only the first sum(op_lengths) bytes: read
             // that total (the scan's last entry) and copy no more.
             int64_t opsBytes = opOffsets[N] - opOffsets[0];
+            size_t early = 0;   // results that have arrived with the total
             if (flags & SQMI_ROWS_PACKED) {
                 int64_t total = 0;
-                if ((err = hipMemcpyAsync(&total, static_cast<const int64_t *>(ctx->b.opStart.p) + N, 8,
-                                          hipMemcpyDeviceToHost, stream)) != hipSuccess ||
+                early = ctx->down.size();
+                if ((err = fetch(ctx, &total, static_cast<const int64_t *>(ctx->b.opStart.p) + N, 8)) != hipSuccess ||
                     (err = hipStreamSynchronize(stream)) != hipSuccess)
                     return hipFail(ctx, err, "reading the packed rows' length");
+                if (ctx->down.size() > early) {
+                    std::memcpy(&total, ctx->down.back().src, 8);
+                    ctx->down.pop_back();
+                }
                 opsBytes = std::min(opsBytes, std::max<int64_t>(total, 0));
             }
-            if (opsBytes > 0 &&
-                (err = hipMemcpyAsync(ops + opOffsets[0], rowsOut + opOffsets[0], (size_t)opsBytes,
-                                      hipMemcpyDeviceToHost, stream)) != hipSuccess)
+            if (opsBytes > 0 && (err = fetch(ctx, ops + opOffsets[0], rowsOut + opOffsets[0], (size_t)opsBytes)) != hipSuccess)
                 return hipFail(ctx, err, "copying rows");
+            deliver(ctx, early);   // while the rows are on their way
         }
     }
     if ((err = hipStreamSynchronize(stream)) != hipSuccess)
         return hipFail(ctx, err, "traceback kernels");
+    deliver(ctx);
+    stageEnd(ctx);
     if ((st = stripCheck(ctx)) != SQMI_OK)
         return st;
     float ms = 0;
@@ -2827,11 +3055,12 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     // The packed kernel's values: the bias covers the longest pair of the
     // call; columns run to the item's longest |H|, a group past the band.
     Drift dr = driftOf(si, local);
+    const int64_t *offH = setH->offsets, *offV = setV->offsets;
     int64_t maxN = 1, maxM = 1;
 #pragma omp parallel for schedule(static) reduction(max : maxN, maxM) if (N > kParallelMin)
     for (int64_t i = 0; i < N; ++i) {
-        maxN = std::max(maxN, setH->offsets[i + 1] - setH->offsets[i]);
-        maxM = std::max(maxM, setV->offsets[i + 1] - setV->offsets[i]);
+        maxN = std::max(maxN, offH[i + 1] - offH[i]);
+        maxM = std::max(maxM, offV[i + 1] - offV[i]);
     }
     if (!local && bandCostsOk)
         dr.bias += (int32_t)std::min<int64_t>(bandDrop(si, dr, W1, maxM), 1 << 20);
@@ -2842,7 +3071,7 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     const bool narrowT = dr.neg == (local ? 2 * dr.d + 2 : dr.cost + 1);   // no t below 0
     bool bandWide = !narrowT;
     const bool packedOk = bandCostsOk;
-    std::vector<int32_t> narrow, wide, rejected, packed;
+    std::vector<int32_t> narrow, wide, rejected;
     int64_t wNarrow = 1, wWide = 0, cells = 0;
     auto toInt32 = [&](int32_t id, int64_t n, int64_t m) {
         const int64_t w = std::min<int64_t>(upper_diag, n) - std::max<int64_t>(lower_diag, -m) + 1;
@@ -2854,80 +3083,109 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
             wWide = std::max(wWide, w);
         }
     };
-    for (int64_t i = 0; i < N; ++i) {
-        const int64_t n = setH->offsets[i + 1] - setH->offsets[i], m = setV->offsets[i + 1] - setV->offsets[i];
-        if (n == 0 || m == 0) {
-            rejected.push_back((int32_t)i);
-            continue;
+    // Every thread routes a contiguous part of the pairs and counts its packed
+    // pairs by |V|; the counts' prefix sums (by |V|, then thread) place them,
+    // in pair order within a |V|.  On 1,048,576 pairs one thread took 5 ms.
+    auto packs = [&](int64_t n, int64_t m) { return packedOk && n <= 30000 && m <= 30000 && bandTop(m) <= 65535; };
+    const int64_t mSlots = std::min<int64_t>(maxM, 30000) + 1;
+    const int parts = N > kParallelMin ? (int)std::max<int64_t>(1, std::min<int64_t>(omp_get_max_threads(), N / mSlots)) : 1;
+    std::vector<int32_t> counts((size_t)parts * mSlots, 0);
+    std::vector<int64_t> nOther((size_t)parts, 0);
+    int64_t firstBad = N, nPacked = 0;
+    bool anyWide = false;
+#pragma omp parallel for schedule(static) num_threads(parts) reduction(+ : cells, nPacked) reduction(min : firstBad) \
+    reduction(|| : anyWide) if (parts > 1)
+    for (int t = 0; t < parts; ++t) {
+        int32_t *cnt = counts.data() + (size_t)t * mSlots;
+        for (int64_t i = N * t / parts; i < N * (t + 1) / parts; ++i) {
+            const int64_t n = offH[i + 1] - offH[i], m = offV[i + 1] - offV[i];
+            if (n != 0 && m != 0 && !bandSupported(n, m, lower_diag, upper_diag, local)) {
+                firstBad = std::min(firstBad, i);
+                continue;
+            }
+            cells += n != 0 && m != 0 ? n * m : 0;
+            if (n != 0 && m != 0 && packs(n, m)) {
+                ++cnt[m];
+                ++nPacked;
+                anyWide = anyWide || bandTop(m) > kDriftNarrowMax;
+            } else {
+                ++nOther[(size_t)t];
+            }
         }
-        if (!bandSupported(n, m, lower_diag, upper_diag, local))
-            return fail(ctx, SQMI_ERR_UNSUPPORTED,
-                        "sqmi_align_score_banded: pair " + std::to_string(i) +
-                            (local ? ": needs |H| >= 2, two diagonals, lower_diag <= |H| - 2 and upper_diag >= 2 - |V|"
-                                   : ": needs |H| >= 2 and lower_diag < min(0, |H| - |V|) < max(0, |H| - |V|) "
-                                     "< upper_diag"));
-        cells += n * m;
-        if (packedOk && n <= 30000 && m <= 30000 && bandTop(m) <= 65535) {
-            packed.push_back((int32_t)i);
-            bandWide |= bandTop(m) > kDriftNarrowMax;
-            continue;
+    }
+    if (firstBad < N)
+        return fail(ctx, SQMI_ERR_UNSUPPORTED,
+                    "sqmi_align_score_banded: pair " + std::to_string(firstBad) +
+                        (local ? ": needs |H| >= 2, two diagonals, lower_diag <= |H| - 2 and upper_diag >= 2 - |V|"
+                               : ": needs |H| >= 2 and lower_diag < min(0, |H| - |V|) < max(0, |H| - |V|) "
+                                 "< upper_diag"));
+    bandWide |= anyWide;
+    for (int t = 0; t < parts; ++t)
+        for (int64_t i = N * t / parts; nOther[(size_t)t] > 0 && i < N * (t + 1) / parts; ++i) {
+            const int64_t n = offH[i + 1] - offH[i], m = offV[i + 1] - offV[i];
+            if (n == 0 || m == 0)
+                rejected.push_back((int32_t)i);
+            else if (!packs(n, m))
+                toInt32((int32_t)i, n, m);
         }
-        toInt32((int32_t)i, n, m);
+    // Packed items: up to 128 pairs of one |V|.
+    RawVec<int32_t> packed((size_t)nPacked);
+    std::vector<WorkItem> bandItems;
+    int bandMaxN = 1;
+    if (nPacked > 0) {
+        int32_t run = 0;
+        for (int64_t mm = 0; mm < mSlots; ++mm) {
+            const int32_t f0 = run;
+            for (int t = 0; t < parts; ++t) {
+                int32_t &c = counts[(size_t)t * mSlots + mm];
+                const int32_t k = c;
+                c = run;
+                run += k;
+            }
+            for (int32_t f = f0; f < run; f += 128)
+                bandItems.push_back(WorkItem{f, std::min<int32_t>(128, run - f) | ((int)mm << 16), 1,
+                                             ((int)mm + bandR) / bandR});
+        }
+#pragma omp parallel for schedule(static) num_threads(parts) if (parts > 1)
+        for (int t = 0; t < parts; ++t) {
+            int32_t *pos = counts.data() + (size_t)t * mSlots;
+            for (int64_t i = N * t / parts; i < N * (t + 1) / parts; ++i) {
+                const int64_t n = offH[i + 1] - offH[i], m = offV[i + 1] - offV[i];
+                if (n != 0 && m != 0 && packs(n, m))
+                    packed[(size_t)pos[m]++] = (int32_t)i;
+            }
+        }
+#pragma omp parallel for schedule(static) reduction(max : bandMaxN) if (parts > 1)
+        for (int64_t k = 0; k < (int64_t)bandItems.size(); ++k) {
+            WorkItem &w = bandItems[(size_t)k];
+            for (int32_t q = w.first; q < w.first + (w.count & 0xffff); ++q)
+                w.maxN = std::max(w.maxN, (int)(offH[packed[q] + 1] - offH[packed[q]]));
+            bandMaxN = std::max(bandMaxN, w.maxN);
+        }
     }
     // Free end gaps and local alignment, few pairs: a packed item takes its
     // whole sweep, however few the items; the int32 kernels, which spread a
     // pair's band over a wave, are done earlier.
     if (mode != 0 && !packed.empty() && !envFlag("SQMI_BAND_PACKED")) {
-        double items = 0, blockCols = 0, lone = 0, full = 0;
-        std::vector<int32_t> perM((size_t)maxM + 1, 0);
-        for (int32_t id : packed) {
-            const int64_t n = setH->offsets[id + 1] - setH->offsets[id], m = setV->offsets[id + 1] - setV->offsets[id];
-            items += perM[(size_t)m]++ % 128 == 0;
-            const double w = (double)std::min<int64_t>(W1 + 1, n + m), chunks = std::ceil(w / 64);
-            blockCols = std::max(blockCols, (double)(m / bandR + 1) * std::min<double>(w + bandR, (double)n));
-            lone = std::max(lone, (double)m * (w <= 64 ? kBandNarrowLone : kBandWideLone * chunks));
-            full += (double)m * (w <= 64 ? kBandNarrowFull * w / 64 : kBandWideFull * chunks);
+        double blockCols = 0, lone = 0, full = 0;
+        for (const WorkItem &it : bandItems) {
+            const double m = (double)((uint32_t)it.count >> 16), w = std::min<double>((double)W1 + 1, it.maxN + m);
+            const double chunks = std::ceil(w / 64);
+            blockCols = std::max(blockCols, it.nblocks * std::min<double>(w + bandR, it.maxN));
+            lone = std::max(lone, m * (w <= 64 ? kBandNarrowLone : kBandWideLone * chunks));
+            full += (it.count & 0xffff) * m * (w <= 64 ? kBandNarrowFull * w / 64 : kBandWideFull * chunks);
         }
         const double simds = 4.0 * std::max(1, ctx->numCUs);
-        if (std::max(lone, full / simds) < std::ceil(items / simds) * blockCols * kBandColumn) {
+        if (std::max(lone, full / simds) < std::ceil(bandItems.size() / simds) * blockCols * kBandColumn) {
             for (int32_t id : packed)
-                toInt32(id, setH->offsets[id + 1] - setH->offsets[id], setV->offsets[id + 1] - setV->offsets[id]);
+                toInt32(id, offH[id + 1] - offH[id], offV[id + 1] - offV[id]);
             packed.clear();
+            bandItems.clear();
         }
     }
     int seg = 1;
     while (seg < wNarrow)
         seg <<= 1;
-    // Packed items: up to 128 pairs of one |V| (counting sort by |V|).
-    std::vector<int32_t> bandOrder;
-    std::vector<WorkItem> bandItems;
-    int bandMaxN = 1;
-    if (!packed.empty()) {
-        int maxM = 0;
-        for (int32_t id : packed)
-            maxM = std::max(maxM, (int)(setV->offsets[id + 1] - setV->offsets[id]));
-        std::vector<int32_t> start((size_t)maxM + 2, 0);
-        for (int32_t id : packed)
-            ++start[(size_t)(setV->offsets[id + 1] - setV->offsets[id]) + 1];
-        for (int mm = 0; mm <= maxM; ++mm)
-            start[(size_t)mm + 1] += start[(size_t)mm];
-        bandOrder.resize(packed.size());
-        {
-            std::vector<int32_t> pos(start.begin(), start.end() - 1);
-            for (int32_t id : packed)
-                bandOrder[(size_t)pos[(size_t)(setV->offsets[id + 1] - setV->offsets[id])]++] = id;
-        }
-        for (int mm = 1; mm <= maxM; ++mm) {
-            for (int32_t f = start[(size_t)mm]; f < start[(size_t)mm + 1]; f += 128) {
-                const int32_t cnt = std::min<int32_t>(128, start[(size_t)mm + 1] - f);
-                int mxN = 1;
-                for (int32_t q = f; q < f + cnt; ++q)
-                    mxN = std::max(mxN, (int)(setH->offsets[bandOrder[q] + 1] - setH->offsets[bandOrder[q]]));
-                bandMaxN = std::max(bandMaxN, mxN);
-                bandItems.push_back(WorkItem{f, cnt | (mm << 16), mxN, (mm + bandR) / bandR});
-            }
-        }
-    }
     ctx->stats.pairs = N;
     ctx->stats.cells = cells;
     ctx->stats.pairs_int32 = (int64_t)(narrow.size() + wide.size());
@@ -2937,22 +3195,24 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     up.join();
     if (upErr != hipSuccess)
         return hipFail(ctx, upErr, "copying residues");
+    hipError_t err;
+    if ((err = stageBegin(ctx, stageInputs(setH, setV, scoring, flags) + stageBytes(4 * (size_t)N) + stageBytes(4 * packed.size()) +
+                                   stageBytes(sizeof(WorkItem) * bandItems.size()) + 1024,
+                          downScores(N, flags))) != hipSuccess)
+        return hipFail(ctx, err, "allocating upload staging");
     if ((st = uploadInputs(ctx, setH, setV, scoring, si, scores, flags, in)) != SQMI_OK)
         return st;
-    hipError_t err;
     const int wideStride = (int)((wWide + 2 + 63) & ~(int64_t)63);
     const int wideGrid = wide.empty() ? 0 : (int)std::min<int64_t>((int64_t)wide.size(), (int64_t)ctx->numCUs * 16);
     const size_t nIds = narrow.size() + wide.size() + rejected.size();
-    if ((err = ensure(ctx->b.bandIds, 4 * std::max<size_t>(nIds, 1))) != hipSuccess ||
-        (wideGrid && (err = ensure(ctx->b.bandScratch, (size_t)wideGrid * 4 * wideStride * 4)) != hipSuccess))
+    if ((wideGrid && (err = ensure(ctx->b.bandScratch, (size_t)wideGrid * 4 * wideStride * 4)) != hipSuccess))
         return hipFail(ctx, err, "allocating banded buffers");
     std::vector<int32_t> all(narrow);
     all.insert(all.end(), wide.begin(), wide.end());
     all.insert(all.end(), rejected.begin(), rejected.end());
-    int32_t *dIds = static_cast<int32_t *>(ctx->b.bandIds.p);
-    if (!all.empty() &&
-        (err = hipMemcpyAsync(dIds, all.data(), 4 * all.size(), hipMemcpyHostToDevice, stream)) != hipSuccess)
+    if ((err = put(ctx, ctx->b.bandIds, all.data(), 4 * nIds)) != hipSuccess)
         return hipFail(ctx, err, "uploading banded pair lists");
+    int32_t *dIds = static_cast<int32_t *>(ctx->b.bandIds.p);
     int bandGrid = 0, bandRowColsN = 0, bandLds = 0;
     BandVariant bandVar{};
     if (!bandItems.empty()) {
@@ -2973,17 +3233,15 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
         const int occ = bandLds ? most : (int)std::max<int64_t>(1, std::min<int64_t>(most, ctx->l2PerCU / (4 * ringBytes)));
         const int64_t nIt = (int64_t)bandItems.size();
         bandGrid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occ, (nIt + 3) / 4));
-        if ((err = ensure(ctx->b.order, 4 * bandOrder.size())) != hipSuccess ||
-            (err = ensure(ctx->b.items, sizeof(WorkItem) * bandItems.size())) != hipSuccess ||
-            (err = ensure(ctx->b.queue, 64)) != hipSuccess ||
+        if ((err = ensure(ctx->b.queue, 64)) != hipSuccess ||
             (err = ensure(ctx->b.rowbuf, bandLds ? 64 : (size_t)bandGrid * 4 * 64 * bandRowColsN * 8)) != hipSuccess)
             return hipFail(ctx, err, "allocating packed banded buffers");
-        if ((err = hipMemcpyAsync(ctx->b.order.p, bandOrder.data(), 4 * bandOrder.size(), hipMemcpyHostToDevice,
-                                  stream)) != hipSuccess ||
-            (err = hipMemcpyAsync(ctx->b.items.p, bandItems.data(), sizeof(WorkItem) * bandItems.size(),
-                                  hipMemcpyHostToDevice, stream)) != hipSuccess)
+        if ((err = put(ctx, ctx->b.order, packed.data(), 4 * packed.size())) != hipSuccess ||
+            (err = put(ctx, ctx->b.items, bandItems.data(), sizeof(WorkItem) * bandItems.size())) != hipSuccess)
             return hipFail(ctx, err, "uploading packed banded work");
     }
+    if ((err = stageFlush(ctx)) != hipSuccess)
+        return hipFail(ctx, err, "uploading");
     if ((err = hipEventRecord(ctx->ev0, stream)) != hipSuccess)
         return hipFail(ctx, err, "event");
     if (!bandItems.empty()) {
@@ -3047,11 +3305,12 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
         return hipFail(ctx, err, "launching fill kernel");
     if ((err = hipEventRecord(ctx->ev1, stream)) != hipSuccess)
         return hipFail(ctx, err, "event");
-    if (!(flags & SQMI_SCORES_ON_DEVICE) &&
-        (err = hipMemcpyAsync(scores, in.dScores, 4 * N, hipMemcpyDeviceToHost, stream)) != hipSuccess)
+    if (!(flags & SQMI_SCORES_ON_DEVICE) && (err = fetch(ctx, scores, in.dScores, 4 * N)) != hipSuccess)
         return hipFail(ctx, err, "copying scores");
     if ((err = hipStreamSynchronize(stream)) != hipSuccess)
         return hipFail(ctx, err, "banded kernels");
+    deliver(ctx);
+    stageEnd(ctx);
     float ms = 0;
     if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess)
         ctx->stats.device_ms = ms;
