@@ -1257,6 +1257,53 @@ void fillStats(const Planned &P, sqmi_stats &st)
     st.padded_cells = padded;
 }
 
+// An item of the trace kernel: up to 128 / lanes pairs of `nblocks` blocks.
+struct TraceItem {
+    int32_t first, count, maxN, nblocks, lanes;
+};
+// 1 KB records of an item (a step of four couples on 16 lanes, four steps of one on 64).
+int64_t traceRecsOf(const TraceItem &w)
+{
+    const int64_t steps = (int64_t)w.nblocks * traceSteps(w.maxN, w.lanes);
+    return w.lanes == 64 ? (steps + 3) / 4 : steps;
+}
+
+// Lanes per couple of the trace kernel, by the time an item takes against the
+// whole call's.  On 16 lanes a step takes a wave 0.53 us (0.47 of a full
+// SIMD) and a block starts about 110 steps behind the one above; on 64 lanes of 4
+// rows 0.2 us for a quarter of the couples, which costs 1.4 times as much.
+// So items go to 64 lanes whose chain of blocks would take more than a share
+// of the call's time on a full chip (with the table, whose lookups weigh more
+// there, a larger one).  SQMI_TRACE_LANES=16 or 64 takes one form for all
+// (tests).  Device time of 8,191 uneven DNA pairs, shares 0.5 / 1 / 2 / 4: 4.3 /
+// 4.7 / 5.5 / 8.7 ms (all on 64 lanes 4.4, on 16 8.6); of 8,192 protein pairs,
+// local: 4.3 / 3.5 / 3.6 / 3.5 (4.2, 3.5); 65,536 pairs of 1 kbp: none, 17.4
+// (all on 64 lanes 20.2).
+constexpr double kTrace64Share = 0.5, kTrace64ShareTab = 1.5;
+void traceItems(const sqmi_sequences &H, const Plan16 &pl, bool dna, std::vector<TraceItem> &out)
+{
+    double total = 0;
+    for (const WorkItem &w : pl.items)
+        total += (double)w.nblocks * traceSteps(w.maxN, 16) * 0.47 / 1024;
+    const char *env = std::getenv("SQMI_TRACE_LANES");
+    const int forced = env && *env ? std::atoi(env) : 0;
+    out.clear();
+    out.reserve(pl.items.size());
+    for (const WorkItem &w : pl.items) {
+        const double chain = (w.maxN + 110.0 * w.nblocks) * 0.53;
+        if (forced == 16 || (forced != 64 && chain <= (dna ? kTrace64Share : kTrace64ShareTab) * total)) {
+            out.push_back(TraceItem{w.first, w.count, w.maxN, w.nblocks, 16});
+            continue;
+        }
+        for (int32_t f = w.first; f < w.first + w.count; f += 2) {
+            TraceItem q{f, std::min<int32_t>(2, w.first + w.count - f), 1, w.nblocks, 64};
+            for (int32_t x = f; x < f + q.count; ++x)
+                q.maxN = std::max(q.maxN, (int32_t)(H.offsets[pl.order[x] + 1] - H.offsets[pl.order[x]]));
+            out.push_back(q);
+        }
+    }
+}
+
 sqmi_status validate(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_sequences *setV,
                      const sqmi_scoring *scoring, uint32_t &mode)
 {
@@ -2490,8 +2537,10 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
     int64_t traceRecs = 0;                  // largest chunk, in steps
     int64_t slotWords = 1, stripWords = 0, nEnds = 0;
     std::vector<int64_t> chunkStrips;       // strip words of each chunk
+    std::vector<TraceItem> tItems;
     if (pl) {
-        const size_t nIt = pl->items.size();
+        traceItems(*setH, *pl, P.dna16, tItems);
+        const size_t nIt = tItems.size();
         const int64_t recBytes = 64 * 16;
         itemOff.resize(nIt);
         endOff.resize(nIt);
@@ -2499,8 +2548,8 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         std::vector<uint8_t> wide(nIt);
         int64_t run = 0;
         for (size_t k = 0; k < nIt; ++k) {
-            const WorkItem &w = pl->items[k];
-            const int64_t recs = (int64_t)w.nblocks * traceSteps(w.maxN);
+            const TraceItem &w = tItems[k];
+            const int64_t recs = traceRecsOf(w);
             if (run > 0 && (run + recs) * recBytes > budget) {
                 chunkEnd.push_back(k);
                 run = 0;
@@ -2512,7 +2561,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         chunkEnd.push_back(nIt);
 #pragma omp parallel for schedule(static) if (N > kParallelMin)
         for (int64_t k = 0; k < (int64_t)nIt; ++k) {
-            const WorkItem &w = pl->items[k];
+            const TraceItem &w = tItems[k];
             bool any = false;
             for (int x = 0; x < w.count; ++x) {
                 const int32_t pid = pl->order[w.first + x];
@@ -2526,23 +2575,25 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         for (size_t c = 0, b = 0; c < chunkEnd.size(); b = chunkEnd[c], ++c) {
             int64_t total = 0, off = 0;
             for (size_t k = b; k < chunkEnd[c]; ++k)
-                total += (int64_t)pl->items[k].nblocks * traceSteps(pl->items[k].maxN);
+                total += (int64_t)tItems[k].nblocks * traceSteps(tItems[k].maxN, tItems[k].lanes);
             for (size_t k = b; k < chunkEnd[c]; ++k) {
-                const WorkItem &w = pl->items[k];
+                const TraceItem &w = tItems[k];
+                const int64_t steps = traceSteps(w.maxN, w.lanes), words = (int64_t)(64 / w.lanes) * (w.maxN + 1);
                 const bool strips = w.nblocks > 1 &&
-                                    (minBlocks < 0 ? (int64_t)w.nblocks * traceSteps(w.maxN) * 4 * kResidentWaves > total
+                                    (minBlocks < 0 ? w.lanes == 64 || w.nblocks * steps * 4 * kResidentWaves > total
                                                    : minBlocks > 0 && w.nblocks >= minBlocks);
-                ScoreUnit u{w.first, w.count, w.maxN, w.nblocks, 16 | 16 << 8, wide[k] ? kUnitWide : 0, -1,
-                            (int32_t)(k - b), 0};
+                const int R = kTraceRows / w.lanes;
+                ScoreUnit u{w.first, w.count, w.maxN, w.nblocks, R | R << 8,
+                            (wide[k] ? kUnitWide : 0) | (w.lanes == 64 ? kUnit64 : 0), -1, (int32_t)(k - b), 0};
                 endOff[k] = nEnds;
                 nEnds += (int64_t)w.count * (strips ? w.nblocks : 1);
                 if (strips) {
                     u.rowOff = off;
-                    off += (int64_t)4 * (w.maxN + 1) * w.nblocks;
+                    off += words * w.nblocks;
                     for (u.block = 0; u.block < w.nblocks; ++u.block)
                         P.units.push_back(u);
                 } else {
-                    slotWords = std::max<int64_t>(slotWords, (int64_t)4 * (w.maxN + 1));
+                    slotWords = std::max<int64_t>(slotWords, words);
                     P.units.push_back(u);
                 }
                 wide[k] = strips;   // from here on: whether the item has strips
@@ -2553,13 +2604,13 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         }
 #pragma omp parallel for schedule(static) if (N > kParallelMin)
         for (int64_t k = 0; k < (int64_t)nIt; ++k) {
-            const WorkItem &w = pl->items[k];
+            const TraceItem &w = tItems[k];
             for (int x = 0; x < w.count; ++x) {
                 const int32_t pid = pl->order[w.first + x];
                 const int64_t m = setV->offsets[pid + 1] - setV->offsets[pid];
-                locs[w.first + x] = TraceLoc{itemOff[k], traceSteps(w.maxN),
-                                             (int32_t)((int64_t)w.nblocks * kTraceRows - 1 - m),
-                                             (x / 2) * kTraceLanes, x % 2, endOff[k] + x, w.count, wide[k] ? w.nblocks : 1};
+                locs[w.first + x] = TraceLoc{itemOff[k], traceSteps(w.maxN, w.lanes),
+                                             (int32_t)((int64_t)w.nblocks * kTraceRows - 1 - m), (x / 2) * kTraceLanes, x % 2,
+                                             w.lanes, endOff[k] + x, w.count, wide[k] ? w.nblocks : 1, 0};
             }
         }
     }
@@ -2590,7 +2641,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         size_t bytes = stageInputs(setH, setV, scoring, flags) + stageBytes(8 * (N + 1)) + stageBytes(4 * P.ids32.size()) + stageBytes(8 * P.ids32.size()) + 4096;
         if (pl)
             bytes += stageBytes(4 * pl->order.size()) + stageBytes(sizeof(ScoreUnit) * P.units.size()) +
-                     2 * stageBytes(8 * pl->items.size()) + stageBytes(sizeof(TraceLoc) * pl->order.size());
+                     2 * stageBytes(8 * tItems.size()) + stageBytes(sizeof(TraceLoc) * pl->order.size());
         size_t down = downScores(N, flags);
         if (down) {
             down += stageBytes((size_t)4 * S * N) + 256;
@@ -2646,7 +2697,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
         return hipFail(ctx, err, "event");
 
     if (pl) {
-        const size_t nIt = pl->items.size(), np = pl->order.size();
+        const size_t nIt = tItems.size(), np = pl->order.size();
         const int wpb = wavesPerBlock16();
         size_t maxUnits = 0;
         for (size_t c = 0, b = 0; c < chunkUnits.size(); b = chunkUnits[c], ++c)
@@ -2701,8 +2752,8 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
             const int cg = std::max(1, std::min(grid, (int)((ue - ub + wpb - 1) / wpb)));
             if ((err = launchTrace16(P.dna16, P.track, a, cg, stream)) != hipSuccess)
                 return hipFail(ctx, err, "launching trace kernel");
-            const int32_t p0 = pl->items[b].first;
-            const int32_t p1 = pl->items[e - 1].first + pl->items[e - 1].count;
+            const int32_t p0 = tItems[b].first;
+            const int32_t p1 = tItems[e - 1].first + tItems[e - 1].count;
             WalkArgs wa{};
             wa.hRes = in.dH;
             wa.vRes = in.dV;

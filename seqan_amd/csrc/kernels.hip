@@ -469,7 +469,14 @@ struct Bits16 {
     __device__ __forceinline__ uint32_t operator()(int i, int j) const
     {
         const int r = loc.p + i;
-        const int b = r / kTraceRows, rr = r % kTraceRows, l = rr / 16, k = rr % 16;
+        const int b = r / kTraceRows, rr = r % kTraceRows;
+        if (loc.lanes == 64) {
+            const int l = rr / 4, sh = rr % 4 + 8 * loc.half;
+            const uint32_t w = reinterpret_cast<const uint32_t *>(trace + loc.rec0 * 64)[((int64_t)b * loc.steps + (j + l)) * 64 + l];
+            return ((w >> sh) & 1u) | (((w >> (sh + 16)) & 1u) << 1) | (((w >> (sh + 4)) & 1u) << 2) |
+                   (((w >> (sh + 20)) & 1u) << 3);
+        }
+        const int l = rr / 16, k = rr % 16;
         const uint4 w = trace[(loc.rec0 + (int64_t)b * loc.steps + (j + l)) * 64 + loc.lane0 + l];
         const uint32_t ef = k < 8 ? w.x : w.y, dx = k < 8 ? w.z : w.w;
         const int sh = (k & 7) + 8 * loc.half;

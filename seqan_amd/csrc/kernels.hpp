@@ -97,11 +97,13 @@ struct TraceLoc {
     int32_t p;                  // item row of the pair's row 0
     int32_t lane0;              // first lane of the pair's group
     int32_t half;               // 0: low int16 half, 1: high
+    int32_t lanes;              // lanes per couple: 16, or 64 (records of one word)
     // The end-cell candidates of the pair's units (strips of the item, or the
     // whole item): ends[end0 + q * endStride], q < nEnds.
     int64_t end0;
     int32_t endStride;
     int32_t nEnds;
+    int32_t pad;
 };
 
 // End-cell candidates a trace unit leaves per pair, values in H: b, the best
@@ -456,10 +458,11 @@ hipError_t launchLong16WalkInit(const LongArgs &args, hipStream_t stream);
 hipError_t launchLong16Round(int R, const LongArgs &args, hipStream_t stream);
 
 // Trace family (trace16.hpp).
-constexpr int kTraceRows = 256;       // rows per block of the trace kernel (G = 16, R = 16)
+constexpr int kTraceRows = 256;       // rows per block of the trace kernel
 constexpr int kTraceLanes = 16;
-inline int traceSteps(int maxN) { return (maxN + kTraceLanes + 3) / 4 * 4; }   // column steps per block
-// Units as ScoreArgs', 256-row blocks throughout, `pad` the item's index.
+inline int traceSteps(int maxN, int lanes) { return (maxN + lanes + 3) / 4 * 4; }   // column steps per block
+// Units as ScoreArgs' (kUnit64: 64 lanes per couple, else 16), 256-row blocks
+// throughout, `pad` the item's index.
 struct TraceArgs {
     const uint8_t *hRes;
     const uint8_t *vRes;

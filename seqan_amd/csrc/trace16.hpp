@@ -4,7 +4,8 @@
 // trace16.hip.
 //
 // The sweep is the score kernel's (score16.hpp): drifted values, LDS rings,
-// strips; G = 16 lanes per pair couple and 16 rows per lane throughout.  Per
+// strips; blocks of 256 rows, by 16 lanes of 16 rows each per pair couple, or
+// by 64 lanes of 4 rows (a step takes a third of the time).  Per
 // cell four decisions are recorded, which is what dp_formula_affine.h:62-126
 // and _maxScore (dp_formula.h:165-201) record, ties resolved the same way:
 //   E  E(i,j) opened a gap:    E(i,j-1) + e <  G(i,j-1)   (TraceBitMap_ HORIZONTAL_OPEN)
@@ -23,14 +24,16 @@
 //   x, y: E of pair A, E of pair B, F of pair A, F of pair B
 //   z, w: D of pair A, D of pair B, X of pair A, X of pair B.
 // Records of block b, step s of an item sit at trace[(traceOff[item] + b *
-// steps + s) * 64 + lane]: one coalesced 1 KB store per wave and step.
+// steps + s) * 64 + lane]: one coalesced 1 KB store per wave and step.  With
+// 64 lanes a record is one word, x | z << 4 (four rows), and a step 256 bytes.
 //
 // What bounds it: vector issue (13 operations per row and the lookup, 90% of
 // the slots) while there are items for every wave; with few items, the sweep
-// of the longest, which strips spread over the chip.  Measured: 65,536 pairs
-// of 1 kbp, global, 17.4 -> 16.2 ms (34 GB of records at 2.1 TB/s beside it);
-// 8,191 uneven pairs, free first and last row, 277 ms with one wave per item
-// -> 7.7 ms; 8,192 protein pairs, local, 11.3 -> 3.3 ms.
+// of the longest, which strips spread over the chip and 64 lanes per couple
+// shorten.  Measured: 65,536 pairs of 1 kbp, global, 17.4 -> 16.2 ms (34 GB of
+// records at 2.1 TB/s beside it); 8,191 uneven pairs, free first and last row,
+// 277 ms with one wave per item -> 8.6 (strips) -> 4.3; 8,192 protein pairs,
+// local, 11.3 -> 3.5 ms.
 //
 // Values are compared as signed halves.  WIDE: stored values are held less
 // 32768, so that the whole 16-bit range is ordered and the differences
@@ -46,7 +49,6 @@
 namespace sqmi {
 namespace {
 
-constexpr int kTR = 16, kTG = 16;   // rows per lane, lanes per couple
 constexpr int kTOutWords = 4 * kPeriod + 64 + kPeriod;
 // Bottom rows with E beside G and F (the end cell's E and F).
 __shared__ uint4 gOutE[kWaves * kTOutWords];
@@ -60,10 +62,12 @@ __device__ __forceinline__ uint32_t signBytes(s16x2 t0, s16x2 t1)
 }
 __device__ __forceinline__ int half16(uint32_t w, int x) { return (int)(int16_t)(x ? w >> 16 : w); }
 
-template <bool DNA, uint32_t TRK, bool WIDE>
+template <int G, bool DNA, uint32_t TRK, bool WIDE>
 struct Trace16 {
     static constexpr bool LOC = (TRK & kTrackLocal) != 0;
-    static constexpr int G = kTG, RB = kTR, QD = kQD, P = kPeriod, RING = kRing<G>;
+    static constexpr int RB = kTraceRows / G, GROUPS = 64 / G, QD = kQD, P = kPeriod, RING = kRing<G>;
+    // A lane's record of a step (file head).
+    using Rec = std::conditional_t<G == 16, uint4, uint32_t>;
 
     __device__ __forceinline__ static uint32_t add(uint32_t a, uint32_t b) { return WIDE ? uadd2(a, b) : a + b; }
     __device__ __forceinline__ static uint32_t sub(uint32_t a, uint32_t b) { return WIDE ? usub2(a, b) : a - b; }
@@ -82,7 +86,7 @@ struct Trace16 {
     template <bool HEAD>
     __device__ __forceinline__ static void sweep(const TraceArgs &a, Couple c, int top, const bool last,
                                                  const bool strip, int Nw, const uint64_t *rowIn, uint64_t *rowOut,
-                                                 const uint32_t *sProf, const char *sT, uint4 *trBlock, Cand &cb,
+                                                 const uint32_t *sProf, const char *sT, Rec *trBlock, Cand &cb,
                                                  Cand &cr, bool &stop)
     {
         // Opaque copies, as in the score kernel.
@@ -160,13 +164,15 @@ struct Trace16 {
         auto hOfG = [&](int g, int ij) { return g + dr.cost - dr.bias - dr.d * ij; };
         auto hOf = [&](int g, int ij) { return g - dr.bias - dr.d * ij; };
 
-        uint4 *ring = gRing + wave * 4 * (RING + QD) + grp * (RING + QD);
-        uint32_t hr[2][2];
-        uint64_t rv[2];
+        constexpr int CPL = G == 16 ? 2 : 1;   // columns per lane of a refill (G = 64: lanes 0..31)
+        uint4 *ring = gRing + wave * 4 * (kRing<16> + QD) + (G == 16 ? grp * (kRing<16> + QD) : 0);
+        uint32_t hr[2][CPL];
+        uint64_t rv[CPL];
+        auto colOf = [&](int s, int q) { return G == 16 ? s + 2 * l + q : s + (l & (P - 1)); };
         auto refillLoad = [&](int s) {
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const int j = s + 2 * l + q;
+            for (int q = 0; q < CPL; ++q) {
+                const int j = colOf(s, q);
 #pragma unroll
                 for (int x = 0; x < 2; ++x)
                     hr[x][q] = c.h[x][min(max(j, 1), max(c.n[x], 1)) - 1];
@@ -183,11 +189,11 @@ struct Trace16 {
         auto refillStore = [&](int s) {
             if constexpr (!HEAD) {
                 if (strip)
-                    waitWords(rv, rowIn, Nw, s + 2 * l, a.error, stop);
+                    waitWords(rv, rowIn, Nw, colOf(s, 0), a.error, stop);
             }
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const int j = s + 2 * l + q, x = (j + G - 1) & (RING - 1);
+            for (int q = 0; q < CPL; ++q) {
+                const int j = colOf(s, q), x = (j + G - 1) & (RING - 1);
                 uint4 w;
                 w.x = prof(j >= 1 && j <= c.n[0] ? min((int)hr[0][q], PAD) : PAD);
                 w.y = prof(j >= 1 && j <= c.n[1] ? min((int)hr[1][q], PAD) : PAD);
@@ -205,9 +211,11 @@ struct Trace16 {
                     w.z = add(w.z, up);
                     w.w = add(w.w, up);
                 }
-                ring[x] = w;
-                if (x < QD)
-                    ring[x + RING] = w;
+                if (G == 16 || l < P) {
+                    ring[x] = w;
+                    if (x < QD)
+                        ring[x + RING] = w;
+                }
             }
             __builtin_amdgcn_wave_barrier();
         };
@@ -221,11 +229,11 @@ struct Trace16 {
         auto flush = [&](int s1, int cnt) {
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const int idx = 2 * l + q, j = s1 - cnt + idx - (G - 1);
-                const uint4 w = outBase[grp * P + idx];
+            for (int q = 0; q < CPL; ++q) {
+                const int idx = G == 16 ? 2 * l + q : l, j = s1 - cnt + idx - (G - 1);
                 if (idx >= cnt || j < 1 || j > Nw)
                     continue;
+                const uint4 w = outBase[grp * P + idx];
                 if (!last) {
                     uint32_t g = w.x, f = w.y;
                     if constexpr (LOC) {
@@ -407,7 +415,10 @@ struct Trace16 {
                         }
                     }
                 }
-                trBlock[(size_t)s * 64] = make_uint4(accEF0, accEF1, accDX0, accDX1);
+                if constexpr (G == 16)
+                    trBlock[(size_t)s * 64] = make_uint4(accEF0, accEF1, accDX0, accDX1);
+                else
+                    trBlock[(size_t)s * 64] = accEF0 | accDX0 << 4;
             }
             out[u] = make_uint4(botG, botF, botE, 0);
         };
@@ -513,9 +524,12 @@ struct Trace16 {
         const bool strip = w.block >= 0;
         const int stride = w.maxN + 1, steps = (w.maxN + G + QD - 1) / QD * QD;
         const int64_t rec0 = a.traceOff[item];
-        if (pairs < 1 || pairs > 8 || w.maxN < 1 || nb < 1 || nb > (1 << 15) || w.block >= nb ||
-            rec0 < 0 || rec0 + (int64_t)nb * steps > a.traceRecs ||
-            (strip ? w.rowOff < 0 || w.rowOff + (int64_t)nb * 4 * stride > a.stripWords : (int64_t)4 * stride > a.slotWords))
+        // (A step of one couple on 64 lanes takes a quarter of one of four on 16.)
+        constexpr int Q = G == 16 ? 1 : 4;
+        if (pairs < 1 || pairs > 2 * GROUPS || w.maxN < 1 || nb < 1 || nb > (1 << 15) || w.block >= nb ||
+            rec0 < 0 || Q * rec0 + (int64_t)nb * steps > Q * a.traceRecs ||
+            (strip ? w.rowOff < 0 || w.rowOff + (int64_t)nb * GROUPS * stride > a.stripWords
+                   : (int64_t)GROUPS * stride > a.slotWords))
             return;
         Couple c;
 #pragma unroll
@@ -544,14 +558,14 @@ struct Trace16 {
             cb.i[x] = cr.i[x] = cb.j[x] = cr.j[x] = 0x7fffffff;
             cb.e[x] = cr.e[x] = cb.f[x] = cr.f[x] = INT32_MIN;
         }
-        uint4 *tr = a.trace + (size_t)rec0 * 64 + lane;
+        Rec *tr = reinterpret_cast<Rec *>(a.trace + (size_t)rec0 * 64) + lane;
         const int b0 = strip ? w.block : 0, b1 = strip ? w.block + 1 : nb;
         for (int b = b0; b < b1; ++b) {
             const bool last = b == nb - 1;
-            const uint64_t *in = strip ? a.strips + w.rowOff + ((int64_t)(b - 1) * 4 + grp) * stride
+            const uint64_t *in = strip ? a.strips + w.rowOff + ((int64_t)(b - 1) * GROUPS + grp) * stride
                                        : slotRow + (int64_t)grp * stride;
-            uint64_t *out = strip ? a.strips + w.rowOff + ((int64_t)b * 4 + grp) * stride : slotRow + (int64_t)grp * stride;
-            uint4 *trBlock = tr + (size_t)b * steps * 64;
+            uint64_t *out = strip ? a.strips + w.rowOff + ((int64_t)b * GROUPS + grp) * stride : slotRow + (int64_t)grp * stride;
+            Rec *trBlock = tr + (size_t)b * steps * 64;
             if (b == 0)
                 sweep<true>(a, c, 0, last, strip, w.maxN, in, out, sProf, sT, trBlock, cb, cr, stop);
             else
@@ -589,10 +603,17 @@ __device__ __forceinline__ void traceRun(const TraceArgs &a)
         if (it >= a.nUnits)
             break;
         const ScoreUnit w = uniformUnit(a.units[it]);
-        if (w.shape & kUnitWide)
-            Trace16<DNA, TRK, true>::unit(a, w, slotRow, sProf, sT, stop);
-        else
-            Trace16<DNA, TRK, false>::unit(a, w, slotRow, sProf, sT, stop);
+        if (w.shape & kUnit64) {
+            if (w.shape & kUnitWide)
+                Trace16<64, DNA, TRK, true>::unit(a, w, slotRow, sProf, sT, stop);
+            else
+                Trace16<64, DNA, TRK, false>::unit(a, w, slotRow, sProf, sT, stop);
+        } else {
+            if (w.shape & kUnitWide)
+                Trace16<16, DNA, TRK, true>::unit(a, w, slotRow, sProf, sT, stop);
+            else
+                Trace16<16, DNA, TRK, false>::unit(a, w, slotRow, sProf, sT, stop);
+        }
     }
 }
 

@@ -90,3 +90,22 @@ def test_local_best_in_an_early_block(ctx, monkeypatch):
                 hs.append(h)
                 vs.append(v)
         _check_rows(ctx, sa.SeqSet.from_list(hs), sa.SeqSet.from_list(vs), score, sa.LOCAL)
+
+
+@pytest.mark.parametrize("budget", ["", "2"])
+@pytest.mark.parametrize("lanes", ["16", "64"])
+def test_lanes_per_couple(ctx, monkeypatch, lanes, budget):
+    # Both forms of the trace kernel for every item, in one chunk and several;
+    # lengths around a block (256 rows) and a lane's rows (4 and 16).
+    monkeypatch.setenv("SQMI_TRACE_LANES", lanes)
+    if budget:
+        monkeypatch.setenv("SQMI_TRACE_BUDGET_MB", budget)
+    rng = np.random.default_rng(15)
+    lengths = [1, 3, 4, 5, 15, 16, 17, 63, 64, 65, 250, 254, 255, 256, 257, 260, 511, 512, 700, 1300]
+    H, V = _set(rng, lengths)
+    for scheme in ((2, -3, -1, -5), (20, -30, -20, -60), (4, -2, -6, -3)):
+        for mode in (0, 9, 15, 2, 4, sa.LOCAL):
+            _check_rows(ctx, H, V, sa.simple_score(*scheme), mode)
+    P, Q = _set(rng, [900, 400, 300, 1200, 255, 31], 24)
+    for mode in (0, 15, sa.LOCAL):
+        _check_rows(ctx, P, Q, sa.blosum62(-1, -11), mode)
