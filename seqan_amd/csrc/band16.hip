@@ -11,18 +11,18 @@
 
 namespace sqmi {
 
-// Rows per block and ring: 8 rows with LDS rings (bands of up to 24
-// diagonals), 12 with either, 16 with rings in memory.
+// Rows per block: 8 and 12 with LDS rings, 16 with either.
 template <bool WIDE>
 static const void *part(int R, bool lds)
 {
     constexpr bool dna = SQMI_BAND_DNA != 0;
     constexpr int kind = SQMI_BAND_KIND;
-    if (R == 8)
-        return lds ? (const void *)&kBand16<8, dna, kind, WIDE, true> : nullptr;
-    if (R == 12)
-        return lds ? (const void *)&kBand16<12, dna, kind, WIDE, true> : (const void *)&kBand16<12, dna, kind, WIDE, false>;
-    return R == 16 && !lds ? (const void *)&kBand16<16, dna, kind, WIDE, false> : nullptr;
+    if (R == 16)
+        return lds ? (const void *)&kBand16<16, dna, kind, WIDE, true> : (const void *)&kBand16<16, dna, kind, WIDE, false>;
+    if (!lds)
+        return nullptr;
+    return R == 12 ? (const void *)&kBand16<12, dna, kind, WIDE, true>
+                   : R == 8 ? (const void *)&kBand16<8, dna, kind, WIDE, true> : nullptr;
 }
 
 const void *SQMI_BAND_PART(int R, bool wide, bool lds) { return wide ? part<true>(R, lds) : part<false>(R, lds); }

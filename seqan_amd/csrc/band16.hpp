@@ -33,11 +33,13 @@
 // sums included) stays there.  Row buffer entries a block reads outside the
 // columns the block above wrote only feed cells outside the band.
 //
-// What bounds it: the issue of one wave per SIMD (the rings of more do not
-// fit the LDS, or one XCD's L2), about 290 ns per column of 12 rows.  1,048,576 pairs of 150
-// bp, band [-16, 16], global: 1.62 -> 1.37 ms against plain saturating values
-// (9 instructions per packed cell, 6.4 now); 65,536 pairs of 1 kbp, band
-// [-100, 100], free ends: 51.8 -> 4.0 ms against a wave per pair in 32 bits.
+// What bounds it: vector issue with two waves per SIMD (8 waves per CU, whose
+// rings fill the LDS) in full calls, an item's blocks in small ones.  1,048,576
+// pairs of 150 bp, band [-16, 16], global: 1.62 ms in plain saturating values
+// (9 instructions per packed cell, 6.4 now), 1.37 in drifted ones with a wave per
+// item, 1.12 with two waves sharing one; 65,536 pairs of 1 kbp, band [-100,
+// 100], free ends: 51.8 (a wave per pair in 32 bits) -> 4.0 -> 2.4 ms, 1,000 of
+// them 0.81.
 #pragma once
 
 #include <type_traits>
@@ -51,8 +53,12 @@ namespace {
 
 constexpr int kBandRebase = 16;   // local: columns between rebases of the drift
 
-// LR: the row-buffer ring lives in LDS (dynamic shared memory, one ring per
-// wave) instead of global memory.  WIDE: values above kDriftNarrowMax.
+// LR: the row-buffer ring lives in LDS (dynamic shared memory) and the waves of
+// a workgroup share an item: wave w takes its blocks w, w + waves, ..., each a few
+// columns behind the block above, whose progress it reads from LDS (all waves
+// of a workgroup run, and block b waits for block b - 1 only, so every wait
+// ends; it is bounded besides).  Otherwise each wave has a ring in global
+// memory and sweeps items of its own.  WIDE: values above kDriftNarrowMax.
 template <int R, bool DNA, int KIND, bool WIDE, bool LR>
 struct Band16 {
     static constexpr int QD = 4;   // columns per group: one dword of residues per pair
@@ -66,6 +72,34 @@ struct Band16 {
     struct Best {
         int2 H;            // global: the best tracked cell (H)
         uint32_t b2;       // local: the best G, without drift
+    };
+    // LR: columns finished, block << 16 | column (0xffff: all), of the wave
+    // that sweeps the block above and of this one.
+    struct Progress {
+        uint32_t *up, *own;
+        uint32_t upBase, ownBase;
+        uint32_t *error;
+        __device__ __forceinline__ void waitFor(int col, uint32_t &seen) const
+        {
+            const uint32_t need = upBase + (uint32_t)min(col, 0xffff);
+            for (int spins = 0; seen < need; ++spins) {
+                seen = (uint32_t)__builtin_amdgcn_readfirstlane(
+                    (int)__hip_atomic_load(up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+                if (seen >= need)
+                    break;
+                if (spins > (1 << 22)) {
+                    __hip_atomic_store(error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    seen = 0xffffffffu;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            asm volatile("" ::: "memory");   // the ring reads stay behind (a wave's LDS operations run in order)
+        }
+        __device__ __forceinline__ void publish(int col) const
+        {
+            asm volatile("" ::: "memory");
+            __hip_atomic_store(own, ownBase + (uint32_t)col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
     };
 
     __device__ __forceinline__ static uint32_t add(uint32_t a, uint32_t b) { return WIDE ? uadd2(a, b) : a + b; }
@@ -96,7 +130,7 @@ struct Band16 {
     // first block's row above starts it and their score (padScore) keeps it.
     __device__ __forceinline__ static void block(const FwdArgs &a, const Couple &c, int i0, int maxN, int minN, bool first,
                                                  bool last, uint2 *rb, const uint32_t *sProf, const int16_t *sT,
-                                                 Best &best)
+                                                 Best &best, const Progress &pg)
     {
         Drift dr = a.drift;
         dr.d = __builtin_amdgcn_readfirstlane(dr.d);
@@ -194,6 +228,9 @@ struct Band16 {
         // The diagonal input of the first swept column, and column 0 of this
         // block's bottom row for the next block.
         const int cm = a.bandCols - 1;
+        uint32_t seen = 0;
+        if (LR && !first)
+            pg.waitFor(jA + QD - 1, seen);
         uint32_t topG = !LOC && topFree ? (uint32_t)(dr.bias - dr.cost) * 0x10001u : neg2;   // first block: G above
         const uint32_t topStep = !LOC && topFree ? d2 : 0u;
         uint32_t upGprev = first ? topG : rb[((jA - 1) & cm) * 64].x;
@@ -262,6 +299,8 @@ struct Band16 {
                     dcol = 0;
                 }
             }
+            if (LR && !first)
+                pg.waitFor(s0 + 2 * QD - 1, seen);
 #pragma unroll
             for (int u = 0; u < QD; ++u)
                 nx[u] = rb[((s0 + QD + u) & cm) * 64];   // read before this block writes them, next group
@@ -375,6 +414,8 @@ struct Band16 {
                 rb[((s0 + u) & cm) * 64] = outv[u];
                 rq[u] = nx[u];
             }
+            if constexpr (LR)
+                pg.publish(s0 + QD - 1);
         };
         int s0 = jA, g = gS;
         // The group's residue bytes; the next group's dwords are loaded
@@ -408,10 +449,14 @@ struct Band16 {
         }
         if constexpr (LOC)
             best.b2 = sub(b2, (uint32_t)dcol * (uint32_t)dr.d * 0x10001u);
-        // The next block reads this block's row-buffer entries from the
-        // same lane: order the stores before those loads.
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        if constexpr (LR) {
+            pg.publish(0xffff);
+        } else {
+            // The next block reads this block's row-buffer entries from the
+            // same lane: order the stores before those loads.
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        }
     }
 
     // Work item: `first` .. first + (count & 0xffff) of `order`, all of length
@@ -448,17 +493,30 @@ struct Band16 {
 
         const int lane = threadIdx.x & 63;
         const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        const size_t slot = (size_t)blockIdx.x * (blockDim.x >> 6) + wave;
+        const int waves = (int)(blockDim.x >> 6);
+        __shared__ uint32_t sProg[kBandWaves], sItem;
+        __shared__ int2 sBest[LR ? kBandWaves * 64 : 1];
         uint2 *rb;
         if constexpr (LR) {
             extern __shared__ uint2 sRing[];
-            rb = sRing + (size_t)wave * a.bandCols * 64 + lane;
+            rb = sRing + lane;
         } else {
-            rb = reinterpret_cast<uint2 *>(a.rowbuf) + slot * (size_t)a.rowCols * 64 + lane;
+            rb = reinterpret_cast<uint2 *>(a.rowbuf) + ((size_t)blockIdx.x * waves + wave) * (size_t)a.rowCols * 64 + lane;
         }
         for (;;) {
-            // Branch-free fetch: every lane takes part (lane 0 adds 1).
-            int it = (int)atomicAdd(a.queue, lane == 0 ? 1u : 0u);
+            int it;
+            if constexpr (LR) {
+                if (threadIdx.x == 0)
+                    sItem = atomicAdd(a.queue, 1u);
+                if (threadIdx.x < kBandWaves)
+                    sProg[threadIdx.x] = 0;
+                __syncthreads();
+                it = (int)sItem;
+                __syncthreads();   // read by every wave before it is set again
+            } else {
+                // Branch-free fetch: every lane takes part (lane 0 adds 1).
+                it = (int)atomicAdd(a.queue, lane == 0 ? 1u : 0u);
+            }
             it = __builtin_amdgcn_readfirstlane(it);
             if (it >= a.nItems)
                 break;
@@ -493,11 +551,25 @@ struct Band16 {
             }
             Best best{make_int2(INT32_MIN, INT32_MIN), (uint32_t)(a.drift.bias - a.drift.cost) * 0x10001u};
             const int p = w.nblocks * R - 1 - m;   // item row of row 0
-            for (int b = 0; b < w.nblocks; ++b)
-                block(a, c, b * R - p, w.maxN, minN, b == 0, b == w.nblocks - 1, rb, sProf, sT, best);
+            for (int b = LR ? wave : 0; b < w.nblocks; b += LR ? waves : 1) {
+                Progress pg{};
+                if constexpr (LR)
+                    pg = Progress{sProg + (b + waves - 1) % waves, sProg + wave, (uint32_t)(b - 1) << 16, (uint32_t)b << 16, a.error};
+                block(a, c, b * R - p, w.maxN, minN, b == 0, b == w.nblocks - 1, rb, sProf, sT, best, pg);
+            }
             if constexpr (LOC)
                 best.H = make_int2((int)(best.b2 & 0xffffu) + a.drift.cost - a.drift.bias,
                                    (int)(best.b2 >> 16) + a.drift.cost - a.drift.bias);
+            if constexpr (LR) {
+                sBest[wave * 64 + lane] = best.H;
+                __syncthreads();
+                if (wave != 0)
+                    continue;
+                for (int q = 1; q < waves; ++q) {
+                    const int2 o = sBest[q * 64 + lane];
+                    best.H = make_int2(max(best.H.x, o.x), max(best.H.y, o.y));
+                }
+            }
             if (c.pid[0] >= 0)
                 a.scores[c.pid[0]] = best.H.x;
             if (c.pid[1] >= 0)
@@ -507,7 +579,7 @@ struct Band16 {
 };
 
 template <int R, bool DNA, int KIND, bool WIDE, bool LR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R >= 12 ? 2 : 3))) void kBand16(FwdArgs a)
+__global__ __launch_bounds__(LR ? 64 * kBandWaves : 256) __attribute__((amdgpu_waves_per_eu(2))) void kBand16(FwdArgs a)
 {
     Band16<R, DNA, KIND, WIDE, LR>::run(a);
 }

@@ -556,12 +556,17 @@ struct LongCost {
     double alone, full;
 };
 constexpr LongCost kLongCosts[] = {{4, 115, 63}, {8, 153, 111}, {16, 230, 203}};
-// Banded scores, ns: a column of a packed item's block (one wave per SIMD);
-// a row of a pair on the int32 kernels, alone and per SIMD of a full chip
-// (wide: of 64 diagonals).  1,000 to 65,536 pairs: free ends, 1 kbp, 201
-// diagonals, packed 3.9-4.0 ms, int32 2.5, 3.3 (4,096), 12.9 (16,384) and
-// 51.8; local, 150 bp, 33 diagonals, 0.19-0.20 against 0.04, 0.06, 0.19, 0.67.
-constexpr double kBandColumn = 310, kBandNarrowLone = 270, kBandNarrowFull = 70, kBandWideLone = 615, kBandWideFull = 202;
+// Waves of a workgroup of the packed banded kernel, by its ring's columns: the
+// ring is the band and a block, and a wave follows the one above by R + 8
+// columns.  (Rings past 256 columns: four waves with rings of their own.)
+int bandWaves(int cols) { return cols > 256 ? 4 : cols > 128 ? 8 : cols > 64 ? 4 : 2; }
+// Banded scores, ns: a column of a packed item's block, by one wave (rings in
+// memory) and with 2, 4 and 8 waves sharing the item; a row of a pair on the
+// int32 kernels, alone and per SIMD of a full chip (wide: of 64 diagonals).
+// 1,000 / 4,096 / 16,384 / 65,536 pairs, free ends, 1 kbp, 201 diagonals: packed
+// 0.81 / 0.81 / 0.84 / 2.5 ms, int32 2.5 / 3.3 / 12.8 / 51.5; local, 150 bp,
+// 33 diagonals: 0.11 / 0.11 / 0.11 / 0.18 against 0.04 / 0.06 / 0.19 / 0.68.
+constexpr double kBandColumnAlone = 335, kBandColumn[3] = {170, 80, 60}, kBandNarrowLone = 270, kBandNarrowFull = 70, kBandWideLone = 615, kBandWideFull = 202;
 // Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
 constexpr int64_t kResidentWaves = 3072;
 // Rows per unit of the group shapes' row counts.
@@ -3091,14 +3096,10 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     const int64_t W1 = upper_diag - lower_diag;
     // Rows per block: more rows share a block's set-up and boundary columns,
     // fewer compute fewer cells outside the band (W - 1 + R columns per
-    // block for W band cells per row).  Band [-16, 16] on 1 M pairs of 150
-    // bp: R = 12 1.64 ms, 16 1.74 ms; [-100, 100] on 65,536 pairs of 1 kbp:
-    // R = 16 4.66 ms, 12 5.10 ms.
-    int bandR = W1 >= 64 ? 16 : W1 >= 24 ? 12 : 8;
-    if (const char *env = std::getenv("SQMI_BAND_ROWS")) {   // tuning knob: 12 or 16 rows per block
-        const int r = std::atoi(env);
-        bandR = W1 >= 24 && (r == 12 || r == 16) ? r : bandR;
-    }
+    // block for W band cells per row).  In plain values, a wave per item: band
+    // [-16, 16] on 1 M pairs of 150 bp: R = 12 1.64 ms, 16 1.74 ms; [-100,
+    // 100] on 65,536 pairs of 1 kbp: R = 16 4.66 ms, 12 5.10 ms.
+    const int bandR = W1 >= 64 ? 16 : W1 >= 24 ? 12 : 8;
     si.dnaDrift = si.dna && si.sMax - si.o - std::max(si.o, si.e) <= 255;
     const bool bandCostsOk = !(flags & SQMI_FORCE_INT32) && W1 >= bandR && si.o <= 0 && si.e <= 0 && si.o >= -1024 &&
                              si.e >= -1024 && si.sMax <= 1024 && si.sMin >= -1024 && si.alpha + 1 <= 33 &&
@@ -3227,7 +3228,10 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
             full += (it.count & 0xffff) * m * (w <= 64 ? kBandNarrowFull * w / 64 : kBandWideFull * chunks);
         }
         const double simds = 4.0 * std::max(1, ctx->numCUs);
-        if (std::max(lone, full / simds) < std::ceil(bandItems.size() / simds) * blockCols * kBandColumn) {
+        const int cols = bandRingCols(bandMaxN, lower_diag, upper_diag, bandR), waves = bandWaves(cols);
+        const double slots = cols > 256 ? simds : 2 * simds / waves;
+        const double column = cols > 256 ? kBandColumnAlone : kBandColumn[waves == 8 ? 2 : waves == 4 ? 1 : 0];
+        if (std::max(lone, full / simds) < std::ceil(bandItems.size() / slots) * blockCols * column) {
             for (int32_t id : packed)
                 toInt32(id, offH[id + 1] - offH[id], offV[id + 1] - offV[id]);
             packed.clear();
@@ -3267,23 +3271,21 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     int bandGrid = 0, bandRowColsN = 0, bandLds = 0;
     BandVariant bandVar{};
     if (!bandItems.empty()) {
-        // Workgroups of 4 waves per CU: the occupancy limit, but no more than
-        // keep the row-buffer rings of a CU's waves within its share of L2
-        // (at least one).  On 1 M pairs of 150 bp, band [-16, 16] (rings of
-        // 32 KB per wave), 1, 2 and 3 workgroups per CU ran 1.92, 2.09 and
-        // 2.61 ms: the rings of more waves than L2 holds go to memory.
-        // Rings of up to 64 columns (128 KB per workgroup) live in LDS, which
-        // also limits the CU to the workgroups whose rings fit.
+        // Rings of up to 256 columns (128 KB) live in LDS, one per workgroup,
+        // whose waves share an item; 8 waves per CU whatever the ring.
+        // Larger ones lie in global memory, one per wave: as many workgroups
+        // of 4 waves as keep a CU's rings within its share of L2 (at least
+        // one; more send the rings to memory).
         bandRowColsN = bandRingCols(bandMaxN, lower_diag, upper_diag, bandR);
-        bandLds = bandR == 16 ? 0 : bandLdsRingBytes(bandRowColsN);
+        bandLds = bandLdsRingBytes(bandRowColsN);
         bandVar = BandVariant{bandR, local ? si.dna : si.dnaDrift,
                               local ? kBandLocal : (mode & (SQMI_FREE_BOTTOM | SQMI_FREE_RIGHT)) ? kBandFree : kBandEnd,
-                              bandWide, bandLds > 0};
+                              bandWide, bandLds > 0, bandWaves(bandRowColsN)};
         const int64_t ringBytes = (int64_t)64 * bandRowColsN * 8;   // per wave
         const int most = occupancyBand16(bandVar, bandLds);
         const int occ = bandLds ? most : (int)std::max<int64_t>(1, std::min<int64_t>(most, ctx->l2PerCU / (4 * ringBytes)));
         const int64_t nIt = (int64_t)bandItems.size();
-        bandGrid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occ, (nIt + 3) / 4));
+        bandGrid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occ, bandLds ? nIt : (nIt + 3) / 4));
         if ((err = ensure(ctx->b.queue, 64)) != hipSuccess ||
             (err = ensure(ctx->b.rowbuf, bandLds ? 64 : (size_t)bandGrid * 4 * 64 * bandRowColsN * 8)) != hipSuccess)
             return hipFail(ctx, err, "allocating packed banded buffers");
@@ -3318,6 +3320,7 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
         f.tTable = static_cast<const int16_t *>(ctx->b.tTable.p);
         f.dnaProfile = static_cast<const uint32_t *>(ctx->b.dnaProf.p);
         f.drift = dr;
+        f.error = ctx->waitFlag;
         f.bandLo = (int32_t)lower_diag;
         f.bandUp = (int32_t)upper_diag;
         if ((err = launchBand16(bandVar, f, bandGrid, bandLds, stream)) != hipSuccess)
@@ -3362,6 +3365,8 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
         return hipFail(ctx, err, "banded kernels");
     deliver(ctx);
     stageEnd(ctx);
+    if ((st = stripCheck(ctx)) != SQMI_OK)
+        return st;
     float ms = 0;
     if (hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1) == hipSuccess)
         ctx->stats.device_ms = ms;

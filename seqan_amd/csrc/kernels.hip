@@ -781,9 +781,9 @@ int bandRingCols(int maxN, int64_t lower, int64_t upper, int R)
 
 int bandLdsRingBytes(int bandCols)
 {
-    // Four waves' rings of bandCols columns x 64 lanes x 8 bytes, when they
-    // leave room for the static tables in the 160 KB of LDS per CU.
-    const int64_t bytes = (int64_t)4 * 64 * bandCols * 8;
+    // A ring of bandCols columns x 64 lanes x 8 bytes, when it leaves room
+    // for the static tables in the 160 KB of LDS per CU.
+    const int64_t bytes = (int64_t)64 * bandCols * 8;
     return bytes > 128 * 1024 ? 0 : (int)bytes;
 }
 
@@ -793,7 +793,7 @@ int occupancyBand16(const BandVariant &v, int ringLdsBytes)
     int blocks = 0;
     if (!k || (v.lds && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, ringLdsBytes) != hipSuccess))
         return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, (size_t)ringLdsBytes) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 64 * v.waves, (size_t)ringLdsBytes) != hipSuccess)
         return 1;
     return blocks > 0 ? blocks : 1;
 }
@@ -805,7 +805,7 @@ hipError_t launchBand16(const BandVariant &v, const FwdArgs &args, int gridBlock
         return hipErrorInvalidValue;
     FwdArgs copy = args;
     void *params[] = {&copy};
-    return hipLaunchKernel(k, dim3(gridBlocks), dim3(256), params, (size_t)ringLdsBytes, stream);
+    return hipLaunchKernel(k, dim3(gridBlocks), dim3(64 * v.waves), params, (size_t)ringLdsBytes, stream);
 }
 
 hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBlocks, hipStream_t stream,

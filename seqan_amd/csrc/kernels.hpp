@@ -86,6 +86,7 @@ struct FwdArgs {
     Drift drift;                // global score kernels
     int32_t bandLo, bandUp;     // banded kernels: cells with bandLo <= j - i <= bandUp
     int32_t bandCols;           // banded kernels: row-buffer ring columns (a power of two <= rowCols)
+    uint32_t *error;            // banded kernels: as in ScoreArgs
 };
 
 // Where the trace records of one pair live: rows are bottom-aligned in the
@@ -250,8 +251,9 @@ int laneRowCols(int maxN, int R);
 // block, bandUp - bandLo >= R; work items hold up to 128 pairs of one length m
 // (WorkItem.count = pairs | m << 16, nblocks = (m + R) / R).  Row buffer per
 // wave slot: a ring of bandRingCols(...) columns x 64 lanes x 8 bytes, in LDS
-// where bandLdsRingBytes() > 0.  R: 8 with LDS rings, 12 with either, 16 with
-// rings in memory.
+// where bandLdsRingBytes() > 0 (one ring per workgroup of `waves` waves, else
+// one per wave of four).  R: 8 and 12 with LDS rings, 16 with either.
+constexpr int kBandWaves = 8;
 enum BandKind : int { kBandEnd = 0, kBandFree = 1, kBandLocal = 2 };   // cell (m, n); free last row / column; local
 struct BandVariant {
     int R;
@@ -259,6 +261,7 @@ struct BandVariant {
     int kind;
     bool wide;      // values above kDriftNarrowMax
     bool lds;
+    int waves;      // per workgroup
 };
 constexpr int bandRowCols(int maxN) { return (maxN + 3) / 4 * 4 + 5; }
 int bandRingCols(int maxN, int64_t lower, int64_t upper, int R);

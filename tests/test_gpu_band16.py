@@ -92,3 +92,23 @@ def test_mismatching_pairs_in_narrow_bands(ctx, monkeypatch):
     for score in (sa.simple_score(2, -3, -1, -5), sa.simple_score(5, -4, -2, -10), sa.simple_score(2, -30, -1, -29)):
         for mode in (0, 9, 15, sa.LOCAL):
             _check(ctx, hs, vs, score, mode, -13, 13)
+
+
+@pytest.mark.parametrize("band", [(-10, 12), (-18, 18), (-40, 60), (-70, 90), (-110, 115), (-200, 150)])
+def test_shared_items(ctx, monkeypatch, band):
+    # 2, 4 and 8 waves on an item's blocks, and one (the widest band): items of
+    # fewer blocks than waves, of many, several items per workgroup.
+    monkeypatch.setenv("SQMI_BAND_PACKED", "1")
+    lo, up = band
+    rng = np.random.default_rng(300 + up)
+    hs, vs = _pairs(rng, 60, lo, up, 4, 60, False)
+    for m in (1, 7, 8, 130, 511, 1200):
+        for _ in range(20):
+            v = rng.integers(0, 4, m).astype(np.uint8)
+            n = max(2, m + int(rng.integers(lo // 2, up // 2)))
+            if not _valid(n, m, lo, up, False):
+                continue
+            hs.append(np.concatenate([v, rng.integers(0, 4, n).astype(np.uint8)])[:n])
+            vs.append(v)
+    for mode in (0, 9, 15, sa.LOCAL):
+        _check(ctx, hs, vs, sa.simple_score(2, -3, -1, -5), mode, lo, up)
