@@ -321,30 +321,34 @@ __device__ __forceinline__ void walkCounts(int n, int m, const uint8_t *h, const
 // the next 16 cells of the diagonal (or of the gap) at once, so a walk waits
 // for memory once per run of equal moves (or per 16 of them) instead of once
 // per move.  What bounds it then is the records' traffic: each cell's record
-// sits in a line of its own (65,536 pairs of 1 kbp 1.85 -> 1.47 ms; 8,191
-// uneven pairs of up to 10 kbp, where the longest walk counts, 13.8 -> 1.2 ms;
-// 8,192 protein pairs local 1.24 -> 0.12 ms; 65,536 banded pairs of 150 bp
+// sits in a line of its own (65,536 pairs of 1 kbp 1.85 -> 1.39 ms; 8,191
+// uneven pairs of up to 10 kbp, where the longest walk counts, 13.8 -> 0.5 ms;
+// 8,192 protein pairs local 1.24 -> 0.1 ms; 65,536 banded pairs of 150 bp
 // 0.67 -> 0.17 ms).  The state is kept alike in all lanes of the group;
 // groups of a wave diverge as they like (a group's lanes never do, outside
 // predicated statements).
+//
+// W lanes per pair: 16, or a whole wave (64) in calls of few pairs, which wait
+// for their longest walk (kWalkWavePairs).
 constexpr int kWalkLanes = 16;
 
-__device__ __forceinline__ uint32_t groupBallot(bool p)
+template <int W>
+__device__ __forceinline__ uint64_t groupBallot(bool p)
 {
-    return (uint32_t)(__ballot(p) >> (threadIdx.x & 48)) & 0xffffu;
+    return W == 64 ? __ballot(p) : (__ballot(p) >> (threadIdx.x & 48)) & 0xffffu;
 }
 
 struct WalkEnd {
     int score, i, j, e, f;   // the end cell
 };
 
-template <class Bits>
+template <int W, class Bits>
 __device__ __forceinline__ void walkGroup(int n, int m, const uint8_t *h, const uint8_t *v, int A, const WalkEnd &end,
                                           const Bits &bits, int32_t *cnt, uint8_t *opEnd, int64_t *opLen, bool local,
                                           int64_t *begins, bool linear, bool alwaysOpen, const int32_t *lTab, int go,
                                           int ge)
 {
-    const int t = threadIdx.x & (kWalkLanes - 1);
+    const int t = threadIdx.x & (W - 1);
     int cur = end.score, i = end.i, j = end.j;
     if (local) {
         m = i;
@@ -361,7 +365,7 @@ __device__ __forceinline__ void walkGroup(int n, int m, const uint8_t *h, const 
         if (k > 0)
             prev = kind;
         if (opEnd)
-            for (int q = t; q < k; q += kWalkLanes)
+            for (int q = t; q < k; q += W)
                 opEnd[-1 - nOps - q] = kind == 0 ? 'M' : kind == 1 ? 'V' : 'H';
         nOps += k;
     };
@@ -379,32 +383,33 @@ __device__ __forceinline__ void walkGroup(int n, int m, const uint8_t *h, const 
         // Aligned pairs from (i, j) up the diagonal.
         const int ii = i - t, jj = j - t;
         const bool valid = ii > 0 && jj > 0;
+        // The residues with the bits, though cells past the run do not need
+        // them: one wait instead of two.
+        const int rh = valid ? h[jj - 1] : 0, rw = valid ? v[ii - 1] : 0;
         const uint32_t b = valid ? bits(ii, jj) : 0;
         int d = valid ? dirOf(b) : 3;
         if (t == 0 && first)
             d = known;
         const bool none = local && !lTab && (b & kBitStop) != 0 && !(first && t == 0);
-        const uint32_t end16 = groupBallot(d != 0 || none);
-        int r = end16 ? __builtin_ctz(end16) : kWalkLanes;
+        const uint64_t stops = groupBallot<W>(d != 0 || none);
+        int r = stops ? __builtin_ctzll(stops) : W;
         bool stopped = false;
-        int hv = 0;
-        if (t < r)
-            hv = min((int)h[jj - 1], A - 1) * A + min((int)v[ii - 1], A - 1);
+        const int hv = min(rh, A - 1) * A + min(rw, A - 1);
         if (lTab) {
             // H along the run; the walk stops on the first cell where it is 0.
             int sum = t < r ? lTab[hv] : 0;
 #pragma unroll
-            for (int q = 1; q < kWalkLanes; q <<= 1) {
-                const int o = __shfl_up(sum, q, kWalkLanes);
+            for (int q = 1; q < W; q <<= 1) {
+                const int o = __shfl_up(sum, q, W);
                 sum += t >= q ? o : 0;
             }
-            const uint32_t zero = groupBallot(t < r && cur == sum && ii > 1 && jj > 1);
+            const uint64_t zero = groupBallot<W>(t < r && cur == sum && ii > 1 && jj > 1);
             if (zero) {
-                r = __builtin_ctz(zero) + 1;
+                r = __builtin_ctzll(zero) + 1;
                 stopped = true;
             }
             if (r > 0)
-                cur -= __shfl(sum, r - 1, kWalkLanes);
+                cur -= __shfl(sum, r - 1, W);
         }
         if (t < r)
             atomicAdd(cnt + hv, 1);
@@ -413,22 +418,22 @@ __device__ __forceinline__ void walkGroup(int n, int m, const uint8_t *h, const 
         j -= r;
         if (stopped || i <= 0 || j <= 0)
             break;
-        if (r == kWalkLanes) {
+        if (r == W) {
             first = false;
             continue;
         }
-        if (__shfl((int)none, r, kWalkLanes))
+        if (__shfl((int)none, r, W))
             break;
-        const bool vert = __shfl(d, r, kWalkLanes) == 1;
+        const bool vert = __shfl(d, r, W) == 1;
         first = false;
         // A gap: up to the cell that opened it, or row / column 1.
         for (;;) {
             const int gi = vert ? i - t : i, gj = vert ? j : j - t, at = vert ? gi : gj;
             const uint32_t gb = at > 0 ? bits(gi, gj) : 0;
             const bool open = alwaysOpen || (gb & (vert ? kBitFOpen : kBitEOpen)) != 0;
-            const uint32_t gEnd = groupBallot(at > 0 && (linear || open || at == 1));
-            const int g = gEnd ? __builtin_ctz(gEnd) + 1 : kWalkLanes;
-            const bool opened = linear || __shfl((int)open, g - 1, kWalkLanes) != 0;
+            const uint64_t gEnd = groupBallot<W>(at > 0 && (linear || open || at == 1));
+            const int g = gEnd ? __builtin_ctzll(gEnd) + 1 : W;
+            const bool opened = linear || __shfl((int)open, g - 1, W) != 0;
             emit(vert ? 1 : 2, g);
             cur -= ge * (g - 1) + (gEnd && opened ? go : ge);
             if (vert)
@@ -527,9 +532,9 @@ __global__ __launch_bounds__(256) void kBandedWalk(BandedWalkArgs a)
         const int up = (int)(a.upper < (int64_t)n ? a.upper : (int64_t)n);
         const BandBits bits{a.trace + a.traceOff[id], a.segLanes, lo, min(up - lo + 1, a.segLanes), n};
         const WalkEnd end{a.scores[pid], a.endIJ[2 * pid], a.endIJ[2 * pid + 1], a.endEF[2 * pid], a.endEF[2 * pid + 1]};
-        walkGroup(n, m, a.hRes + ho, a.vRes + vo, A, end, bits, cnt, a.ops ? a.ops + a.opOff[pid + 1] : nullptr,
-                  a.ops ? a.opLen + pid : nullptr, a.local != 0, a.begins ? a.begins + 2 * pid : nullptr,
-                  a.linear != 0, false, nullptr, 0, 0);
+        walkGroup<kWalkLanes>(n, m, a.hRes + ho, a.vRes + vo, A, end, bits, cnt,
+                              a.ops ? a.ops + a.opOff[pid + 1] : nullptr, a.ops ? a.opLen + pid : nullptr, a.local != 0,
+                              a.begins ? a.begins + 2 * pid : nullptr, a.linear != 0, false, nullptr, 0, 0);
     }
     __syncthreads();
     if (id < a.nIds) {
@@ -539,14 +544,15 @@ __global__ __launch_bounds__(256) void kBandedWalk(BandedWalkArgs a)
     }
 }
 
+template <int W>
 __global__ __launch_bounds__(256) void kWalk16(WalkArgs a)
 {
     extern __shared__ int32_t sCnt[];
     const int A = a.alpha, S = A * A + 2;
-    const int t = threadIdx.x & (kWalkLanes - 1), q = threadIdx.x / kWalkLanes;
-    const int id = blockIdx.x * (blockDim.x / kWalkLanes) + q;
+    const int t = threadIdx.x & (W - 1), q = threadIdx.x / W;
+    const int id = blockIdx.x * (blockDim.x / W) + q;
     int32_t *cnt = sCnt + q * S;
-    for (int k = t; k < S; k += kWalkLanes)
+    for (int k = t; k < S; k += W)
         cnt[k] = 0;
     __syncthreads();
     if (id < a.nPairs) {
@@ -558,7 +564,7 @@ __global__ __launch_bounds__(256) void kWalk16(WalkArgs a)
         // column order.  Global: the last unit's bottom-row candidate, unless
         // a cell of column n beats it (rows ascend with the units).
         WalkEnd end{INT32_MIN, 0x7fffffff, 0x7fffffff, INT32_MIN, INT32_MIN};
-        for (int k = t; k < loc.nEnds; k += kWalkLanes) {
+        for (int k = t; k < loc.nEnds; k += W) {
             const TraceEnd c = a.ends[loc.end0 + (int64_t)k * loc.endStride];
             const bool take = a.local ? c.v > end.score || (c.v == end.score && (c.j < end.j || (c.j == end.j && c.i < end.i)))
                                       : c.rv > end.score || (c.rv == end.score && c.ri < end.i);
@@ -566,10 +572,10 @@ __global__ __launch_bounds__(256) void kWalk16(WalkArgs a)
                 end = a.local ? WalkEnd{c.v, c.i, c.j, c.e, c.f} : WalkEnd{c.rv, c.ri, c.rj, c.re, c.rf};
         }
 #pragma unroll
-        for (int d = 1; d < kWalkLanes; d <<= 1) {
-            const WalkEnd o{__shfl_xor(end.score, d, kWalkLanes), __shfl_xor(end.i, d, kWalkLanes),
-                            __shfl_xor(end.j, d, kWalkLanes), __shfl_xor(end.e, d, kWalkLanes),
-                            __shfl_xor(end.f, d, kWalkLanes)};
+        for (int d = 1; d < W; d <<= 1) {
+            const WalkEnd o{__shfl_xor(end.score, d, W), __shfl_xor(end.i, d, W),
+                            __shfl_xor(end.j, d, W), __shfl_xor(end.e, d, W),
+                            __shfl_xor(end.f, d, W)};
             if (o.score > end.score || (o.score == end.score && (o.j < end.j || (o.j == end.j && o.i < end.i))))
                 end = o;
         }
@@ -584,14 +590,14 @@ __global__ __launch_bounds__(256) void kWalk16(WalkArgs a)
         if (t == 0)
             a.scores[pid] = end.score;
         const Bits16 bits{a.trace, loc};
-        walkGroup(n, m, a.hRes + ho, a.vRes + vo, A, end, bits, cnt, a.ops ? a.ops + a.opOff[pid + 1] : nullptr,
+        walkGroup<W>(n, m, a.hRes + ho, a.vRes + vo, A, end, bits, cnt, a.ops ? a.ops + a.opOff[pid + 1] : nullptr,
                   a.ops ? a.opLen + pid : nullptr, a.local != 0, a.begins ? a.begins + 2 * pid : nullptr,
                   a.linear != 0, a.gapExtend < a.gapOpen, a.local ? a.table : nullptr, a.gapOpen, a.gapExtend);
     }
     __syncthreads();
     if (id < a.nPairs) {
         int32_t *out = a.counts + (int64_t)a.ids[id] * S;
-        for (int k = t; k < S; k += kWalkLanes)
+        for (int k = t; k < S; k += W)
             out[k] = cnt[k];
     }
 }
@@ -838,14 +844,24 @@ int occupancyTrace16(bool dna, uint32_t track)
     return blocks > 0 ? blocks : 1;
 }
 
+// Up to this many pairs (a wave each fills the chip's SIMDs 16 times) the
+// longest walk bounds the kernel, and 64 lanes read four times as far at once:
+// 8,191 uneven pairs of up to 10 kbp 0.51 ms against 1.08 with 16 lanes, 8,192
+// protein pairs local 0.095 / 0.11; 65,536 pairs of 1 kbp, bound by the
+// records' traffic, 2.1 / 1.39.
+constexpr int kWalkWavePairs = 16384;
+
 hipError_t launchWalk16(const WalkArgs &args, hipStream_t stream)
 {
     if (args.nPairs <= 0)
         return hipSuccess;
-    const int threads = walkThreads(args.alpha), pairs = threads / kWalkLanes;
-    hipLaunchKernelGGL(kWalk16, dim3((args.nPairs + pairs - 1) / pairs), dim3(threads),
-                       (size_t)pairs * (args.alpha * args.alpha + 2) * sizeof(int32_t), stream, args);
-    return hipGetLastError();
+    const bool wave = args.nPairs <= kWalkWavePairs;
+    const int threads = walkThreads(args.alpha), pairs = threads / (wave ? 64 : kWalkLanes);
+    const void *k = wave ? (const void *)&kWalk16<64> : (const void *)&kWalk16<kWalkLanes>;
+    WalkArgs copy = args;
+    void *params[] = {&copy};
+    return hipLaunchKernel(k, dim3((args.nPairs + pairs - 1) / pairs), dim3(threads), params,
+                           (size_t)pairs * (args.alpha * args.alpha + 2) * sizeof(int32_t), stream);
 }
 
 hipError_t launchBandedWalk(const BandedWalkArgs &args, hipStream_t stream)

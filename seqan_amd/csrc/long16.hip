@@ -659,12 +659,15 @@ __global__ __launch_bounds__(64) void kLong16Walk(LongArgs a)
     while (inside && i > 0 && j > 0) {
         if (mode == 0) {
             const int ii = i - t, jj = j - t;
-            const int b = ii > 0 && jj > 0 ? bits(ii, jj) : -1;
+            // The residues with the bits: one wait instead of two.
+            const bool valid = ii > 0 && jj > 0;
+            const int rh = valid ? h[jj - 1] : 0, rw = valid ? v[ii - 1] : 0;
+            const int b = valid ? bits(ii, jj) : -1;
             const int d = b < 0 ? 3 : (b & 4) ? ((b & 8) ? 2 : 1) : 0;
             const uint64_t other = __ballot(d != 0);
             const int r = other ? __builtin_ctzll(other) : 64;
             if (t < r)
-                atomicAdd(&sCnt[min((int)h[jj - 1], A - 1) * A + min((int)v[ii - 1], A - 1)], 1);
+                atomicAdd(&sCnt[min(rh, A - 1) * A + min(rw, A - 1)], 1);
             emit(0, r);
             i -= r;
             j -= r;
