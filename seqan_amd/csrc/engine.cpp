@@ -2123,7 +2123,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             need += arenaBytes(4 * nOrder) + arenaBytes(sizeof(WorkItem) * nItems);
         if (!P.units.empty()) {
             need += arenaBytes(4 * P.order16.size()) + arenaBytes(sizeof(ScoreUnit) * P.units.size());
-            minRb = std::max(minRb, (size_t)wavesPerBlock16() * P.slotWords * 8);
+            minRb = std::max(minRb, (size_t)scoreWaves(P.dna16, (int64_t)P.units.size(), ctx->numCUs) * P.slotWords * 8);
         }
         if (!plans.empty() || !P.units.empty())
             need += arenaBytes(64 * (plans.size() + 1));
@@ -2219,7 +2219,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             a.queue = static_cast<uint32_t *>(ctx->b.queue.p) + k;
             a.rowbuf = static_cast<uint64_t *>(ctx->b.rowbuf.p);
             a.slotWords = slotWords;
-            if ((err = launchScore16(P.dna16, kind, a, 1, stream, 64)) != hipSuccess)
+            if ((err = launchScore16(P.dna16, kind, a, 1, 1, stream)) != hipSuccess)
                 return hipFail(ctx, err, "launching plain kernel");
         }
         plans.clear();
@@ -2239,11 +2239,12 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         std::vector<size_t> orderOff(plans.size() + 1, unitOrder), itemOff(plans.size() + 1, 0);
         std::vector<int> grids(plans.size()), rowColsOf(plans.size());
         size_t rbMax = 0;
-        int unitGrid = 0;
+        int unitGrid = 0, unitWaves = 4;
         if (!P.units.empty()) {
-            unitGrid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occupancyScore16(P.dna16, kind),
-                                                          ((int64_t)P.units.size() + wpb - 1) / wpb));
-            const size_t perBlock = std::max<size_t>((size_t)wpb * P.slotWords * 8, 8);
+            unitWaves = scoreWaves(P.dna16, (int64_t)P.units.size(), ctx->numCUs);
+            unitGrid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occupancyScore16(P.dna16, kind, unitWaves),
+                                                          ((int64_t)P.units.size() + unitWaves - 1) / unitWaves));
+            const size_t perBlock = std::max<size_t>((size_t)unitWaves * P.slotWords * 8, 8);
             if (ctx->noAlloc)   // the persistent grid shrinks to the scratch that is left
                 unitGrid = (int)std::max<size_t>(1, std::min<size_t>((size_t)unitGrid, rowbufBudget / perBlock));
             rbMax = (size_t)unitGrid * perBlock;
@@ -2304,7 +2305,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
                     });
             }
             const bool dna = P.dna16;
-            launches.push_back([=] { return launchScore16(dna, kind, a, unitGrid, stream); });
+            launches.push_back([=] { return launchScore16(dna, kind, a, unitGrid, unitWaves, stream); });
         }
         for (size_t k = 0; k < plans.size(); ++k) {
             const Plan16 &pl = plans[k];

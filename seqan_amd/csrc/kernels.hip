@@ -758,10 +758,10 @@ const void *scoreKernel(bool dna, int kind)
 
 }  // namespace
 
-int occupancyScore16(bool dna, int kind)
+int occupancyScore16(bool dna, int kind, int waves)
 {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, scoreKernel(dna, kind), 256, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, scoreKernel(dna, kind), 64 * waves, 0) != hipSuccess)
         return 1;
     return blocks > 0 ? blocks : 1;
 }
@@ -814,15 +814,14 @@ hipError_t launchBand16(const BandVariant &v, const FwdArgs &args, int gridBlock
     return hipLaunchKernel(k, dim3(gridBlocks), dim3(64 * v.waves), params, (size_t)ringLdsBytes, stream);
 }
 
-hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBlocks, hipStream_t stream,
-                         int threadsPerBlock)
+hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBlocks, int waves, hipStream_t stream)
 {
     const void *k = scoreKernel(dna, kind);
     if (!k)
         return hipErrorInvalidValue;
     ScoreArgs copy = args;
     void *params[] = {&copy};
-    return hipLaunchKernel(k, dim3(gridBlocks), dim3(threadsPerBlock), params, 0, stream);
+    return hipLaunchKernel(k, dim3(gridBlocks), dim3(64 * waves), params, 0, stream);
 }
 
 hipError_t launchTrace16(bool dna, uint32_t track, const TraceArgs &args, int gridBlocks, hipStream_t stream)

@@ -225,9 +225,12 @@ struct ScoreArgs {
     const uint32_t *dnaProfile;
     Drift drift;
 };
-hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBlocks, hipStream_t stream,
-                         int threadsPerBlock = 256);
-int occupancyScore16(bool dna, int kind);
+// Waves per workgroup of a launch of `units` units: 4, or 8 with the table where
+// the units fill the chip's SIMDs twice.
+constexpr int kScoreTabWaves = 8;
+inline int scoreWaves(bool dna, int64_t units, int numCUs) { return dna || units <= (int64_t)4 * numCUs ? 4 : kScoreTabWaves; }
+hipError_t launchScore16(bool dna, int kind, const ScoreArgs &args, int gridBlocks, int waves, hipStream_t stream);
+int occupancyScore16(bool dna, int kind, int waves);
 
 // Kernel variant of the packed int16 family.
 struct Variant16 {

@@ -27,7 +27,7 @@
 // first row needs no subtraction: its neighbour's values are one step old.)  The floor H >= 0 rides in E's maximum (E >= z, z the stored 0):
 //   E = max3(E, G, z); F = max(F, G) - drift; H = max3(D, E, F); G = H - cost
 // and one maximum per two rows keeps the best cell: 6.5 operations and the
-// lookup against 9.  262,144 protein pairs (Blosum62): 20.9 ms against 27.2.
+// lookup against 9.  262,144 protein pairs (Blosum62): 20.35 ms against 27.2.
 //
 // WIDE (values past kDriftNarrowMax, or scores t < 0): the same recurrences
 // in packed 16-bit operations with two maxima for max3.
@@ -77,7 +77,13 @@ __device__ __forceinline__ uint32_t shiftIn(uint32_t v, uint32_t first)
     return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, ctrl, 0xf, 0xf, false);
 }
 
-constexpr int kWaves = 4;        // waves per workgroup, independent of each other
+// Waves per workgroup, independent of each other: at most 4, or 8 where they
+// share a table of 32 copies (score kernels).
+#if defined(SQMI_SCORE_DNA) && !SQMI_SCORE_DNA
+constexpr int kWaves = kScoreTabWaves, kTabCopies = 32;
+#else
+constexpr int kWaves = 4, kTabCopies = 16;
+#endif
 constexpr int kPeriod = 32;      // steps between refills of the ring and flushes of the bottom row
 constexpr int kQD = 4;           // steps per chunk
 constexpr int kRebase = 16;      // local: steps between rebases of the drift
@@ -99,8 +105,11 @@ __shared__ uint2 gOut[kWaves * kOutWords];
 
 // Substitution table of the table kernels in LDS: word (h, v), copy c of
 // kTabCopies, holds t << 16 (lane c mod kTabCopies reads its own copy).  Pair
-// A reads the word's high half (t), pair B the word (t << 16).
-constexpr int kTabCopies = 16;
+// A reads the word's high half (t), pair B the word (t << 16).  With 32 copies
+// the 32 lanes that read at once never meet in a bank; with 16 two lanes do
+// whenever their words agree modulo 4.  The trace kernels have no room for 32
+// beside their rings.  262,144 protein pairs, local: 21.0 -> 20.35 ms, 64 to 65,536 of them
+// 1-4% faster.
 constexpr int kTabLdsBytes = kTabMaxCodes * kTabMaxCodes * 4 * kTabCopies;
 
 __device__ __forceinline__ uint64_t rowLoad(const uint64_t *p, bool strip)
@@ -173,11 +182,14 @@ __device__ __forceinline__ void loadScores(const Args &a, int tAdd, uint32_t *sP
             sProf[threadIdx.x] = w;
         }
     } else {
+        // A word per thread, its copies from the lane's own on, so that the
+        // lanes' stores spread over the banks.
         const int TW = a.alpha + 1;
-        for (int i = threadIdx.x; i < TW * TW * kTabCopies; i += blockDim.x) {
-            const int w = i / kTabCopies, h = w / TW, v = w % TW;
+        for (int w = threadIdx.x; w < TW * TW; w += blockDim.x) {
+            const int h = w / TW, v = w % TW;
             const uint32_t t = (h == a.alpha || v == a.alpha) ? 0u : (uint32_t)(uint16_t)(a.tTable[w] + tAdd);
-            *reinterpret_cast<uint32_t *>(sT + 4 * i) = t << 16;
+            for (int c = 0; c < kTabCopies; ++c)
+                *reinterpret_cast<uint32_t *>(sT + 4 * (w * kTabCopies + (((int)threadIdx.x + c) & (kTabCopies - 1)))) = t << 16;
         }
     }
     __syncthreads();
@@ -727,7 +739,7 @@ __device__ __forceinline__ void scoreRun(const ScoreArgs &a)
 // Three waves per SIMD (168 registers) with the DNA profile, two (256) with
 // the table, whose row offsets and scores read ahead would spill at three.
 template <bool DNA, int KIND>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DNA ? 3 : 2))) void kScore16(ScoreArgs a)
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(DNA ? 3 : 2))) void kScore16(ScoreArgs a)
 {
     scoreRun<DNA, KIND>(a);
 }
