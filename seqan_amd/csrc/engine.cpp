@@ -830,6 +830,36 @@ int stripMinBlocks()
 // Units of the packed score kernel from the sorted keys of the group shapes,
 // which come first, in slot order (the longest items first).  starts /
 // itemOff: the buckets' first keys and items.
+// Strips in the order a wave should claim them: by the steps from a strip's
+// start to its item's end (its columns, and kStripLag for every block from it
+// on), the most first.  The strip above always comes earlier.  Claimed item
+// by item, an item's lower strips held waves that only waited for the upper
+// ones.  The whole items follow in their order.  Rows of 8,192 protein
+// pairs, local: trace kernel 3.35 -> 2.9 ms.  (Score calls measured the same
+// either way and keep their items' order.)
+constexpr int32_t kStripLag = 128;
+void orderStrips(RawVec<ScoreUnit> &units, size_t begin)
+{
+    constexpr int kShift = 3, kBuckets = 1 << 13;   // 8 steps per bucket, up to 65,536 steps
+    auto bucket = [](const ScoreUnit &u) {
+        const int64_t left = u.maxN + (int64_t)kStripLag * (u.nblocks - u.block);
+        return u.block < 0 ? kBuckets : kBuckets - 1 - (int)std::min<int64_t>(left >> kShift, kBuckets - 1);
+    };
+    bool strips = false;
+    for (size_t k = begin; k < units.size() && !strips; ++k)
+        strips = units[k].block > 0;
+    if (!strips)
+        return;
+    std::vector<uint32_t> at(kBuckets + 2, 0);
+    for (size_t k = begin; k < units.size(); ++k)
+        ++at[bucket(units[k]) + 1];
+    for (int b = 0; b <= kBuckets; ++b)
+        at[b + 1] += at[b];
+    const std::vector<ScoreUnit> from(units.begin() + begin, units.end());
+    for (const ScoreUnit &u : from)
+        units[begin + at[bucket(u)]++] = u;
+}
+
 void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &starts,
                const std::vector<size_t> &itemOff, int R16, int R64, double cellsStrip, bool noStrips)
 {
@@ -2604,6 +2634,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
                 }
                 wide[k] = strips;   // from here on: whether the item has strips
             }
+            orderStrips(P.units, chunkUnits.empty() ? 0 : chunkUnits.back());
             chunkUnits.push_back(P.units.size());
             chunkStrips.push_back(off);
             stripWords = std::max(stripWords, off);

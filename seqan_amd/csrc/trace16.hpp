@@ -32,8 +32,8 @@
 // of the longest, which strips spread over the chip and 64 lanes per couple
 // shorten.  Measured: 65,536 pairs of 1 kbp, global, 17.4 -> 16.2 ms (34 GB of
 // records at 2.1 TB/s beside it); 8,191 uneven pairs, free first and last row,
-// 277 ms with one wave per item -> 8.6 (strips) -> 4.3; 8,192 protein pairs,
-// local, 11.3 -> 3.5 ms.
+// 277 ms with one wave per item -> 8.6 (strips) -> 3.2 (64 lanes); 8,192
+// protein pairs, local, 11.3 -> 2.9 ms.
 //
 // Values are compared as signed halves.  WIDE: stored values are held less
 // 32768, so that the whole 16-bit range is ordered and the differences
