@@ -25,7 +25,7 @@
 //                  residue codes of the next row are loaded one row ahead.
 //   kBandedWide:   wider bands; one wave per pair, the band in chunks of 64
 //                  lanes, the previous row in a per-wave global buffer.
-//   kBandedTrace:  kBandedNarrow with one trace byte per cell and the end
+//   kBandedTrace, kBandedTraceWide: kBandedNarrow with one trace byte per cell and the end
 //                  cell's position, E and F, for banded rows and counts
 //                  (walked by kBandedWalk in kernels.hip).
 #include "kernels.hpp"
@@ -390,6 +390,159 @@ __global__ __launch_bounds__(256) void kBandedTrace(BandedArgs a)
     }
 }
 
+// kBandedTrace for bands of up to 64 C diagonals: one wave per pair, lane k owns
+// diagonals k C .. k C + C - 1 of the band in registers.  The horizontal gap's
+// scan runs over a lane's own cells first, then over the lanes' maxima.  Trace
+// rows hold 64 C bytes.  What bounds it: the issue of about 25 instructions a
+// cell, in a call of few pairs their rows one after the other.  Rows calls from
+// host buffers, against one thread per pair with the whole matrix in scratch
+// (kCounts32): 1,000 pairs of 1 kbp, 201 diagonals 175 -> 1.3 ms; 500 of 2 kbp,
+// 301 diagonals 997 -> 2.7 ms; 30,000 of 300 bp, 141 diagonals 57 -> 4.0 ms.
+constexpr int kMaxBandC = kMaxBandTrace / 64;
+template <int C>
+__global__ __launch_bounds__(256) void kBandedTraceWide(BandedArgs a)
+{
+    constexpr int S = 64 * C;
+    constexpr uint32_t kEOpen = 1, kFOpen = 2, kNotDiag = 4, kHori = 8, kStop = 16;
+    __shared__ int32_t sTab[32 * 32];
+    __shared__ uint8_t sV[4][kChunkRows];
+    __shared__ uint8_t sH[4][kChunkRows + S];
+    for (int x = threadIdx.x; x < a.alpha * a.alpha; x += blockDim.x)
+        sTab[x] = a.table[x];
+    __syncthreads();
+    const int k = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int t = blockIdx.x * (blockDim.x >> 6) + wv;
+    if (t >= a.nIds)
+        return;   // the whole wave is past the end
+    const BandPair P = loadPair(a, a.ids[t]);
+    const int32_t o = a.gapOpen, e = a.gapExtend, g = max(o, e);
+    const int A = a.alpha;
+    const bool local = (a.mode & SQMI_LOCAL) != 0;
+    const bool freeTop = (a.mode & (SQMI_FREE_TOP | SQMI_LOCAL)) != 0;
+    const bool freeLeft = (a.mode & (SQMI_FREE_LEFT | SQMI_LOCAL)) != 0;
+    const int32_t floorH = local ? 0 : kNegB;
+    uint8_t *rowT = a.trace + a.traceOff[t];
+    // End cell candidate of this lane (its cells do not come in column order).
+    int32_t bv = kNegB, be = kNegB, bf = kNegB;
+    int bi = 0x7fffffff, bj = 0x7fffffff;
+    int32_t hPrev[C], fPrev[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int q = k * C + c, d = P.lo + q;
+        hPrev[c] = fPrev[c] = kNegB;
+        if (q < P.w && d >= 0 && d <= P.n) {
+            hPrev[c] = rowZero(d, freeTop, o, g);
+            if (P.track(0, d, a.mode) && hPrev[c] > bv) {   // row 0 comes in column order
+                bv = hPrev[c];
+                be = (d == 0 || freeTop) ? kNegB : hPrev[c];
+                bi = 0;
+                bj = d;
+            }
+        }
+    }
+    uint8_t *myV = sV[wv], *myH = sH[wv];
+    for (int i = 1; i <= P.m; ++i) {
+        const int r = (i - 1) % kChunkRows;
+        if (r == 0) {
+            // As in kBandedNarrow: the residues of the next rows and of the columns they meet.
+            __builtin_amdgcn_wave_barrier();
+            for (int x = k; x < kChunkRows; x += 64) {
+                const int row = i + x;
+                myV[x] = row <= P.m ? P.v[row - 1] : 0;
+            }
+            for (int c = k; c < kChunkRows + S - 1; c += 64) {
+                const int col = i + P.lo + c;
+                myH[c] = (col >= 1 && col <= P.n) ? P.h[col - 1] : 0;
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+        const int vb = min((int)myV[r], A - 1);
+        // The next lane's first diagonal of the row above; every lane runs the moves.
+        const int32_t hNext = dpp<kDppWaveShl1>(hPrev[0]), fNext = dpp<kDppWaveShl1>(fPrev[0]);
+        int32_t D[C], F0[C], X[C], hUp[C], fUp[C];
+        int32_t run = 0, before[C];   // maxima of the biased scan values (0: minus infinity)
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int q = k * C + c, j = i + P.lo + q;
+            const bool valid = q < P.w && j >= 0 && j <= P.n, col0 = j == 0, upOut = q + 1 >= P.w;
+            hUp[c] = upOut ? kNegB : c + 1 < C ? hPrev[c + 1] : hNext;
+            fUp[c] = upOut ? kNegB : c + 1 < C ? fPrev[c + 1] : fNext;
+            D[c] = hPrev[c] + sTab[min((int)myH[r + q], A - 1) * A + vb];
+            F0[c] = max(fUp[c] + e, hUp[c] + o);
+            const int32_t x0 = col0 ? (freeLeft ? 0 : F0[c]) : max(max(D[c], F0[c]), floorH);
+            X[c] = valid ? x0 : kNegB;
+            before[c] = run;
+            run = max(run, valid ? max(x0 - kNegB + o - q * g, 0) : 0);
+        }
+        const int32_t lanes = dpp0<kDppWaveShr1>(prefixMaxDpp<64>(run, k));   // of the lanes before
+        int32_t H[C], E[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int q = k * C + c, j = i + P.lo + q;
+            const bool valid = q < P.w && j >= 0 && j <= P.n, col0 = j == 0;
+            E[c] = q == 0 ? kNegB : max(lanes, before[c]) + kNegB + (q - 1) * g;
+            H[c] = valid ? (col0 ? X[c] : max(X[c], E[c])) : kNegB;
+        }
+        const int32_t hLast = dpp<kDppWaveShr1>(H[C - 1]), eLast = dpp<kDppWaveShr1>(E[C - 1]);
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int q = k * C + c, j = i + P.lo + q;
+            const bool valid = q < P.w && j >= 0 && j <= P.n, col0 = j == 0;
+            const int32_t hLeft = q == 0 ? kNegB : c > 0 ? H[c > 0 ? c - 1 : 0] : hLast;
+            const int32_t eLeft = q == 0 ? kNegB : c > 0 ? E[c > 0 ? c - 1 : 0] : eLast;
+            uint32_t tb = kStop;   // as in kBandedTrace: no byte of a row stays unwritten
+            if (valid && !col0) {
+                const int32_t extE = eLeft + e, opnE = hLeft + o;
+                tb = extE < opnE ? kEOpen : 0u;
+                const int32_t ei = max(extE, opnE);
+                tb |= (fUp[c] + e) < (hUp[c] + o) ? kFOpen : 0u;
+                const int32_t fe = max(F0[c], ei);
+                int32_t x = D[c];
+                if (D[c] < fe) {
+                    x = fe;
+                    tb |= kNotDiag | (F0[c] < ei ? kHori : 0u);
+                }
+                if (local && !(0 < x))
+                    tb = kStop;
+            }
+            rowT[(int64_t)(i - 1) * S + q] = (uint8_t)tb;
+            const int32_t f = (valid && !(col0 && freeLeft)) ? F0[c] : kNegB;
+            if (valid && P.track(i, j, a.mode) && (H[c] > bv || (H[c] == bv && (j < bj || (j == bj && i < bi))))) {
+                bv = H[c];
+                be = col0 ? kNegB : E[c];
+                bf = f;
+                bi = i;
+                bj = j;
+            }
+            fPrev[c] = f;
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            hPrev[c] = H[c];
+    }
+    // Larger value, then smaller column, then smaller row.
+#pragma unroll
+    for (int x = 32; x >= 1; x >>= 1) {
+        const int32_t ov = __shfl_xor(bv, x), oe = __shfl_xor(be, x), of = __shfl_xor(bf, x);
+        const int oi = __shfl_xor(bi, x), oj = __shfl_xor(bj, x);
+        const bool take = ov > bv || (ov == bv && (oj < bj || (oj == bj && oi < bi)));
+        bv = take ? ov : bv;
+        be = take ? oe : be;
+        bf = take ? of : bf;
+        bi = take ? oi : bi;
+        bj = take ? oj : bj;
+    }
+    if (k == 0) {
+        if (bi == P.m && (int64_t)bj - bi == a.lower)   // as in kBandedTrace
+            bf = kNegB;
+        a.scores[P.pid] = bv;
+        a.endIJ[2 * P.pid] = bi;
+        a.endIJ[2 * P.pid + 1] = bj;
+        a.endEF[2 * P.pid] = be;
+        a.endEF[2 * P.pid + 1] = bf;
+    }
+}
+
 // One wave per pair; rows of the band (H and F, double-buffered) in the
 // wave's slice of `scratch`: 4 * (wmax + 2) int32.  blockDim = 64, so the
 // workgroup barrier between rows orders this wave's own global writes and
@@ -499,6 +652,16 @@ hipError_t launchBandedTrace(const BandedArgs &args, int segLanes, hipStream_t s
 {
     if (args.nIds <= 0)
         return hipSuccess;
+    if (segLanes > 64) {
+        if (segLanes % 64 != 0 || segLanes / 64 > kMaxBandC)
+            return hipErrorInvalidValue;
+        using Kernel = void (*)(BandedArgs);
+        static constexpr Kernel wide[kMaxBandC - 1] = {kBandedTraceWide<2>, kBandedTraceWide<3>, kBandedTraceWide<4>,
+                                                       kBandedTraceWide<5>, kBandedTraceWide<6>, kBandedTraceWide<7>,
+                                                       kBandedTraceWide<8>};
+        hipLaunchKernelGGL(wide[segLanes / 64 - 2], dim3((args.nIds + 3) / 4), dim3(256), 0, stream, args);
+        return hipGetLastError();
+    }
     const int pairsPerWave = 64 / segLanes;
     const int waves = (args.nIds + pairsPerWave - 1) / pairsPerWave;
     const dim3 grid((waves + 3) / 4), block(256);

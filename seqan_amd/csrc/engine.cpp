@@ -2819,9 +2819,10 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
             ub = ue;
         }
     }
-    // Banded pairs whose band, clipped to the matrix, has at most 64
+    // Banded pairs whose band, clipped to the matrix, has at most 512
     // diagonals: the lane-per-diagonal trace kernel (S trace bytes per row,
-    // S = the widest band rounded up to a power of two) and a walk, in
+    // S = the widest band rounded up to a power of two), or up to 8 diagonals
+    // per lane (S a multiple of 64), and a walk, in
     // chunks whose trace bytes fit the trace budget (offsets restart at 0 in
     // every chunk; the chunks run one after another on the call's stream).
     // SQMI_BANDED_TRACE_INT32=1 keeps them on the int32 kernel.
@@ -2835,10 +2836,12 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
             const int64_t n = setH->offsets[id + 1] - setH->offsets[id], m = setV->offsets[id + 1] - setV->offsets[id];
             wmax = std::max(wmax, std::min(band[1], n) - std::max(band[0], -m) + 1);
         }
-        if (wmax <= 64) {
+        if (wmax <= kMaxBandTrace) {
             bandLanes = 1;
-            while (bandLanes < wmax)
+            while (bandLanes < std::min<int64_t>(wmax, 64))
                 bandLanes <<= 1;
+            if (wmax > 64)
+                bandLanes = (int)((wmax + 63) / 64 * 64);
             bandOff.resize(P.ids32.size());
             int64_t run = 0;
             for (size_t k = 0; k < P.ids32.size(); ++k) {

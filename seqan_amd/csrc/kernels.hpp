@@ -304,8 +304,10 @@ struct BandedArgs {
 // segLanes: 1..64 (power of two >= every band width: kBandedNarrow), or 0
 // (kBandedWide on wideGrid workgroups).
 hipError_t launchBanded(const BandedArgs &args, int segLanes, int wideGrid, hipStream_t stream);
-// Forward with trace bytes for bands of at most 64 diagonals (segLanes as in
-// launchBanded), then one thread per pair walks (kBandedWalk).
+// Forward with trace bytes for bands of at most kMaxBandTrace diagonals
+// (segLanes: as in launchBanded up to 64, then a multiple of 64), then 16
+// lanes per pair walk (kBandedWalk).
+constexpr int kMaxBandTrace = 512;
 hipError_t launchBandedTrace(const BandedArgs &args, int segLanes, hipStream_t stream);
 struct BandedWalkArgs {
     const uint8_t *hRes;
