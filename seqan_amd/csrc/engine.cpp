@@ -567,6 +567,21 @@ int bandWaves(int cols) { return cols > 256 ? 4 : cols > 128 ? 8 : cols > 64 ? 4
 // 0.81 / 0.81 / 0.84 / 2.5 ms, int32 2.5 / 3.3 / 12.8 / 51.5; local, 150 bp,
 // 33 diagonals: 0.11 / 0.11 / 0.11 / 0.18 against 0.04 / 0.06 / 0.19 / 0.68.
 constexpr double kBandColumnAlone = 335, kBandColumn[3] = {170, 80, 60}, kBandNarrowLone = 270, kBandNarrowFull = 70, kBandWideLone = 615, kBandWideFull = 202;
+// Calls of pairs of about one size (the largest at most four times the mean):
+// 64 lanes for all of them cost more than twice the instructions, and their
+// skew of 64 steps weighs on short pairs.  In cycles: a pair alone on 16 lanes
+// about 2.9 a cell (more waves per SIMD: up to twice that), on 64 lanes 0.93 and
+// the skew.  Whether 16 lanes are about as fast.  Device time of 53,121 pairs of 68 bp, local:
+// 64 lanes 413 us, 16 152; 4,000 of them 71, 40; 53,121 of 150 bp 457, 268;
+// 20,000 of 300 bp 413, 348.  Past 512 rows 64 lanes have rows enough to cost
+// the same: 20,000 of 1 kbp, global, 2.24 ms, 16 lanes 2.42.
+bool evenOn16(double most, double pairs, double cells)
+{
+    const double waves = pairs / 8 / 1024, skew = (std::sqrt(most) + 64) / std::max(1.0, std::sqrt(most));
+    const double t16 = std::max(2.9 * most * std::max(1.0, 0.66 * std::min(3.0, waves)), 2.3e-4 * cells);
+    const double t64 = std::max(0.93 * most, 2.1 * 2.3e-4 * cells) * skew;
+    return most <= 512.0 * 512.0 && t64 * 1.3 >= t16;
+}
 // Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
 constexpr int64_t kResidentWaves = 3072;
 // Rows per unit of the group shapes' row counts.
@@ -1062,10 +1077,10 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
         shapes.push_back(Variant16{1, 32, dna16, track});
         shapes.push_back(Variant16{1, forcedG == 1 ? forcedR : 16, dna16, track, true});
         // Pairs per length bin and cells of the int16 route.
-        int64_t binCount[16] = {}, cells16 = 0;
+        int64_t binCount[16] = {}, cells16 = 0, most16 = 0;
 #pragma omp parallel if (N > kParallelMin)
         {
-            int64_t local16[16] = {}, localCells = 0;
+            int64_t local16[16] = {}, localCells = 0, localMost = 0;
 #pragma omp for schedule(static) nowait
             for (int64_t i = 0; i < N; ++i) {
                 const int64_t n = H.offsets[i + 1] - H.offsets[i];
@@ -1073,6 +1088,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
                 if (n != 0 && m != 0 && route16(n, m)) {
                     ++local16[lengthBin(m)];
                     localCells += n * m;
+                    localMost = std::max(localMost, n * m);
                 }
             }
 #pragma omp critical
@@ -1080,6 +1096,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
                 for (int b = 0; b < 16; ++b)
                     binCount[b] += local16[b];
                 cells16 += localCells;
+                most16 = std::max(most16, localMost);
             }
         }
         int64_t pairs16 = 0;
@@ -1087,6 +1104,8 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
             pairs16 += binCount[b];
         cells64 = kCouple64Share * (double)cells16;
         cellsStrip = kStripShare * (double)cells16;
+        if ((double)most16 * (double)pairs16 <= 4.0 * (double)cells16 && evenOn16((double)most16, (double)pairs16, (double)cells16))
+            cells64 = cellsStrip = 1e300;
         if (fixedShapeRule()) {
             std::fill(binG, binG + 16, 16);
         } else {
