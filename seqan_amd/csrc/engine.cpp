@@ -573,14 +573,15 @@ constexpr double kBandColumnAlone = 335, kBandColumn[3] = {170, 80, 60}, kBandNa
 // about 2.9 a cell (more waves per SIMD: up to twice that), on 64 lanes 0.93 and
 // the skew.  Whether 16 lanes are about as fast.  Device time of 53,121 pairs of 68 bp, local:
 // 64 lanes 413 us, 16 152; 4,000 of them 71, 40; 53,121 of 150 bp 457, 268;
-// 20,000 of 300 bp 413, 348.  Past 512 rows 64 lanes have rows enough to cost
-// the same: 20,000 of 1 kbp, global, 2.24 ms, 16 lanes 2.42.
+// 20,000 of 300 bp 413, 348.  Past 512 rows (mean) 64 lanes have rows enough to cost
+// the same: 20,000 of 1 kbp, global, 2.24 ms, 16 lanes 2.42.  62,172 protein
+// pairs of 50-372 by 50-744, local: 1.35 ms, 16 lanes 1.02.
 bool evenOn16(double most, double pairs, double cells)
 {
     const double waves = pairs / 8 / 1024, skew = (std::sqrt(most) + 64) / std::max(1.0, std::sqrt(most));
     const double t16 = std::max(2.9 * most * std::max(1.0, 0.66 * std::min(3.0, waves)), 2.3e-4 * cells);
     const double t64 = std::max(0.93 * most, 2.1 * 2.3e-4 * cells) * skew;
-    return most <= 512.0 * 512.0 && t64 * 1.3 >= t16;
+    return cells <= 512.0 * 512.0 * pairs && t64 * 1.3 >= t16;
 }
 // Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
 constexpr int64_t kResidentWaves = 3072;
