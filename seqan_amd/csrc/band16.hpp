@@ -474,7 +474,8 @@ struct Band16 {
         __shared__ uint32_t sProf[16];
         __shared__ int16_t sT[33 * 33];
         // t = s - o, and the second half of a diagonal step's drift (global);
-        // the rows' padding code: 0, or what keeps a free first row at H = 0.
+        // the rows' padding code: 0, or what keeps a free first row at H = 0
+        // (-gapOpen; DNA: a byte, the caller takes the table form above 255).
         const int tAdd = LOC ? 0 : a.drift.d;
         const int padScore = !LOC && (a.mode & SQMI_FREE_TOP) ? a.drift.cost + a.drift.d : 0;
         if constexpr (DNA) {

@@ -3333,7 +3333,11 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
         // one; more send the rings to memory).
         bandRowColsN = bandRingCols(bandMaxN, lower_diag, upper_diag, bandR);
         bandLds = bandLdsRingBytes(bandRowColsN);
-        bandVar = BandVariant{bandR, local ? si.dna : si.dnaDrift,
+        // The DNA form keeps scores in bytes, also the one that holds row 0 at
+        // H = 0 under a free first row: -gapOpen, which only schemes whose
+        // scores are all negative let past 255.  The table holds it in 16 bits.
+        const bool padFits = !(mode & SQMI_FREE_TOP) || si.o >= -255;
+        bandVar = BandVariant{bandR, padFits && (local ? si.dna : si.dnaDrift),
                               local ? kBandLocal : (mode & (SQMI_FREE_BOTTOM | SQMI_FREE_RIGHT)) ? kBandFree : kBandEnd,
                               bandWide, bandLds > 0, bandWaves(bandRowColsN)};
         const int64_t ringBytes = (int64_t)64 * bandRowColsN * 8;   // per wave
