@@ -583,6 +583,20 @@ bool evenOn16(double most, double pairs, double cells)
     const double t64 = std::max(0.93 * most, 2.1 * 2.3e-4 * cells) * skew;
     return cells <= 512.0 * 512.0 * pairs && t64 * 1.3 >= t16;
 }
+// Global pairs whose drifted values need all 16 bits (Variant16::wide), one per
+// lane with 32 rows: in the length bins up to kWideLane[k].bin when the call
+// holds that many of them there, `alone` or beside pairs that stay on groups
+// (the lane kernel's sweep of its longest pair then comes on top).  Device ms,
+// match 1, mismatch -4, gaps -1 / -2, global and all ends free, groups -> lanes: 524,288 pairs
+// of 30-40 bp 0.92 / 0.98 -> 0.31 / 0.37; 20,000 of 10-20 bp 0.08 / 0.08 -> 0.05 / 0.07;
+// 30,000 of 17-30 bp 0.09 / 0.09 -> 0.06 / 0.09; of 34-62 bp 131,072 0.28 / 0.28 ->
+// 0.18 / 0.24 and 60,000 0.16 / 0.17 -> 0.17 / 0.22; of 66-126 bp 262,144 0.80 / 0.83 ->
+// 0.72 / 0.76 and 131,072 0.43 / 0.47 -> 0.56 / 0.66.
+struct WideLane {
+    int bin;
+    int64_t alone, beside;
+};
+constexpr WideLane kWideLane[] = {{7, 262144, 1048576}, {6, 131072, 262144}, {5, 24576, 65536}, {4, 16384, 49152}};
 // Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
 constexpr int64_t kResidentWaves = 3072;
 // Rows per unit of the group shapes' row counts.
@@ -1066,6 +1080,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
     int R16 = 16, R64 = 0;          // rows per lane of the group shapes (R64 = 0: by the rule)
     int binLane[16] = {};           // one-pair-per-lane rows of a length bin, or 0
     int binG[16] = {};              // forced group size of a bin, or 0 (the rule)
+    int wideLaneBin = -1;           // global pairs of wide values: the last bin on lanes (kWideLane)
     double cells64 = 0, cellsStrip = 0;
     if (traceShape) {
         shapes.push_back(Variant16{kTraceLanes, kTraceRows / kTraceLanes, dna16, track});
@@ -1076,26 +1091,33 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
             shapes.push_back(Variant16{16, 16, dna16, track, w != 0});
         shapes.push_back(Variant16{1, 16, dna16, track});
         shapes.push_back(Variant16{1, 32, dna16, track});
-        shapes.push_back(Variant16{1, forcedG == 1 ? forcedR : 16, dna16, track, true});
-        // Pairs per length bin and cells of the int16 route.
-        int64_t binCount[16] = {}, cells16 = 0, most16 = 0;
+        shapes.push_back(Variant16{1, forcedG == 1 ? forcedR : 32, dna16, track, true});
+        // Pairs per length bin and cells of the int16 route; global pairs of
+        // wide values where there may be enough of them for lanes.
+        int64_t binCount[16] = {}, binWide[16] = {}, cells16 = 0, most16 = 0;
+        const bool countWide = !local && N >= kWideLane[3].alone;
 #pragma omp parallel if (N > kParallelMin)
         {
-            int64_t local16[16] = {}, localCells = 0, localMost = 0;
+            int64_t local16[16] = {}, localWide[16] = {}, localCells = 0, localMost = 0;
 #pragma omp for schedule(static) nowait
             for (int64_t i = 0; i < N; ++i) {
                 const int64_t n = H.offsets[i + 1] - H.offsets[i];
                 const int64_t m = V.offsets[i + 1] - V.offsets[i];
                 if (n != 0 && m != 0 && route16(n, m)) {
-                    ++local16[lengthBin(m)];
+                    const int b = lengthBin(m);
+                    ++local16[b];
+                    if (countWide)
+                        localWide[b] += !driftNarrow(si, dr, local, n, m);
                     localCells += n * m;
                     localMost = std::max(localMost, n * m);
                 }
             }
 #pragma omp critical
             {
-                for (int b = 0; b < 16; ++b)
+                for (int b = 0; b < 16; ++b) {
                     binCount[b] += local16[b];
+                    binWide[b] += localWide[b];
+                }
                 cells16 += localCells;
                 most16 = std::max(most16, localMost);
             }
@@ -1112,6 +1134,13 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
         } else {
             for (int b = 0; b < 16; ++b)
                 binLane[b] = laneRows(shapeCategory(dna16, local), b, pairs16);
+            for (const WideLane &q : kWideLane) {
+                int64_t below = 0;
+                for (int b = 0; b <= q.bin; ++b)
+                    below += binWide[b];
+                if (countWide && wideLaneBin < 0 && below >= (below == pairs16 ? q.alone : q.beside))
+                    wideLaneBin = q.bin;
+            }
         }
         // SQMI_BIN_SHAPES="b:G:R,...": the shape of bin b (the shape tuner
         // times whole calls with it); forced shapes: every bin's.
@@ -1152,7 +1181,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
         }
         const int b = lengthBin(m);
         const bool wide = !driftNarrow(si, dr, local, n, m);
-        if (binLane[b] && (local || !wide || forcedG == 1)) {
+        if (local || !wide || forcedG == 1 ? binLane[b] != 0 : b <= wideLaneBin && !binG[b]) {
             const uint32_t slot = !local && wide ? kSlotLaneWide : binLane[b] == 32 ? kSlotLane32 : kSlotLane16;
             units = blocksFor(shapes[slot], m);
             if (units <= kMaxBlocks16)
