@@ -148,6 +148,9 @@ sqmi_status fail(sqmi_context *ctx, sqmi_status st, const std::string &msg)
 
 sqmi_status hipFail(sqmi_context *ctx, hipError_t err, const char *what)
 {
+    // The runtime keeps an error until it is read: without this the next
+    // call's check after a launch would report it again.
+    (void)hipGetLastError();
     std::string msg = std::string(what) + ": " + hipGetErrorString(err);
     return fail(ctx, err == hipErrorOutOfMemory ? SQMI_ERR_OUT_OF_MEMORY : SQMI_ERR_DEVICE, msg);
 }
