@@ -59,7 +59,7 @@ struct Buffers
     // Traceback (sqmi_align_counts).
     DevBuf trace, traceOff, locs, ends, endOff, endEF, endIJ, counts;
     // Long pairs (tiled int32 kernels).
-    DevBuf longCk, longPairs, longWalk, longTrace, longBest, longSched;
+    DevBuf longCk, longRows, longPairs, longWalk, longTrace, longBest, longSched;
     // Alignment rows (sqmi_align_rows, sqmi_align_local_rows).
     DevBuf ops, opOff, opLen, begins, opsPacked, opStart;
     // Banded scores (sqmi_align_score_banded).
@@ -70,7 +70,7 @@ struct Buffers
     {
         for (DevBuf *b : {&hRes, &vRes, &hOff, &vOff, &order, &items, &queue, &rowbuf, &strips, &scores, &tTable, &dnaProf,
                           &ids32, &scratchOff32, &scratch32, &table32, &emptyIds, &trace, &traceOff, &locs, &ends, &endOff, &endEF,
-                          &endIJ, &counts, &longCk, &longPairs, &longWalk, &longTrace, &longBest, &longSched, &ops, &opOff, &opLen,
+                          &endIJ, &counts, &longCk, &longRows, &longPairs, &longWalk, &longTrace, &longBest, &longSched, &ops, &opOff, &opLen,
                           &begins, &opsPacked, &opStart, &bandIds, &bandScratch})
             f(*b);
     }
@@ -1682,7 +1682,9 @@ sqmi_status runLong16(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_
         return fail(ctx, SQMI_ERR_UNSUPPORTED, "long pairs: too many strips for one launch");
     hipError_t err;
     const size_t qWords = 16 * chunkEnd.size();
-    if ((err = ensure(ctx->b.strips, (size_t)maxRows * 8)) != hipSuccess ||
+    // (Bottom rows apart from the score and trace kernels' strips: the same
+    // call's launches may hold those by address already.)
+    if ((err = ensure(ctx->b.longRows, (size_t)maxRows * 8)) != hipSuccess ||
         (err = ensure(ctx->b.longPairs, sizeof(LongCouple) * nc)) != hipSuccess ||
         (err = ensure(ctx->b.longSched, 4 * qWords + sizeof(int2) * units.size())) != hipSuccess ||
         (err = ensure(ctx->b.endEF, (size_t)8 * N)) != hipSuccess)
@@ -1721,7 +1723,7 @@ sqmi_status runLong16(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_
         a.units = dUnits + ub;
         a.nUnits = (int32_t)(ue - ub);
         a.queue = queues + 16 * k;
-        a.rows = static_cast<uint64_t *>(ctx->b.strips.p);
+        a.rows = static_cast<uint64_t *>(ctx->b.longRows.p);
         a.state = dCounts ? static_cast<uint32_t *>(ctx->b.longCk.p) : nullptr;
         a.error = ctx->waitFlag;
         a.target = longTarget(P.si, P.drift);
