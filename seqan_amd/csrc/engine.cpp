@@ -553,6 +553,10 @@ int laneRows(int category, int bin, int64_t pairs16)
 // waves of one workgroup used to share an item's blocks; 1,048,576 of them
 // 99 -> 69 ms, of which the shorter recurrence gives most.
 constexpr double kCouple64Share = 1.0e-5, kStripShare = 4.0e-5;
+// Device memory of a score call's strips, at most (and SQMI_TRACE_BUDGET_MB):
+// the shares alone let 25,000 pairs of 13 kbp take 17 GB.  (16,000 of 13 kbp,
+// all strips, 11 GB: 330 ms; within 4 GB: 291.)
+constexpr int64_t kMaxStripBytes = (int64_t)4 << 30;
 // Time of a strip's step (ns), by its rows per lane: alone on a SIMD, and of a full one.
 struct LongCost {
     int rows;
@@ -894,7 +898,7 @@ void orderStrips(RawVec<ScoreUnit> &units, size_t begin)
 }
 
 void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &starts,
-               const std::vector<size_t> &itemOff, int R16, int R64, double cellsStrip, bool noStrips)
+               const std::vector<size_t> &itemOff, int R16, int R64, double cellsStrip, int64_t stripBytes)
 {
     const RawVec<Key> &keys = P.keys16;
     const size_t nb = starts.size() - 1;
@@ -910,7 +914,7 @@ void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &s
 #pragma omp parallel for schedule(static) if (par)
     for (int64_t k = 0; k < (int64_t)nPairs; ++k)
         P.order16[k] = keys[k].id;
-    const int minBlocks = noStrips ? 0 : fixedShapeRule() && stripMinBlocks() < 0 ? 0 : stripMinBlocks();
+    const int minBlocks = stripBytes <= 0 ? 0 : fixedShapeRule() && stripMinBlocks() < 0 ? 0 : stripMinBlocks();
     // An item as one unit, with its row units in `pad`.  Few pairs: the
     // units of its tallest pair (buckets may be coarse).
     auto item = [&](size_t b, size_t k, size_t e) {
@@ -965,21 +969,50 @@ void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &s
             stripR *= 2;
     }
     P.units.reserve(nItems);
+    std::vector<ScoreUnit> wave;
+    wave.reserve(n64);
+    const int64_t budget = stripBytes / 8;
+    int64_t all = 0;   // words of every item that qualifies
     for (size_t b = 0; b < b64; ++b)
         for (size_t k = starts[b]; k < starts[b + 1]; k += 2) {
             ScoreUnit u = item(b, k, std::min(starts[b + 1], k + 2));
             split(u, R64 ? R64 : stripR);
-            const bool s = strips(u);
-            if (!s && !R64)
-                split(u, 16);
-            P.padded16 += padded(u);
-            if (s) {
-                addStrips(u);
-            } else {
-                P.slotWords = std::max(P.slotWords, words(u));
-                P.units.push_back(u);
-            }
+            u.block = strips(u) ? 0 : -1;
+            all += u.block < 0 ? 0 : words(u) * u.nblocks;
+            wave.push_back(u);
         }
+    // Past the budget: strips for the first items (the longest: a chain of its
+    // own) and for the last ones (they level the waves' ends), the items in
+    // between whole.  A quarter of the budget covers some hundred of the longest.
+    if (all > budget) {
+        int64_t used = 0;
+        size_t from = 0, to = wave.size();
+        auto take = [&](const ScoreUnit &u, int64_t limit) {
+            const int64_t w = u.block < 0 ? 0 : words(u) * u.nblocks;
+            const bool fits = used + w <= limit;
+            used += fits ? w : 0;
+            return fits;
+        };
+        while (from < to && take(wave[from], budget / 4))
+            ++from;
+        while (to > from && take(wave[to - 1], budget))
+            --to;
+        for (size_t k = from; k < to; ++k)
+            wave[k].block = -1;
+    }
+    for (ScoreUnit &u : wave) {
+        const bool s = u.block >= 0;
+        u.block = -1;
+        if (!s && !R64)
+            split(u, 16);
+        P.padded16 += padded(u);
+        if (s) {
+            addStrips(u);
+        } else {
+            P.slotWords = std::max(P.slotWords, words(u));
+            P.units.push_back(u);
+        }
+    }
     // 16 lanes: whole items (strips on request only).
     if (minBlocks > 0) {
         for (size_t b = b64; b < bG; ++b)
@@ -987,7 +1020,7 @@ void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &s
                 ScoreUnit u = item(b, k, std::min(starts[b + 1], k + 8));
                 split(u, R16);
                 P.padded16 += padded(u);
-                if (strips(u)) {
+                if (strips(u) && P.stripWords + words(u) * u.nblocks <= budget) {
                     addStrips(u);
                 } else {
                     P.slotWords = std::max(P.slotWords, words(u));
@@ -1017,7 +1050,7 @@ void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &s
 // Routing (empty / int16 / int32) and length bucketing into work items.
 // Pure host code: needs no device.
 void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &scoring, uint32_t mode,
-          uint32_t flags, Planned &P, bool traceShape = false, bool noLong = false, bool noStrips = false)
+          uint32_t flags, Planned &P, bool traceShape = false, bool noLong = false, int64_t stripBytes = kMaxStripBytes)
 {
     P.flags = flags;
     const int64_t N = H.count;
@@ -1284,7 +1317,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
     }
     std::vector<Plan16> &plans = P.plans;
     if (!traceShape)
-        makeUnits(V, P, starts, itemOff, R16, R64, cellsStrip, noStrips);
+        makeUnits(V, P, starts, itemOff, R16, R64, cellsStrip, stripBytes);
     for (uint32_t v = traceShape ? 0 : kSlotLane16; v < (uint32_t)shapes.size(); ++v) {
         // The shape's contiguous range of buckets and of sorted pairs.
         size_t b0 = 0;
@@ -2170,7 +2203,14 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
     Planned &P = *ctx->planned;
     P.reset();
     const auto tPlan = std::chrono::steady_clock::now();
-    plan(*setH, *setV, *scoring, mode, flags, P, false, false, ctx->noAlloc);
+    plan(*setH, *setV, *scoring, mode, flags, P, false, false,
+         ctx->noAlloc ? 0 : std::min(kMaxStripBytes, traceBudget(ctx)));
+    if (P.stripWords && ensure(ctx->b.strips, (size_t)P.stripWords * 8) != hipSuccess) {
+        // No room for the strips: whole items need a row buffer per wave only.
+        (void)hipGetLastError();
+        P.reset();
+        plan(*setH, *setV, *scoring, mode, flags, P, false, false, 0);
+    }
     ctx->stats.host_plan_ms = msSince(tPlan);
     fillStats(P, ctx->stats);
     const ScoringInfo &si = P.si;
@@ -2362,8 +2402,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         if ((err = put(ctx, ctx->b.order, orders.data(), orders.size())) != hipSuccess ||
             (err = put(ctx, ctx->b.items, lists.data(), lists.size())) != hipSuccess)
             return hipFail(ctx, err, "uploading work lists");
-        if ((err = ensure(ctx->b.queue, 4 * nq)) != hipSuccess || (err = ensure(ctx->b.rowbuf, rbMax)) != hipSuccess ||
-            (P.stripWords && (err = ensure(ctx->b.strips, (size_t)P.stripWords * 8)) != hipSuccess))
+        if ((err = ensure(ctx->b.queue, 4 * nq)) != hipSuccess || (err = ensure(ctx->b.rowbuf, rbMax)) != hipSuccess)
             return hipFail(ctx, err, "allocating work lists");
         uint32_t *dQueues = static_cast<uint32_t *>(ctx->b.queue.p);
         launches.push_back([=] { return launchZero32(dQueues, nq, stream); });
