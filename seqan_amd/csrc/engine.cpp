@@ -266,10 +266,14 @@ void release(DevBuf &b)
 // gathered in pinned memory and sent together: a copy from pageable memory
 // takes 8-12 us each, whatever its size, and large ones run at one thread's
 // memcpy.  Results come back the same way (20 MB to pageable memory 1.13 ms,
-// to pinned memory 0.38 and 0.03 from there).  stageBegin: `bytes` bounds what the call will put (each array
-// rounded up to 256 bytes), `down` what it will fetch; more than kMaxDown goes
-// straight to the caller's memory.
-constexpr size_t kMaxDown = (size_t)256 << 20;
+// to pinned memory 0.38 and 0.03 from there).  stageBegin: `bytes` bounds what
+// the call will put (each array rounded up to 256 bytes), `down` what it will
+// fetch.  The pinned memory stays with the context, so it has a bound: results
+// past kMaxDown go straight to the caller's memory, of uploads past kMaxUp
+// (about 10 million pairs) the arrays that do not fit are copied by themselves;
+// without pinned or device memory for the stage all are.  SQMI_STAGE_MB sets
+// both bounds (0: no staging; tests).
+constexpr size_t kMaxUp = (size_t)512 << 20, kMaxDown = (size_t)256 << 20;
 hipError_t stageBegin(sqmi_context *ctx, size_t bytes, size_t down = 0)
 {
     ctx->pinOn = false;
@@ -281,30 +285,44 @@ hipError_t stageBegin(sqmi_context *ctx, size_t bytes, size_t down = 0)
             return e;
         ctx->pinBusy = false;
     }
-    if (ctx->noAlloc)
+    size_t maxUp = kMaxUp, maxDown = kMaxDown;
+    if (const char *env = std::getenv("SQMI_STAGE_MB"))
+        if (*env)
+            maxUp = maxDown = (size_t)std::max(0ll, std::min(512ll, std::atoll(env))) << 20;
+    if (ctx->noAlloc || maxUp == 0)
         return hipSuccess;
-    if (down > kMaxDown)
+    bytes = std::min(bytes, maxUp);
+    if (down > maxDown)
         down = 0;
-    if (ctx->pinCap < std::max(bytes, down)) {
+    const size_t most = std::max(bytes, down);
+    if (ctx->pinCap < most) {
         if (ctx->pin)
             (void)hipHostFree(ctx->pin);
         ctx->pin = nullptr;
         ctx->pinCap = 0;
-        const size_t cap = std::max(bytes, down) + std::max(bytes, down) / 4;
+        const size_t cap = std::min(most + most / 4, kMaxUp);
         void *p = nullptr;
-        const hipError_t e = hipHostMalloc(&p, cap, hipHostMallocDefault);
-        if (e != hipSuccess)
-            return e;
+        if (hipHostMalloc(&p, cap, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return hipSuccess;
+        }
         ctx->pin = static_cast<char *>(p);
         ctx->pinCap = cap;
     }
-    const hipError_t e = ensure(ctx->stage, bytes);
-    if (e != hipSuccess)
-        return e;
+    if (ensure(ctx->stage, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipSuccess;
+    }
     ctx->downCap = down;
     ctx->pinUsed = ctx->pinSent = 0;
     ctx->pinOn = true;
     return hipSuccess;
+}
+
+// Whether the stage has room for `bytes` more.
+bool stageFits(const sqmi_context *ctx, size_t bytes)
+{
+    return ctx->pinOn && ctx->pinUsed + bytes <= std::min(ctx->pinCap, ctx->stage.cap);
 }
 
 // Sends what has been put since the last flush.
@@ -377,7 +395,7 @@ hipError_t put(sqmi_context *ctx, DevBuf &b, const Piece *pieces, size_t n)
     size_t bytes = 0, at = 0;
     for (size_t k = 0; k < n; ++k)
         bytes += pieces[k].bytes;
-    if (!ctx->pinOn || ctx->pinUsed + stageBytes(bytes) > std::min(ctx->pinCap, ctx->stage.cap)) {
+    if (!stageFits(ctx, stageBytes(bytes))) {
         hipError_t e = ensure(b, bytes);
         for (size_t k = 0; k < n && e == hipSuccess; at += pieces[k++].bytes)
             if (pieces[k].bytes)
@@ -1523,14 +1541,14 @@ hipError_t uploadResidues(sqmi_context *ctx, const sqmi_sequences *setH, const s
     const int64_t N = setH->count;
     const int64_t hTot = setH->offsets[N], vTot = setV->offsets[N];
     hipError_t err;
-    if (ctx->pinOn && hTot + vTot <= kStageResidues) {
-        // (64 bytes of slack after the residues, as below.)
+    if (hTot + vTot <= kStageResidues && stageFits(ctx, stageBytes(hTot) + stageBytes(vTot) + 512)) {
+        // (256 bytes of slack after the residues, 64 below.)
         if ((err = put(ctx, ctx->b.hRes, setH->residues, hTot)) != hipSuccess)
             return err;
-        ctx->pinUsed = std::min(std::min(ctx->pinCap, ctx->stage.cap), ctx->pinUsed + 256);
+        ctx->pinUsed += 256;
         if ((err = put(ctx, ctx->b.vRes, setV->residues, vTot)) != hipSuccess)
             return err;
-        ctx->pinUsed = std::min(std::min(ctx->pinCap, ctx->stage.cap), ctx->pinUsed + 256);
+        ctx->pinUsed += 256;
     } else if ((err = ensure(ctx->b.hRes, hTot + 64)) != hipSuccess || (err = ensure(ctx->b.vRes, vTot + 64)) != hipSuccess ||
         (err = hipMemcpyAsync(ctx->b.hRes.p, setH->residues, hTot, hipMemcpyHostToDevice, ctx->stream)) !=
             hipSuccess ||
