@@ -274,10 +274,14 @@ void release(DevBuf &b)
 // without pinned or device memory for the stage all are.  SQMI_STAGE_MB sets
 // both bounds (0: no staging; tests).
 constexpr size_t kMaxUp = (size_t)512 << 20, kMaxDown = (size_t)256 << 20;
-hipError_t stageBegin(sqmi_context *ctx, size_t bytes, size_t down = 0)
+
+// stageResume: a call that replays the last one's launches; what that one put
+// stays in place, results have `down` bytes of the pinned memory that is there.
+hipError_t stageResume(sqmi_context *ctx, size_t down)
 {
     ctx->pinOn = false;
-    ctx->downUsed = ctx->downCap = 0;
+    ctx->downUsed = 0;
+    ctx->downCap = down <= std::min(ctx->pinCap, kMaxDown) ? down : 0;
     ctx->down.clear();
     if (ctx->pinBusy) {   // an earlier call failed between its uploads and its end
         const hipError_t e = hipDeviceSynchronize();
@@ -285,6 +289,14 @@ hipError_t stageBegin(sqmi_context *ctx, size_t bytes, size_t down = 0)
             return e;
         ctx->pinBusy = false;
     }
+    return hipSuccess;
+}
+
+hipError_t stageBegin(sqmi_context *ctx, size_t bytes, size_t down = 0)
+{
+    const hipError_t e = stageResume(ctx, 0);
+    if (e != hipSuccess)
+        return e;
     size_t maxUp = kMaxUp, maxDown = kMaxDown;
     if (const char *env = std::getenv("SQMI_STAGE_MB"))
         if (*env)
@@ -420,6 +432,19 @@ hipError_t put(sqmi_context *ctx, DevBuf &b, const void *src, size_t bytes)
 {
     const Piece one{src, bytes};
     return put(ctx, b, &one, 1);
+}
+
+// New contents for two buffers that the last call put, in one copy.
+hipError_t restage(sqmi_context *ctx, const DevBuf &a, const void *srcA, size_t bytesA, const DevBuf &b, const void *srcB,
+                   size_t bytesB)
+{
+    char *stage = static_cast<char *>(ctx->stage.p);
+    const size_t atA = static_cast<char *>(a.p) - stage, atB = static_cast<char *>(b.p) - stage;
+    copyBytes(ctx->pin + atA, srcA, bytesA);
+    copyBytes(ctx->pin + atB, srcB, bytesB);
+    const size_t from = std::min(atA, atB), to = std::max(atA + bytesA, atB + bytesB);
+    ctx->pinBusy = true;
+    return hipMemcpyAsync(stage + from, ctx->pin + from, to - from, hipMemcpyHostToDevice, ctx->stream);
 }
 
 struct ScoringInfo
@@ -2182,10 +2207,19 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             const double keyMs = msSince(tKey);
             const uint8_t *rH = setH->residues, *rV = setV->residues;
             const int64_t hTot = setH->offsets[N], vTot = setV->offsets[N];
-            if (!(flags & SQMI_RESIDUES_ON_DEVICE) &&
-                ((err = hipMemcpyAsync(ctx->b.hRes.p, rH, hTot, hipMemcpyHostToDevice, stream)) != hipSuccess ||
-                 (err = hipMemcpyAsync(ctx->b.vRes.p, rV, vTot, hipMemcpyHostToDevice, stream)) != hipSuccess))
-                return hipFail(ctx, err, "copying residues");
+            // Residues that were staged are staged again, at their places, and
+            // the scores come back through the stage too (by
+            // three pageable copies 256 pairs of 150 bp take 122 us, so 82).
+            if ((err = stageResume(ctx, downScores(N, flags))) != hipSuccess)
+                return hipFail(ctx, err, "waiting for an earlier call");
+            if (!(flags & SQMI_RESIDUES_ON_DEVICE)) {
+                if (ctx->b.hRes.view && ctx->b.vRes.view)
+                    err = restage(ctx, ctx->b.hRes, rH, hTot, ctx->b.vRes, rV, vTot);
+                else if ((err = hipMemcpyAsync(ctx->b.hRes.p, rH, hTot, hipMemcpyHostToDevice, stream)) == hipSuccess)
+                    err = hipMemcpyAsync(ctx->b.vRes.p, rV, vTot, hipMemcpyHostToDevice, stream);
+                if (err != hipSuccess)
+                    return hipFail(ctx, err, "copying residues");
+            }
             if (!ctx->replay.exec)
                 captureReplay(ctx);
             if ((err = hipEventRecord(ctx->ev0, stream)) != hipSuccess)
@@ -2200,11 +2234,12 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             }
             if ((err = hipEventRecord(ctx->ev1, stream)) != hipSuccess)
                 return hipFail(ctx, err, "event");
-            if (!(flags & SQMI_SCORES_ON_DEVICE) &&
-                (err = hipMemcpyAsync(scores, ctx->b.scores.p, 4 * N, hipMemcpyDeviceToHost, stream)) != hipSuccess)
+            if (!(flags & SQMI_SCORES_ON_DEVICE) && (err = fetch(ctx, scores, ctx->b.scores.p, 4 * N)) != hipSuccess)
                 return hipFail(ctx, err, "copying scores");
             if ((err = hipStreamSynchronize(stream)) != hipSuccess)
                 return hipFail(ctx, err, "alignment kernels");
+            deliver(ctx);
+            stageEnd(ctx);
             if ((st = stripCheck(ctx)) != SQMI_OK)
                 return st;
             ctx->stats = ctx->replay.stats;
