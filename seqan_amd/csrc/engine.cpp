@@ -1185,7 +1185,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
                 if (n != 0 && m != 0 && route16(n, m)) {
                     const int b = lengthBin(m);
                     ++local16[b];
-                    if (countWide)
+                    if (countWide && b <= kWideLane[0].bin)
                         localWide[b] += !driftNarrow(si, dr, local, n, m);
                     localCells += n * m;
                     localMost = std::max(localMost, n * m);
