@@ -1091,9 +1091,12 @@ void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &s
 }
 
 // Routing (empty / int16 / int32) and length bucketing into work items.
-// Pure host code: needs no device.
+// Pure host code: needs no device.  stripBytes: what strips may take (0: none).
+// tight: the smallest lists, for a no-allocation call near its limit (16
+// lanes per couple, every bin of the shape table's on lanes whatever its values).
 void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &scoring, uint32_t mode,
-          uint32_t flags, Planned &P, bool traceShape = false, bool noLong = false, int64_t stripBytes = kMaxStripBytes)
+          uint32_t flags, Planned &P, bool traceShape = false, bool noLong = false, int64_t stripBytes = kMaxStripBytes,
+          bool tight = false)
 {
     P.flags = flags;
     const int64_t N = H.count;
@@ -1208,6 +1211,8 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
         cellsStrip = kStripShare * (double)cells16;
         if ((double)most16 * (double)pairs16 <= 4.0 * (double)cells16 && evenOn16((double)most16, (double)pairs16, (double)cells16))
             cells64 = cellsStrip = 1e300;
+        if (tight)
+            cells64 = 1e300;
         if (fixedShapeRule()) {
             std::fill(binG, binG + 16, 16);
         } else {
@@ -1260,7 +1265,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
         }
         const int b = lengthBin(m);
         const bool wide = !driftNarrow(si, dr, local, n, m);
-        if (local || !wide || forcedG == 1 ? binLane[b] != 0 : b <= wideLaneBin && !binG[b]) {
+        if (local || !wide || forcedG == 1 || tight ? binLane[b] != 0 : b <= wideLaneBin && !binG[b]) {
             const uint32_t slot = !local && wide ? kSlotLaneWide : binLane[b] == 32 ? kSlotLane32 : kSlotLane16;
             units = blocksFor(shapes[slot], m);
             if (units <= kMaxBlocks16)
@@ -2277,12 +2282,16 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
 
     // The no-allocation call: everything but the row buffers has a fixed
     // size; the row buffers need at least one workgroup's worth per shape.
+    // A request that does not fit is planned once more in its tightest form.
     size_t rowbufBudget = 0;
-    if (ctx->noAlloc) {
+    int unitWaves = scoreWaves(P.dna16, (int64_t)P.units.size(), ctx->numCUs);
+    RawVec<SlimUnit> slim;
+    for (bool tight = false; ctx->noAlloc; tight = true) {
         if (!P.idsLong.empty())
             return fail(ctx, SQMI_ERR_UNSUPPORTED,
                         "sqmi_align_score_noalloc: pairs on the long-pair route need sqmi_align_score");
         const int64_t A2 = (int64_t)si.alpha * si.alpha, hTot = setH->offsets[N], vTot = setV->offsets[N];
+        const size_t nSlim = (P.units.size() + 3) / 4 * 4;   // the lists after them start on 16 bytes
         size_t need = 0;
         if (!(flags & SQMI_RESIDUES_ON_DEVICE))
             need += arenaBytes(hTot + 64) + arenaBytes(vTot + 64);
@@ -2290,18 +2299,16 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         if (!(flags & SQMI_SCORES_ON_DEVICE))
             need += arenaBytes(4 * N);
         need += arenaBytes(2 * (si.alpha + 1) * (si.alpha + 1)) + arenaBytes(64) + arenaBytes(4 * A2);
-        size_t nOrder = 0, nItems = 0, minRb = 0;
+        size_t nOrder = 0, nItems = 0, laneRb = 0;
         for (const Plan16 &pl : plans) {
             nOrder += pl.order.size();
             nItems += pl.items.size();
-            minRb = std::max(minRb, (size_t)wavesPerBlock16() * 64 * laneRowCols(pl.maxN, pl.var.R) * 8);
+            laneRb = std::max(laneRb, (size_t)wavesPerBlock16() * 64 * laneRowCols(pl.maxN, pl.var.R) * 8);
         }
         if (!plans.empty())
             need += arenaBytes(4 * nOrder) + arenaBytes(sizeof(WorkItem) * nItems);
-        if (!P.units.empty()) {
-            need += arenaBytes(4 * P.order16.size()) + arenaBytes(sizeof(ScoreUnit) * P.units.size());
-            minRb = std::max(minRb, (size_t)scoreWaves(P.dna16, (int64_t)P.units.size(), ctx->numCUs) * P.slotWords * 8);
-        }
+        if (!P.units.empty())
+            need += arenaBytes(4 * P.order16.size()) + arenaBytes(sizeof(SlimUnit) * nSlim);
         if (!plans.empty() || !P.units.empty())
             need += arenaBytes(64 * (plans.size() + 1));
         if (!ids32.empty())
@@ -2309,12 +2316,25 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         if (!emptyIds.empty())
             need += arenaBytes(4 * emptyIds.size());
         const size_t cap = ctx->arena.cap - ctx->arena.used;
-        if (need + arenaBytes(minRb) > cap)
+        unitWaves = scoreWaves(P.dna16, (int64_t)P.units.size(), ctx->numCUs);
+        auto rowbufs = [&] { return arenaBytes(std::max(laneRb, (size_t)unitWaves * P.slotWords * 8)); };
+        if (need + rowbufs() > cap)
+            unitWaves = std::min(unitWaves, 4);
+        if (need + rowbufs() <= cap) {
+            rowbufBudget = (cap - need) & ~(size_t)255;   // holds rowbufs()
+            slim.resize(nSlim);
+            for (size_t k = 0; k < nSlim; ++k)
+                slim[k] = k < P.units.size() ? SlimUnit::of(P.units[k]) : SlimUnit{};
+            break;
+        }
+        if (tight)
             return fail(ctx, SQMI_ERR_OUT_OF_MEMORY,
-                        "sqmi_align_score_noalloc: the request needs " + std::to_string(need + arenaBytes(minRb)) +
+                        "sqmi_align_score_noalloc: the request needs " + std::to_string(need + rowbufs()) +
                             " bytes of device scratch, more than the " + std::to_string(cap) +
                             " of SQMI_NOALLOC_SCRATCH_BYTES; use sqmi_align_score");
-        rowbufBudget = (cap - need) & ~(size_t)255;   // holds arenaBytes(minRb), see above
+        P.reset();
+        plan(*setH, *setV, *scoring, mode, flags, P, false, false, 0, true);
+        fillStats(P, ctx->stats);
     }
 
     // ---- device buffers --------------------------------------------------
@@ -2412,13 +2432,13 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
     // buffers, which a launch only uses while it runs.
     if (!plans.empty() || !P.units.empty()) {
         const int wpb = wavesPerBlock16();
-        const size_t unitBytes = sizeof(ScoreUnit) * P.units.size(), unitOrder = P.order16.size();
+        const size_t unitBytes = ctx->noAlloc ? sizeof(SlimUnit) * slim.size() : sizeof(ScoreUnit) * P.units.size();
+        const size_t unitOrder = P.order16.size();
         std::vector<size_t> orderOff(plans.size() + 1, unitOrder), itemOff(plans.size() + 1, 0);
         std::vector<int> grids(plans.size()), rowColsOf(plans.size());
         size_t rbMax = 0;
-        int unitGrid = 0, unitWaves = 4;
+        int unitGrid = 0;
         if (!P.units.empty()) {
-            unitWaves = scoreWaves(P.dna16, (int64_t)P.units.size(), ctx->numCUs);
             unitGrid = std::max(1, (int)std::min<int64_t>((int64_t)ctx->numCUs * occupancyScore16(P.dna16, kind, unitWaves),
                                                           ((int64_t)P.units.size() + unitWaves - 1) / unitWaves));
             const size_t perBlock = std::max<size_t>((size_t)unitWaves * P.slotWords * 8, 8);
@@ -2446,7 +2466,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
         std::vector<Piece> orders, lists;
         if (!P.units.empty()) {
             orders.push_back({P.order16.data(), 4 * unitOrder});
-            lists.push_back({P.units.data(), unitBytes});
+            lists.push_back({ctx->noAlloc ? (const void *)slim.data() : P.units.data(), unitBytes});
         }
         for (const Plan16 &pl : plans) {
             orders.push_back({pl.order.data(), 4 * pl.order.size()});
@@ -2463,6 +2483,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
             ScoreArgs a = sa;
             a.order = static_cast<const int32_t *>(ctx->b.order.p);
             a.units = static_cast<const ScoreUnit *>(ctx->b.items.p);
+            a.slim = ctx->noAlloc ? static_cast<const SlimUnit *>(ctx->b.items.p) : nullptr;
             a.nUnits = (int32_t)P.units.size();
             a.queue = dQueues;
             a.rowbuf = static_cast<uint64_t *>(ctx->b.rowbuf.p);

@@ -204,6 +204,24 @@ struct ScoreUnit {
     int32_t pad;
     int64_t rowOff;     // strips: the item's words in ScoreArgs::strips (nblocks x 64 / G x (maxN + 1))
 };
+// A unit without strips in 12 bytes: the list's form in the no-allocation call,
+// whose scratch array holds it (40 bytes per 8 pairs of 16 lanes would refuse
+// calls of 2.7 million short pairs on).
+struct SlimUnit {
+    int32_t first;
+    uint32_t size;      // maxN | nblocks << 16
+    uint32_t form;      // count | shape << 8 | rows << 16
+    __host__ __device__ static SlimUnit of(const ScoreUnit &u)
+    {
+        return SlimUnit{u.first, (uint32_t)u.maxN | (uint32_t)u.nblocks << 16,
+                        (uint32_t)u.count | (uint32_t)u.shape << 8 | (uint32_t)u.rows << 16};
+    }
+    __host__ __device__ ScoreUnit unit() const
+    {
+        return ScoreUnit{first, (int32_t)(form & 0xff), (int32_t)(size & 0xffff), (int32_t)(size >> 16), (int32_t)(form >> 16),
+                         (int32_t)(form >> 8 & 0xff), -1, 0, 0};
+    }
+};
 struct ScoreArgs {
     const uint8_t *hRes;
     const uint8_t *vRes;
@@ -211,6 +229,7 @@ struct ScoreArgs {
     const int64_t *vOff;
     const int32_t *order;
     const ScoreUnit *units;
+    const SlimUnit *slim;       // in place of `units`, or null
     int32_t nUnits;
     uint32_t *queue;            // unit counter (zeroed before the launch)
     uint64_t *rowbuf;           // slotWords (G, F) words per wave of the grid

@@ -721,7 +721,7 @@ __device__ __forceinline__ void scoreRun(const ScoreArgs &a)
         it = __builtin_amdgcn_readfirstlane(it);
         if (it >= a.nUnits)
             break;
-        const ScoreUnit w = uniformUnit(a.units[it]);
+        const ScoreUnit w = uniformUnit(a.slim ? a.slim[it].unit() : a.units[it]);
         if (w.shape & kUnit64) {
             if (w.shape & kUnitWide)
                 Score16<64, DNA, KIND, true>::unit(a, w, slotRow, sProf, sT, stop);
