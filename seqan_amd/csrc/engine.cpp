@@ -3310,11 +3310,20 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     // call; columns run to the item's longest |H|, a group past the band.
     Drift dr = driftOf(si, local);
     const int64_t *offH = setH->offsets, *offV = setV->offsets;
-    int64_t maxN = 1, maxM = 1;
-#pragma omp parallel for schedule(static) reduction(max : maxN, maxM) if (N > kParallelMin)
-    for (int64_t i = 0; i < N; ++i) {
-        maxN = std::max(maxN, offH[i + 1] - offH[i]);
-        maxM = std::max(maxM, offV[i + 1] - offV[i]);
+    int64_t maxN = 1, maxM = 1, nTop = 1;   // nTop: |H| of a pair of the most rows (calls of one thread)
+    if (N > kParallelMin) {
+#pragma omp parallel for schedule(static) reduction(max : maxN, maxM)
+        for (int64_t i = 0; i < N; ++i) {
+            maxN = std::max(maxN, offH[i + 1] - offH[i]);
+            maxM = std::max(maxM, offV[i + 1] - offV[i]);
+        }
+    } else if (bandCostsOk) {
+        for (int64_t i = 0; i < N; ++i) {
+            const int64_t n = offH[i + 1] - offH[i], m = offV[i + 1] - offV[i];
+            maxN = std::max(maxN, n);
+            nTop = m > maxM ? n : nTop;
+            maxM = std::max(maxM, m);
+        }
     }
     if (!local && bandCostsOk)
         dr.bias += (int32_t)std::min<int64_t>(bandDrop(si, dr, W1, maxM), 1 << 20);
@@ -3324,7 +3333,34 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     };
     const bool narrowT = dr.neg == (local ? 2 * dr.d + 2 : dr.cost + 1);   // no t below 0
     bool bandWide = !narrowT;
-    const bool packedOk = bandCostsOk;
+    // Free end gaps and local alignment, few pairs: a packed item takes its
+    // whole sweep, however few the items; the int32 kernels, which spread a
+    // pair's band over a wave, are done earlier.  Times in ns: a call's items
+    // on the packed kernel, a pair on int32 (alone; its share of a full chip).
+    const double simds = 4.0 * std::max(1, ctx->numCUs);
+    auto packedTime = [&](double items, double blockCols, int64_t most) {
+        const int cols = bandRingCols((int)most, lower_diag, upper_diag, bandR), waves = bandWaves(cols);
+        const double slots = cols > 256 ? simds : 2 * simds / waves;
+        const double column = cols > 256 ? kBandColumnAlone : kBandColumn[waves == 8 ? 2 : waves == 4 ? 1 : 0];
+        return std::ceil(items / slots) * blockCols * column;
+    };
+    auto loneTime = [&](double m, double w) { return m * (w <= 64 ? kBandNarrowLone : kBandWideLone * std::ceil(w / 64)); };
+    auto fullTime = [&](double m, double w) {
+        return m * (w <= 64 ? kBandNarrowFull * w / 64 : kBandWideFull * std::ceil(w / 64)) / simds;
+    };
+    const bool choose = mode != 0 && !envFlag("SQMI_BAND_PACKED");
+    bool packedOk = bandCostsOk;
+    if (choose && packedOk && N <= kParallelMin && maxN <= 30000 && maxM <= 30000) {
+        // From the sums alone, where the least that the packed kernel takes
+        // (the tallest pair's item) exceeds the most that int32 does: the
+        // pairs need not be placed first (20,000 pairs of 1 kbp, 11 diagonals,
+        // local: a call 0.69 -> 0.54 ms).
+        const double w = std::min<double>((double)W1 + 1, (double)(maxN + maxM));
+        const double wTop = std::min<double>((double)W1 + 1, (double)(nTop + maxM));
+        const double blockCols = ((maxM + bandR) / bandR) * std::min<double>(wTop + bandR, (double)nTop);
+        packedOk = std::max(loneTime((double)maxM, w), fullTime((double)(offV[N] - offV[0]), w)) >=
+                   packedTime(std::ceil((double)N / 128), blockCols, nTop);
+    }
     std::vector<int32_t> narrow, wide, rejected;
     int64_t wNarrow = 1, wWide = 0, cells = 0;
     auto toInt32 = [&](int32_t id, int64_t n, int64_t m) {
@@ -3347,11 +3383,26 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
     std::vector<int64_t> nOther((size_t)parts, 0);
     int64_t firstBad = N, nPacked = 0;
     bool anyWide = false;
+    const bool routed = !packedOk && parts == 1;   // one pass: no pair is packed
+    if (routed) {
+        narrow.reserve((size_t)N);
+        for (int64_t i = 0; i < N && firstBad == N; ++i) {
+            const int64_t n = offH[i + 1] - offH[i], m = offV[i + 1] - offV[i];
+            if (n == 0 || m == 0) {
+                rejected.push_back((int32_t)i);
+            } else if (!bandSupported(n, m, lower_diag, upper_diag, local)) {
+                firstBad = i;
+            } else {
+                cells += n * m;
+                toInt32((int32_t)i, n, m);
+            }
+        }
+    }
 #pragma omp parallel for schedule(static) num_threads(parts) reduction(+ : cells, nPacked) reduction(min : firstBad) \
     reduction(|| : anyWide) if (parts > 1)
     for (int t = 0; t < parts; ++t) {
         int32_t *cnt = counts.data() + (size_t)t * mSlots;
-        for (int64_t i = N * t / parts; i < N * (t + 1) / parts; ++i) {
+        for (int64_t i = N * t / parts; i < N * (t + 1) / parts && !routed; ++i) {
             const int64_t n = offH[i + 1] - offH[i], m = offV[i + 1] - offV[i];
             if (n != 0 && m != 0 && !bandSupported(n, m, lower_diag, upper_diag, local)) {
                 firstBad = std::min(firstBad, i);
@@ -3417,23 +3468,15 @@ sqmi_status sqmi_align_score_banded(sqmi_context *ctx, const sqmi_sequences *set
             bandMaxN = std::max(bandMaxN, w.maxN);
         }
     }
-    // Free end gaps and local alignment, few pairs: a packed item takes its
-    // whole sweep, however few the items; the int32 kernels, which spread a
-    // pair's band over a wave, are done earlier.
-    if (mode != 0 && !packed.empty() && !envFlag("SQMI_BAND_PACKED")) {
+    if (choose && !packed.empty()) {
         double blockCols = 0, lone = 0, full = 0;
         for (const WorkItem &it : bandItems) {
             const double m = (double)((uint32_t)it.count >> 16), w = std::min<double>((double)W1 + 1, it.maxN + m);
-            const double chunks = std::ceil(w / 64);
             blockCols = std::max(blockCols, it.nblocks * std::min<double>(w + bandR, it.maxN));
-            lone = std::max(lone, m * (w <= 64 ? kBandNarrowLone : kBandWideLone * chunks));
-            full += (it.count & 0xffff) * m * (w <= 64 ? kBandNarrowFull * w / 64 : kBandWideFull * chunks);
+            lone = std::max(lone, loneTime(m, w));
+            full += (it.count & 0xffff) * fullTime(m, w);
         }
-        const double simds = 4.0 * std::max(1, ctx->numCUs);
-        const int cols = bandRingCols(bandMaxN, lower_diag, upper_diag, bandR), waves = bandWaves(cols);
-        const double slots = cols > 256 ? simds : 2 * simds / waves;
-        const double column = cols > 256 ? kBandColumnAlone : kBandColumn[waves == 8 ? 2 : waves == 4 ? 1 : 0];
-        if (std::max(lone, full / simds) < std::ceil(bandItems.size() / slots) * blockCols * column) {
+        if (std::max(lone, full) < packedTime((double)bandItems.size(), blockCols, bandMaxN)) {
             for (int32_t id : packed)
                 toInt32(id, offH[id + 1] - offH[id], offV[id + 1] - offV[id]);
             packed.clear();
