@@ -750,6 +750,26 @@ struct Planned
         plans.clear();
         scratch32 = slotWords = stripWords = items16 = padded16 = cells = 0;
     }
+
+    // Back to an empty plan of its own after a call whose arrays a context
+    // should not keep: past 128 MB (some 5 million pairs) faulting them in
+    // again is a small part of the next such call.
+    static constexpr size_t kKeepBytes = (size_t)128 << 20;
+    void trim()
+    {
+        auto of = [](const auto &v) { return v.capacity() * sizeof(v[0]); };
+        size_t bytes = of(emptyIds) + of(ids32) + of(idsLong) + of(scratchOff32) + of(keys16) + of(keysTmp) + of(order16) + of(units);
+        for (const Plan16 &p : plans)
+            bytes += of(p.order) + of(p.items);
+        if (bytes > kKeepBytes)
+            *this = Planned{};
+    }
+};
+
+// Trims the context's plan when the call ends.
+struct PlanUse {
+    Planned &p;
+    ~PlanUse() { p.trim(); }
 };
 
 // int32 pairs whose sides are both at least this long (and that are DNA,
@@ -2259,6 +2279,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
     dropReplay(ctx);
 
     Planned &P = *ctx->planned;
+    const PlanUse use{P};
     P.reset();
     const auto tPlan = std::chrono::steady_clock::now();
     plan(*setH, *setV, *scoring, mode, flags, P, false, false,
@@ -2703,6 +2724,7 @@ static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, 
     hipStream_t stream = ctx->stream;
 
     Planned &P = *ctx->planned;
+    const PlanUse use{P};
     P.reset();
     Inputs in;
     // Host residue sets of 4 MB and more are copied in on a second host
