@@ -617,21 +617,30 @@ int bandWaves(int cols) { return cols > 256 ? 4 : cols > 128 ? 8 : cols > 64 ? 4
 // 0.81 / 0.81 / 0.84 / 2.5 ms, int32 2.5 / 3.3 / 12.8 / 51.5; local, 150 bp,
 // 33 diagonals: 0.11 / 0.11 / 0.11 / 0.18 against 0.04 / 0.06 / 0.19 / 0.68.
 constexpr double kBandColumnAlone = 335, kBandColumn[3] = {170, 80, 60}, kBandNarrowLone = 270, kBandNarrowFull = 70, kBandWideLone = 615, kBandWideFull = 202;
+// Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
+constexpr int64_t kResidentWaves = 3072;
 // Calls of pairs of about one size (the largest at most four times the mean):
-// 64 lanes for all of them cost more than twice the instructions, and their
-// skew of 64 steps weighs on short pairs.  In cycles: a pair alone on 16 lanes
-// about 2.9 a cell (more waves per SIMD: up to twice that), on 64 lanes 0.93 and
-// the skew.  Whether 16 lanes are about as fast.  Device time of 53,121 pairs of 68 bp, local:
-// 64 lanes 413 us, 16 152; 4,000 of them 71, 40; 53,121 of 150 bp 457, 268;
-// 20,000 of 300 bp 413, 348.  Past 512 rows (mean) 64 lanes have rows enough to cost
-// the same: 20,000 of 1 kbp, global, 2.24 ms, 16 lanes 2.42.  62,172 protein
-// pairs of 50-372 by 50-744, local: 1.35 ms, 16 lanes 1.02.
-bool evenOn16(double most, double pairs, double cells)
+// 64 lanes for all of them cost more than twice the instructions, their skew
+// of 64 steps weighs on short pairs, and four times the units and more (strips)
+// are claimed one by one.  In cycles: a pair alone on 16 lanes about 3.2 a cell,
+// with the table 4 (more waves per SIMD: up to twice that), on 64 lanes 0.93
+// (1.2), the skew and 4,000; 40 a unit.  Whether 16 lanes are the faster.  Device us, 64
+// lanes / 16: 4,096 pairs of 20-60 bp 66 / 31, of 66-126 71 / 43, of 150 76 / 61, of
+// 100-200 80 / 77, of 400 205 / 203; 2,048 of 66-126 46 / 40, of 150 53 / 55, of 200
+// 60 / 77; 53,121 of 68 bp, local, 413 / 152; 20,000 of 300 bp 413 / 348.  Proteins:
+// 4,096 of 66-126 78 / 54, of 100-200 84 / 107, of 300 198 / 189; 8,192 of 200-400
+// 236 / 345; 62,172 of 50-372 by 50-744, local, 1,350 / 1,020.  Past 512 rows (mean)
+// 64 lanes have rows enough to cost the same: 20,000 of 1 kbp, global, 2,240 / 2,420.
+bool evenOn16(double most, double pairs, double cells, bool dna)
 {
-    const double waves = pairs / 8 / 1024, skew = (std::sqrt(most) + 64) / std::max(1.0, std::sqrt(most));
-    const double t16 = std::max(2.9 * most * std::max(1.0, 0.66 * std::min(3.0, waves)), 2.3e-4 * cells);
-    const double t64 = std::max(0.93 * most, 2.1 * 2.3e-4 * cells) * skew;
-    return cells <= 512.0 * 512.0 * pairs && t64 * 1.3 >= t16;
+    const double alone16 = dna ? 3.2 : 4.0, alone64 = dna ? 0.93 : 1.2, side = std::max(1.0, std::sqrt(most));
+    const double waves = pairs / 8 / 1024, skew = (side + 64) / side;
+    double blocks = pairs * kStripShare < 1 ? std::ceil((side + 1) / 256) : 1;   // makeUnits: strips of 4 rows per lane, or more
+    while (blocks > 1 && blocks * pairs / 2 > 2 * kResidentWaves)
+        blocks = std::ceil(blocks / 2);
+    const double t16 = std::max(alone16 * most * std::max(1.0, 0.66 * std::min(3.0, waves)), 2.3e-4 * cells) + 40 * pairs / 8;
+    const double t64 = std::max(alone64 * most, 2.1 * 2.3e-4 * cells) * skew + 40 * blocks * pairs / 2 + 4000;
+    return cells <= 512.0 * 512.0 * pairs && 1.03 * t64 >= t16;
 }
 // Global pairs whose drifted values need all 16 bits (Variant16::wide), one per
 // lane with 32 rows: in the length bins up to kWideLane[k].bin when the call
@@ -647,8 +656,6 @@ struct WideLane {
     int64_t alone, beside;
 };
 constexpr WideLane kWideLane[] = {{7, 262144, 1048576}, {6, 131072, 262144}, {5, 24576, 65536}, {4, 16384, 49152}};
-// Waves of the packed score kernel that the chip holds (256 CUs, 4 SIMDs, 3).
-constexpr int64_t kResidentWaves = 3072;
 // Rows per unit of the group shapes' row counts.
 constexpr int kUnitRows = 64;
 inline int64_t unitsOfRows(int64_t m) { return (m + kUnitRows) / kUnitRows; }   // m + 1 rows
@@ -1229,7 +1236,7 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
             pairs16 += binCount[b];
         cells64 = kCouple64Share * (double)cells16;
         cellsStrip = kStripShare * (double)cells16;
-        if ((double)most16 * (double)pairs16 <= 4.0 * (double)cells16 && evenOn16((double)most16, (double)pairs16, (double)cells16))
+        if ((double)most16 * (double)pairs16 <= 4.0 * (double)cells16 && evenOn16((double)most16, (double)pairs16, (double)cells16, dna16))
             cells64 = cellsStrip = 1e300;
         if (tight)
             cells64 = 1e300;
