@@ -124,14 +124,15 @@ struct sqmi_context
     Arena arena;
     bool noAlloc = false;   // inside sqmi_align_score_noalloc
     // The last sqmi_align_score call, kept for an identical next call: the
-    // key of its inputs, its statistics and its launches, from the second
-    // such call on as an instantiated HIP graph (to capture and instantiate one
-    // takes 60-80 us, which a call that comes once does not get back).  Its plan lives on in the context's device buffers, so any
-    // other call on the context drops it.
+    // key of its inputs, its statistics and its launches; more than
+    // kDirectLaunches of them, from the second such call on, as an instantiated
+    // HIP graph (to capture and instantiate one takes 60-80 us, which a call that
+    // comes once does not get back).  Its plan lives on in the context's device
+    // buffers, so any other call on the context drops it.
     struct Replay {
         bool valid = false;
         uint64_t key = 0;
-        std::vector<std::function<hipError_t()>> launches;   // until the second such call captures them
+        std::vector<std::function<hipError_t()>> launches;   // until a graph holds them
         hipGraphExec_t exec = nullptr;
         sqmi_stats stats{};
     } replay;
@@ -208,6 +209,10 @@ void dropReplay(sqmi_context *ctx)
         (void)hipGraphExecDestroy(ctx->replay.exec);
     ctx->replay = sqmi_context::Replay{};
 }
+
+// A replayed call of up to this many launches runs them one by one: a graph of
+// two takes 8-10 us longer than they do.
+constexpr size_t kDirectLaunches = 4;
 
 // The kept launches as an instantiated graph; a capture the runtime refuses
 // leaves them to be run one by one.
@@ -2252,7 +2257,7 @@ static sqmi_status alignScore(sqmi_context *ctx, const sqmi_sequences *setH, con
                 if (err != hipSuccess)
                     return hipFail(ctx, err, "copying residues");
             }
-            if (!ctx->replay.exec)
+            if (!ctx->replay.exec && ctx->replay.launches.size() > kDirectLaunches)
                 captureReplay(ctx);
             if ((err = hipEventRecord(ctx->ev0, stream)) != hipSuccess)
                 return hipFail(ctx, err, "event");
