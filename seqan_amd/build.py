@@ -52,7 +52,7 @@ NBINS = 16
 
 def shape_table_source(path: str = SHAPE_TABLE) -> str:
     """C++ initializers of the planner's shape table (length bin x count
-    class -> kernel shape), from the committed JSON table."""
+    class -> groups or rows per lane), from the committed JSON table."""
     with open(path) as f:
         t = json.load(f)
     shapes = [tuple(int(x) for x in s) for s in t["shapes"]]
@@ -72,12 +72,10 @@ def shape_table_source(path: str = SHAPE_TABLE) -> str:
     prov = json.dumps(t.get("provenance", {}), sort_keys=True).replace("\\", "\\\\").replace('"', '\\"')
     return "\n".join([
         "// Generated by seqan_amd/build.py from seqan_amd/tuning/shapes.json; do not edit.",
-        f"constexpr int kTabNShapes = {len(shapes)};",
         "constexpr int kTabShapes[][2] = {" + ", ".join(f"{{{g}, {r}}}" for g, r in shapes) + "};",
         f"constexpr int kTabNClasses = {len(classes)};",
         "constexpr int64_t kTabCountClasses[4] = {" + ", ".join(str(c) for c in classes + [0] * (4 - len(classes))) + "};",
         "constexpr uint8_t kTabChoice[4][16][4] = {" + ",\n    ".join(rows) + "};",
-        f"constexpr int kTabCoopMinBlocks = {int(t.get('coop_min_blocks', 10))};",
         f'constexpr const char *kTabProvenance = "{prov}";',
         ""])
 

@@ -550,11 +550,11 @@ bool shapeSupported(const Variant16 &v)
     return (v.G == 16 && (v.R == 8 || v.R == 16)) || (v.G == 64 && (v.R == 4 || v.R == 8 || v.R == 16));
 }
 
-// The planner's shape table (seqan_amd/tuning/shapes.json, turned into C++
-// by the build): per category (DNA byte profile or substitution table,
-// global or local), length bin b (2^(b-1) < |V| + 1 <= 2^b) and count class
-// (the bin's pairs in this call, at least kTabCountClasses[c]), an index
-// into kTabShapes.
+// The planner's table (seqan_amd/tuning/shapes.json, turned into C++ by the
+// build): per category (DNA byte profile or substitution table, global or
+// local), length bin b (2^(b-1) < |V| + 1 <= 2^b) and count class (the call's
+// pairs on the packed route, at least kTabCountClasses[c]), an index into
+// kTabShapes: groups (0, 0) or one pair couple per lane (1, rows).
 #include "shape_table.inc"
 
 int lengthBin(int64_t m)
@@ -1258,9 +1258,14 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
                     wideLaneBin = q.bin;
             }
         }
-        // SQMI_BIN_SHAPES="b:G:R,...": the shape of bin b (the shape tuner
-        // times whole calls with it); forced shapes: every bin's.
+        // SQMI_BIN_SHAPES="b:G:R,...": the form of bin b in place of the
+        // table's (the tuner times calls with it): 1:R one pair per lane, 0:0
+        // groups by the rule, or a group shape, whose rows R then hold for
+        // every bin of that group size (units have one row count each); forced
+        // shapes: every bin's.
         auto force = [&](int b, int g, int r) {
+            if (g == 0 && r == 0)
+                binG[b] = binLane[b] = 0;
             if (!shapeSupported(Variant16{g, r, dna16, track}))
                 return;
             binG[b] = g == 1 ? 0 : g;

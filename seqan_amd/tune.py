@@ -1,23 +1,28 @@
-"""Shape autotuner of the packed int16 forward (run on the GPU):
+"""Autotuner of the planner's lane table (run on the GPU):
 
     python -m seqan_amd.tune [--out seqan_amd/tuning/shapes.json] [--cells 3e10]
 
-For every category of the planner's shape table (DNA byte profile or
-substitution table, global or local), every length bin b (2^(b-1) < |V| + 1
-<= 2^b) and every count class (how many pairs of a call take the packed
-route, over all bins: the launches of a call's shapes run side by side, so
-the whole call is what fills the GPU), it times one call of the library on
-synthetic pairs of that bin with each
-compiled shape forced (G = 16 with R = 16 / 8: a 16-lane group per pair
-couple; G = 1 with R = 16 / 32: one pair couple per lane; G = 64 with
-R = 4 / 8: a wavefront per pair couple), checks that all
-shapes give the same scores, and keeps the fastest.  A class is timed on
-its representative pair count, cut to --cells cells per call but never
-below FILL pairs (enough to fill the GPU with every group shape), so that
-the large classes of long bins measure the shapes' full-GPU rates; a class
-that would repeat a smaller class's count takes that class's choice.  The table it
-writes replaces seqan_amd/tuning/shapes.json; rebuild the library
-(python -m seqan_amd.build) to compile it into the planner.
+The planner spreads a pair couple over 16 or 64 lanes by a rule of its own
+(engine.cpp: evenOn16, kCouple64Share, kStripShare); what it takes from the
+table is whether a length bin's pairs go to the one-pair-per-lane kernel
+instead, and with how many rows per lane.  For every category (DNA byte
+profile or substitution table, global or local), every length bin b (2^(b-1)
+< |V| + 1 <= 2^b) and every count class (how many pairs of a call take the
+packed route, over all bins: the call's launches share the GPU) it times one
+call of the library on synthetic pairs of that bin with groups by the rule
+and with 16 and 32 rows per lane, checks that all give the same scores, and
+keeps the fastest (lanes only where they are 2% faster).  A class is timed on
+its representative pair count, cut to --cells cells per call; a class that
+would repeat a smaller class's count takes that class's choice.  Then the
+representative workloads are timed as whole calls while one bin at a time
+takes each other form.  Last, each category and class keeps the committed
+table's choices unless the new ones are 2% faster over calls of one bin and of
+mixed short lengths together and slow none of them by more than 3%: a call
+whose bins are split between lanes and groups pays for both launches, which
+single bins do not show.  (Global pairs whose values need all 16 bits have a
+rule of their own, kWideLane.)  The table it writes replaces
+seqan_amd/tuning/shapes.json; rebuild the library (python -m seqan_amd.build)
+to compile it into the planner.
 
 The knob this mirrors is the reference's block size / number of parallel
 alignments of its wavefront execution policy
@@ -36,26 +41,34 @@ import time
 import numpy as np
 
 from . import (LOCAL, FREE_TOP, FREE_BOTTOM, WL_DNA1K, WL_DNA_LOGNORMAL, WL_PROTEIN, Context, DeviceBuffer,
-               SeqSet, blosum62, force_shape, simple_score, synchronize, workload)
+               SeqSet, blosum62, simple_score, workload)
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 TABLE = os.path.join(HERE, "tuning", "shapes.json")
-SHAPES = [(16, 16), (16, 8), (1, 16), (1, 32), (64, 4), (64, 8)]
+FORMS = [(0, 0), (1, 16), (1, 32)]    # groups by the planner's rule; rows of one pair couple per lane
 COUNT_CLASSES = [0, 16384, 131072, 524288]
 CLASS_REP = [4096, 32768, 262144, 1048576]   # pairs timed for each class
-FILL = 24576   # pairs that fill the GPU with G = 16 (256 CU x 12 waves x 8 pairs)
 CATEGORIES = ["dna", "dna_local", "table", "table_local"]
-# Measured bins per category: up to the largest bin whose pairs all stay in
-# the packed kernels' int16 window (2 x 16k DNA pairs, or 11 x 4k Blosum62
-# pairs, would not); smaller bins copy bin 4, larger ones the last measured.
-BINS = {"dna": list(range(4, 14)), "dna_local": list(range(4, 14)), "table": list(range(4, 12)),
-        "table_local": list(range(4, 12))}
+# Measured bins: smaller ones copy the first, larger ones take groups (a
+# lane's sweep of 1,024 rows outlasts a call's of the same pairs on groups).
+BINS = list(range(4, 11))
+
+
+ABOUT = ("One pair couple per lane or groups, per length bin, for the packed int16 score kernels. bins[b] covers pairs "
+         "with 2^(b-1) < |V|+1 <= 2^b rows; each bin lists, per count class, the form used when the call holds at least "
+         "that many pairs on the packed route (over all bins): (0, 0) groups of 16 or 64 lanes by the planner's rule "
+         "(kScore16), (1, R) one pair couple per lane with R rows (kLane16). Written by seqan_amd/tune.py from "
+         "measurements on the GPU.")
 
 
 def pairs_for(rng, count, bin_, alpha):
-    """count pairs with |V| + 1 uniform in bin_ and |H| within 10% of |V|;
-    V is H with 10% substitutions (both residues uniform)."""
-    lo, hi = (1 << (bin_ - 1)), (1 << bin_) - 1          # |V| in [lo, hi]
+    """count pairs with |V| + 1 uniform in bin_."""
+    return pairs_between(rng, count, 1 << (bin_ - 1), (1 << bin_) - 1, alpha)
+
+
+def pairs_between(rng, count, lo, hi, alpha):
+    """count pairs with |V| uniform in lo..hi and |H| within 10% of it; V is H
+    with 10% substitutions (both residues uniform)."""
     m = rng.integers(lo, hi + 1, count)
     n = np.maximum(1, (m * rng.uniform(0.9, 1.1, count)).astype(np.int64))
     H = rng.integers(0, alpha, int(n.sum()), dtype=np.uint8)
@@ -73,43 +86,27 @@ def pairs_for(rng, count, bin_, alpha):
     return SeqSet(H, hoff), SeqSet(V, voff)
 
 
-def time_call(ctx, H, V, score, mode, flags, dh, dv, ds, reps):
-    ctx.align_score(H, V, score, mode, flags=flags, h_dev=dh.address, v_dev=dv.address, scores_dev=ds.address)
-    best = float("inf")
-    for _ in range(reps):
-        synchronize()
-        t = time.perf_counter()
-        ctx.align_score(H, V, score, mode, flags=flags, h_dev=dh.address, v_dev=dv.address, scores_dev=ds.address)
-        best = min(best, time.perf_counter() - t)
-    return best * 1e3
+def form_name(form):
+    return "groups" if form[0] == 0 else f"lanes{form[1]}"
 
 
-def smooth(choice, byClass, bins, log, margin=0.9):
-    """A call's bins run as one launch per distinct shape, so a mixture of
-    shapes costs more than the bins' separate timings add up to (each launch
-    has its own tail, and launches of different register budgets share the
-    CUs badly).  Per count class, the single shape with the smallest summed
-    slowdown over the long bins (b >= 8) is preferred in every long bin where
-    the bin's own best beats it by less than 10% (margin)."""
-    long_bins = [b for b in bins if b >= 8]
-    for k in range(len(COUNT_CLASSES)):
-        timed = [(b, byClass[(b, k)]) for b in long_bins if (b, k) in byClass]
-        if not timed:
-            continue
-        names = set.intersection(*(set(t) for _, t in timed))
-        if not names:
-            continue
-        dom = min(names, key=lambda nm: sum(t[nm] / min(t.values()) for _, t in timed))
-        di = next(i for i, sh in enumerate(SHAPES) if f"{sh[0]}x{sh[1]}" == dom)
-        for b, t in timed:
-            if min(t.values()) >= margin * t[dom] and choice[b][k] != di:
-                log(f"  class {k} bin {b}: {SHAPES[choice[b][k]]} -> {SHAPES[di]} (one shape for the long bins)")
-                choice[b][k] = di
+def device_ms(ctx, H, V, score, mode, forms, dev, reps):
+    """Device time of a call whose bin b takes forms[b] (best of reps)."""
+    dh, dv, ds = dev
+    os.environ["SQMI_BIN_SHAPES"] = ",".join(f"{b}:{g}:{r}" for b, (g, r) in sorted(forms.items()))
+    try:
+        best = float("inf")
+        for _ in range(reps + 1):
+            ctx.align_score(H, V, score, mode, h_dev=dh.address, v_dev=dv.address, scores_dev=ds.address)
+            best = min(best, ctx.stats()["device_ms"])
+        return best
+    finally:
+        os.environ.pop("SQMI_BIN_SHAPES", None)
 
 
 # Whole-call refinement: per (category, count class), a representative
 # workload of that class (the benchmark workloads), timed as one call while
-# one bin at a time takes each other shape (SQMI_BIN_SHAPES).
+# one bin at a time takes each other form.
 REFINE = [("dna", "1,048,576 uneven DNA pairs, semi-global", WL_DNA_LOGNORMAL, 0x5EED0002, 1 << 20,
            FREE_TOP | FREE_BOTTOM),
           ("dna", "65,536 DNA pairs of 1 kbp, global", WL_DNA1K, 0x5EED0004, 1 << 16, 0),
@@ -125,81 +122,76 @@ def count_class(pairs):
     return k
 
 
-def refine(ctx, setups, choice, allClass, log, reps=2):
-    """Per representative workload: first every group shape for all the bins
-    holding >= 1% of its cells at once, then coordinate descent over those
-    bins, heaviest first, each trying the shapes its own timing put within
-    2x of its best; a change is kept when the whole call gets >= 2% faster."""
+def refine(ctx, setups, choice, log, reps=2):
+    """Coordinate descent over the bins that hold 0.1% of the pairs of each
+    representative workload, most pairs first; a change is kept when the whole
+    call gets >= 2% faster."""
     notes = {}
     for cat, what, wl, seed, count, mode in REFINE:
         score = setups[cat][0]
-        byClass = allClass[cat]
         H, V = workload(wl, seed, 0, count)
         k = count_class(count)
-        m = np.diff(V.offsets)
-        cells = m * np.diff(H.offsets)
-        bins = np.ceil(np.log2(m + 1)).astype(int)
-        share = {int(b): float(cells[bins == b].sum() / cells.sum()) for b in np.unique(bins)}
-        pshare = {int(b): float((bins == b).mean()) for b in np.unique(bins)}
-        order = sorted((b for b, f in share.items() if f >= 0.01), key=lambda b: -share[b])
-        # Light bins (few cells, but their pairs may be wide: a shape with a
-        # long per-pair latency there can set the whole call's time).
-        light = sorted((b for b in share if share[b] < 0.01 and pshare[b] >= 0.001), key=lambda b: -share[b])
-        cur = {b: SHAPES[choice[cat][b][k]] for b in share}
-        dh, dv = DeviceBuffer.from_array(H.residues), DeviceBuffer.from_array(V.residues)
-        ds = DeviceBuffer(4 * count)
-
-        def timed(shapes):
-            os.environ["SQMI_BIN_SHAPES"] = ",".join(f"{b}:{g}:{r}" for b, (g, r) in sorted(shapes.items()))
-            try:
-                ctx.align_score(H, V, score, mode, h_dev=dh.address, v_dev=dv.address, scores_dev=ds.address)
-                best = float("inf")
-                for _ in range(reps):
-                    ctx.align_score(H, V, score, mode, h_dev=dh.address, v_dev=dv.address, scores_dev=ds.address)
-                    best = min(best, ctx.stats()["device_ms"])
-                return best
-            finally:
-                os.environ.pop("SQMI_BIN_SHAPES", None)
-
-        t0 = timed(cur)
-        best_t = t0
-        # One shape for all the heavy bins first (mixtures of shapes pay for
-        # sharing the GPU between launches, so single-bin moves alone can
-        # stall short of a uniform choice), then one bin at a time.
-        for sh in SHAPES:
-            if sh[0] == 1 or all(cur[b] == sh for b in order):
-                continue
-            t = timed({**cur, **{b: sh for b in order}})
-            if t < 0.98 * best_t:
-                log(f"  refine {cat} class {k} ({what}): heavy bins -> {sh}: {best_t:.2f} -> {t:.2f} ms")
-                cur.update({b: sh for b in order})
-                best_t = t
-        if light and order:
-            # The light bins on the heavy bins' leading shape.
-            sh = cur[order[0]]
-            if any(cur[b] != sh for b in light):
-                t = timed({**cur, **{b: sh for b in light}})
-                if t < 0.98 * best_t:
-                    log(f"  refine {cat} class {k} ({what}): light bins -> {sh}: {best_t:.2f} -> {t:.2f} ms")
-                    cur.update({b: sh for b in light})
-                    best_t = t
-        for b in order + light:
-            own = byClass.get((min(max(b, 4), 15), k)) or {}
-            fast = min(own.values()) if own else None
-            for sh in SHAPES:
-                if sh == cur[b] or (own and (f"{sh[0]}x{sh[1]}" not in own or own[f"{sh[0]}x{sh[1]}"] > 2 * fast)):
+        bins = np.ceil(np.log2(np.diff(V.offsets) + 1)).astype(int)
+        share = {int(b): float((bins == b).mean()) for b in np.unique(bins)}
+        cur = {b: FORMS[choice[cat][b][k]] for b in share}
+        dev = [DeviceBuffer.from_array(H.residues), DeviceBuffer.from_array(V.residues), DeviceBuffer(4 * count)]
+        t0 = best = device_ms(ctx, H, V, score, mode, cur, dev, reps)
+        for b in sorted((b for b in share if share[b] >= 0.001 and b <= BINS[-1]), key=lambda b: -share[b]):
+            for form in FORMS:
+                if form == cur[b]:
                     continue
-                t = timed({**cur, b: sh})
-                if t < 0.98 * best_t:
-                    log(f"  refine {cat} class {k} ({what}): bin {b} {cur[b]} -> {sh}: {best_t:.2f} -> {t:.2f} ms")
-                    cur[b], best_t = sh, t
-        for b, sh in cur.items():
-            if 0 <= b < 16:
-                choice[cat][b][k] = SHAPES.index(sh)
-        for x in (dh, dv, ds):
+                t = device_ms(ctx, H, V, score, mode, {**cur, b: form}, dev, reps)
+                if t < 0.98 * best:
+                    log(f"  refine {cat} class {k} ({what}): bin {b} {form_name(cur[b])} -> {form_name(form)}: "
+                        f"{best:.2f} -> {t:.2f} ms")
+                    cur[b], best = form, t
+        for b, form in cur.items():
+            choice[cat][b][k] = FORMS.index(form)
+        for x in dev:
             x.free()
-        notes[f"{cat}_class{k}"] = {"workload": what, "device_ms_table": round(t0, 3), "device_ms_refined": round(best_t, 3)}
-        log(f"refine {cat} class {k} ({what}): {t0:.2f} -> {best_t:.2f} ms")
+        notes[f"{cat}_class{k}"] = {"workload": what, "device_ms_table": round(t0, 3), "device_ms_refined": round(best, 3)}
+        log(f"refine {cat} class {k} ({what}): {t0:.2f} -> {best:.2f} ms")
+    return notes
+
+
+MIXTURES = [(8, 14), (17, 30), (34, 62), (66, 126), (20, 60), (50, 100), (20, 120), (100, 200), (8, 300)]
+
+
+def committed():
+    """The committed table's choices, as indices into FORMS."""
+    with open(TABLE) as f:
+        t = json.load(f)
+    form = [FORMS.index((1, r)) if g == 1 else 0 for g, r in t["shapes"]]
+    return {c: [[form[i] for i in b] for b in t["categories"][c]] for c in CATEGORIES}
+
+
+def settle(ctx, setups, choice, cells_budget, log, reps=3):
+    """Back to the committed choices per category and class (see the top)."""
+    rng = np.random.default_rng(77)
+    old, notes = committed(), {}
+    for cat in CATEGORIES:
+        score, mode, alpha = setups[cat]
+        for k, rep in enumerate(CLASS_REP):
+            if all(choice[cat][b][k] == old[cat][b][k] for b in range(16)):
+                continue
+            times = []
+            for lo, hi in MIXTURES:
+                H, V = pairs_between(rng, min(rep, int(cells_budget / hi ** 2)), lo, hi, alpha)
+                dev = [DeviceBuffer.from_array(H.residues), DeviceBuffer.from_array(V.residues),
+                       DeviceBuffer(4 * len(H))]
+                times.append([device_ms(ctx, H, V, score, mode, {b: FORMS[t[cat][b][k]] for b in range(16)}, dev, reps)
+                              for t in (old, choice)])
+                for x in dev:
+                    x.free()
+            was, now = np.array(times).T
+            keep = now.sum() < 0.98 * was.sum() and (now / was).max() <= 1.03
+            log(f"settle {cat} class {k}: committed {np.round(was, 3)} new {np.round(now, 3)} -> "
+                f"{'new' if keep else 'committed'}")
+            notes[f"{cat}_class{k}"] = {"committed_ms": [round(float(x), 3) for x in was],
+                                        "new_ms": [round(float(x), 3) for x in now], "taken": "new" if keep else "committed"}
+            if not keep:
+                for b in range(16):
+                    choice[cat][b][k] = old[cat][b][k]
     return notes
 
 
@@ -212,64 +204,39 @@ def tune(cells_budget=2e11, reps=2, log=print):
               "table_local": (blosum62(-1, -11), LOCAL, 24)}
     choice = {c: [[0] * len(COUNT_CLASSES) for _ in range(16)] for c in CATEGORIES}
     meas = {c: {} for c in CATEGORIES}
-    allClass = {}
     for cat in CATEGORIES:
         score, mode, alpha = setups[cat]
-        byClass = {}
-        for b in BINS[cat]:
+        for b in BINS:
             mean_cells = ((1 << (b - 1)) + (1 << b)) ** 2 / 4
-            measured = []
-            last = 0
-            contenders = list(SHAPES)
+            last, measured = 0, -1
             for k, rep in enumerate(CLASS_REP):
-                count = rep
-                if count * mean_cells > cells_budget:
-                    floor = 256 if k == 0 else min(rep, FILL)
-                    count = max(floor, int(cells_budget / mean_cells))
+                count = min(rep, int(cells_budget / mean_cells))
                 if count <= last:
                     break
                 last = count
                 H, V = pairs_for(rng, count, b, alpha)
-                dh, dv = DeviceBuffer.from_array(H.residues), DeviceBuffer.from_array(V.residues)
-                ds = DeviceBuffer(4 * count)
-                times, ref = {}, None
-                for G, R in SHAPES:
-                    if (G, R) not in contenders:
-                        continue
-                    ms = time_call(ctx, H, V, score, mode, force_shape(G, R), dh, dv, ds, reps)
-                    got = ds.to_array(np.int32, count)
-                    if ref is None:
-                        ref = got
-                    elif not np.array_equal(got, ref):
-                        raise AssertionError(f"{cat} bin {b} count {count}: shape {G}x{R} disagrees")
-                    times[f"{G}x{R}"] = round(ms, 3)
-                for x in (dh, dv, ds):
+                dev = [DeviceBuffer.from_array(H.residues), DeviceBuffer.from_array(V.residues), DeviceBuffer(4 * count)]
+                times, ref = [], None
+                for form in FORMS:
+                    times.append(round(device_ms(ctx, H, V, score, mode, {x: form for x in range(16)}, dev, reps), 3))
+                    got = dev[2].to_array(np.int32, count)
+                    if ref is not None and not np.array_equal(got, ref):
+                        raise AssertionError(f"{cat} bin {b} count {count}: {form_name(form)} disagrees")
+                    ref = got
+                for x in dev:
                     x.free()
-                best = min((i for i in range(len(SHAPES)) if SHAPES[i] in contenders),
-                           key=lambda i: times[f"{SHAPES[i][0]}x{SHAPES[i][1]}"])
-                # At a count that fills the GPU, shapes 2.5x slower than the
-                # best drop out of this bin's larger classes (they only fall
-                # further behind; below FILL the group shapes may just lack
-                # pairs to fill the GPU).
-                fastest = times[f"{SHAPES[best][0]}x{SHAPES[best][1]}"]
-                if count >= FILL:
-                    contenders = [sh for sh in contenders if times[f"{sh[0]}x{sh[1]}"] <= 2.5 * fastest]
-                choice[cat][b][k] = best
-                measured.append(k)
-                meas[cat][f"bin{b}_count{count}"] = times
-                byClass[(b, k)] = times
-                log(f"{cat} bin {b} count {count}: {times} -> {SHAPES[best]}")
-            for k in range(len(COUNT_CLASSES)):
-                if k not in measured:
-                    choice[cat][b][k] = choice[cat][b][max(measured)]
-                    byClass[(b, k)] = byClass[(b, max(measured))]
-        smooth(choice[cat], byClass, BINS[cat], log)
-        for b in range(0, BINS[cat][0]):
-            choice[cat][b] = list(choice[cat][BINS[cat][0]])
-        for b in range(BINS[cat][-1] + 1, 16):
-            choice[cat][b] = list(choice[cat][BINS[cat][-1]])
-        allClass[cat] = byClass
-    meas["refine"] = refine(ctx, setups, choice, allClass, log)
+                best = int(np.argmin(times))
+                choice[cat][b][k] = best if times[best] < 0.98 * times[0] else 0
+                measured = k
+                meas[cat][f"bin{b}_count{count}"] = {form_name(f): t for f, t in zip(FORMS, times)}
+                log(f"{cat} bin {b} count {count}: {meas[cat][f'bin{b}_count{count}']} -> "
+                    f"{form_name(FORMS[choice[cat][b][k]])}")
+            for k in range(measured + 1, len(COUNT_CLASSES)):
+                choice[cat][b][k] = choice[cat][b][measured]
+        for b in range(0, BINS[0]):
+            choice[cat][b] = list(choice[cat][BINS[0]])
+    meas["refine"] = refine(ctx, setups, choice, log)
+    meas["settle"] = settle(ctx, setups, choice, cells_budget, log)
     return choice, meas
 
 
@@ -307,18 +274,15 @@ def main():
     args = ap.parse_args()
     t0 = time.time()
     choice, meas = tune(args.cells, args.reps, log=lambda *a: print(*a, flush=True))
-    with open(TABLE) as f:
-        about = json.load(f)["about"]
     table = {
-        "about": about,
+        "about": ABOUT,
         "provenance": {"kind": "measured", "measured": True, "tool": "python -m seqan_amd.tune",
                        "gpu": gpu_name(), "host": platform.node(),
                        "date": datetime.datetime.utcnow().strftime("%Y-%m-%d %H:%M UTC"),
                        "cells_per_call": args.cells, "reps": args.reps, "seconds": round(time.time() - t0, 1)},
-        "shapes": [list(s) for s in SHAPES],
+        "shapes": [list(f) for f in FORMS],
         "count_classes": COUNT_CLASSES,
         "categories": choice,
-        "coop_min_blocks": 10,
         "measurements_ms": meas,
     }
     with open(args.out, "w") as f:
