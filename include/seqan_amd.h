@@ -96,10 +96,11 @@ enum {
 };
 /* Tuning knob: force the packed kernel shape instead of the planner's choice
  * (0 means automatic): lanes per pair group G and rows per lane R, G = 16
- * with R in {8, 16} (a group of 16 lanes sweeps a pair couple as a skewed
- * wavefront) or G = 1 with R in {16, 32} (one pair couple per lane).  The
- * automatic choice follows the shape table built from
- * seqan_amd/tuning/shapes.json, per length bin and number of pairs. */
+ * with R in {8, 16} or G = 64 with R in {4, 8, 16} (a group of lanes sweeps a
+ * pair couple as a skewed wavefront) or G = 1 with R in {16, 32} (one pair
+ * couple per lane).  The automatic choice takes G = 1 by the table built from
+ * seqan_amd/tuning/shapes.json, per length bin and number of pairs, and 16 or
+ * 64 lanes by a pair's share of the call. */
 #define SQMI_FORCE_SHAPE(G, R) ((((uint32_t)(G) & 0xFFu) << 8) | (((uint32_t)(R) & 0xFFu) << 16))
 
 /* A set of sequences: concatenated residue ordinals (Dna: A0 C1 G2 T3;

@@ -33,8 +33,9 @@
 // sums included) stays there.  Row buffer entries a block reads outside the
 // columns the block above wrote only feed cells outside the band.
 //
-// What bounds it: vector issue with two waves per SIMD (8 waves per CU, whose
-// rings fill the LDS) in full calls, an item's blocks in small ones.  1,048,576
+// What bounds it: two waves per SIMD (8 waves per CU, whose rings fill the LDS),
+// which use 73% of the vector issue slots on the first call below and 57% on
+// the second (two rounds of items); an item's blocks in small calls.  1,048,576
 // pairs of 150 bp, band [-16, 16], global: 1.62 ms in plain saturating values
 // (9 instructions per packed cell, 6.4 now), 1.37 in drifted ones with a wave per
 // item, 1.12 with two waves sharing one; 65,536 pairs of 1 kbp, band [-100,

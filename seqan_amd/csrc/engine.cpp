@@ -784,9 +784,6 @@ struct PlanUse {
     ~PlanUse() { p.trim(); }
 };
 
-// int32 pairs whose sides are both at least this long (and that are DNA,
-// global) run the tiled long-pair kernels instead of one thread per pair
-// (2048, or SQMI_LONG_MIN_SIDE).
 // The packed long-pair kernels (long16.hip) hold values relative to a base;
 // target: where a strip's top row is kept; a strip of 64 R rows needs every
 // value below kDriftNarrowMax, the cells of a wave growing by at most sMax + 2
@@ -818,6 +815,9 @@ bool envFlag(const char *name)
     return env && *env == '1';
 }
 
+// Pairs outside the int16 window whose sides are both at least this long (and
+// that are DNA) run the long-pair kernels instead of one thread per pair (2048,
+// or SQMI_LONG_MIN_SIDE).
 int64_t longMinSide()
 {
     const char *env = std::getenv("SQMI_LONG_MIN_SIDE");
@@ -939,9 +939,6 @@ int stripMinBlocks()
     return env && *env ? std::max(0, std::atoi(env)) : -1;
 }
 
-// Units of the packed score kernel from the sorted keys of the group shapes,
-// which come first, in slot order (the longest items first).  starts /
-// itemOff: the buckets' first keys and items.
 // Strips in the order a wave should claim them: by the steps from a strip's
 // start to its item's end (its columns, and kStripLag for every block from it
 // on), the most first.  The strip above always comes earlier.  Claimed item
@@ -972,6 +969,10 @@ void orderStrips(RawVec<ScoreUnit> &units, size_t begin)
         units[begin + at[bucket(u)]++] = u;
 }
 
+// Units of the packed score kernel from the sorted keys of the group shapes,
+// which come first, in slot order (the longest items first).  starts /
+// itemOff: the buckets' first keys and items; stripBytes: what their strips may
+// take (0: none).
 void makeUnits(const sqmi_sequences &V, Planned &P, const std::vector<size_t> &starts,
                const std::vector<size_t> &itemOff, int R16, int R64, double cellsStrip, int64_t stripBytes)
 {
@@ -1172,10 +1173,10 @@ void plan(const sqmi_sequences &H, const sqmi_sequences &V, const sqmi_scoring &
     P.track = track;
     P.mode = mode;
     // Route every pair and give it a bucket key (see bucketOf).  The int16
-    // pairs' shape slots: the trace shape, a forced shape, or per length bin
-    // the shape table's choice for the number of the call's pairs in that
-    // bin (a pair that needs more than 255 row blocks of its bin's shape
-    // takes G = 16, R = 16).
+    // pairs' shape slots: the trace shape, a forced shape, or lanes where the
+    // table (wide global values: kWideLane) gives a pair's length bin to them,
+    // else 16 or 64 lanes by its share of the call's cells (a pair that needs
+    // more than 255 row blocks on lanes takes groups).
     RawVec<Key> &keys = P.keys16;
     keys.resize((size_t)N);
     int64_t cells = 0;
@@ -1674,11 +1675,6 @@ sqmi_status uploadInputs(sqmi_context *ctx, const sqmi_sequences *setH, const sq
     return SQMI_OK;
 }
 
-// Long pairs: the tiled int32 forward (one launch per tile anti-diagonal),
-// then, with `dCounts`, the checkpointed traceback: per round every
-// unfinished pair's current tile is recomputed with trace records and
-// walked.  Pairs run in chunks whose checkpoints fit traceBudget().  `pairs`
-// holds the host copy of the descriptors until the caller synchronises.
 // Device addresses of the alignment rows output (all null: no rows).
 struct RowsDev {
     uint8_t *ops = nullptr;
@@ -1888,6 +1884,12 @@ sqmi_status runLong16(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_
     return SQMI_OK;
 }
 
+// Long pairs: the packed kernels (runLong16) where the scoring allows and the
+// alignment is global, else the tiled int32 forward (one launch per tile
+// anti-diagonal), then, with `dCounts`, the checkpointed traceback: per round
+// every unfinished pair's current window is recomputed with trace records and
+// walked.  Pairs run in chunks whose checkpoints fit traceBudget().  `stage`
+// holds the host copies of the descriptors until the caller synchronises.
 sqmi_status runLong(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_sequences *setV, const Planned &P,
                     const Inputs &in, uint32_t flags, int32_t *dCounts, const RowsDev &rows,
                     LongStage &stage, Deferred *deferred = nullptr)
@@ -2699,10 +2701,12 @@ sqmi_status sqmi_plan_stats(const sqmi_sequences *setH, const sqmi_sequences *se
 
 // Traceback: the packed forward pass writes 4 trace bits per cell into a
 // buffer of at most traceBudget() bytes, so the work items run in chunks;
-// after each chunk one thread per pair walks its path.  Pairs outside the
-// int16 window, every pair under SQMI_FORCE_INT32 and every banded pair
-// (band given) run the int32 kernel with one trace byte per cell, chunked by
-// the same budget.
+// after each chunk 16 or 64 lanes per pair walk its path.  Banded pairs (band
+// given) whose band has at most kMaxBandTrace diagonals inside the matrix run
+// the banded trace kernels (one byte per cell of the band); wider bands, pairs
+// outside the int16 window and every pair under SQMI_FORCE_INT32 run the int32
+// kernel with one trace byte per cell of the matrix.  All are chunked by the
+// same budget.
 static sqmi_status alignBackward(sqmi_context *ctx, const sqmi_sequences *setH, const sqmi_sequences *setV,
                                  const sqmi_scoring *scoring, uint32_t mode, int32_t *scores, int32_t *counts,
                                  uint8_t *ops, const int64_t *opOffsets, int64_t *opLengths, int64_t *begins,

@@ -116,7 +116,7 @@ struct TraceEnd {
     int32_t rv, ri, rj, re, rf;
 };
 
-// Traceback walk: 16 lanes per pair.
+// Traceback walk: 16 lanes per pair, or a whole wave in calls of few pairs.
 struct WalkArgs {
     const uint8_t *hRes;
     const uint8_t *vRes;

@@ -381,9 +381,10 @@ struct Lane16 {
     }
 };
 
-// Register budgets without spills in the column loops: four waves per SIMD
-// (128 VGPRs) for 16 rows per lane, three for local alignment (its running
-// maximum and padding masks), two for 32 rows.
+// Register budgets: four waves per SIMD (128 VGPRs) for 16 rows per lane, three
+// for local alignment (its running maximum and padding masks), two for 32 rows.
+// What the compiler spills there (up to 108 registers) belongs to the blocks'
+// set-up, but for a free first row's block, whose column loop reads some back.
 template <int R, uint32_t TRK>
 constexpr int laneWaves() { return R >= 32 ? 2 : (TRK & kTrackLocal) ? 3 : 4; }
 

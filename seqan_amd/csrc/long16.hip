@@ -37,13 +37,14 @@
 // of the next 64 cells of the diagonal (or the gap), so a run of equal moves
 // costs one memory wait.
 //
-// What bounds it: vector issue (6.4 instructions per packed cell, 4.9 cycles
-// each) once the strips fill the SIMDs, the sweep of one strip and the start
-// of the ones below before.  64 pairs of 100 kbp (6.4e11 cells): forward 270 ->
-// 67 ms against one launch per tile anti-diagonal with plain values, 8
-// rows per lane (16: 77, of which a fourth round of 64 strips on 1,024 SIMDs
-// takes 16; 4: 76); records 8 ms and walks 6 ms of 46 rounds, 43 before
-// (one thread per pair walked); scores and counts 315 -> 80 ms.
+// What bounds it: vector issue (6.6 instructions per packed cell, 80% of the
+// slots on 64 pairs, whose last round of strips leaves SIMDs idle) once the
+// strips fill the SIMDs, the sweep of one strip and the start of the ones below
+// before.  64 pairs of 100 kbp (6.4e11 cells): forward 270 -> 67 ms against one
+// launch per tile anti-diagonal with plain values, 8 rows per lane (16: 77, of
+// which a fourth round of 64 strips on 1,024 SIMDs takes 16; 4: 76); records 6
+// ms and walks 6 ms of 82 rounds, 43 before (one thread per pair walked);
+// scores and counts 315 -> 80 ms.
 #include <algorithm>
 
 #include "score16.hpp"

@@ -27,13 +27,16 @@
 // steps + s) * 64 + lane]: one coalesced 1 KB store per wave and step.  With
 // 64 lanes a record is one word, x | z << 4 (four rows), and a step 256 bytes.
 //
-// What bounds it: vector issue (13 operations per row and the lookup, 90% of
-// the slots) while there are items for every wave; with few items, the sweep
-// of the longest, which strips spread over the chip and 64 lanes per couple
-// shorten.  Measured: 65,536 pairs of 1 kbp, global, 17.4 -> 16.2 ms (34 GB of
-// records at 2.1 TB/s beside it); 8,191 uneven pairs, free first and last row,
-// 277 ms with one wave per item -> 8.6 (strips) -> 3.2 (64 lanes); 8,192
-// protein pairs, local, 11.3 -> 2.9 ms.
+// What bounds it: vector issue while there are items for every wave (65,536
+// pairs of 1 kbp: 93% of the slots, 15.3 instructions per packed row with the
+// lookup and the sweep's own; local 96%, 23); with few items, the sweep of the
+// longest, which strips spread over the chip and 64 lanes per couple shorten
+// (8,191 uneven pairs: 49%).  Measured: 65,536 pairs of 1 kbp, global, 17.4 ->
+// 15.0 ms (34 GB of records at 2.4 TB/s beside it); 8,191 uneven pairs, free
+// first and last row, 277 ms with one wave per item -> 8.6 (strips) -> 3.1 (64
+// lanes); 8,192 protein pairs, local, 11.3 -> 2.9 ms.  The DNA kernels spill 38 to
+// 247 registers of their four bodies' set-up at three waves per SIMD; the
+// column loops read none back.
 //
 // Values are compared as signed halves.  WIDE: stored values are held less
 // 32768, so that the whole 16-bit range is ordered and the differences
