@@ -884,14 +884,25 @@ void radixSort(RawVec<Key> &keys, RawVec<Key> &tmp, std::vector<uint32_t> &hist)
 #pragma omp barrier
 #pragma omp single
             {
+                // One thread: the sums of one array.  (The nested loop took 7 to
+                // 20 us more for its 2 x 16,384 digits, by where the compiler
+                // put its branches: 4,096 pairs of 150 bp 169 us, so 154.)
                 uint32_t run = 0;
-                for (int d = 0; d < NB; ++d)
-                    for (int u = 0; u < T; ++u) {
-                        uint32_t &c = hist[(size_t)u * NB + d];
-                        const uint32_t v = c;
-                        c = run;
+                if (T == 1) {
+                    for (int d = 0; d < NB; ++d) {
+                        const uint32_t v = h[d];
+                        h[d] = run;
                         run += v;
                     }
+                } else {
+                    for (int d = 0; d < NB; ++d)
+                        for (int u = 0; u < T; ++u) {
+                            uint32_t &c = hist[(size_t)u * NB + d];
+                            const uint32_t v = c;
+                            c = run;
+                            run += v;
+                        }
+                }
             }
             for (size_t k = lo; k < hi; ++k)
                 tmp[h[(keys[k].key >> shift) & mask]++] = keys[k];
